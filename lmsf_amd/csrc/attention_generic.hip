@@ -25,7 +25,20 @@
 
 #define GEN_THREADS 256
 
-template <typename T>
+// four neighbouring elements in one load
+__device__ __forceinline__ void gen_load4(const float* p, float* x) {
+  const float4 v = *reinterpret_cast<const float4*>(p);
+  x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+}
+__device__ __forceinline__ void gen_load4(const bf16_t* p, float* x) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xffff0000u);
+  x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xffff0000u);
+}
+
+// VEC: the key pages start on a boundary of four elements (every row does then: d is a multiple of 4), and a key is read
+// four elements a load.
+template <typename T, bool VEC>
 __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
     const T* __restrict__ q, long q_stride, T* __restrict__ out, long out_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ block_tables, int bt_width, const int* __restrict__ seg,
@@ -34,8 +47,9 @@ __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
   extern __shared__ float smem[];
   float* sq = smem;                       // [d] query, pre-scaled
   float* sp = sq + d;                     // [256] scores, then probabilities
-  int* srow = (int*)(sp + GEN_THREADS);   // [256] (page * nkv + g) * ps + offset of each key
-  float* sacc = (float*)(srow + GEN_THREADS);  // [256] partial outputs of the key groups
+  int* shead = (int*)(sp + GEN_THREADS);  // [256] page * nkv + g of each key
+  int* soff = shead + GEN_THREADS;        // [256] its offset in the page
+  float* sacc = (float*)(soff + GEN_THREADS);  // [256] partial outputs of the key groups
   __shared__ float red[16];
 
   const int t = blockIdx.x, h = blockIdx.y;
@@ -61,14 +75,22 @@ __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
     const int j = j0 + tid;
     float sc = -INFINITY;
     if (j <= p) {
-      const int page = bt[j / ps];
-      const int row = (page * nkv + g) * ps + j % ps;
-      srow[tid] = row;
-      const T* kr = k_pages + (long)row * d;
+      const int block = j / ps, off = j - block * ps;
+      const int head_base = bt[block] * nkv + g;
+      shead[tid] = head_base;
+      soff[tid] = off;
+      const T* kr = k_pages + ((long)head_base * ps + off) * d;
       float dot = 0.f;
+#pragma unroll 8
       for (int i = 0; i < d; i += 4) {
-        dot += sq[i] * to_f32<T>(kr[i]) + sq[i + 1] * to_f32<T>(kr[i + 1]) + sq[i + 2] * to_f32<T>(kr[i + 2]) +
-               sq[i + 3] * to_f32<T>(kr[i + 3]);
+        float k4[4];
+        if (VEC) {
+          gen_load4(kr + i, k4);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) k4[e] = to_f32<T>(kr[i + e]);
+        }
+        dot += sq[i] * k4[0] + sq[i + 1] * k4[1] + sq[i + 2] * k4[2] + sq[i + 3] * k4[3];
       }
       sc = softcap > 0.f ? softcap * tanhf(dot / softcap) : dot;   // scores bounded by cap tanh(s / cap)
       if (bias) sc -= r1 * log1pf(r2 * (float)(p - j));            // what the distance takes off
@@ -77,7 +99,7 @@ __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
     const float m_new = fmaxf(m, cmax);
     const float e = (j <= p) ? expf(sc - m_new) : 0.f;
     sp[tid] = e;
-    const float csum = block_sum(e, red);  // has barriers: sp and srow are visible afterwards
+    const float csum = block_sum(e, red);  // has barriers: sp, shead and soff are visible afterwards
     const float corr = (m == -INFINITY) ? 0.f : expf(m - m_new);
     l = l * corr + csum;
     acc *= corr;
@@ -88,8 +110,22 @@ __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
     __syncthreads();
     if (pv_active) {
       const int n = min(GEN_THREADS, p - j0 + 1);
-      for (int jj = og; jj < n; jj += ngroups) {
-        const int row = srow[jj], head_base = row / ps, off = row - head_base * ps;
+      int jj = og;
+      // (up to 256 output dims: eight values of a group's keys are asked for at a time; one by one every value waits for
+      // the one before it, 300 keys of 32 dims in float32 14.0 -> 12.2 us)
+      if (d <= GEN_THREADS)
+        for (; jj + 7 * ngroups < n; jj += 8 * ngroups) {
+          float v[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const int key = jj + u * ngroups;
+            v[u] = to_f32<T>(v_pages[((long)shead[key] * d + oi) * ps + soff[key]]);
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u) acc += sp[jj + u * ngroups] * v[u];
+        }
+      for (; jj < n; jj += ngroups) {
+        const int head_base = shead[jj], off = soff[jj];
         acc += sp[jj] * to_f32<T>(v_pages[((long)head_base * d + oi) * ps + off]);
         if (d > GEN_THREADS) {
 #pragma unroll
@@ -137,16 +173,19 @@ extern "C" int lmsf_paged_attention_generic_biased(const void* q, long q_stride,
   LMSF_CHECK(q_stride >= (long)nh * d && out_stride >= (long)nh * d, "paged_attention: row strides too small");
   LMSF_CHECK(nh <= 65535, "paged_attention: too many heads");
   if (n_tokens == 0) return 0;
-  const size_t smem = (size_t)(d + 3 * GEN_THREADS) * 4;
+  const size_t smem = (size_t)(d + 4 * GEN_THREADS) * 4;
   dim3 grid(n_tokens, nh), block(GEN_THREADS);
-  if (dtype == LMSF_F32)
-    hipLaunchKernelGGL((paged_attention_generic_kernel<float>), grid, block, smem, stream, (const float*)q, q_stride,
-                       (float*)out, out_stride, (const float*)k_pages, (const float*)v_pages, block_tables, bt_width,
-                       seg, pos, nh, nkv, d, ps, scale, window, softcap, bias, sink);
-  else
-    hipLaunchKernelGGL((paged_attention_generic_kernel<bf16_t>), grid, block, smem, stream, (const bf16_t*)q, q_stride,
-                       (bf16_t*)out, out_stride, (const bf16_t*)k_pages, (const bf16_t*)v_pages, block_tables,
-                       bt_width, seg, pos, nh, nkv, d, ps, scale, window, softcap, bias, sink);
+#define GENERIC(T_, VEC_)                                                                                               \
+  hipLaunchKernelGGL((paged_attention_generic_kernel<T_, VEC_>), grid, block, smem, stream, (const T_*)q, q_stride,     \
+                     (T_*)out, out_stride, (const T_*)k_pages, (const T_*)v_pages, block_tables, bt_width, seg, pos,    \
+                     nh, nkv, d, ps, scale, window, softcap, bias, sink)
+  const bool vec = (size_t)k_pages % (4 * lmsf_elem_size(dtype)) == 0;
+  if (dtype == LMSF_F32) {
+    if (vec) GENERIC(float, true); else GENERIC(float, false);
+  } else {
+    if (vec) GENERIC(bf16_t, true); else GENERIC(bf16_t, false);
+  }
+#undef GENERIC
   LMSF_LAUNCH_CHECK("paged_attention_generic");
   return 0;
 }

@@ -1,0 +1,81 @@
+"""The float32 product split over the waves of a workgroup, and general attention's values read eight keys at a time."""
+import pytest
+import torch
+
+from torch_ops import TorchOps
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from lmsf_amd.ops import get_ops
+    return get_ops()
+
+
+# the edges of its row forms (8, 16, 32 rows a workgroup) and columns (16), K below, at and beyond a piece for every wave
+# and four pieces for every wave, K that is no multiple of 4, and both sides of the line to the 64x64 tiles
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 16, 4), (8, 17, 31), (9, 15, 32), (16, 33, 36), (17, 64, 127), (32, 16, 128),
+                                   (33, 70, 132), (65, 130, 260), (7, 128, 352), (1024, 512, 20), (1025, 512, 20),
+                                   (2, 16384, 12), (2, 16385, 12)])
+@pytest.mark.parametrize("types", [(torch.float32, torch.float32, torch.float32), (torch.float32, torch.bfloat16, torch.float32),
+                                   (torch.bfloat16, torch.float32, torch.float32), (torch.bfloat16, torch.float32, torch.bfloat16)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_product_of_few_outputs(ops, M, N, K, types, shift):
+    ta, tw, to = types
+    g = torch.Generator().manual_seed(M * 7 + N + K + shift)
+
+    def rows(n, dtype):        # rows that start ``shift`` elements off a 16-byte boundary
+        pad = (-K) % 8 + (8 if shift else 0)
+        buf = torch.full((n * (K + pad) + 8,), float("nan"), dtype=dtype, device="cuda:0")
+        t = buf[shift:shift + n * (K + pad)].view(n, K + pad)[:, :K]
+        t.copy_(torch.randn(n, K, generator=g).to(dtype))
+        return t
+    x, w = rows(M, ta), rows(N, tw)
+    b = torch.randn(N, generator=g).to(tw).to("cuda:0")
+    y = ops.linear(x, w, b, out_dtype=to).double()
+    exact = x.double() @ w.double().T + b.double()
+    # a wave adds K / 8 products and one more piece of up to 4 in turn, the waves' eight sums and the bias come on top;
+    # the tiles add all K in turn
+    split = N <= 16384 and M * N <= 1 << 19
+    chain = (K / 8 + 4 + 9) if split else K + 1
+    bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * chain * 2.0 ** -24
+    if to == torch.bfloat16:
+        bound = bound + exact.abs() * 2.0 ** -8
+    assert ((y - exact).abs() <= bound + 1e-30).all()
+
+
+# keys just below, at and beyond eight a group (256 / d groups), a second round of 256 keys, pages of odd sizes
+@pytest.mark.parametrize("d,ps", [(32, 16), (4, 3), (96, 16), (256, 8), (260, 16)])
+@pytest.mark.parametrize("context", [1, 7, 8, 63, 64, 65, 256, 257, 300])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_general_attention(ops, d, ps, context, dtype, shift):
+    nh, nkv, scale = 4, 2, d ** -0.5
+    g = torch.Generator().manual_seed(d + context)
+    blocks = -(-context // ps)
+    pages = blocks + 3
+
+    def cache():                # pages that start ``shift`` elements off a 16-byte boundary
+        buf = torch.empty(pages * nkv * ps * d + 8, dtype=dtype, device="cuda:0")
+        t = buf[shift:shift + pages * nkv * ps * d]
+        t.copy_(torch.randn(t.shape, generator=g).to(dtype))
+        return t
+    k, v = cache().view(pages, nkv, ps, d), cache().view(pages, nkv, d, ps)
+    q = torch.randn(2, nh * d, generator=g).to(dtype).to("cuda:0")
+    table = torch.randperm(pages, generator=g)[:blocks].to(torch.int32).view(1, -1).to("cuda:0")
+    seg = torch.zeros(2, dtype=torch.int32, device="cuda:0")
+    pos = torch.tensor([context - 1, max(0, context - 2)], dtype=torch.int32, device="cuda:0")
+    got = ops.paged_attention(q, k, v, table, seg, pos, nh, nkv, d, scale, kernel="generic").double().cpu()
+    keys = k[table[0].long()].permute(1, 0, 2, 3).reshape(nkv, -1, d)[:, :context].double().cpu()
+    vals = v[table[0].long()].permute(1, 0, 3, 2).reshape(nkv, -1, d)[:, :context].double().cpu()
+    for t in range(2):
+        n = int(pos[t]) + 1
+        for h in range(nh):
+            s = keys[h // 2, :n] @ q[t, h * d:(h + 1) * d].double().cpu() * scale
+            want = torch.softmax(s, 0) @ vals[h // 2, :n]
+            # scores of a few units to 2^-21, weights that add up to one over values of up to 5 units
+            tol = 2e-5 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+            assert ((got[t, h * d:(h + 1) * d] - want).abs() <= tol).all()
+
+
