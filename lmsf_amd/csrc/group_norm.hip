@@ -14,17 +14,15 @@
 //   out[row] = wn ? gn(x; wn) : x                           the norm *before* the next sublayer
 //
 // All arithmetic is float32; branch and out are float32 or bfloat16, the weights float32. One workgroup a row
-// (256 to 1,024 threads), the row kept in LDS between the passes; the stream's row and the earlier results are asked
-// for before the first pass, so that the passes do not each wait for memory.
+// (256 to 1,024 threads), the row kept in LDS between the passes (in registers where its groups allow it: further
+// down); the stream's row and the earlier results are asked for before the first pass, so that the passes do not each
+// wait for memory.
 #include "common.h"
 
 #include <math.h>
 
 #define GN_MAX_THREADS 1024
 #define GN_THREADS ((int)blockDim.x)
-
-template <typename T>
-__device__ __forceinline__ float gn_load(const void* p, long i) { return to_f32<T>(((const T*)p)[i]); }
 
 // divides the row in LDS by its groups' root mean squares and multiplies by w; ``red`` is block_sum's scratch
 __device__ __forceinline__ void gn_normalize(float* row, const float* __restrict__ w, int W, int groups, float eps,
@@ -95,11 +93,149 @@ __global__ __launch_bounds__(GN_MAX_THREADS) void group_norm_kernel(
   }
 }
 
+// four neighbours an access
+template <typename T> struct Na4;
+template <> struct Na4<float> {
+  static __device__ __forceinline__ void load(const float* p, float* x) {
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+  }
+  static __device__ __forceinline__ void store(float* p, const float* x) {
+    *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
+  }
+};
+template <> struct Na4<bf16_t> {
+  static __device__ __forceinline__ void load(const bf16_t* p, float* x) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xffff0000u);
+    x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xffff0000u);
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, const float* x) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack2_bf16(x[0], x[1]), pack2_bf16(x[2], x[3]));
+  }
+};
+
+// The same with the row in registers, for groups of whole 256 columns (or one group) and rows that start on 16-byte
+// boundaries: a thread holds E groups of four neighbours, 64 lanes stand for 256 columns, so a wave's sum belongs to one
+// group and a norm costs one sum over the lanes and one barrier. Everything that comes from memory is asked for in one
+// go. What bounds it with few rows is that trip and the launch (8 rows of 2,048 in 2 groups, branch, stream and output:
+// 8.9 -> 4.9 us), with many rows memory (2,000 such rows 31.0 -> 15.9 us).
+#define GN_SLOTS 64     // 256-column parts of a row: W <= 16,384
+
+// the sum of group g's parts, in their order
+__device__ __forceinline__ float gn_group_sum(const float* red, int g, int per_group) {
+  float s = 0.f;
+  for (int k = 0; k < per_group; ++k) s += red[g * per_group + k];
+  return s;
+}
+
+template <typename TB, typename TO, int E>
+__global__ __launch_bounds__(GN_MAX_THREADS) void group_norm_vec_kernel(
+    const TB* __restrict__ branch, long branch_stride, const float* __restrict__ wb, float* __restrict__ residual,
+    float* __restrict__ hist, long hist_stride, int hist_index, const float* __restrict__ mix,
+    const float* __restrict__ wn, TO* __restrict__ out, long out_stride, const int* __restrict__ rows, int W,
+    int per_group, float gw, float eps_b, float eps_n) {
+  __shared__ float red[2][GN_SLOTS];
+  const long n = blockIdx.x, src = rows ? rows[n] : n;
+  const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE, n_waves = blockDim.x / LMSF_WAVE;
+  float x[E][4], res[E][4], ave[E][4], vb[E][4], vn[E][4];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = (threadIdx.x + e * blockDim.x) * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[e][j] = res[e][j] = ave[e][j] = 0.f;
+    if (i < W) {
+      if (branch) {
+        Na4<TB>::load(branch + n * branch_stride + i, x[e]);
+        Na4<float>::load(wb + i, vb[e]);
+      }
+      if (residual) Na4<float>::load(residual + src * W + i, res[e]);
+      if (wn) Na4<float>::load(wn + i, vn[e]);
+    }
+  }
+  if (hist) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = (threadIdx.x + e * blockDim.x) * 4;
+      if (i >= W) continue;
+#pragma unroll 8
+      for (int k = 0; k < hist_index; ++k) {
+        float h[4];
+        Na4<float>::load(hist + (long)k * hist_stride + n * W + i, h);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ave[e][j] += mix[k] * h[j];
+      }
+    }
+  }
+  auto normalize = [&](const float (&w)[E][4], float eps, float* sums) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      float s = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s += x[e][j] * x[e][j];
+      s = wave_sum(s);
+      if (lane == 0) sums[e * n_waves + wave] = s;      // parts beyond W hold 0
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = (threadIdx.x + e * blockDim.x) * 4;
+      if (i >= W) continue;
+      const float rms = sqrtf(gn_group_sum(sums, i / 256 / per_group, per_group) / gw + eps);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[e][j] = x[e][j] / rms * w[e][j];
+    }
+  };
+  if (branch) normalize(vb, eps_b, red[0]);
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int i = (threadIdx.x + e * blockDim.x) * 4;
+    if (i >= W) continue;
+    if (residual) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[e][j] = res[e][j] + x[e][j];
+      if (branch && !rows && !hist) Na4<float>::store(residual + n * W + i, x[e]);
+    }
+    if (hist) {
+      Na4<float>::store(hist + (long)hist_index * hist_stride + n * W + i, x[e]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[e][j] = ave[e][j] + mix[hist_index] * x[e][j];
+      Na4<float>::store(residual + n * W + i, x[e]);
+    }
+  }
+  if (out) {
+    if (wn) normalize(vn, eps_n, red[1]);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int i = (threadIdx.x + e * blockDim.x) * 4;
+      if (i < W) Na4<TO>::store(out + n * out_stride + i, x[e]);
+    }
+  }
+}
+
 template <typename TB, typename TO>
 static void gn_launch(int n_rows, size_t smem, hipStream_t stream, const void* branch, long branch_stride,
                       const float* wb, float* residual, float* hist, long hist_stride, int hist_index,
                       const float* mix, const float* wn, void* out, long out_stride, const int* rows, int W,
                       int groups, float eps_b, float eps_n) {
+  const int gw = W / groups;
+  const bool vec = W % 4 == 0 && (groups == 1 || gw % 256 == 0) && W <= 256 * GN_SLOTS && branch_stride % 4 == 0 &&
+                   out_stride % 4 == 0 && hist_stride % 4 == 0 && lmsf_aligned16(branch) && lmsf_aligned16(wb) &&
+                   lmsf_aligned16(residual) && lmsf_aligned16(hist) && lmsf_aligned16(wn) && lmsf_aligned16(out);
+  if (vec) {
+    // few rows: as many threads as a row has groups of four; many rows: smaller workgroups with several each
+    const int quads = W / 4, per_thread = n_rows >= 512 ? 2 : 1;
+    int threads = 64;
+    while (threads < GN_MAX_THREADS && threads * per_thread < quads) threads *= 2;
+    const int need = (quads + threads - 1) / threads, per_group = (gw + 255) / 256;
+#define GN_VEC(E_)                                                                                                     \
+  hipLaunchKernelGGL((group_norm_vec_kernel<TB, TO, E_>), dim3(n_rows), dim3(threads), 0, stream, (const TB*)branch,   \
+                     branch_stride, wb, residual, hist, hist_stride, hist_index, mix, wn, (TO*)out, out_stride, rows,  \
+                     W, per_group, (float)gw, eps_b, eps_n)
+    if (need <= 1) GN_VEC(1); else if (need <= 2) GN_VEC(2); else GN_VEC(4);
+#undef GN_VEC
+    return;
+  }
   // few rows: a row's passes wait for memory one after the other, so many threads with few elements each; many
   // rows fill the chip with smaller workgroups
   const int threads = n_rows >= 1024 || W <= 256 ? 256 : W <= 1024 ? 512 : 1024;
@@ -148,27 +284,6 @@ extern "C" int lmsf_group_norm(const void* branch, int branch_dtype, long branch
 //
 // (two mixers side by side are joined on the way: nothing of v goes through memory). A workgroup a row, the row in
 // registers, four neighbours an access; everything that comes from memory is asked for before the first sum.
-
-template <typename T> struct Na4;
-template <> struct Na4<float> {
-  static __device__ __forceinline__ void load(const float* p, float* x) {
-    const float4 v = *reinterpret_cast<const float4*>(p);
-    x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
-  }
-  static __device__ __forceinline__ void store(float* p, const float* x) {
-    *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
-  }
-};
-template <> struct Na4<bf16_t> {
-  static __device__ __forceinline__ void load(const bf16_t* p, float* x) {
-    const uint2 v = *reinterpret_cast<const uint2*>(p);
-    x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xffff0000u);
-    x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xffff0000u);
-  }
-  static __device__ __forceinline__ void store(bf16_t* p, const float* x) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(pack2_bf16(x[0], x[1]), pack2_bf16(x[2], x[3]));
-  }
-};
 
 // E: groups of four entries a thread holds
 template <typename T, bool PAIR, int E>
