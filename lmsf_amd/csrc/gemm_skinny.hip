@@ -76,7 +76,9 @@ struct NormAroundArgs {
 // 4 add to the stream and prepare the norm that follows (y receives bf16(stream * w))
 // XROWS: rows of a tile of x that are fetched and staged, 16 or (one row tile of up to 8 rows) 8; the columns of the
 // result that belong to the others are never stored.
-template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH, bool SCALED, int XROWS>
+// WROWS: rows of a tile of W that are fetched, 16 or 8. With 8 the upper half of the tile in LDS holds whatever it held,
+// and the outputs that belong to it are never stored; every product is added up in the same order.
+template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH, bool SCALED, int XROWS, int WROWS>
 __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __restrict__ x, long ldx,
                                                               const bf16_t* __restrict__ W, long ldw,
                                                               const bf16_t* __restrict__ bias, TOut* __restrict__ y,
@@ -85,6 +87,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   using T = SkinnyTile<KC>;
   constexpr int WT = ((ACT >= 1 && ACT <= 3) || ACT >= 5) ? 2 : 1;   // W tiles per chunk: gate and up, the two halves of a head, or one
   constexpr int XLOADS = (XROWS + T::ROWS_PER_LOAD - 1) / T::ROWS_PER_LOAD;   // load instructions per tile of x
+  constexpr int WLOADS = (WROWS + T::ROWS_PER_LOAD - 1) / T::ROWS_PER_LOAD;   // of a tile of W
+  static_assert(WROWS == 16 || (WROWS == 8 && MT == 1 && WLOADS < T::LOADS), "8 rows of W: one row tile, and a whole load fewer");
+  static_assert(WROWS == 16 || ACT != 4, "the sums of squares before a norm are over 16 columns");
   static_assert(XROWS == 16 || (XROWS == 8 && MT == 1 && XLOADS < T::LOADS), "8 rows of x: one row tile, and a whole load fewer");
   static_assert(!(SCALED || ACT == 4) || MT == 1, "the forms around a norm take up to 16 rows");
   static_assert(ACT != 4 || NW >= 4, "the epilogue of the product before a norm has a thread for each of the tile's 256 elements");
@@ -93,7 +98,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   const int wave = tid / 64, lane = tid % 64;
   const int half = rc.d / 2;
   // first row of the first tile; the second tile starts tile_step rows further
-  const int n0 = ACT == 3 ? (blockIdx.x / (half / 16)) * rc.d + (blockIdx.x % (half / 16)) * 16 : blockIdx.x * 16;
+  const int n0 = ACT == 3 ? (blockIdx.x / (half / WROWS)) * rc.d + (blockIdx.x % (half / WROWS)) * WROWS : blockIdx.x * WROWS;
   const int tile_step = ACT == 3 ? half : N;
   unsigned char* my = lds + (size_t)wave * (WT + MT) * T::TILE_BYTES;
 
@@ -143,6 +148,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
     const bool live_ = (live);                                                                  \
     _Pragma("unroll") for (int i = 0; i < T::LOADS; ++i) {                                      \
       _Pragma("unroll") for (int wt = 0; wt < WT; ++wt) {                                       \
+        if (i >= WLOADS) break;                                                                 \
         const bf16_t* from_ = live_ ? W + woff[wt][i] : x + xoff[0][i];                         \
         wreg[buf][wt][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(from_ + kk_)); \
       }                                                                                         \
@@ -201,7 +207,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
       for (int i = 0; i < T::LOADS; ++i) {
         const int off = (lrow + i * T::ROWS_PER_LOAD) * T::ROW_BYTES + lcol * 2;
 #pragma unroll
-        for (int wt = 0; wt < WT; ++wt) *reinterpret_cast<u32x4_t*>(my + wt * T::TILE_BYTES + off) = wreg[b][wt][i];
+        for (int wt = 0; wt < WT; ++wt)
+          if (i < WLOADS) *reinterpret_cast<u32x4_t*>(my + wt * T::TILE_BYTES + off) = wreg[b][wt][i];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
           if (i < XLOADS) *reinterpret_cast<u32x4_t*>(my + (WT + mt) * T::TILE_BYTES + off) = xreg[b][mt][i];
@@ -240,6 +247,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   __syncthreads();
   for (int e = tid; e < MT * 256; e += NW * 64) {
     const int mt = e / 256, l = (e % 256) / 4, j = e % 4;
+    if (WROWS < 16 && (l / 16) * 4 + j >= WROWS) continue;       // the half that was not fetched
     float sum[WT];
 #pragma unroll
     for (int wt = 0; wt < WT; ++wt) {
@@ -345,7 +353,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   }
 }
 
-template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH, bool SCALED, int XROWS>
+template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH, bool SCALED, int XROWS, int WROWS>
 static int launch_skinny_x(const void* x, long ldx, const void* W, long ldw, const void* bias, void* y, long ldy, int M,
                            int N, int K, hipStream_t stream, RopeCacheArgs rc, NormAroundArgs na) {
   using T = SkinnyTile<KC>;
@@ -353,7 +361,7 @@ static int launch_skinny_x(const void* x, long ldx, const void* W, long ldw, con
   const size_t stage = (size_t)NW * (WT + MT) * T::TILE_BYTES;
   const size_t red = (size_t)NW * WT * MT * 64 * 4 * sizeof(float) + ((SCALED || ACT == 4) ? 256 * sizeof(float) : 0);
   const size_t smem = stage > red ? stage : red;
-  auto kernel = gemm_skinny_kernel<MT, KC, NW, TOut, ACT, DEPTH, SCALED, XROWS>;
+  auto kernel = gemm_skinny_kernel<MT, KC, NW, TOut, ACT, DEPTH, SCALED, XROWS, WROWS>;
   static bool configured = false;   // per instantiation
   if (!configured) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -364,12 +372,18 @@ static int launch_skinny_x(const void* x, long ldx, const void* W, long ldw, con
     }
     configured = true;
   }
-  // the gated form has a workgroup per 16 outputs, the rotary form one per 32 rows of W, the plain one per 16
-  const int blocks = ACT == 3 ? N / 32 : (N + 15) / 16;
+  // the gated form has a workgroup per WROWS outputs, the rotary form one per 2 WROWS rows of W, the plain one per WROWS
+  const int blocks = ACT == 3 ? N / (2 * WROWS) : (N + WROWS - 1) / WROWS;
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(NW * 64), smem, stream, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw,
                      (const bf16_t*)bias, (TOut*)y, ldy, M, N, K, rc, na);
   return 0;
 }
+
+// Whether a product of M rows with so many outputs (pairs of outputs in the rotary form) runs with tiles of 8 rows of W:
+// where such tiles all fit on the chip at once, tiles of 16 leave half of its compute units or more without a workgroup.
+// Measured at 8 rows, tiles of 16 -> 8: 2,048 x 1,024 to 4,096 (128 -> 256 workgroups) 6.8 -> 6.0 us, 2,048 x 8,192 10.4 ->
+// 8.7, QKV of 3,072 x 2,048 with rotation (96 -> 192) 7.7 -> 7.0; but of 6,144 x 4,096 (192 -> 384) 12.4 -> 13.2.
+static bool skinny_narrow(int M, int outputs) { return M <= 16 && (outputs + 7) / 8 <= lmsf_compute_units(); }
 
 template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH = 1, bool SCALED = false>
 static int launch_skinny(const void* x, long ldx, const void* W, long ldw, const void* bias, void* y, long ldy, int M,
@@ -377,10 +391,18 @@ static int launch_skinny(const void* x, long ldx, const void* W, long ldw, const
                          NormAroundArgs na = NormAroundArgs()) {
   // up to 8 rows (and tiles whose loads cover 8 rows each): half of x's tile is neither fetched nor staged
   if constexpr (MT == 1 && SkinnyTile<KC>::ROWS_PER_LOAD <= 8) {
-    if (M <= 8)
-      return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, 8>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na);
+#define GO(X_, W_) \
+  return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, X_, W_>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na)
+    if constexpr (ACT != 4) {
+      if (skinny_narrow(M, ACT == 3 ? N / 2 : N)) {
+        if (M <= 8) GO(8, 8);
+        GO(16, 8);
+      }
+    }
+    if (M <= 8) GO(8, 16);
+#undef GO
   }
-  return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, 16>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na);
+  return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, 16, 16>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na);
 }
 
 // x [M, K] bfloat16 (row stride ldx), W [N, K] bfloat16 (row stride ldw), bias [N] bfloat16 or null,

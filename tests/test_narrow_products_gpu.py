@@ -1,0 +1,60 @@
+"""The few-rows products whose workgroups own 8 rows of the weight instead of 16: at both sides of the line between the
+two every output is added up in the same order, so the same rows give the same bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from lmsf_amd.ops import get_ops
+    return get_ops()
+
+
+def rnd(g, *shape):
+    return (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).bfloat16().to("cuda:0")
+
+
+# 8 compute units' worth of columns more than the line (2,048 on 256 units), odd numbers of columns, one column
+@pytest.mark.parametrize("N", [1, 7, 8, 9, 24, 1000, 2041, 2048])
+@pytest.mark.parametrize("M", [2, 8, 9, 16])
+@pytest.mark.parametrize("K", [8, 64, 1096, 4096])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_product(ops, M, N, K, out):
+    g = torch.Generator().manual_seed(N * K + M)
+    w, b, x = rnd(g, 8192, K), rnd(g, 8192), rnd(g, M, K)
+    assert torch.equal(ops.linear(x, w[:N], b[:N], out_dtype=out), ops.linear(x, w, b, out_dtype=out)[:, :N])
+
+
+@pytest.mark.parametrize("I", [1, 8, 23, 2048])
+@pytest.mark.parametrize("M", [3, 8, 13])
+@pytest.mark.parametrize("kind", ["silu", "gelu", "gelu_tanh"])
+def test_gated_product(ops, M, I, kind):
+    g = torch.Generator().manual_seed(I + M)
+    K, more = 1032, 4096
+    gate, up, x = rnd(g, more, K), rnd(g, more, K), rnd(g, M, K)
+    few = ops.linear_gated(x, torch.cat([gate[:I], up[:I]]), None, kind)
+    assert torch.equal(few, ops.linear_gated(x, torch.cat([gate, up]), None, kind)[:, :I])
+
+
+@pytest.mark.parametrize("M", [3, 8, 15])
+@pytest.mark.parametrize("d,heads", [(32, 2), (96, 5), (64, 62)])
+def test_qkv_product_with_rotation(ops, M, d, heads):
+    """Few heads beside the same query heads among many: tiles of 8 pairs beside tiles of 16."""
+    g = torch.Generator().manual_seed(d + heads + M)
+    K, many, ps, pages = 520, 260, 8, 4
+    wq, wkv, x = rnd(g, many * d, K), rnd(g, 2 * d, K), rnd(g, M, K)
+    pos = torch.randint(0, 40, (M,), generator=g, dtype=torch.int32).to("cuda:0")
+    ang = torch.arange(40)[:, None] * torch.rand(d // 2, generator=g)[None, :]
+    table = torch.cat([ang.cos(), ang.sin()], 1).contiguous().to("cuda:0")
+    slots = torch.randperm(pages * ps, generator=g)[:M].to(torch.int32).to("cuda:0")
+
+    def run(n):
+        k = torch.zeros(pages, 1, ps, d, dtype=torch.bfloat16, device="cuda:0")
+        v = torch.zeros(pages, 1, d, ps, dtype=torch.bfloat16, device="cuda:0")
+        y = ops.qkv_rope_cache(x, torch.cat([wq[:n * d], wkv]), None, n, 1, d, pos, table, d, True, slots, k, v)
+        return y, k, v
+    (a, ka, va), (b, kb, vb) = run(heads), run(many)
+    assert torch.equal(a[:, :heads * d], b[:, :heads * d]) and torch.equal(ka, kb) and torch.equal(va, vb)
+    assert ka.abs().sum() > 0
