@@ -153,6 +153,171 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
   }
 }
 
+// ---------------------------------------------------------------- few tokens, rows that allow 16-byte loads
+//
+// The same two products with everything that comes from memory asked for in one go, and an expert that several pairs
+// have chosen read once for all of them. A wave reads its rows of the matrix and the same entries of the vectors
+// (which the caches hold) with 16-byte loads, MOE_AHEAD pieces of 512 or 256 entries of each row on their way at a time;
+// nothing goes through LDS and no wave waits for another. Every output is added up in the order of the kernels above.
+// The outputs vary fastest over the workgroups, so that an expert's rows are read by all eight dies (with the pairs
+// fastest, a pair's whole expert falls to one die: gate and up 26.5 us). What bounds them is memory and, for an expert
+// of several pairs, the multiply-adds of a wave (8 tokens, 2 of 16 experts of 2,048 -> 2 x 1,024 -> 2,048 a token: gate
+// and up 24.4 -> 21.2 us, down 15.1 -> 11.6; 4 pieces ahead, 2 pairs a read, 1 or 4 outputs a wave: 23.4 to 28.4 us).
+#define MOE_AHEAD 2
+#define MOE_FEW_PAIRS 64      // a lane each
+#define MOE_SHARED_PAIRS 4    // pairs of one expert that share a read of its rows
+#define MOE_FEW_OUT 2         // outputs a wave owns
+
+// a[q][r] += sum over this lane's entries of rows r against the vectors of the pairs, each times its scale
+template <typename T, int ROWS, int PAIRS>
+__device__ __forceinline__ void moe_few_dot(const T* const (&w)[ROWS], const T* const (&x)[PAIRS], const float (&scale)[PAIRS],
+                                            int n_pairs, int W, int lane, float (&a)[PAIRS][ROWS]) {
+  constexpr int V = Vec16<T>::N, STEP = LMSF_WAVE * V;
+  for (int i0 = lane * V; i0 < W; i0 += MOE_AHEAD * STEP) {
+    Vec16<T> p[MOE_AHEAD][ROWS], xv[PAIRS][MOE_AHEAD];
+#pragma unroll
+    for (int u = 0; u < MOE_AHEAD; ++u) {
+      const int i = i0 + u * STEP;
+      if (i < W) {
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) p[u][r].load(w[r] + i);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q) {
+      if (q >= n_pairs) break;
+#pragma unroll
+      for (int u = 0; u < MOE_AHEAD; ++u)
+        if (i0 + u * STEP < W) xv[q][u].load(x[q] + i0 + u * STEP);
+    }
+#pragma unroll
+    for (int q = 0; q < PAIRS; ++q) {
+      if (q >= n_pairs) break;
+#pragma unroll
+      for (int u = 0; u < MOE_AHEAD; ++u) {
+        if (i0 + u * STEP >= W) break;
+#pragma unroll
+        for (int e = 0; e < V; ++e) {
+          const float f = scale[q] * xv[q][u].get(e);
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r) a[q][r] += p[u][r].get(e) * f;
+        }
+      }
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
+    const T* __restrict__ h, long h_stride, const T* __restrict__ Wgu, const int* __restrict__ ids,
+    const int* __restrict__ table, int vocab, int top, int E, T* __restrict__ act, int F, int W, int n_pairs,
+    const float* __restrict__ pair_scale, int gated, float limit, int identity) {
+  const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE;
+  const int f0 = (blockIdx.x * MOE_WAVES + wave) * MOE_FEW_OUT;
+  if (f0 >= F) return;
+  int mine = -1;                  // the expert of pair ``lane``
+  if (lane < n_pairs) {
+    const int n = lane / top, id = min(max(ids ? ids[n] : n, 0), vocab - 1);
+    mine = min(max(table[(long)id * top + lane - n * top], 0), E + identity - 1);
+  }
+  const int e = __shfl(mine, blockIdx.y, LMSF_WAVE);
+  if (e >= E) return;             // (what an expert without matrices returns is its input: the kernel below)
+  unsigned long long pairs = __ballot(mine == e);
+  if (__ffsll(pairs) - 1 != (int)blockIdx.y) return;     // the first pair of an expert stands for all of them
+  const T* We = Wgu + (long)e * (gated ? 2 : 1) * F * W;
+  const int valid = min(MOE_FEW_OUT, F - f0);
+  const T* w[2 * MOE_FEW_OUT];
+#pragma unroll
+  for (int r = 0; r < MOE_FEW_OUT; ++r) {
+    w[r] = We + (long)(f0 + min(r, valid - 1)) * W;
+    w[MOE_FEW_OUT + r] = gated ? w[r] + (long)F * W : w[r];
+  }
+  while (pairs) {
+    const T* x[MOE_SHARED_PAIRS];
+    float scale[MOE_SHARED_PAIRS], a[MOE_SHARED_PAIRS][2 * MOE_FEW_OUT];
+    int pair[MOE_SHARED_PAIRS], count = 0;
+#pragma unroll
+    for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
+      pair[q] = 0;
+      if (pairs) {
+        pair[q] = __ffsll(pairs) - 1;
+        pairs &= pairs - 1;
+        ++count;
+      }
+      x[q] = h + (long)(pair[q] / top) * h_stride;
+      scale[q] = pair_scale ? pair_scale[pair[q]] : 1.f;
+#pragma unroll
+      for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = 0.f;
+    }
+    moe_few_dot<T, 2 * MOE_FEW_OUT, MOE_SHARED_PAIRS>(w, x, scale, count, W, lane, a);
+#pragma unroll
+    for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
+      if (q >= count) break;
+#pragma unroll
+      for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = wave_sum(a[q][r]);
+      if (lane < valid) {
+        // the products are rounded as stored activations are, then the activation in float32
+        const float gg = to_f32<T>(from_f32<T>(lane == 0 ? a[q][0] : a[q][1]));
+        const float uu = to_f32<T>(from_f32<T>(lane == 0 ? a[q][MOE_FEW_OUT] : a[q][MOE_FEW_OUT + 1]));
+        float y;
+        if (!gated) {
+          const float up = fmaxf(gg, 0.f);      // one matrix an expert: relu(W_up h)^2
+          y = up * up;
+        } else {
+          y = limit > 0.f ? bounded_gate(gg, uu, limit) : gg / (1.f + expf(-gg)) * uu;
+        }
+        act[(long)pair[q] * F + f0 + lane] = from_f32<T>(y);
+      }
+    }
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(MOE_THREADS) void moe_down_few_kernel(
+    const T* __restrict__ act, const T* __restrict__ Wd, const int* __restrict__ ids, const int* __restrict__ table,
+    int vocab, int top, int E, float weight, const T* __restrict__ base, long base_stride, T* __restrict__ out,
+    long out_stride, int F, int W, const float* __restrict__ base_scale, const float* __restrict__ out_scale,
+    int identity, const T* __restrict__ h, long h_stride, const float* __restrict__ pair_scale) {
+  const int n = blockIdx.y;
+  const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE;
+  const int o0 = (blockIdx.x * MOE_WAVES + wave) * MOE_FEW_OUT;
+  if (o0 >= W) return;
+  const int valid = min(MOE_FEW_OUT, W - o0);
+  const int id = min(max(ids ? ids[n] : n, 0), vocab - 1);
+  float total[MOE_FEW_OUT];
+#pragma unroll
+  for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] = 0.f;
+  float b = 0.f;
+  if (lane < valid && base) b = to_f32<T>(base[(long)n * base_stride + o0 + lane]);
+#pragma unroll 2
+  for (int k = 0; k < top; ++k) {
+    const int e = min(max(table[(long)id * top + k], 0), E + identity - 1);
+    const float os = out_scale ? out_scale[(long)n * top + k] : 1.f;
+    if (e >= E) {      // an expert without matrices returns its input
+      const float f = os * (pair_scale ? pair_scale[(long)n * top + k] : 1.f);
+#pragma unroll
+      for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] += f * to_f32<T>(h[(long)n * h_stride + o0 + min(r, valid - 1)]);
+      continue;
+    }
+    const T* w[MOE_FEW_OUT];
+    const T* x[1] = {act + ((long)n * top + k) * F};
+    const float one[1] = {1.f};
+    float a[1][MOE_FEW_OUT];
+#pragma unroll
+    for (int r = 0; r < MOE_FEW_OUT; ++r) {
+      w[r] = Wd + ((long)e * W + o0 + min(r, valid - 1)) * F;
+      a[0][r] = 0.f;
+    }
+    moe_few_dot<T, MOE_FEW_OUT, 1>(w, x, one, 1, F, lane, a);
+#pragma unroll
+    for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] += os * wave_sum(a[0][r]);
+  }
+  if (lane < valid) {
+    if (base_scale) b *= base_scale[n];
+    out[(long)n * out_stride + o0 + lane] = from_f32<T>(b + weight * (lane == 0 ? total[0] : total[1]));
+  }
+}
+
 // ---------------------------------------------------------------- many tokens: grouped by expert, matrix cores
 
 #define MOE_TILE 128         // pairs a tile holds
@@ -438,6 +603,25 @@ extern "C" int lmsf_table_moe_act(const void* h, int dtype, long h_stride, const
     if (vec) MOE_COMBINE(true); else MOE_COMBINE(false);
 #undef MOE_COMBINE
     LMSF_LAUNCH_CHECK("table_moe (grouped)");
+    return 0;
+  }
+  const int es16 = 16 / lmsf_elem_size(dtype);
+  if ((long)n_tokens * top <= MOE_FEW_PAIRS && W % es16 == 0 && F % es16 == 0 && h_stride % es16 == 0 && lmsf_aligned16(h) &&
+      lmsf_aligned16(Wgu) && lmsf_aligned16(Wd) && lmsf_aligned16(act)) {
+    const int outs = MOE_WAVES * MOE_FEW_OUT, P = n_tokens * top;
+    const dim3 f1((F + outs - 1) / outs, P), f2((W + outs - 1) / outs, n_tokens);
+#define MOE_FEW(T_)                                                                                                   \
+  do {                                                                                                                \
+    hipLaunchKernelGGL((moe_gate_up_few_kernel<T_>), f1, dim3(MOE_THREADS), 0, stream, (const T_*)h, h_stride,        \
+                       (const T_*)Wgu, ids, table, vocab, top, E, (T_*)act, F, W, P, pair_scale, gated, limit,        \
+                       identity);                                                                                     \
+    hipLaunchKernelGGL((moe_down_few_kernel<T_>), f2, dim3(MOE_THREADS), 0, stream, (const T_*)act, (const T_*)Wd,    \
+                       ids, table, vocab, top, E, weight, (const T_*)base, base_stride, (T_*)out, out_stride, F, W,   \
+                       base_scale, out_scale, identity, (const T_*)h, h_stride, pair_scale);                          \
+  } while (0)
+    if (dtype == LMSF_F32) MOE_FEW(float); else MOE_FEW(bf16_t);
+#undef MOE_FEW
+    LMSF_LAUNCH_CHECK("table_moe (few)");
     return 0;
   }
   const int per_block = MOE_WAVES * MOE_OUT_PER_WAVE;
