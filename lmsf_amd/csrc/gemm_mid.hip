@@ -4,7 +4,7 @@
 //
 // The product is still a stream of the weight matrix, but with this many rows the activations are no
 // longer negligible: a workgroup that owns 16 rows of W reads four times as many bytes of x as of W. Here
-// a workgroup owns 64 rows of W (16 per wave) and all rows of x, so x is read once per 64 rows of W; where
+// a workgroup owns up to 64 rows of W (16 per wave) and all rows of x, so x is read once per 64 rows of W; where
 // that leaves too few workgroups to fill the chip (N = 4096: 64 of them), K is split over several
 // workgroups, which write float32 partial sums that a second small kernel adds in a fixed order (and
 // applies bias and activation to). The reference leaves these products to cuBLASLt
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
                                                        const bf16_t* __restrict__ W, long ldw,
                                                        const bf16_t* __restrict__ bias, TOut* __restrict__ y,
                                                        long ldy, float* __restrict__ part, int M, int N, int K,
-                                                       int n_split, MidRowScale rs) {
+                                                       int n_split, int U, MidRowScale rs) {
   constexpr int WP = ACT ? 2 : 1;      // projections: gate and up, or the only one
   constexpr int WT = WP * TW;          // tiles of 16 rows of W per wave: TW of each projection
   constexpr int STAGES = MID_STAGES_OF(TW);
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
   constexpr int LPW = 2 * WT + XL;     // transfers per wave and step
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r = l & 15, g = l >> 4;
-  const int n0 = blockIdx.x * (64 * TW), split = blockIdx.y;
+  const int n0 = blockIdx.x * U, split = blockIdx.y;   // this workgroup's U outputs, at most 64 TW
   const int chunks = K / 64;
   const int c_begin = (int)((long)split * chunks / n_split), c_end = (int)((long)(split + 1) * chunks / n_split);
   const int n_steps = c_end - c_begin;
@@ -114,8 +114,8 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
       const int row = 8 * h + trow, piece = (tslot - row) & 7;
       // tile t of this wave: projection t / TW (0 the gate's rows or the only ones, 1 the up projection's), the
       // wave's 16 outputs number t % TW
-      int n = n0 + 16 * (w * TW + t % TW) + row;
-      if (n > N - 1) n = N - 1;        // rows beyond the matrix repeat the last row and are not stored
+      int n = n0 + min(16 * (w * TW + t % TW) + row, U - 1);
+      if (n > N - 1) n = N - 1;        // rows beyond the workgroup's or the matrix repeat the last row and are not stored
       src[t * 2 + h] = W + (long)(n + (t / TW) * N) * ldw + piece * 8 + (long)c_begin * 64;
       dst[t * 2 + h] = (w * WT + t) * MID_TILE + h * 1024;
     }
@@ -209,7 +209,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
 #pragma unroll
   for (int tw = 0; tw < TW; ++tw) {
     const int n = n0 + 16 * (w * TW + tw) + 4 * g;
-    if (n >= N) continue;              // N is a multiple of 4 where it is not a multiple of 64 (checked by the host)
+    if (n >= N || n - n0 >= U) continue;       // N is a multiple of 4 (checked by the host), U of 8
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int m = mt * 16 + r;
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) void gemm_mid_reduce_kernel(const float* __res
 }
 
 template <int MT, int ACT, bool PARTIAL, typename TOut, int TW = 1>
-static int launch_mid(dim3 grid, hipStream_t stream, const bf16_t* x, long ldx, const bf16_t* W, long ldw,
+static int launch_mid(dim3 grid, int U, hipStream_t stream, const bf16_t* x, long ldx, const bf16_t* W, long ldw,
                       const bf16_t* bias, TOut* y, long ldy, float* part, int M, int N, int K, int n_split,
                       MidRowScale rs) {
   static_assert(TW == 1 || TW == 2, "one or two tiles of each projection per wave");
@@ -283,7 +283,7 @@ static int launch_mid(dim3 grid, hipStream_t stream, const bf16_t* x, long ldx, 
     }
     configured = true;
   }
-  hipLaunchKernelGGL(kernel, grid, dim3(256), smem, stream, x, ldx, W, ldw, bias, y, ldy, part, M, N, K, n_split, rs);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), smem, stream, x, ldx, W, ldw, bias, y, ldy, part, M, N, K, n_split, U, rs);
   return 0;
 }
 
@@ -336,17 +336,38 @@ static int mid_check(const void* x, long ldx, const void* W, long ldw, int M, in
   return 0;
 }
 
+// Outputs a workgroup owns: 64, or, where such workgroups leave compute units without one, as few (in steps of 8, at
+// least 32) as the chip still takes at once. QKV of 6,144 x 4,096 in 2 parts at 64 rows: 192 workgroups of 64 outputs
+// 18.1 us, 256 of 48 14.7; gate_up of 28,672 x 4,096: 224 of 64 42.6, 256 of 56 41.5. The gated product after a norm (up to
+// 16 rows), whose x is small, stays at 64 (37.5 against 37.8 at 8 rows).
+static int mid_outputs(int N, int n_split, bool after_norm) {
+  const int cus = lmsf_compute_units();
+  if (after_norm || (long)((N + 63) / 64) * n_split >= cus) return 64;
+  int U = 64;
+  while (U > 32 && (long)((N + U - 9) / (U - 8)) * n_split <= cus) U -= 8;
+  return U;
+}
+
 // The product's kernel: the result into y (n_split == 1) or partial sums into scratch.
 static int mid_product(const bf16_t* xb, long ldx, const bf16_t* Wb, long ldw, const bf16_t* bb, void* y, int out_dtype,
                        long ldy, int M, int N, int K, int act, int n_split, float* scratch, hipStream_t stream,
                        MidRowScale rs = MidRowScale{nullptr, 0, 0.f, 0, 0.f}) {
-  dim3 grid((N + 63) / 64, n_split);
+  const int U = mid_outputs(N, n_split, rs.sumsq != nullptr);
+  dim3 grid((N + U - 1) / U, n_split);
   int rc = 0;
 #define MID(MT_, ACT_, T_)                                                                                          \
   rc = n_split > 1                                                                                                  \
-           ? launch_mid<MT_, ACT_, true, T_>(grid, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs) \
-           : launch_mid<MT_, ACT_, false, T_>(grid, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs)
-  if (out_dtype == LMSF_F32) {
+           ? launch_mid<MT_, ACT_, true, T_>(grid, U, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs) \
+           : launch_mid<MT_, ACT_, false, T_>(grid, U, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs)
+  // Many more outputs than the chip has workgroups for (an LM head): 128 a workgroup, so that x, which every workgroup
+  // reads whole from the caches, is read half as often. 128,256 x 4,096 in float32 at 32 / 64 / 128 rows: 194 / 230 / 300
+  // us with 64 outputs a workgroup, 183 / 211 / 245 with 128.
+  if (out_dtype == LMSF_F32 && n_split == 1 && (N + 127) / 128 >= 2 * lmsf_compute_units()) {
+    const dim3 wide((N + 127) / 128, 1);
+#define WIDE(MT_) rc = launch_mid<MT_, 0, false, float, 2>(wide, 128, stream, xb, ldx, Wb, ldw, bb, (float*)y, ldy, scratch, M, N, K, 1, rs)
+    if (M <= 32) WIDE(2); else if (M <= 64) WIDE(4); else if (M <= 96) WIDE(6); else WIDE(8);
+#undef WIDE
+  } else if (out_dtype == LMSF_F32) {
     if (M <= 32) MID(2, 0, float); else if (M <= 64) MID(4, 0, float); else if (M <= 96) MID(6, 0, float); else MID(8, 0, float);
   } else if (M <= 32) {
     if (act == 0) MID(2, 0, bf16_t); else if (act == 1) MID(2, 1, bf16_t); else if (act == 2) MID(2, 2, bf16_t); else MID(2, 6, bf16_t);
@@ -442,9 +463,9 @@ extern "C" int lmsf_gemm_mid_scaled(const void* x, long ldx, const void* W, long
   const MidRowScale rs = {sumsq, in_tiles, eps, K, 0.f};
   if (mid_scaled_outputs(N) == 128) {
     const dim3 grid((N + 127) / 128, 1);
-    const int rc = act == 1 ? launch_mid<2, 1, false, bf16_t, 2>(grid, stream, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw,
+    const int rc = act == 1 ? launch_mid<2, 1, false, bf16_t, 2>(grid, 128, stream, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw,
                                                                  (const bf16_t*)bias, (bf16_t*)y, ldy, nullptr, M, N, K, 1, rs)
-                            : launch_mid<2, 2, false, bf16_t, 2>(grid, stream, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw,
+                            : launch_mid<2, 2, false, bf16_t, 2>(grid, 128, stream, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw,
                                                                  (const bf16_t*)bias, (bf16_t*)y, ldy, nullptr, M, N, K, 1, rs);
     if (rc) return rc;
     LMSF_LAUNCH_CHECK("gemm_mid_scaled");

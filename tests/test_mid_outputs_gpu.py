@@ -1,0 +1,60 @@
+"""The 17-and-more-rows product with fewer than 64 outputs a workgroup, and with 128: every output is added up in the same
+order, so the same rows of the weight give the same bits as among many."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from lmsf_amd.ops import get_ops
+    return get_ops()
+
+
+def rnd(g, *shape):
+    return (torch.randn(*shape, generator=g) * shape[-1] ** -0.5).bfloat16().to("cuda:0")
+
+
+def product(ops, x, w, bias, out, splits, gated):
+    from lmsf_amd.ops.hip_ops import _ptr
+    M, K, N = x.shape[0], x.shape[1], w.shape[0] // (2 if gated else 1)
+    y = torch.full((M, N + 4), float("nan"), dtype=out, device="cuda:0")[:, :N]
+    scratch = torch.empty(max(4, ops.lib.lmsf_gemm_mid_scratch_floats(M, N, splits, int(gated))), device="cuda:0")
+    ops._check(ops.lib.lmsf_gemm_mid(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(bias), _ptr(y),
+                                     0 if out == torch.float32 else 1, y.stride(0), M, N, K, 1 if gated else 0, splits,
+                                     _ptr(scratch), ops._stream()))
+    return y
+
+
+# 32, 40, 48, 56 and 64 outputs a workgroup on 256 units (in one part and in 2), remainders of a workgroup, of 8 and of 4
+@pytest.mark.parametrize("N,splits", [(4, 1), (36, 1), (8192, 1), (8196, 1), (10240, 1), (14332, 1), (16380, 1), (4096, 2),
+                                      (6144, 2), (6148, 2), (4100, 4)])
+@pytest.mark.parametrize("M", [17, 33, 64, 97])
+@pytest.mark.parametrize("gated", [False, True])
+def test_outputs_a_workgroup(ops, N, splits, M, gated):
+    if gated and M > 64:
+        pytest.skip("the gated form takes up to 64 rows")
+    g = torch.Generator().manual_seed(N + M)
+    K, many = 512, 20480               # 320 workgroups of 64 outputs: more than the chip takes at once
+    a, b, x = rnd(g, many, K), rnd(g, many, K), rnd(g, M, K)
+    ba, bb = rnd(g, many), rnd(g, many)
+    w = lambda n: torch.cat([a[:n], b[:n]]) if gated else a[:n]          # noqa: E731
+    bias = lambda n: torch.cat([ba[:n], bb[:n]]) if gated else ba[:n].clone()    # noqa: E731
+    for out in (torch.bfloat16,) if gated else (torch.bfloat16, torch.float32):
+        few = product(ops, x, w(N), bias(N), out, splits, gated)
+        assert torch.equal(few, product(ops, x, w(many), bias(many), out, splits, gated)[:, :N])
+
+
+# both sides of the line to 128 outputs a workgroup (65,408 = 511 such workgroups, 65,412 = 512), remainders
+@pytest.mark.parametrize("N", [65412, 65536, 128252])
+@pytest.mark.parametrize("M", [17, 64, 65, 128])
+def test_float32_output_of_many_columns(ops, N, M):
+    g = torch.Generator().manual_seed(N + M)
+    K = 64
+    w, x = rnd(g, N, K), rnd(g, M, K)
+    wide = product(ops, x, w, None, torch.float32, 1, False)
+    assert torch.equal(wide[:, :65408], product(ops, x, w[:65408], None, torch.float32, 1, False))
+    exact = x.double() @ w.double().T
+    # 64 products and their sums in float32
+    assert ((wide.double() - exact).abs() <= 66 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
