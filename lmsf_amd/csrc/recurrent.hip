@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
     long bc_stride, int b_at, int c_at, const T* __restrict__ z, long z_stride, const float* __restrict__ A_log,
     const float* __restrict__ Dw, float* __restrict__ state, long state_stride, const int* __restrict__ seg_starts,
     const int* __restrict__ state_slots, T* __restrict__ y, long y_stride, int inner, int nstate, int chunk,
-    const int* __restrict__ scratch_base, float* __restrict__ scratch) {
+    const int* __restrict__ scratch_base, float* __restrict__ scratch, int vec) {
   __shared__ float sB[SCANL_TT * NS], sC[SCANL_TT * NS];
   const int tid = threadIdx.x;
   const int c = blockIdx.x * 256 + tid;
@@ -394,18 +394,32 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
   const long entry = (long)inner * (nstate + 1);
   float* st = state + (long)state_slots[s] * state_stride + (long)cc * nstate;
   float a[NS], S[NS];
+  if (vec && base < 0) {
+    // a channel's NS rates and state entries, 16 bytes a load (one by one every load asks for 64 cache lines: 8 single
+    // tokens of 4,096 channels by 16 entries 10.6 -> 5.7 us)
 #pragma unroll
-  for (int n = 0; n < NS; ++n) {
-    const bool ok = n < nstate;
-    a[n] = ok ? -expf(A_log[(long)cc * nstate + n]) : 0.f;
-    S[n] = 0.f;
-    if (ok) {
-      if (base < 0) {
-        S[n] = st[n];
-      } else if (SUMMARY) {
-        if (j == 0 && live) scratch[(long)base * entry + (long)c * nstate + n] = st[n];     // the entry before the first chunk
-      } else {
-        S[n] = scratch[(long)(base + j) * entry + (long)cc * nstate + n];    // folded by selective_scan_fold_kernel
+    for (int n = 0; n + 3 < NS; n += 4) {
+      const float4 s4 = *reinterpret_cast<const float4*>(st + n);
+      const float4 a4 = *reinterpret_cast<const float4*>(A_log + (long)cc * NS + n);
+      S[n] = s4.x; S[n + 1] = s4.y; S[n + 2] = s4.z; S[n + 3] = s4.w;
+      a[n] = a4.x; a[n + 1] = a4.y; a[n + 2] = a4.z; a[n + 3] = a4.w;
+    }
+#pragma unroll
+    for (int n = 0; n < NS; ++n) a[n] = -expf(a[n]);
+  } else {
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      const bool ok = n < nstate;
+      a[n] = ok ? -expf(A_log[(long)cc * nstate + n]) : 0.f;
+      S[n] = 0.f;
+      if (ok) {
+        if (base < 0) {
+          S[n] = st[n];
+        } else if (SUMMARY) {
+          if (j == 0 && live) scratch[(long)base * entry + (long)c * nstate + n] = st[n];     // the entry before the first chunk
+        } else {
+          S[n] = scratch[(long)(base + j) * entry + (long)cc * nstate + n];    // folded by selective_scan_fold_kernel
+        }
       }
     }
   }
@@ -457,9 +471,15 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
       if (n < nstate) ent[(long)c * nstate + n] = S[n];
     ent[(long)inner * nstate + c] = sum_dt;
   } else if (j == n_chunks - 1) {
+    if (vec) {
 #pragma unroll
-    for (int n = 0; n < NS; ++n)
-      if (n < nstate) st[n] = S[n];
+      for (int n = 0; n + 3 < NS; n += 4)
+        *reinterpret_cast<float4*>(st + n) = make_float4(S[n], S[n + 1], S[n + 2], S[n + 3]);
+    } else {
+#pragma unroll
+      for (int n = 0; n < NS; ++n)
+        if (n < nstate) st[n] = S[n];
+    }
   }
 }
 
@@ -491,10 +511,13 @@ extern "C" int lmsf_selective_scan(const void* x, int dtype, long x_stride, cons
   if (n_tokens == 0 || n_segments == 0) return 0;
   if (nstate <= 32) {
     dim3 lgrid((inner + 255) / 256, chunked ? max_chunks : 1, n_segments), lblock(256);
+    // (the kernel holds exactly these numbers of entries, and every channel's lie on a 16-byte boundary)
+    const int vec = (nstate == 4 || nstate == 8 || nstate == 16 || nstate == 32) && state_stride % 4 == 0 &&
+                    lmsf_aligned16(state) && lmsf_aligned16(A_log);
 #define SCANL(T, NS, SUM)                                                                                              \
   hipLaunchKernelGGL((selective_scan_lane_kernel<T, NS, SUM>), lgrid, lblock, 0, stream, (const T*)x, x_stride, dt_pre, \
                      dt_stride, (const T*)bc, bc_stride, b_at, c_at, (const T*)z, z_stride, A_log, Dw, state,          \
-                     state_stride, seg_starts, state_slots, (T*)y, y_stride, inner, nstate, chunk, scratch_base, scratch)
+                     state_stride, seg_starts, state_slots, (T*)y, y_stride, inner, nstate, chunk, scratch_base, scratch, vec)
 #define SCANL_T(T, SUM)                      \
   do {                                       \
     if (nstate <= 4) SCANL(T, 4, SUM);       \
