@@ -6,8 +6,8 @@
 // (tops/csrc/tops/tensorrt_llm/common/cublasMMWrapper.cpp:182-210) and adds the bias afterwards
 // (core/src/model_executor/layers/linear.rs:101-104).
 //
-// Many outputs: a 64x64 tile per workgroup of 256 threads, 4x4 outputs per thread, K in slabs of 16 staged
-// through LDS; few outputs: K split over the waves (further down). Any M, N, K; rows may be strided (lda, ldw, ldc in elements).
+// K split over the waves of a workgroup (further down), or, for many outputs whose rows do not allow wide loads, a 64x64
+// tile per workgroup of 256 threads, 4x4 outputs per thread, K in slabs of 16 staged through LDS. Any M, N, K; rows may be strided (lda, ldw, ldc in elements).
 #include "common.h"
 
 #define GP_TILE 64
@@ -162,117 +162,120 @@ static void launch_gemm_plain_few(const void* A, long lda, const void* W, long l
 #undef FEW
 }
 
-// The product where the 64x64 tiles above are too few to fill the chip: every wave of a workgroup takes a share of K.
-// A workgroup of eight waves owns 8 MR rows by 16 columns; lane (r, c) = (l / 8, l % 8) of every wave holds the outputs of
-// rows r, r + 8, ... and columns c, c + 8, and wave w takes the pieces of V elements w, w + 8, w + 16, ... of K, so that
-// the eight waves read a row's neighbouring pieces at the same time and GP_AHEAD pieces of every row are on their way in
-// each. The waves' sums are added in wave order at the end: a fixed order, and shorter chains of additions than the tile's
-// single one. No LDS and no barrier inside the loop; what bounds it is a compute unit's rate of loads from the cache (a
-// row's piece goes to eight lanes; with twice as many pieces asked for at a time 8 rows, 128 columns, K = 352 take 10.4 us).
-// 8 rows, 128 columns, K = 352 in float32: 34.6 us in the tiles, 7.9 here; relative error of the result 3.3e-7 -> 1.3e-7.
-#define GP_AHEAD 4
-// Where it runs. The tiles take about 0.1 us for each k, whatever M and N, until they fill the chip several times; this
-// form takes N K at 0.8 TB/s of float32 weights or 2 M N K at 12.6 TFLOP/s, whichever is longer (every workgroup reads its
-// rows and columns for itself). Measured in float32, tiles -> this form: 1 x 6,144 x 4,096 390 -> 128 us, 64 x 6,144 x
-// 4,096 454 -> 256, 256 x 2,048 x 2,048 218 -> 173, 70 x 6,144 x 4,096 439 -> 420, but 128 x 6,144 x 4,096 445 -> 507.
-#define GP_SPLIT_COLS 16384
-#define GP_SPLIT_OUTPUTS (1L << 19)
-template <typename T, int V> struct GpPiece;
-template <> struct GpPiece<float, 4> {
-  float4 v;
-  __device__ __forceinline__ void load(const float* p) { v = *reinterpret_cast<const float4*>(p); }
-  __device__ __forceinline__ float get(int i) const { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
-};
-template <> struct GpPiece<bf16_t, 4> {
-  uint2 v;
-  __device__ __forceinline__ void load(const bf16_t* p) { v = *reinterpret_cast<const uint2*>(p); }
-  __device__ __forceinline__ float get(int i) const {
-    const uint32_t w = i < 2 ? v.x : v.y;
-    return __uint_as_float((i & 1) ? (w & 0xffff0000u) : (w << 16));
-  }
-};
-template <typename T> struct GpPiece<T, 1> {
-  T v;
-  __device__ __forceinline__ void load(const T* p) { v = *p; }
-  __device__ __forceinline__ float get(int) const { return to_f32<T>(v); }
-};
+// The product with K split over the waves of a workgroup.
+// A workgroup of eight waves owns 8 MR rows by 16 columns; wave w takes the steps of 32 k w, w + 8, w + 16, ... A step's
+// rows are read whole cache lines at a time (lane (r, c) = (l / 8, l % 8) reads four entries c of rows r, r + 8, ...), the
+// next step's while this one is multiplied, and go through an area of LDS that belongs to the wave, from which lane (r, c)
+// takes rows r, r + 8, ... and columns c, c + 8 for the outputs it holds: no barrier inside the loop. The waves' sums
+// are added in wave order at the end: a fixed order, and shorter chains of additions than the tile's single one.
+// (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of every wave and each
+// line is asked for by all eight waves: 7.9 us where this form takes 4.3.) What bounds it is the trip to memory
+// with few outputs, the reads of LDS (12 bytes a multiply-add with 32 rows) with many.
+// 8 rows, 128 columns, K = 352 in float32: 34.6 us in the tiles, 4.3 here; relative error 3.3e-7 -> 9.4e-8.
+// Where it runs: wherever the rows allow wide loads. Measured in float32, tiles -> this form: 8 x 6,144 x 4,096 401 -> 23 us,
+// 64 x 4,096 x 14,336 1,644 -> 163 (error 2.1e-6 -> 3.9e-7), 8 x 128,256 x 4,096 1,341 -> 394, 2,048 x 2,048 x 2,048 465 ->
+// 352, 2,048 x 28,672 x 4,096 12.7 -> 9.8 ms (38 -> 49 TFLOP/s; the card's rate without packed instructions is 79). With rows of any alignment
+// up to so many outputs: 512 x 1,001 x 333 38.2 -> 16.4 us, 1,024 rows 39.3 -> 28.7, but 2,048 rows 49.7 -> 52.1.
+#define GP_SPLIT_OUTPUTS (1L << 20)
+#define GP_STEP 32
+#define GP_ROW (GP_STEP + 4)      // floats a row takes in LDS: eight rows at a time lie on distinct banks
 
-template <typename TA, typename TW, typename TO, int MR, int V>
+// four neighbouring entries; VEC: in one load (K is a multiple of 4 then), else one by one, those from K on as zeros
+template <bool VEC>
+__device__ __forceinline__ float4 gp_load4(const float* p, int k, int K) {
+  if (VEC) return k < K ? *reinterpret_cast<const float4*>(p + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+  return make_float4(k < K ? p[k] : 0.f, k + 1 < K ? p[k + 1] : 0.f, k + 2 < K ? p[k + 2] : 0.f, k + 3 < K ? p[k + 3] : 0.f);
+}
+template <bool VEC>
+__device__ __forceinline__ float4 gp_load4(const bf16_t* p, int k, int K) {
+  if (VEC) {
+    const uint2 v = k < K ? *reinterpret_cast<const uint2*>(p + k) : make_uint2(0u, 0u);
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                       __uint_as_float(v.y & 0xffff0000u));
+  }
+  return make_float4(k < K ? bf16_to_f32(p[k]) : 0.f, k + 1 < K ? bf16_to_f32(p[k + 1]) : 0.f,
+                     k + 2 < K ? bf16_to_f32(p[k + 2]) : 0.f, k + 3 < K ? bf16_to_f32(p[k + 3]) : 0.f);
+}
+
+template <typename TA, typename TW, typename TO, int MR, bool VEC>
 __global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restrict__ A, long lda,
                                                                const TW* __restrict__ W, long ldw,
                                                                const TW* __restrict__ bias, TO* __restrict__ C,
                                                                long ldc, int M, int N, int K) {
-  __shared__ float sums[8][MR * 2 * 64];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  constexpr int ROWS = 8 * MR + 16;                 // of A, then of W
+  static_assert(ROWS * GP_ROW >= MR * 128, "the waves' sums lie where their steps lay");
+  __shared__ __align__(16) float area[8][ROWS * GP_ROW];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane >> 3, c = lane & 7;
   const int m0 = blockIdx.y * (8 * MR), n0 = blockIdx.x * 16;
+  float* mine = area[wave];
   const TA* a[MR];
   const TW* w[2];
 #pragma unroll
-  for (int i = 0; i < MR; ++i) a[i] = A + (long)min(m0 + lane / 8 + 8 * i, M - 1) * lda;   // rows beyond M: not written
+  for (int i = 0; i < MR; ++i) a[i] = A + (long)min(m0 + r + 8 * i, M - 1) * lda;   // rows beyond M: not written
 #pragma unroll
-  for (int j = 0; j < 2; ++j) w[j] = W + (long)min(n0 + lane % 8 + 8 * j, N - 1) * ldw;
-  float acc[MR][2];
+  for (int j = 0; j < 2; ++j) w[j] = W + (long)min(n0 + r + 8 * j, N - 1) * ldw;
+  float acc[MR][2][4];        // of k = 0, 1, 2, 3 mod 4: four short chains instead of one
 #pragma unroll
-  for (int i = 0; i < MR; ++i) acc[i][0] = acc[i][1] = 0.f;
-  const int pieces = K / V;            // (V divides K)
-  int p = wave;
-  for (; p + 8 * (GP_AHEAD - 1) < pieces; p += 8 * GP_AHEAD) {
-    GpPiece<TA, V> x[GP_AHEAD][MR];
-    GpPiece<TW, V> y[GP_AHEAD][2];
+  for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int u = 0; u < GP_AHEAD; ++u) {
-      const long k = (long)(p + 8 * u) * V;
+    for (int e = 0; e < 4; ++e) acc[i][0][e] = acc[i][1][e] = 0.f;
+  float4 x[MR], y[2];
+  auto fetch = [&](int k0) {
 #pragma unroll
-      for (int i = 0; i < MR; ++i) x[u][i].load(a[i] + k);
+    for (int i = 0; i < MR; ++i) x[i] = gp_load4<VEC>(a[i], k0 + 4 * c, K);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) y[u][j].load(w[j] + k);
-    }
+    for (int j = 0; j < 2; ++j) y[j] = gp_load4<VEC>(w[j], k0 + 4 * c, K);
+  };
+  int k0 = wave * GP_STEP;
+  if (k0 < K) fetch(k0);
+  for (; k0 < K; k0 += 8 * GP_STEP) {
 #pragma unroll
-    for (int u = 0; u < GP_AHEAD; ++u)
+    for (int i = 0; i < MR; ++i) *reinterpret_cast<float4*>(mine + (r + 8 * i) * GP_ROW + 4 * c) = x[i];
 #pragma unroll
-      for (int e = 0; e < V; ++e)
+    for (int j = 0; j < 2; ++j) *reinterpret_cast<float4*>(mine + (8 * MR + r + 8 * j) * GP_ROW + 4 * c) = y[j];
+    if (k0 + 8 * GP_STEP < K) fetch(k0 + 8 * GP_STEP);
+    __builtin_amdgcn_wave_barrier();                // (a wave's LDS accesses are carried out in their order)
+#pragma unroll
+    for (int q = 0; q < GP_STEP; q += 4) {
+      float xe[MR][4], ye[2][4];
+#pragma unroll
+      for (int i = 0; i < MR; ++i)
+        *reinterpret_cast<float4*>(xe[i]) = *reinterpret_cast<const float4*>(mine + (r + 8 * i) * GP_ROW + q);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        *reinterpret_cast<float4*>(ye[j]) = *reinterpret_cast<const float4*>(mine + (8 * MR + c + 8 * j) * GP_ROW + q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int i = 0; i < MR; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] = fmaf(x[u][i].get(e), y[u][j].get(e), acc[i][j]);
-  }
-  for (; p < pieces; p += 8) {
-    GpPiece<TA, V> x[MR];
-    GpPiece<TW, V> y[2];
-#pragma unroll
-    for (int i = 0; i < MR; ++i) x[i].load(a[i] + (long)p * V);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) y[j].load(w[j] + (long)p * V);
-#pragma unroll
-    for (int e = 0; e < V; ++e)
-#pragma unroll
-      for (int i = 0; i < MR; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = fmaf(x[i].get(e), y[j].get(e), acc[i][j]);
+          for (int j = 0; j < 2; ++j) acc[i][j][e] = fmaf(xe[i][e], ye[j][e], acc[i][j][e]);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) sums[wave][(i * 2 + j) * 64 + lane] = acc[i][j];
+    for (int j = 0; j < 2; ++j) mine[(i * 2 + j) * 64 + lane] = (acc[i][j][0] + acc[i][j][1]) + (acc[i][j][2] + acc[i][j][3]);
   __syncthreads();
   for (int e = tid; e < MR * 128; e += 512) {
     const int l = e & 63, j = (e >> 6) & 1, i = e >> 7;
     const int m = m0 + l / 8 + 8 * i, n = n0 + l % 8 + 8 * j;
     if (m >= M || n >= N) continue;
-    float r = 0.f;
+    float s = 0.f;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) r += sums[v][e];
-    if (bias) r += to_f32<TW>(bias[n]);
-    C[(long)m * ldc + n] = from_f32<TO>(r);
+    for (int v = 0; v < 8; ++v) s += area[v][e];
+    if (bias) s += to_f32<TW>(bias[n]);
+    C[(long)m * ldc + n] = from_f32<TO>(s);
   }
 }
 
-template <typename TA, typename TW, typename TO, int V>
+template <typename TA, typename TW, typename TO, bool VEC>
 static void launch_gemm_plain_split(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                                     int M, int N, int K, hipStream_t stream) {
   const dim3 block(512);
 #define SPLIT(MR_)                                                                                                     \
-  hipLaunchKernelGGL((gemm_plain_split_kernel<TA, TW, TO, MR_, V>), dim3((N + 15) / 16, (M + 8 * MR_ - 1) / (8 * MR_)), \
+  hipLaunchKernelGGL((gemm_plain_split_kernel<TA, TW, TO, MR_, VEC>), dim3((N + 15) / 16, (M + 8 * MR_ - 1) / (8 * MR_)), \
                      block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw, (const TW*)bias, (TO*)C, ldc, M, N, K)
   if (M <= 8) SPLIT(1); else if (M <= 16) SPLIT(2); else SPLIT(4);
 #undef SPLIT
@@ -282,13 +285,14 @@ template <typename TA, typename TW, typename TO>
 static void launch_gemm_plain(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                               int M, int N, int K, hipStream_t stream) {
   dim3 grid((N + GP_TILE - 1) / GP_TILE, (M + GP_TILE - 1) / GP_TILE), block(256);
-  if (N <= GP_SPLIT_COLS && (long)M * N <= GP_SPLIT_OUTPUTS) {
-    const bool wide = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (size_t)A % (4 * sizeof(TA)) == 0 &&
-                      (size_t)W % (4 * sizeof(TW)) == 0;
-    if (wide)
-      launch_gemm_plain_split<TA, TW, TO, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
-    else
-      launch_gemm_plain_split<TA, TW, TO, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+  const bool wide = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (size_t)A % (4 * sizeof(TA)) == 0 &&
+                    (size_t)W % (4 * sizeof(TW)) == 0;
+  if (wide) {
+    launch_gemm_plain_split<TA, TW, TO, true>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
+    return;
+  }
+  if ((long)M * N <= GP_SPLIT_OUTPUTS) {
+    launch_gemm_plain_split<TA, TW, TO, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
     return;
   }
   hipLaunchKernelGGL((gemm_plain_kernel<TA, TW, TO>), grid, block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw,

@@ -13,11 +13,11 @@ def ops():
     return get_ops()
 
 
-# the edges of its row forms (8, 16, 32 rows a workgroup) and columns (16), K below, at and beyond a piece for every wave
-# and four pieces for every wave, K that is no multiple of 4, and both sides of the line to the 64x64 tiles
+# the edges of its row forms (8, 16, 32 rows a workgroup) and columns (16), K below, at and beyond a step of 32 and a step
+# for every wave, K that is no multiple of 4, and both sides of the line to the 64x64 tiles (2^20 outputs)
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 16, 4), (8, 17, 31), (9, 15, 32), (16, 33, 36), (17, 64, 127), (32, 16, 128),
-                                   (33, 70, 132), (65, 130, 260), (7, 128, 352), (1024, 512, 20), (1025, 512, 20),
-                                   (2, 16384, 12), (2, 16385, 12)])
+                                   (33, 70, 132), (65, 130, 260), (7, 128, 352), (5, 20, 256), (5, 20, 257), (5, 20, 515), (1024, 1024, 21), (1025, 1024, 21), (1025, 1024, 20),
+                                   (2, 20000, 12)])
 @pytest.mark.parametrize("types", [(torch.float32, torch.float32, torch.float32), (torch.float32, torch.bfloat16, torch.float32),
                                    (torch.bfloat16, torch.float32, torch.float32), (torch.bfloat16, torch.float32, torch.bfloat16)])
 @pytest.mark.parametrize("shift", [0, 1])
@@ -35,10 +35,10 @@ def test_product_of_few_outputs(ops, M, N, K, types, shift):
     b = torch.randn(N, generator=g).to(tw).to("cuda:0")
     y = ops.linear(x, w, b, out_dtype=to).double()
     exact = x.double() @ w.double().T + b.double()
-    # a wave adds K / 8 products and one more piece of up to 4 in turn, the waves' eight sums and the bias come on top;
-    # the tiles add all K in turn
-    split = N <= 16384 and M * N <= 1 << 19
-    chain = (K / 8 + 4 + 9) if split else K + 1
+    # a wave adds 8 products of every 256 in turn, four such sums, the waves' eight and the bias come on top; the tiles add
+    # all K in turn
+    split = M * N <= 1 << 20 or (K % 4 == 0 and shift == 0)
+    chain = 8 * -(-K // 256) + 11 if split else K + 1
     bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * chain * 2.0 ** -24
     if to == torch.bfloat16:
         bound = bound + exact.abs() * 2.0 ** -8
