@@ -214,11 +214,11 @@ __global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restr
   for (int i = 0; i < MR; ++i) a[i] = A + (long)min(m0 + r + 8 * i, M - 1) * lda;   // rows beyond M: not written
 #pragma unroll
   for (int j = 0; j < 2; ++j) w[j] = W + (long)min(n0 + r + 8 * j, N - 1) * ldw;
-  float acc[MR][2][4];        // of k = 0, 1, 2, 3 mod 4: four short chains instead of one
+  float acc[MR][2][2];        // of the even and of the odd k: two short chains instead of one
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[i][0][e] = acc[i][1][e] = 0.f;
+    for (int e = 0; e < 2; ++e) acc[i][0][e] = acc[i][1][e] = 0.f;
   float4 x[MR], y[2];
   auto fetch = [&](int k0) {
 #pragma unroll
@@ -249,14 +249,14 @@ __global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restr
 #pragma unroll
         for (int i = 0; i < MR; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j][e] = fmaf(xe[i][e], ye[j][e], acc[i][j][e]);
+          for (int j = 0; j < 2; ++j) acc[i][j][e & 1] = fmaf(xe[i][e], ye[j][e], acc[i][j][e & 1]);
     }
     __builtin_amdgcn_wave_barrier();
   }
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) mine[(i * 2 + j) * 64 + lane] = (acc[i][j][0] + acc[i][j][1]) + (acc[i][j][2] + acc[i][j][3]);
+    for (int j = 0; j < 2; ++j) mine[(i * 2 + j) * 64 + lane] = acc[i][j][0] + acc[i][j][1];
   __syncthreads();
   for (int e = tid; e < MR * 128; e += 512) {
     const int l = e & 63, j = (e >> 6) & 1, i = e >> 7;

@@ -35,10 +35,10 @@ def test_product_of_few_outputs(ops, M, N, K, types, shift):
     b = torch.randn(N, generator=g).to(tw).to("cuda:0")
     y = ops.linear(x, w, b, out_dtype=to).double()
     exact = x.double() @ w.double().T + b.double()
-    # a wave adds 8 products of every 256 in turn, four such sums, the waves' eight and the bias come on top; the tiles add
+    # a wave adds 16 products of every 256 in turn, two such sums, the waves' eight and the bias come on top; the tiles add
     # all K in turn
     split = M * N <= 1 << 20 or (K % 4 == 0 and shift == 0)
-    chain = 8 * -(-K // 256) + 11 if split else K + 1
+    chain = 16 * -(-K // 256) + 10 if split else K + 1
     bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * chain * 2.0 ** -24
     if to == torch.bfloat16:
         bound = bound + exact.abs() * 2.0 ** -8
