@@ -171,9 +171,9 @@ static void launch_gemm_plain_few(const void* A, long lda, const void* W, long l
 // (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of every wave and each
 // line is asked for by all eight waves: 7.9 us where this form takes 4.3.) What bounds it is the trip to memory
 // with few outputs, the reads of LDS (12 bytes a multiply-add with 32 rows) with many.
-// 8 rows, 128 columns, K = 352 in float32: 34.6 us in the tiles, 4.3 here; relative error 3.3e-7 -> 9.4e-8.
-// Where it runs: wherever the rows allow wide loads. Measured in float32, tiles -> this form: 8 x 6,144 x 4,096 401 -> 23 us,
-// 64 x 4,096 x 14,336 1,644 -> 163 (error 2.1e-6 -> 3.9e-7), 8 x 128,256 x 4,096 1,341 -> 394, 2,048 x 2,048 x 2,048 465 ->
+// 8 rows, 128 columns, K = 352 in float32: 34.6 us in the tiles, 4.3 here; relative error 3.3e-7 -> 1.1e-7.
+// Where it runs: wherever the rows allow wide loads. Measured in float32, tiles -> this form: 8 x 6,144 x 4,096 401 -> 24 us (error 1.15e-6 -> 2.9e-7),
+// 64 x 4,096 x 14,336 1,644 -> 163, 8 x 128,256 x 4,096 1,341 -> 394, 2,048 x 2,048 x 2,048 465 ->
 // 352, 2,048 x 28,672 x 4,096 12.7 -> 9.8 ms (38 -> 49 TFLOP/s; the card's rate without packed instructions is 79). With rows of any alignment
 // up to so many outputs: 512 x 1,001 x 333 38.2 -> 16.4 us, 1,024 rows 39.3 -> 28.7, but 2,048 rows 49.7 -> 52.1.
 #define GP_SPLIT_OUTPUTS (1L << 20)
