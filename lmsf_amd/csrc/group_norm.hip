@@ -116,48 +116,63 @@ template <> struct Na4<bf16_t> {
 };
 
 // The same with the row in registers, for groups of whole 256 columns (or one group) and rows that start on 16-byte
-// boundaries: a thread holds E groups of four neighbours, 64 lanes stand for 256 columns, so a wave's sum belongs to one
-// group and a norm costs one sum over the lanes and one barrier. Everything that comes from memory is asked for in one
-// go. What bounds it with few rows is that trip and the launch (8 rows of 2,048 in 2 groups, branch, stream and output:
-// 8.9 -> 4.9 us), with many rows memory (2,000 such rows 31.0 -> 15.9 us).
-#define GN_SLOTS 64     // 256-column parts of a row: W <= 16,384
+// boundaries, to the bits of the kernel above: what a layer rounds to bfloat16 after a norm must not hang on which of the
+// two ran. There thread c % T of T adds up the squares of columns c, c + T, ... of a group, 64 threads' sums meet in a
+// butterfly, the waves' sums are added in turn. Here a thread stands for four neighbouring threads of that kernel: it
+// holds columns 4 q + j + k T, chains them over k for every j, 16 lanes carry a wave's butterfly (its first four steps
+// between lanes, the last two within a thread), and the waves' sums lie in LDS: a norm costs four steps between lanes and
+// one barrier. Everything that comes from memory is asked for in one go (the weights only before they are needed where a
+// thread holds more than four groups of four). What bounds it with few rows is that trip and the launch, with many rows
+// memory: branch, stream and output of rows of 2,048 in 2 groups, LDS -> here: 8 rows 7.4 -> 3.9 us, 2,000 rows 22.9
+// -> 11.7.
+#define GN_PARTS 256    // sums of 64 threads in a row: W / 64 at most
 
-// the sum of group g's parts, in their order
-__device__ __forceinline__ float gn_group_sum(const float* red, int g, int per_group) {
-  float s = 0.f;
-  for (int k = 0; k < per_group; ++k) s += red[g * per_group + k];
-  return s;
+// keeps a rounded product from being taken into the addition that follows (the row goes through LDS above)
+__device__ __forceinline__ float gn_rounded(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
 }
 
-template <typename TB, typename TO, int E>
-__global__ __launch_bounds__(GN_MAX_THREADS) void group_norm_vec_kernel(
+// A thread holds CHAIN groups of four of each of up to PER groups of columns: of groups slot, slot + at_once, ..., where
+// ``quads`` threads side by side have a group (a multiple of 16).
+template <typename TB, typename TO, int CHAIN, int PER, int THREADS>
+__global__ __launch_bounds__(THREADS) void group_norm_vec_kernel(
     const TB* __restrict__ branch, long branch_stride, const float* __restrict__ wb, float* __restrict__ residual,
     float* __restrict__ hist, long hist_stride, int hist_index, const float* __restrict__ mix,
-    const float* __restrict__ wn, TO* __restrict__ out, long out_stride, const int* __restrict__ rows, int W,
-    int per_group, float gw, float eps_b, float eps_n) {
-  __shared__ float red[2][GN_SLOTS];
+    const float* __restrict__ wn, TO* __restrict__ out, long out_stride, const int* __restrict__ rows, int gw, int groups,
+    int T, int quads, int at_once, float eps_b, float eps_n) {
+  __shared__ __align__(16) float red[2][GN_PARTS];
+  constexpr int E = CHAIN * PER;
+  const int W = gw * groups;
   const long n = blockIdx.x, src = rows ? rows[n] : n;
-  const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE, n_waves = blockDim.x / LMSF_WAVE;
-  float x[E][4], res[E][4], ave[E][4], vb[E][4], vn[E][4];
+  const int slot = threadIdx.x / quads, q4 = (threadIdx.x - slot * quads) * 4;
+  // column of the thread's e-th group of four, or -1
+  auto column = [&](int e) {
+    const int g = slot + e / CHAIN * at_once, c = q4 + e % CHAIN * T;
+    return slot < at_once && g < groups && c < gw ? g * gw + c : -1;
+  };
+  constexpr bool EARLY = E <= 4;
+  float x[E][4], res[E][4], ave[E][4], vb[EARLY ? E : 1][4], vn[EARLY ? E : 1][4];
+  int col[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = (threadIdx.x + e * blockDim.x) * 4;
+    const int i = col[e] = column(e);
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[e][j] = res[e][j] = ave[e][j] = 0.f;
-    if (i < W) {
+    if (i >= 0) {
       if (branch) {
         Na4<TB>::load(branch + n * branch_stride + i, x[e]);
-        Na4<float>::load(wb + i, vb[e]);
+        if (EARLY) Na4<float>::load(wb + i, vb[EARLY ? e : 0]);
       }
       if (residual) Na4<float>::load(residual + src * W + i, res[e]);
-      if (wn) Na4<float>::load(wn + i, vn[e]);
+      if (EARLY && wn) Na4<float>::load(wn + i, vn[EARLY ? e : 0]);
     }
   }
   if (hist) {
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int i = (threadIdx.x + e * blockDim.x) * 4;
-      if (i >= W) continue;
+      const int i = col[e];
+      if (i < 0) continue;
 #pragma unroll 8
       for (int k = 0; k < hist_index; ++k) {
         float h[4];
@@ -167,30 +182,53 @@ __global__ __launch_bounds__(GN_MAX_THREADS) void group_norm_vec_kernel(
       }
     }
   }
-  auto normalize = [&](const float (&w)[E][4], float eps, float* sums) {
+  auto normalize = [&](const float* __restrict__ w, const float (&held)[EARLY ? E : 1][4], float eps, float* sums) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      float s = 0.f;
+    for (int p = 0; p < PER; ++p) {
+      float s[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s += x[e][j] * x[e][j];
-      s = wave_sum(s);
-      if (lane == 0) sums[e * n_waves + wave] = s;      // parts beyond W hold 0
+      for (int k = 0; k < CHAIN; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = fmaf(x[p * CHAIN + k][j], x[p * CHAIN + k][j], s[j]);   // (0 where there is no column)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[j] = gn_rounded(s[j]);
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += __shfl_xor(s[j], o, LMSF_WAVE);
+      if (threadIdx.x % 16 == 0) sums[(p * blockDim.x + threadIdx.x) / 16] = (s[0] + s[2]) + (s[1] + s[3]);
     }
     __syncthreads();
+    float rms = 1.f;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int i = (threadIdx.x + e * blockDim.x) * 4;
-      if (i >= W) continue;
-      const float rms = sqrtf(gn_group_sum(sums, i / 256 / per_group, per_group) / gw + eps);
+      if (e % CHAIN == 0 && slot < at_once && slot + e / CHAIN * at_once < groups) {
+        const float4* part = reinterpret_cast<const float4*>(sums + (e / CHAIN * blockDim.x + slot * quads) / 16);
+        float total = 0.f;
+#pragma unroll 4
+        for (int k = 0; k < (quads + 63) / 64; ++k) {
+          const float4 v = part[k];
+          total = (((total + v.x) + v.y) + v.z) + v.w;
+        }
+        rms = sqrtf(total / (float)gw + eps);
+      }
+      if (col[e] < 0) continue;
+      float v[4];
+      if (EARLY) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[e][j] = x[e][j] / rms * w[e][j];
+        for (int j = 0; j < 4; ++j) v[j] = held[EARLY ? e : 0][j];
+      } else {
+        Na4<float>::load(w + col[e], v);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[e][j] = gn_rounded(x[e][j] / rms * v[j]);
     }
   };
-  if (branch) normalize(vb, eps_b, red[0]);
+  if (branch) normalize(wb, vb, eps_b, red[0]);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int i = (threadIdx.x + e * blockDim.x) * 4;
-    if (i >= W) continue;
+    const int i = col[e];
+    if (i < 0) continue;
     if (residual) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) x[e][j] = res[e][j] + x[e][j];
@@ -204,12 +242,10 @@ __global__ __launch_bounds__(GN_MAX_THREADS) void group_norm_vec_kernel(
     }
   }
   if (out) {
-    if (wn) normalize(vn, eps_n, red[1]);
+    if (wn) normalize(wn, vn, eps_n, red[1]);
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int i = (threadIdx.x + e * blockDim.x) * 4;
-      if (i < W) Na4<TO>::store(out + n * out_stride + i, x[e]);
-    }
+    for (int e = 0; e < E; ++e)
+      if (col[e] >= 0) Na4<TO>::store(out + n * out_stride + col[e], x[e]);
   }
 }
 
@@ -218,27 +254,31 @@ static void gn_launch(int n_rows, size_t smem, hipStream_t stream, const void* b
                       const float* wb, float* residual, float* hist, long hist_stride, int hist_index,
                       const float* mix, const float* wn, void* out, long out_stride, const int* rows, int W,
                       int groups, float eps_b, float eps_n) {
-  const int gw = W / groups;
-  const bool vec = W % 4 == 0 && (groups == 1 || gw % 256 == 0) && W <= 256 * GN_SLOTS && branch_stride % 4 == 0 &&
-                   out_stride % 4 == 0 && hist_stride % 4 == 0 && lmsf_aligned16(branch) && lmsf_aligned16(wb) &&
-                   lmsf_aligned16(residual) && lmsf_aligned16(hist) && lmsf_aligned16(wn) && lmsf_aligned16(out);
-  if (vec) {
-    // few rows: as many threads as a row has groups of four; many rows: smaller workgroups with several each
-    const int quads = W / 4, per_thread = n_rows >= 512 ? 2 : 1;
-    int threads = 64;
-    while (threads < GN_MAX_THREADS && threads * per_thread < quads) threads *= 2;
-    const int need = (quads + threads - 1) / threads, per_group = (gw + 255) / 256;
-#define GN_VEC(E_)                                                                                                     \
-  hipLaunchKernelGGL((group_norm_vec_kernel<TB, TO, E_>), dim3(n_rows), dim3(threads), 0, stream, (const TB*)branch,   \
-                     branch_stride, wb, residual, hist, hist_stride, hist_index, mix, wn, (TO*)out, out_stride, rows,  \
-                     W, per_group, (float)gw, eps_b, eps_n)
-    if (need <= 1) GN_VEC(1); else if (need <= 2) GN_VEC(2); else GN_VEC(4);
-#undef GN_VEC
-    return;
-  }
   // few rows: a row's passes wait for memory one after the other, so many threads with few elements each; many
   // rows fill the chip with smaller workgroups
   const int threads = n_rows >= 1024 || W <= 256 ? 256 : W <= 1024 ? 512 : 1024;
+  const int gw = W / groups;
+  // (a thread with more than four groups of four reads its weights late: the norm of a branch alone, which has nothing
+  // else to ask for, then takes 3 to 9 % longer than in LDS with up to 1,024 rows of one group)
+  const bool late = gw > 4 * threads && !residual && (groups == 1 || n_rows < 1024);
+  if (!late && W % 4 == 0 && (groups == 1 || gw % 256 == 0) && branch_stride % 4 == 0 && out_stride % 4 == 0 &&
+      hist_stride % 4 == 0 && lmsf_aligned16(branch) && lmsf_aligned16(wb) && lmsf_aligned16(residual) &&
+      lmsf_aligned16(hist) && lmsf_aligned16(wn) && lmsf_aligned16(out)) {
+    // (16 lanes for every 64 threads of the other kernel that have a column of a group)
+    const int quads = (min(gw, threads) + 63) / 64 * 16, chain = (gw + threads - 1) / threads;
+    const int at_once = min(groups, GN_MAX_THREADS / quads), block = (at_once * quads + 63) / 64 * 64;
+    const int per = (groups + at_once - 1) / at_once;
+#define GN_VEC(CHAIN_, PER_, THREADS_)                                                                                 \
+  if (chain <= CHAIN_ && per <= PER_ && block <= THREADS_) {                                                           \
+    hipLaunchKernelGGL((group_norm_vec_kernel<TB, TO, CHAIN_, PER_, THREADS_>), dim3(n_rows), dim3(block), 0, stream,  \
+                       (const TB*)branch, branch_stride, wb, residual, hist, hist_stride, hist_index, mix, wn,         \
+                       (TO*)out, out_stride, rows, gw, groups, threads, quads, at_once, eps_b, eps_n);                 \
+    return;                                                                                                            \
+  }
+    GN_VEC(1, 1, 1024) GN_VEC(2, 1, 1024) GN_VEC(4, 1, 1024) GN_VEC(8, 1, 512) GN_VEC(16, 1, 256)
+    GN_VEC(1, 2, 1024) GN_VEC(2, 2, 1024) GN_VEC(1, 4, 1024)
+#undef GN_VEC
+  }
   hipLaunchKernelGGL((group_norm_kernel<TB, TO>), dim3(n_rows), dim3(threads), smem, stream, (const TB*)branch,
                      branch_stride, wb, residual, hist, hist_stride, hist_index, mix, wn, (TO*)out, out_stride, rows,
                      W, groups, eps_b, eps_n);

@@ -66,3 +66,28 @@ def test_group_norm(ops, W, groups, rows, dtype, form):
         grow = gn(scale, wb.double().abs(), groups, eps) * (scale.view(rows, groups, -1).pow(2).mean(-1) /
                                                             mixed.view(rows, groups, -1).pow(2).mean(-1)).sqrt().amax(-1, keepdim=True)
         assert ((out.double() - want).abs() <= 4e-6 * (1 + grow) + rel * want.abs()).all()
+
+
+# rows below and from 1,024 on (other numbers of threads), one to sixteen groups of four a thread, several groups a thread
+@pytest.mark.parametrize("W,groups", [(4, 1), (252, 1), (260, 1), (512, 2), (768, 3), (1024, 1), (1020, 1), (2048, 2), (2048, 1),
+                                      (2048, 8), (3072, 3), (4096, 1), (4100, 1), (8192, 1), (8192, 8), (13312, 52), (13312, 4),
+                                      (12800, 5), (13632, 1)])
+@pytest.mark.parametrize("rows", [1, 9, 1024])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_same_bits_in_registers_and_in_lds(ops, W, groups, rows, dtype):
+    """Weights off a 16-byte boundary keep the row in LDS; the results are the same bits either way."""
+    g = torch.Generator(device="cuda:0").manual_seed(W + rows)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda:0")      # noqa: E731
+    x, res, hist, mix = r(rows, W).to(dtype), r(rows, W), r(4, rows, W), r(4)
+    wa, wb = r(W), r(W)
+    off = lambda t: torch.empty(t.numel() + 1, device="cuda:0")[1:].copy_(t)      # noqa: E731
+
+    def run(a, b):
+        args = dict(groups=groups, x_eps=1e-5, out_eps=1e-6, out_dtype=dtype)
+        out = [ops.group_norm(x=x, x_weight=a, **args), ops.group_norm(residual=res.clone(), out_weight=b, **args)]
+        for more in ({}, dict(history=hist.clone(), index=3, mix=mix)):
+            s = res.clone()
+            out += [ops.group_norm(x=x, x_weight=a, residual=s, out_weight=b, **args, **more), s, more.get("history", s)]
+        return out
+    for got, want in zip(run(wa, wb), run(off(wa), off(wb))):
+        assert torch.equal(got, want)
