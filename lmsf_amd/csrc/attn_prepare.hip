@@ -298,13 +298,16 @@ __global__ __launch_bounds__(256) void rms_pair_kernel(const T* __restrict__ a, 
 }
 
 // The same with both rows in registers, E pieces of 16 bytes a thread, where the rows allow such loads: everything is asked
-// for at once, both sums cross the workgroup together (8 rows of 2,048 7.4 -> 2.9 us).
+// for at once, both sums cross the workgroup together. The rows also go through LDS, from which thread t adds up the squares
+// of entries t, t + 256, ... as the kernel above does, so that both give the same bits (8
+// rows of 2,048 4.7 -> 2.9 us, 2,048 rows 8.5 -> 6.6).
 template <typename T, int E>
 __global__ __launch_bounds__(256) void rms_pair_vec_kernel(const T* __restrict__ a, long a_stride, const T* __restrict__ b,
                                                            long b_stride, const float* __restrict__ wa,
                                                            const float* __restrict__ wb, T* __restrict__ out, int W,
                                                            float eps, float scale) {
   constexpr int V = Vec16<T>::N;
+  __shared__ __align__(16) T row[2][E * 256 * V];
   __shared__ float red[2][4];
   const long n = blockIdx.x;
   const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE;
@@ -324,15 +327,20 @@ __global__ __launch_bounds__(256) void rms_pair_vec_kernel(const T* __restrict__
     }
   }
 #pragma unroll
-  for (int e = 0; e < E; ++e)
-    if ((e * 256 + threadIdx.x) * V < W) {
-#pragma unroll
-      for (int j = 0; j < V; ++j) {
-        const float x = va[e].get(j), y = vb[e].get(j);
-        sa += x * x;
-        sb += y * y;
-      }
+  for (int e = 0; e < E; ++e) {
+    const int i = (e * 256 + threadIdx.x) * V;
+    if (i < W) {
+      va[e].store(row[0] + i);
+      vb[e].store(row[1] + i);
     }
+  }
+  __syncthreads();
+#pragma unroll 8
+  for (int i = threadIdx.x; i < W; i += 256) {
+    const float x = to_f32<T>(row[0][i]), y = to_f32<T>(row[1][i]);
+    sa += x * x;
+    sb += y * y;
+  }
   sa = wave_sum(sa);
   sb = wave_sum(sb);
   if (lane == 0) {
@@ -340,8 +348,8 @@ __global__ __launch_bounds__(256) void rms_pair_vec_kernel(const T* __restrict__
     red[1][wave] = sb;
   }
   __syncthreads();
-  sa = red[0][0] + red[0][1] + red[0][2] + red[0][3];
-  sb = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+  sa = ((red[0][0] + red[0][1]) + red[0][2]) + red[0][3];
+  sb = ((red[1][0] + red[1][1]) + red[1][2]) + red[1][3];
   const float ia = 1.f / sqrtf(sa / (float)W + eps), ib = 1.f / sqrtf(sb / (float)W + eps);
 #pragma unroll
   for (int e = 0; e < E; ++e) {

@@ -77,3 +77,13 @@ def test_selective_scan_state_on_and_off_the_boundary(ops, n, lens):
         return y, state[:, :inner * n].clone()
     (ya, sa), (yb, sb) = run(inner * n), run(inner * n + 1)       # (the second one's rows start off 16-byte boundaries)
     assert torch.equal(ya, yb) and torch.equal(sa, sb) and not torch.equal(sa, first)
+
+
+@pytest.mark.parametrize("W", [8, 12, 248, 2048, 2056, 4096, 8192])
+@pytest.mark.parametrize("N", [1, 300])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rms_pair_on_and_off_the_boundary(ops, W, N, dtype):
+    g = torch.Generator().manual_seed(W + N)
+    a, b = (torch.randn(N, W, generator=g).to(dtype).to("cuda:0") for _ in range(2))
+    wa, wb = (torch.randn(W, generator=g).to("cuda:0") for _ in range(2))
+    assert torch.equal(ops.rms_pair(a, b, wa, wb, 1e-5, 0.5), ops.rms_pair(a, b, off(wa), wb, 1e-5, 0.5))
