@@ -108,6 +108,15 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_gate_up_kernel(
   }
 }
 
+// total + f v for output o: rounded once, and for every fourth output with the product rounded first, so that the two
+// kernels that add up a token's experts give the same bits (left to itself the compiler shares one addition between the
+// kinds of experts for the last output that a wave owns, which is not the same one in both).
+__device__ __forceinline__ float moe_add(float total, float f, float v, int o) {
+  float p = f * v;
+  asm volatile("" : "+v"(p));
+  return (o & 3) == 3 ? total + p : fmaf(f, v, total);
+}
+
 // out[n, o] = base[n, o] + weight * sum_k Wd_{e_k}[o] . act[n * top + k]
 template <typename T>
 __global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
@@ -135,12 +144,13 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
     if (e >= E) {      // an expert without matrices returns its input
       const float f = os * (pair_scale ? pair_scale[(long)n * top + k] : 1.f);
 #pragma unroll
-      for (int r = 0; r < MOE_OUT_PER_WAVE; ++r) total[r] += f * to_f32<T>(h[(long)n * h_stride + o0 + min(r, valid - 1)]);
+      for (int r = 0; r < MOE_OUT_PER_WAVE; ++r)
+        total[r] = moe_add(total[r], f, to_f32<T>(h[(long)n * h_stride + o0 + min(r, valid - 1)]), o0 + r);
       continue;
     }
     moe_rows_dot<T, MOE_OUT_PER_WAVE>(Wd + ((long)e * W + o0) * F, F, valid, sa + k * F, F, lane, vec, part);
 #pragma unroll
-    for (int r = 0; r < MOE_OUT_PER_WAVE; ++r) total[r] += os * part[r];
+    for (int r = 0; r < MOE_OUT_PER_WAVE; ++r) total[r] = moe_add(total[r], os, part[r], o0 + r);
   }
   if (lane < valid) {
     float mine = 0.f;
@@ -296,7 +306,8 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_few_kernel(
     if (e >= E) {      // an expert without matrices returns its input
       const float f = os * (pair_scale ? pair_scale[(long)n * top + k] : 1.f);
 #pragma unroll
-      for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] += f * to_f32<T>(h[(long)n * h_stride + o0 + min(r, valid - 1)]);
+      for (int r = 0; r < MOE_FEW_OUT; ++r)
+        total[r] = moe_add(total[r], f, to_f32<T>(h[(long)n * h_stride + o0 + min(r, valid - 1)]), o0 + r);
       continue;
     }
     const T* w[MOE_FEW_OUT];
@@ -310,7 +321,7 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_few_kernel(
     }
     moe_few_dot<T, MOE_FEW_OUT, 1>(w, x, one, 1, F, lane, a);
 #pragma unroll
-    for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] += os * wave_sum(a[0][r]);
+    for (int r = 0; r < MOE_FEW_OUT; ++r) total[r] = moe_add(total[r], os, wave_sum(a[0][r]), o0 + r);
   }
   if (lane < valid) {
     if (base_scale) b *= base_scale[n];

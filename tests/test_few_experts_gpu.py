@@ -67,3 +67,19 @@ def test_experts_of_few_tokens(ops, N, top, E, W, F, dtype, form):
     # the other way, and the result's own rounding
     tol = 1e-4 if dtype == torch.float32 else 6e-2
     assert ((got.double() - want).abs() <= tol * (1 + want.abs())).all()
+
+
+@pytest.mark.parametrize("W,F", [(8, 8), (520, 264), (2048, 1024)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_scaled_results_of_experts_have_the_same_bits(ops, W, F, dtype):
+    """Factors on what experts return, experts without matrices among them: rows on and off a 16-byte boundary."""
+    g = torch.Generator().manual_seed(W)
+    N, top, E = 9, 3, 4
+    r = lambda *s: torch.randn(*s, generator=g).to("cuda:0")     # noqa: E731
+    gu, dn = (r(E, 2 * F, W) * W ** -0.5).to(dtype), (r(E, W, F) * F ** -0.5).to(dtype)
+    h, scale = r(N, W).to(dtype), r(N, top).abs()
+    table = torch.randint(0, E + 2, (N, top), generator=g, dtype=torch.int32).to("cuda:0")
+    off = torch.empty(N * (W + 16) + 1, dtype=dtype, device="cuda:0")[1:].view(N, W + 16)[:, :W]
+    off.copy_(h)
+    args = dict(out_scale=scale, limit=3.0, identity=2)
+    assert torch.equal(ops.table_moe(h, gu, dn, None, table, 0.5, **args), ops.table_moe(off, gu, dn, None, table, 0.5, **args))
