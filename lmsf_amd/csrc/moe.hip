@@ -165,18 +165,25 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
 
 // ---------------------------------------------------------------- few tokens, rows that allow 16-byte loads
 //
-// The same two products with everything that comes from memory asked for in one go, and an expert that several pairs
-// have chosen read once for all of them. A wave reads its rows of the matrix and the same entries of the vectors
-// (which the caches hold) with 16-byte loads, MOE_AHEAD pieces of 512 or 256 entries of each row on their way at a time;
-// nothing goes through LDS and no wave waits for another. Every output is added up in the order of the kernels above.
-// The outputs vary fastest over the workgroups, so that an expert's rows are read by all eight dies (with the pairs
-// fastest, a pair's whole expert falls to one die: gate and up 26.5 us). What bounds them is memory and, for an expert
-// of several pairs, the multiply-adds of a wave (8 tokens, 2 of 16 experts of 2,048 -> 2 x 1,024 -> 2,048 a token: gate
-// and up 24.4 -> 21.2 us, down 15.1 -> 11.6; 4 pieces ahead, 2 pairs a read, 1 or 4 outputs a wave: 23.4 to 28.4 us).
+// The same two products with everything that comes from memory asked for in one go, and a read of an expert's rows
+// shared by up to MOE_SHARED_PAIRS of the pairs that have chosen it (where more have, other workgroups take the next ones
+// side by side). A wave reads its rows of the matrix and the same entries of the vectors (which the caches hold) with
+// 16-byte loads, MOE_AHEAD pieces of 512 or 256 entries of each row on their way at a time; nothing goes through LDS and
+// no wave waits for another. Every output is added up in the order of the kernels above. The outputs vary fastest over the
+// workgroups, so that an expert's rows are read by all eight dies (with the pairs fastest, a pair's whole expert falls to
+// one die: gate and up 26.5 us). What bounds them is memory and, for an expert of several pairs, the multiply-adds of a
+// wave. Both products of 2,048 -> 2 x 1,024 -> 2,048 in bfloat16, kernels above -> these: 8 tokens with 2 of 16 experts
+// each 38.6 -> 27.6 us, 31 tokens with one expert 40.1 -> 27.0 (in float32 45.5 -> 35.4, and 69.7 with one workgroup taking
+// all of an expert's pairs in turn); 4 pieces ahead, 2 pairs a read, 1 or 4 outputs a wave: up to a third slower.
 #define MOE_AHEAD 2
 #define MOE_FEW_PAIRS 64      // a lane each
 #define MOE_SHARED_PAIRS 4    // pairs of one expert that share a read of its rows
 #define MOE_FEW_OUT 2         // outputs a wave owns
+// Smaller experts stay with the kernels above, which share a vector between a workgroup's waves: what counts there is the
+// way from a wave's first load to its last sum (2 x 512 x 256 entries, 30 pairs of two experts from memory: 10.6 -> 12.6
+// us here; 2 x 1,024 x 512 level to 1.14 times as long with all pairs on one expert, 0.75 times with the pairs spread;
+// from 2 x 1,536 x 512 on nothing is slower).
+#define MOE_FEW_ENTRIES (3L << 18)
 
 // a[q][r] += sum over this lane's entries of rows r against the vectors of the pairs, each times its scale
 template <typename T, int ROWS, int PAIRS>
@@ -232,8 +239,11 @@ __global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
   }
   const int e = __shfl(mine, blockIdx.y, LMSF_WAVE);
   if (e >= E) return;             // (what an expert without matrices returns is its input: the kernel below)
+  // of an expert's pairs every MOE_SHARED_PAIRS-th stands for itself and the ones up to the next such pair
   unsigned long long pairs = __ballot(mine == e);
-  if (__ffsll(pairs) - 1 != (int)blockIdx.y) return;     // the first pair of an expert stands for all of them
+  const unsigned long long before = pairs & ((1ull << blockIdx.y) - 1);
+  if (__popcll(before) % MOE_SHARED_PAIRS) return;
+  pairs ^= before;
   const T* We = Wgu + (long)e * (gated ? 2 : 1) * F * W;
   const int valid = min(MOE_FEW_OUT, F - f0);
   const T* w[2 * MOE_FEW_OUT];
@@ -242,42 +252,40 @@ __global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
     w[r] = We + (long)(f0 + min(r, valid - 1)) * W;
     w[MOE_FEW_OUT + r] = gated ? w[r] + (long)F * W : w[r];
   }
-  while (pairs) {
-    const T* x[MOE_SHARED_PAIRS];
-    float scale[MOE_SHARED_PAIRS], a[MOE_SHARED_PAIRS][2 * MOE_FEW_OUT];
-    int pair[MOE_SHARED_PAIRS], count = 0;
+  const T* x[MOE_SHARED_PAIRS];
+  float scale[MOE_SHARED_PAIRS], a[MOE_SHARED_PAIRS][2 * MOE_FEW_OUT];
+  int pair[MOE_SHARED_PAIRS], count = 0;
 #pragma unroll
-    for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
-      pair[q] = 0;
-      if (pairs) {
-        pair[q] = __ffsll(pairs) - 1;
-        pairs &= pairs - 1;
-        ++count;
-      }
-      x[q] = h + (long)(pair[q] / top) * h_stride;
-      scale[q] = pair_scale ? pair_scale[pair[q]] : 1.f;
-#pragma unroll
-      for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = 0.f;
+  for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
+    pair[q] = 0;
+    if (pairs) {
+      pair[q] = __ffsll(pairs) - 1;
+      pairs &= pairs - 1;
+      ++count;
     }
-    moe_few_dot<T, 2 * MOE_FEW_OUT, MOE_SHARED_PAIRS>(w, x, scale, count, W, lane, a);
+    x[q] = h + (long)(pair[q] / top) * h_stride;
+    scale[q] = pair_scale ? pair_scale[pair[q]] : 1.f;
 #pragma unroll
-    for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
-      if (q >= count) break;
+    for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = 0.f;
+  }
+  moe_few_dot<T, 2 * MOE_FEW_OUT, MOE_SHARED_PAIRS>(w, x, scale, count, W, lane, a);
 #pragma unroll
-      for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = wave_sum(a[q][r]);
-      if (lane < valid) {
-        // the products are rounded as stored activations are, then the activation in float32
-        const float gg = to_f32<T>(from_f32<T>(lane == 0 ? a[q][0] : a[q][1]));
-        const float uu = to_f32<T>(from_f32<T>(lane == 0 ? a[q][MOE_FEW_OUT] : a[q][MOE_FEW_OUT + 1]));
-        float y;
-        if (!gated) {
-          const float up = fmaxf(gg, 0.f);      // one matrix an expert: relu(W_up h)^2
-          y = up * up;
-        } else {
-          y = limit > 0.f ? bounded_gate(gg, uu, limit) : gg / (1.f + expf(-gg)) * uu;
-        }
-        act[(long)pair[q] * F + f0 + lane] = from_f32<T>(y);
+  for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
+    if (q >= count) break;
+#pragma unroll
+    for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = wave_sum(a[q][r]);
+    if (lane < valid) {
+      // the products are rounded as stored activations are, then the activation in float32
+      const float gg = to_f32<T>(from_f32<T>(lane == 0 ? a[q][0] : a[q][1]));
+      const float uu = to_f32<T>(from_f32<T>(lane == 0 ? a[q][MOE_FEW_OUT] : a[q][MOE_FEW_OUT + 1]));
+      float y;
+      if (!gated) {
+        const float up = fmaxf(gg, 0.f);      // one matrix an expert: relu(W_up h)^2
+        y = up * up;
+      } else {
+        y = limit > 0.f ? bounded_gate(gg, uu, limit) : gg / (1.f + expf(-gg)) * uu;
       }
+      act[(long)pair[q] * F + f0 + lane] = from_f32<T>(y);
     }
   }
 }
@@ -617,7 +625,7 @@ extern "C" int lmsf_table_moe_act(const void* h, int dtype, long h_stride, const
     return 0;
   }
   const int es16 = 16 / lmsf_elem_size(dtype);
-  if ((long)n_tokens * top <= MOE_FEW_PAIRS && W % es16 == 0 && F % es16 == 0 && h_stride % es16 == 0 && lmsf_aligned16(h) &&
+  if ((long)n_tokens * top <= MOE_FEW_PAIRS && (long)W * F >= MOE_FEW_ENTRIES && W % es16 == 0 && F % es16 == 0 && h_stride % es16 == 0 && lmsf_aligned16(h) &&
       lmsf_aligned16(Wgu) && lmsf_aligned16(Wd) && lmsf_aligned16(act)) {
     const int outs = MOE_WAVES * MOE_FEW_OUT, P = n_tokens * top;
     const dim3 f1((F + outs - 1) / outs, P), f2((W + outs - 1) / outs, n_tokens);

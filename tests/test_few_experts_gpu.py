@@ -69,7 +69,7 @@ def test_experts_of_few_tokens(ops, N, top, E, W, F, dtype, form):
     assert ((got.double() - want).abs() <= tol * (1 + want.abs())).all()
 
 
-@pytest.mark.parametrize("W,F", [(8, 8), (520, 264), (2048, 1024)])
+@pytest.mark.parametrize("W,F", [(8, 8), (520, 264), (2048, 1024), (392, 2056)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_scaled_results_of_experts_have_the_same_bits(ops, W, F, dtype):
     """Factors on what experts return, experts without matrices among them: rows on and off a 16-byte boundary."""
@@ -83,3 +83,12 @@ def test_scaled_results_of_experts_have_the_same_bits(ops, W, F, dtype):
     off.copy_(h)
     args = dict(out_scale=scale, limit=3.0, identity=2)
     assert torch.equal(ops.table_moe(h, gu, dn, None, table, 0.5, **args), ops.table_moe(off, gu, dn, None, table, 0.5, **args))
+
+
+# experts on both sides of the line to those whose rows are shared (786,432 entries), odd pieces of rows
+@pytest.mark.parametrize("N,top,E", [(1, 1, 1), (9, 1, 1), (15, 2, 3), (31, 1, 2), (64, 1, 5)])
+@pytest.mark.parametrize("W,F", [(1024, 760), (1024, 768), (1032, 776), (392, 2056), (2056, 392)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("form", ["table", "router", "one matrix", "bounded"])
+def test_experts_about_the_line_to_shared_rows(ops, N, top, E, W, F, dtype, form):
+    test_experts_of_few_tokens(ops, N, top, E, W, F, dtype, form)
