@@ -287,11 +287,13 @@ static void launch_gemm_plain(const void* A, long lda, const void* W, long ldw, 
   dim3 grid((N + GP_TILE - 1) / GP_TILE, (M + GP_TILE - 1) / GP_TILE), block(256);
   const bool wide = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (size_t)A % (4 * sizeof(TA)) == 0 &&
                     (size_t)W % (4 * sizeof(TW)) == 0;
-  if (wide) {
+  // (the split form has a row of workgroups per 32 rows, the tiles per 64: beyond what a grid takes of the former, tiles)
+  const bool fits = (M + 31) / 32 <= 65535;
+  if (fits && wide) {
     launch_gemm_plain_split<TA, TW, TO, true>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
     return;
   }
-  if ((long)M * N <= GP_SPLIT_OUTPUTS) {
+  if (fits && (long)M * N <= GP_SPLIT_OUTPUTS) {
     launch_gemm_plain_split<TA, TW, TO, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
     return;
   }

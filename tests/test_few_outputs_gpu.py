@@ -45,6 +45,16 @@ def test_product_of_few_outputs(ops, M, N, K, types, shift):
     assert ((y - exact).abs() <= bound + 1e-30).all()
 
 
+# as many rows as the grid of the split form takes (32 a workgroup), and one more
+@pytest.mark.parametrize("M", [65535 * 32, 65535 * 32 + 1])
+def test_product_of_very_many_rows(ops, M):
+    g = torch.Generator(device="cuda:0").manual_seed(M)
+    x, w = torch.randn(M, 4, generator=g, device="cuda:0"), torch.randn(3, 4, generator=g, device="cuda:0")
+    exact = x.double() @ w.double().T
+    # four products and their sums in float32
+    assert ((ops.linear(x, w).double() - exact).abs() <= 5 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
+
+
 # keys just below, at and beyond eight a group (256 / d groups), a second round of 256 keys, pages of odd sizes
 @pytest.mark.parametrize("d,ps", [(32, 16), (4, 3), (96, 16), (256, 8), (260, 16)])
 @pytest.mark.parametrize("context", [1, 7, 8, 63, 64, 65, 256, 257, 300])
