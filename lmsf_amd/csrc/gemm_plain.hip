@@ -2,55 +2,94 @@
 //
 // This is the true 32-bit matrix product of the float32 path (no matrix-core instruction, no
 // reduced-precision input mode), and the fallback of the bfloat16 path for shapes the fast kernels
-// refuse. Inputs may be float32 or bfloat16; products and sums are float32, added over k in a fixed order. The reference calls cuBLASLt with float32 compute
+// refuse. Inputs may be float32 or bfloat16; products and sums are float32. The reference calls cuBLASLt with float32 compute
 // (tops/csrc/tops/tensorrt_llm/common/cublasMMWrapper.cpp:182-210) and adds the bias afterwards
 // (core/src/model_executor/layers/linear.rs:101-104).
 //
-// K split over the waves of a workgroup (further down), or, for many outputs whose rows do not allow wide loads, a 64x64
-// tile per workgroup of 256 threads, 4x4 outputs per thread, K in slabs of 16 staged through LDS. Any M, N, K; rows may be strided (lda, ldw, ldc in elements).
+// Two forms: K split over the waves of a workgroup (further down), or a 64x64 tile per workgroup of 256 threads, 4x4
+// outputs per thread, K in slabs of 16 staged through LDS. Both add up an output in one order, so that which of them runs,
+// and with it the number of rows multiplied together, changes no bit: the ceil(K / 32) steps of 32 k are cut into eight
+// consecutive parts (gp_part), the even and the odd k of a part are two chains of fused multiply-adds, and the parts' sums
+// (even + odd) are added in turn. Any M, N, K; rows may be strided (lda, ldw, ldc in elements).
 #include "common.h"
 
 #define GP_TILE 64
 #define GP_BK 16
+#define GP_STEP 32      // k of a step
+#define GP_PARTS 8
 
+// the first k of part p
+__device__ __forceinline__ int gp_part(int p, int K) {
+  const long steps = (K + GP_STEP - 1) / GP_STEP;
+  return (int)(p * steps / GP_PARTS) * GP_STEP;
+}
+
+// The tiles. Up to K the four entries that a thread reads of a row carry no test; with one for every entry, rows outside the
+// matrix included, the tests took half of the time (2,048 x 2,048 x 512 in float32 123 us, now 68).
 template <typename TA, typename TW, typename TO>
 __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ A, long lda, const TW* __restrict__ W,
                                                          long ldw, const TW* __restrict__ bias, TO* __restrict__ C,
                                                          long ldc, int M, int N, int K) {
-  __shared__ float As[GP_BK][GP_TILE + 4];
-  __shared__ float Ws[GP_BK][GP_TILE + 4];
+  __shared__ __align__(16) float As[GP_BK][GP_TILE + 4];
+  __shared__ __align__(16) float Ws[GP_BK][GP_TILE + 4];
   const int tid = threadIdx.x;
   const int tx = tid % 16, ty = tid / 16;
   const int m0 = blockIdx.y * GP_TILE, n0 = blockIdx.x * GP_TILE;
   const int lrow = tid / 4, lk = (tid % 4) * 4;
-  float acc[4][4];
+  const TA* arow = A + (long)min(m0 + lrow, M - 1) * lda + lk;    // rows beyond the matrix repeat the last: not written
+  const TW* wrow = W + (long)min(n0 + lrow, N - 1) * ldw + lk;
+  float sum[4][4], acc[4][4][2];      // the parts so far; the even and the odd k of the present one
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int j = 0; j < 4; ++j) sum[i][j] = acc[i][j][0] = acc[i][j][1] = 0.f;
 
-  for (int k0 = 0; k0 < K; k0 += GP_BK) {
-    const int gm = m0 + lrow, gn = n0 + lrow;
+  for (int p = 0; p < GP_PARTS; ++p) {
+    const int end = min(gp_part(p + 1, K), K);
+    for (int k0 = gp_part(p, K); k0 < end; k0 += GP_BK) {
+      float av[4], wv[4];
+      if (k0 + GP_BK <= K) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int k = k0 + lk + e;
-      As[lk + e][lrow] = (gm < M && k < K) ? to_f32<TA>(A[(long)gm * lda + k]) : 0.f;
-      Ws[lk + e][lrow] = (gn < N && k < K) ? to_f32<TW>(W[(long)gn * ldw + k]) : 0.f;
+        for (int e = 0; e < 4; ++e) {
+          av[e] = to_f32<TA>(arow[k0 + e]);
+          wv[e] = to_f32<TW>(wrow[k0 + e]);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          av[e] = k0 + lk + e < K ? to_f32<TA>(arow[k0 + e]) : 0.f;
+          wv[e] = k0 + lk + e < K ? to_f32<TW>(wrow[k0 + e]) : 0.f;
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        As[lk + e][lrow] = av[e];
+        Ws[lk + e][lrow] = wv[e];
+      }
+      __syncthreads();
+      float a[2][4], w[2][4];      // the next k's operands are read while the present one's are multiplied
+      auto read = [&](int kk) {
+        *reinterpret_cast<float4*>(a[kk & 1]) = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
+        *reinterpret_cast<float4*>(w[kk & 1]) = *reinterpret_cast<const float4*>(&Ws[kk][tx * 4]);
+      };
+      read(0);
+#pragma unroll
+      for (int kk = 0; kk < GP_BK; ++kk) {
+        if (kk + 1 < GP_BK) read(kk + 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j][kk & 1] = fmaf(a[kk & 1][i], w[kk & 1][j], acc[i][j][kk & 1]);
+      }
+      __syncthreads();
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < GP_BK; ++kk) {
-      float a[4], w[4];
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) w[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
-    }
-    __syncthreads();
+      for (int j = 0; j < 4; ++j) {
+        sum[i][j] += acc[i][j][0] + acc[i][j][1];
+        acc[i][j][0] = acc[i][j][1] = 0.f;
+      }
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -60,7 +99,7 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
     for (int j = 0; j < 4; ++j) {
       const int gn = n0 + tx * 4 + j;
       if (gn >= N) continue;
-      float r = acc[i][j];
+      float r = sum[i][j];
       if (bias) r += to_f32<TW>(bias[gn]);
       C[(long)gm * ldc + gn] = from_f32<TO>(r);
     }
@@ -163,21 +202,14 @@ static void launch_gemm_plain_few(const void* A, long lda, const void* W, long l
 }
 
 // The product with K split over the waves of a workgroup.
-// A workgroup of eight waves owns 8 MR rows by 16 columns; wave w takes the steps of 32 k w, w + 8, w + 16, ... A step's
-// rows are read whole cache lines at a time (lane (r, c) = (l / 8, l % 8) reads four entries c of rows r, r + 8, ...), the
-// next step's while this one is multiplied, and go through an area of LDS that belongs to the wave, from which lane (r, c)
-// takes rows r, r + 8, ... and columns c, c + 8 for the outputs it holds: no barrier inside the loop. The waves' sums
-// are added in wave order at the end: a fixed order, and shorter chains of additions than the tile's single one.
-// (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of every wave and each
-// line is asked for by all eight waves: 7.9 us where this form takes 4.3.) What bounds it is the trip to memory
-// with few outputs, the reads of LDS (12 bytes a multiply-add with 32 rows) with many.
-// 8 rows, 128 columns, K = 352 in float32: 34.6 us in the tiles, 4.3 here; relative error 3.3e-7 -> 1.1e-7.
-// Where it runs: wherever the rows allow wide loads. Measured in float32, tiles -> this form: 8 x 6,144 x 4,096 401 -> 24 us (error 1.15e-6 -> 2.9e-7),
-// 64 x 4,096 x 14,336 1,644 -> 163, 8 x 128,256 x 4,096 1,341 -> 394, 2,048 x 2,048 x 2,048 465 ->
-// 352, 2,048 x 28,672 x 4,096 12.7 -> 9.8 ms (38 -> 49 TFLOP/s; the card's rate without packed instructions is 79). With rows of any alignment
-// up to so many outputs: 512 x 1,001 x 333 38.2 -> 16.4 us, 1,024 rows 39.3 -> 28.7, but 2,048 rows 49.7 -> 52.1.
+// A workgroup of eight waves owns 8 MR rows by 16 columns; wave w takes part w of K, step by step. A step's rows are read
+// whole cache lines at a time (lane (r, c) = (l / 8, l % 8) reads four entries c of rows r, r + 8, ...), the next step's
+// while this one is multiplied, and go through an area of LDS that belongs to the wave, from which lane (r, c) takes rows
+// r, r + 8, ... and columns c, c + 8 for the outputs it holds: no barrier inside the loop. The waves' sums are added in
+// wave order at the end. (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of
+// every wave and each line is asked for by all eight waves: 7.9 us where this form took 4.3.) What bounds it is the trip
+// to memory with few outputs; with many the tiles are ahead.
 #define GP_SPLIT_OUTPUTS (1L << 20)
-#define GP_STEP 32
 #define GP_ROW (GP_STEP + 4)      // floats a row takes in LDS: eight rows at a time lie on distinct banks
 
 // four neighbouring entries; VEC: in one load (K is a multiple of 4 then), else one by one, those from K on as zeros
@@ -198,14 +230,14 @@ __device__ __forceinline__ float4 gp_load4(const bf16_t* p, int k, int K) {
 }
 
 template <typename TA, typename TW, typename TO, int MR, bool VEC>
-__global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restrict__ A, long lda,
+__global__ __launch_bounds__(512, 4) void gemm_plain_split_kernel(const TA* __restrict__ A, long lda,
                                                                const TW* __restrict__ W, long ldw,
                                                                const TW* __restrict__ bias, TO* __restrict__ C,
                                                                long ldc, int M, int N, int K) {
   constexpr int ROWS = 8 * MR + 16;                 // of A, then of W
   static_assert(ROWS * GP_ROW >= MR * 128, "the waves' sums lie where their steps lay");
   __shared__ __align__(16) float area[8][ROWS * GP_ROW];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r = lane >> 3, c = lane & 7;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane >> 3, c = lane & 7;
   const int m0 = blockIdx.y * (8 * MR), n0 = blockIdx.x * 16;
   float* mine = area[wave];
   const TA* a[MR];
@@ -226,14 +258,15 @@ __global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restr
 #pragma unroll
     for (int j = 0; j < 2; ++j) y[j] = gp_load4<VEC>(w[j], k0 + 4 * c, K);
   };
-  int k0 = wave * GP_STEP;
-  if (k0 < K) fetch(k0);
-  for (; k0 < K; k0 += 8 * GP_STEP) {
+  int k0 = gp_part(wave, K);
+  const int end = min(gp_part(wave + 1, K), K);
+  if (k0 < end) fetch(k0);
+  for (; k0 < end; k0 += GP_STEP) {
 #pragma unroll
     for (int i = 0; i < MR; ++i) *reinterpret_cast<float4*>(mine + (r + 8 * i) * GP_ROW + 4 * c) = x[i];
 #pragma unroll
     for (int j = 0; j < 2; ++j) *reinterpret_cast<float4*>(mine + (8 * MR + r + 8 * j) * GP_ROW + 4 * c) = y[j];
-    if (k0 + 8 * GP_STEP < K) fetch(k0 + 8 * GP_STEP);
+    if (k0 + GP_STEP < end) fetch(k0 + GP_STEP);
     __builtin_amdgcn_wave_barrier();                // (a wave's LDS accesses are carried out in their order)
 #pragma unroll
     for (int q = 0; q < GP_STEP; q += 4) {
@@ -264,7 +297,7 @@ __global__ __launch_bounds__(512) void gemm_plain_split_kernel(const TA* __restr
     if (m >= M || n >= N) continue;
     float s = 0.f;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) s += area[v][e];
+    for (int v = 0; v < GP_PARTS; ++v) s += area[v][e];
     if (bias) s += to_f32<TW>(bias[n]);
     C[(long)m * ldc + n] = from_f32<TO>(s);
   }

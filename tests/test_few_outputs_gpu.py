@@ -45,6 +45,19 @@ def test_product_of_few_outputs(ops, M, N, K, types, shift):
     assert ((y - exact).abs() <= bound + 1e-30).all()
 
 
+# few rows and many, in both forms of the product: K of one step of 32, of fewer steps than parts, of uneven parts, odd rows
+@pytest.mark.parametrize("M,N,K", [(1100, 1001, 21), (1100, 1001, 333), (2100, 1001, 1030), (9000, 65, 33), (4200, 260, 20),
+                                   (4200, 260, 36), (4200, 260, 132), (4100, 600, 260), (2100, 2050, 800)])
+@pytest.mark.parametrize("types", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
+def test_a_row_does_not_hang_on_the_number_of_rows(ops, M, N, K, types):
+    g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
+    x, w = (torch.randn(n, K, generator=g, device="cuda:0").to(t) for n, t in zip((M, N), types))
+    y = ops.linear(x, w, out_dtype=torch.float32)
+    for rows in (1, 9, 40, 700):
+        assert torch.equal(ops.linear(x[:rows], w, out_dtype=torch.float32), y[:rows])
+    assert torch.equal(ops.linear(x[-33:], w, out_dtype=torch.float32), y[-33:])
+
+
 # as many rows as the grid of the split form takes (32 a workgroup), and one more
 @pytest.mark.parametrize("M", [65535 * 32, 65535 * 32 + 1])
 def test_product_of_very_many_rows(ops, M):
