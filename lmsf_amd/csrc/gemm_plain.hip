@@ -18,10 +18,10 @@
 #define GP_STEP 32      // k of a step
 #define GP_PARTS 8
 
-// the first k of part p
+// the first k of part p (of part GP_PARTS: K)
 __device__ __forceinline__ int gp_part(int p, int K) {
-  const long steps = (K + GP_STEP - 1) / GP_STEP;
-  return (int)(p * steps / GP_PARTS) * GP_STEP;
+  const unsigned steps = ((unsigned)K + GP_STEP - 1) / GP_STEP;      // (below 2^26)
+  return (int)min(p * steps / GP_PARTS * GP_STEP, (unsigned)K);
 }
 
 // The tiles. Up to K the four entries that a thread reads of a row carry no test; with one for every entry, rows outside the
@@ -44,9 +44,10 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
 #pragma unroll
     for (int j = 0; j < 4; ++j) sum[i][j] = acc[i][j][0] = acc[i][j][1] = 0.f;
 
-  for (int p = 0; p < GP_PARTS; ++p) {
-    const int end = min(gp_part(p + 1, K), K);
-    for (int k0 = gp_part(p, K); k0 < end; k0 += GP_BK) {
+  for (int p = 0, k0 = 0; p < GP_PARTS; ++p) {
+    const int end = gp_part(p + 1, K);
+    if (k0 >= end) continue;      // a part without a step
+    for (; k0 < end; k0 += GP_BK) {
       float av[4], wv[4];
       if (k0 + GP_BK <= K) {
 #pragma unroll
@@ -209,7 +210,6 @@ static void launch_gemm_plain_few(const void* A, long lda, const void* W, long l
 // wave order at the end. (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of
 // every wave and each line is asked for by all eight waves: 7.9 us where this form took 4.3.) What bounds it is the trip
 // to memory with few outputs; with many the tiles are ahead.
-#define GP_SPLIT_OUTPUTS (1L << 20)
 #define GP_ROW (GP_STEP + 4)      // floats a row takes in LDS: eight rows at a time lie on distinct banks
 
 // four neighbouring entries; VEC: in one load (K is a multiple of 4 then), else one by one, those from K on as zeros
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(512, 4) void gemm_plain_split_kernel(const TA* __re
     for (int j = 0; j < 2; ++j) y[j] = gp_load4<VEC>(w[j], k0 + 4 * c, K);
   };
   int k0 = gp_part(wave, K);
-  const int end = min(gp_part(wave + 1, K), K);
+  const int end = gp_part(wave + 1, K);
   if (k0 < end) fetch(k0);
   for (; k0 < end; k0 += GP_STEP) {
 #pragma unroll
@@ -314,24 +314,35 @@ static void launch_gemm_plain_split(const void* A, long lda, const void* W, long
 #undef SPLIT
 }
 
+// Whether the split form runs. It takes rows in pieces of 32 x 16 outputs, which fill the chip where 64x64 tiles leave compute
+// units without one, and K in eight parts, of which a K of one or two steps leaves most waves without work: the tiles are
+// ahead from a number of pieces a compute unit on that falls with K and with rows that are read entry by entry. Split form
+// -> tiles in us by the number of pieces on 256 units (2,048 are 2^20 outputs), float32: K = 16 with 1,024 5.9 -> 5.1, with
+// 2,048 10.0 -> 6.7; K = 64 with 2,048 11.2 -> 9.6; K = 128 with 4,096 22.7 -> 15.4; K = 512 with 2,048 25.3 -> 35.2, with
+// 4,096 47.4 -> 41.5, with 8,192 89.1 -> 67.7; rows of 33 entries with 1,024 8.0 -> 8.5; of 1,001 with 2,048 79.5 -> 77.1,
+// with 4,096 149.8 -> 86.5. Up to 32 rows tiles of 64 would be half empty.
+static bool gp_split(int M, int N, int K, bool wide) {
+  const long rows = ((long)M + 31) / 32, pieces = rows * (((long)N + 15) / 16), cus = lmsf_compute_units();
+  if (rows > 65535 || N > 1 << 26) return false;      // beyond what a grid takes
+  if (M <= 32) return true;
+  if (wide) return 2 * pieces < (K <= 32 ? 8 : K <= 128 ? 15 : 30) * cus;
+  return 2 * pieces < (K <= 64 ? 7 : 15) * cus;
+}
+
 template <typename TA, typename TW, typename TO>
 static void launch_gemm_plain(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                               int M, int N, int K, hipStream_t stream) {
-  dim3 grid((N + GP_TILE - 1) / GP_TILE, (M + GP_TILE - 1) / GP_TILE), block(256);
   const bool wide = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (size_t)A % (4 * sizeof(TA)) == 0 &&
                     (size_t)W % (4 * sizeof(TW)) == 0;
-  // (the split form has a row of workgroups per 32 rows, the tiles per 64: beyond what a grid takes of the former, tiles)
-  const bool fits = (M + 31) / 32 <= 65535;
-  if (fits && wide) {
+  if (!gp_split(M, N, K, wide)) {
+    const dim3 grid((N + GP_TILE - 1) / GP_TILE, (M + GP_TILE - 1) / GP_TILE), block(256);
+    hipLaunchKernelGGL((gemm_plain_kernel<TA, TW, TO>), grid, block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw,
+                       (const TW*)bias, (TO*)C, ldc, M, N, K);
+  } else if (wide) {
     launch_gemm_plain_split<TA, TW, TO, true>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
-    return;
-  }
-  if (fits && (long)M * N <= GP_SPLIT_OUTPUTS) {
+  } else {
     launch_gemm_plain_split<TA, TW, TO, false>(A, lda, W, ldw, bias, C, ldc, M, N, K, stream);
-    return;
   }
-  hipLaunchKernelGGL((gemm_plain_kernel<TA, TW, TO>), grid, block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw,
-                     (const TW*)bias, (TO*)C, ldc, M, N, K);
 }
 
 // Supported (a, w, c) dtypes: (f32,f32,f32), (bf16,bf16,bf16), (bf16,bf16,f32), (f32,bf16,f32),
