@@ -359,13 +359,16 @@ static int mid_product(const bf16_t* xb, long ldx, const bf16_t* Wb, long ldw, c
   rc = n_split > 1                                                                                                  \
            ? launch_mid<MT_, ACT_, true, T_>(grid, U, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs) \
            : launch_mid<MT_, ACT_, false, T_>(grid, U, stream, xb, ldx, Wb, ldw, bb, (T_*)y, ldy, scratch, M, N, K, n_split, rs)
-  // Many more outputs than the chip has workgroups for (an LM head): 128 a workgroup, so that x, which every workgroup
-  // reads whole from the caches, is read half as often. 128,256 x 4,096 in float32 at 32 / 64 / 128 rows: 194 / 230 / 300
-  // us with 64 outputs a workgroup, 183 / 211 / 245 with 128.
-  if (out_dtype == LMSF_F32 && n_split == 1 && (N + 127) / 128 >= 2 * lmsf_compute_units()) {
+  // Beyond 64 rows and many more outputs than the chip has workgroups for (an LM head): 128 a workgroup, so that x, which
+  // every workgroup reads whole from the caches, is read half as often. 64 -> 128 outputs a workgroup in float32: 128,256 x
+  // 4,096 at 96 / 128 rows 293 / 325 -> 247 / 265 us, 66,560 x 2,048 (520 workgroups of 128, a last round that is nearly
+  // empty) 93 / 105 -> 90 / 95. Up to 64 rows there is too little to share and 64 is ahead, by 2 to 23 %
+  // from 65,536 to 110,000 columns of 2,048 to 8,192 (only beyond 128,000 columns of 4,096 are 64 rows 4 % faster with
+  // 128).
+  if (out_dtype == LMSF_F32 && n_split == 1 && M > 64 && (N + 127) / 128 >= 2 * lmsf_compute_units()) {
     const dim3 wide((N + 127) / 128, 1);
 #define WIDE(MT_) rc = launch_mid<MT_, 0, false, float, 2>(wide, 128, stream, xb, ldx, Wb, ldw, bb, (float*)y, ldy, scratch, M, N, K, 1, rs)
-    if (M <= 32) WIDE(2); else if (M <= 64) WIDE(4); else if (M <= 96) WIDE(6); else WIDE(8);
+    if (M <= 96) WIDE(6); else WIDE(8);
 #undef WIDE
   } else if (out_dtype == LMSF_F32) {
     if (M <= 32) MID(2, 0, float); else if (M <= 64) MID(4, 0, float); else if (M <= 96) MID(6, 0, float); else MID(8, 0, float);
