@@ -8,7 +8,7 @@ exactly the tokens it was given, and commits them to the cache. Sampling is a se
 trace replay can take the logits.
 """
 from collections import OrderedDict
-from typing import Hashable, Optional, Sequence, Tuple
+from typing import Hashable, List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -36,8 +36,7 @@ class ModelExecutor:
             raise ValueError("max_model_len %d exceeds the positions the parts were built for (%d)"
                              % (self.max_model_len, rt.max_positions))
         self.vocab_size = model.spec.vocab_size
-        self._staging = [_Staging() for _ in range(_STAGING_BUFFERS)]     # a step's metadata on its way to the device
-        self._staging_turn = 0
+        self._staging = _Staging(rt.device)     # a step's metadata on its way to the device
         self._prev_tokens: Optional[torch.Tensor] = None   # the step before's sampled tokens, while a step is built
         # steps of single tokens run at a padded batch size and are captured as HIP graphs, one per padded
         # size and context bucket, the least recently used dropped beyond max_graphs
@@ -264,10 +263,8 @@ class ModelExecutor:
         if self.program is not None and static is None and N != S:
             plan_at, plan_cap = total, self.program.plan_capacity(N)
             total += plan_cap
-        staging = self._staging[self._staging_turn]
-        self._staging_turn = (self._staging_turn + 1) % len(self._staging)
-        host_np = staging.take(total, self.rt.device)
-        host = staging.buffer[:total]
+        part, host_np = self._staging.take(total)
+        host = part[:total]
         if single:
             host_np[order_at:order_at + N] = np.argsort(-starts_a, kind="stable")
             if n_all > N:
@@ -311,12 +308,12 @@ class ModelExecutor:
         if plan_cap:
             used, plan_info = self.program.write_plan(lens, starts, host_np[plan_at:plan_at + plan_cap], plan_cap)
             total = plan_at + _pad4(max(used, 1))
-            host = staging.buffer[:total]
+            host = part[:total]
         # The copy waits for the steps before it on the stream, the host does not wait for the copy: it goes on to launch
         # this step while they run, and the staging buffer is filled again only when its event says it has been read
         # (the GPU stood still about 10 us a step: 8 requests at Takosun sizes 25.5 -> 25.0 ms for 25 steps).
         if static is not None:
-            staging.send(static.device_buffer, host)
+            self._staging.send(static.device_buffer, host)
             if self._prev_tokens is not None:
                 self.rt.ops.patch_tokens(static.device_buffer[offsets["token_ids"][0]:offsets["token_ids"][0] + n_all],
                                          static.device_buffer[src_at:src_at + n_all], self._prev_tokens)
@@ -325,7 +322,7 @@ class ModelExecutor:
             dev = static.device_buffer
         elif self.rt.device.type == "cuda":
             dev = torch.empty(total, dtype=torch.int32, device=self.rt.device)
-            staging.send(dev, host)
+            self._staging.send(dev, host)
         else:
             dev = host.clone()
 
@@ -449,38 +446,49 @@ def _pad4(n: int) -> int:
     return (n + 3) // 4 * 4
 
 
-_STAGING_BUFFERS = 4      # steps whose metadata may be on its way to the device at a time
-
-
 class _Staging:
-    """A pinned host buffer that a step's metadata travels through, and the event behind its last copy."""
+    """The pinned host memory that steps' metadata travels through: one block in four parts that take turns, each with
+    the event behind its last copy. It grows to the next power of two, all parts at once, so that the first steps do not
+    each pay for a pinned allocation and longer ones do so seldom."""
 
-    def __init__(self):
-        self.buffer: Optional[torch.Tensor] = None
-        self._np: Optional[np.ndarray] = None
-        self._event = None
-        self._sent = False
+    PARTS = 4      # steps whose metadata may be on its way to the device at a time
 
-    def take(self, total: int, device: torch.device) -> np.ndarray:
-        """The buffer as an array of at least ``total`` int32, free to be filled: waits for its last copy."""
-        if self._sent:
-            self._event.synchronize()
-            self._sent = False
-        if self.buffer is None or self.buffer.numel() < total:
-            self.buffer = torch.empty(max(total, 4096), dtype=torch.int32, pin_memory=device.type == "cuda")
-            self._np = self.buffer.numpy()
-        return self._np
+    def __init__(self, device: torch.device):
+        self._device = device
+        self._size = 0                     # int32 a part
+        self._parts: List[Tuple[torch.Tensor, np.ndarray]] = []
+        self._events: list = [None] * self.PARTS
+        self._sent = [False] * self.PARTS
+        self._turn = 0
+
+    def _wait(self, turn: int) -> None:
+        if self._sent[turn]:
+            self._events[turn].synchronize()
+            self._sent[turn] = False
+
+    def take(self, total: int) -> Tuple[torch.Tensor, np.ndarray]:
+        """The next part, of at least ``total`` int32, free to be filled (its last copy is waited for)."""
+        self._turn = (self._turn + 1) % self.PARTS
+        if total > self._size:
+            for turn in range(self.PARTS):
+                self._wait(turn)
+            size = max(4096, 1 << (total - 1).bit_length())
+            block = torch.empty((self.PARTS, size), dtype=torch.int32, pin_memory=self._device.type == "cuda")
+            self._parts = [(part, part.numpy()) for part in block]
+            self._size = size
+        self._wait(self._turn)
+        return self._parts[self._turn]
 
     def send(self, to: torch.Tensor, host: torch.Tensor) -> None:
-        """Copy ``host`` (the buffer's first elements) to ``to`` in the current stream's order."""
+        """Copy ``host`` (the first elements of the part last taken) to ``to`` in the current stream's order."""
         if to.device.type != "cuda":
             to.copy_(host)
             return
-        if self._event is None:
-            self._event = torch.cuda.Event()
+        if self._events[self._turn] is None:
+            self._events[self._turn] = torch.cuda.Event()
         to.copy_(host, non_blocking=True)
-        self._event.record(torch.cuda.current_stream(to.device))
-        self._sent = True
+        self._events[self._turn].record(torch.cuda.current_stream(to.device))
+        self._sent[self._turn] = True
 
 
 class _StaticBatch:
