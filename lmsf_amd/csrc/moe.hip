@@ -169,20 +169,24 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_kernel(
 // shared by up to MOE_SHARED_PAIRS of the pairs that have chosen it (where more have, other workgroups take the next ones
 // side by side). A wave reads its rows of the matrix and the same entries of the vectors (which the caches hold) with
 // 16-byte loads, MOE_AHEAD pieces of 512 or 256 entries of each row on their way at a time; nothing goes through LDS and
-// no wave waits for another. Every output is added up in the order of the kernels above. The outputs vary fastest over the
-// workgroups, so that an expert's rows are read by all eight dies (with the pairs fastest, a pair's whole expert falls to
-// one die: gate and up 26.5 us). What bounds them is memory and, for an expert of several pairs, the multiply-adds of a
-// wave. Both products of 2,048 -> 2 x 1,024 -> 2,048 in bfloat16, kernels above -> these: 8 tokens with 2 of 16 experts
-// each 38.6 -> 27.6 us, 31 tokens with one expert 40.1 -> 27.0 (in float32 45.5 -> 35.4, and 69.7 with one workgroup taking
-// all of an expert's pairs in turn); 4 pieces ahead, 2 pairs a read, 1 or 4 outputs a wave: up to a third slower.
+// no wave waits for another. Every output is added up in the order of the kernels above. In the first product the outputs
+// vary fastest over the workgroups, so that an expert's rows are read by all eight dies (with the pairs fastest, a pair's
+// whole expert falls to one die: gate and up 26.5 us). In the second the tokens vary fastest within a die, so that a row
+// that several tokens need comes to a die once: 32 tokens in float32, 4,096 -> 2 x 1,536 -> 4,096, with one pair of
+// experts 268 -> 203 us, with experts of their own choice 380 -> 305. What bounds them is memory and, for an expert of
+// several pairs, the multiply-adds of a wave. Both products of 2,048 -> 2 x 1,024 -> 2,048 in bfloat16, kernels above ->
+// these: 8 tokens with 2 of 16 experts each 40.6 -> 33.1 us, 31 tokens with one expert 38.6 -> 28.3 (in float32 44.3 ->
+// 34.3); of one matrix 28.9 -> 22.4 and 30.0 -> 22.7; 4 pieces ahead, 2 pairs a read, 1 or 4 outputs a wave: up to a
+// third slower.
 #define MOE_AHEAD 2
 #define MOE_FEW_PAIRS 64      // a lane each
 #define MOE_SHARED_PAIRS 4    // pairs of one expert that share a read of its rows
 #define MOE_FEW_OUT 2         // outputs a wave owns
 // Smaller experts stay with the kernels above, which share a vector between a workgroup's waves: what counts there is the
 // way from a wave's first load to its last sum (2 x 512 x 256 entries, 30 pairs of two experts from memory: 10.6 -> 12.6
-// us here; 2 x 1,024 x 512 level to 1.14 times as long with all pairs on one expert, 0.75 times with the pairs spread;
-// from 2 x 1,536 x 512 on nothing is slower).
+// us here; 2 x 1,024 x 512 level to 1.14 times as long with all pairs on one expert, 0.75 times with the pairs spread). From
+// 1,536 x 512 on everything measured is faster but 31 pairs on one expert of one matrix of that size, 18.5 -> 20.9 us in
+// float32 (spread over 16 experts 32.3 -> 19.4).
 #define MOE_FEW_ENTRIES (3L << 18)
 
 // a[q][r] += sum over this lane's entries of rows r against the vectors of the pairs, each times its scale
@@ -224,11 +228,11 @@ __device__ __forceinline__ void moe_few_dot(const T* const (&w)[ROWS], const T* 
   }
 }
 
-template <typename T>
+template <typename T, bool GATED>
 __global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
     const T* __restrict__ h, long h_stride, const T* __restrict__ Wgu, const int* __restrict__ ids,
     const int* __restrict__ table, int vocab, int top, int E, T* __restrict__ act, int F, int W, int n_pairs,
-    const float* __restrict__ pair_scale, int gated, float limit, int identity) {
+    const float* __restrict__ pair_scale, float limit, int identity) {
   const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE;
   const int f0 = (blockIdx.x * MOE_WAVES + wave) * MOE_FEW_OUT;
   if (f0 >= F) return;
@@ -244,16 +248,17 @@ __global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
   const unsigned long long before = pairs & ((1ull << blockIdx.y) - 1);
   if (__popcll(before) % MOE_SHARED_PAIRS) return;
   pairs ^= before;
-  const T* We = Wgu + (long)e * (gated ? 2 : 1) * F * W;
+  const T* We = Wgu + (long)e * (GATED ? 2 : 1) * F * W;
   const int valid = min(MOE_FEW_OUT, F - f0);
-  const T* w[2 * MOE_FEW_OUT];
+  constexpr int ROWS = (GATED ? 2 : 1) * MOE_FEW_OUT;
+  const T* w[ROWS];
 #pragma unroll
   for (int r = 0; r < MOE_FEW_OUT; ++r) {
     w[r] = We + (long)(f0 + min(r, valid - 1)) * W;
-    w[MOE_FEW_OUT + r] = gated ? w[r] + (long)F * W : w[r];
+    if (GATED) w[ROWS - MOE_FEW_OUT + r] = w[r] + (long)F * W;
   }
   const T* x[MOE_SHARED_PAIRS];
-  float scale[MOE_SHARED_PAIRS], a[MOE_SHARED_PAIRS][2 * MOE_FEW_OUT];
+  float scale[MOE_SHARED_PAIRS], a[MOE_SHARED_PAIRS][ROWS];
   int pair[MOE_SHARED_PAIRS], count = 0;
 #pragma unroll
   for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
@@ -266,20 +271,20 @@ __global__ __launch_bounds__(MOE_THREADS, 4) void moe_gate_up_few_kernel(
     x[q] = h + (long)(pair[q] / top) * h_stride;
     scale[q] = pair_scale ? pair_scale[pair[q]] : 1.f;
 #pragma unroll
-    for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = 0.f;
+    for (int r = 0; r < ROWS; ++r) a[q][r] = 0.f;
   }
-  moe_few_dot<T, 2 * MOE_FEW_OUT, MOE_SHARED_PAIRS>(w, x, scale, count, W, lane, a);
+  moe_few_dot<T, ROWS, MOE_SHARED_PAIRS>(w, x, scale, count, W, lane, a);
 #pragma unroll
   for (int q = 0; q < MOE_SHARED_PAIRS; ++q) {
     if (q >= count) break;
 #pragma unroll
-    for (int r = 0; r < 2 * MOE_FEW_OUT; ++r) a[q][r] = wave_sum(a[q][r]);
+    for (int r = 0; r < ROWS; ++r) a[q][r] = wave_sum(a[q][r]);
     if (lane < valid) {
       // the products are rounded as stored activations are, then the activation in float32
       const float gg = to_f32<T>(from_f32<T>(lane == 0 ? a[q][0] : a[q][1]));
-      const float uu = to_f32<T>(from_f32<T>(lane == 0 ? a[q][MOE_FEW_OUT] : a[q][MOE_FEW_OUT + 1]));
+      const float uu = to_f32<T>(from_f32<T>(lane == 0 ? a[q][ROWS - 2] : a[q][ROWS - 1]));
       float y;
-      if (!gated) {
+      if (!GATED) {
         const float up = fmaxf(gg, 0.f);      // one matrix an expert: relu(W_up h)^2
         y = up * up;
       } else {
@@ -295,10 +300,10 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_few_kernel(
     const T* __restrict__ act, const T* __restrict__ Wd, const int* __restrict__ ids, const int* __restrict__ table,
     int vocab, int top, int E, float weight, const T* __restrict__ base, long base_stride, T* __restrict__ out,
     long out_stride, int F, int W, const float* __restrict__ base_scale, const float* __restrict__ out_scale,
-    int identity, const T* __restrict__ h, long h_stride, const float* __restrict__ pair_scale) {
-  const int n = blockIdx.y;
+    int identity, const T* __restrict__ h, long h_stride, const float* __restrict__ pair_scale, int n_tokens) {
   const int wave = threadIdx.x / LMSF_WAVE, lane = threadIdx.x % LMSF_WAVE;
-  const int o0 = (blockIdx.x * MOE_WAVES + wave) * MOE_FEW_OUT;
+  const int i = blockIdx.x / 8, n = i % n_tokens;
+  const int o0 = ((i / n_tokens * 8 + blockIdx.x % 8) * MOE_WAVES + wave) * MOE_FEW_OUT;
   if (o0 >= W) return;
   const int valid = min(MOE_FEW_OUT, W - o0);
   const int id = min(max(ids ? ids[n] : n, 0), vocab - 1);
@@ -625,21 +630,23 @@ extern "C" int lmsf_table_moe_act(const void* h, int dtype, long h_stride, const
     return 0;
   }
   const int es16 = 16 / lmsf_elem_size(dtype);
-  if ((long)n_tokens * top <= MOE_FEW_PAIRS && (long)W * F >= MOE_FEW_ENTRIES && W % es16 == 0 && F % es16 == 0 && h_stride % es16 == 0 && lmsf_aligned16(h) &&
-      lmsf_aligned16(Wgu) && lmsf_aligned16(Wd) && lmsf_aligned16(act)) {
+  if ((long)n_tokens * top <= MOE_FEW_PAIRS && (long)W * F >= MOE_FEW_ENTRIES && W % es16 == 0 && F % es16 == 0 &&
+      h_stride % es16 == 0 && lmsf_aligned16(h) && lmsf_aligned16(Wgu) && lmsf_aligned16(Wd) && lmsf_aligned16(act)) {
     const int outs = MOE_WAVES * MOE_FEW_OUT, P = n_tokens * top;
-    const dim3 f1((F + outs - 1) / outs, P), f2((W + outs - 1) / outs, n_tokens);
+    const dim3 f1((F + outs - 1) / outs, P), f2((W + 8 * outs - 1) / (8 * outs) * 8 * n_tokens);
+#define MOE_GATE_UP_FEW(T_, GATED_)                                                                                   \
+  hipLaunchKernelGGL((moe_gate_up_few_kernel<T_, GATED_>), f1, dim3(MOE_THREADS), 0, stream, (const T_*)h, h_stride,  \
+                     (const T_*)Wgu, ids, table, vocab, top, E, (T_*)act, F, W, P, pair_scale, limit, identity)
 #define MOE_FEW(T_)                                                                                                   \
   do {                                                                                                                \
-    hipLaunchKernelGGL((moe_gate_up_few_kernel<T_>), f1, dim3(MOE_THREADS), 0, stream, (const T_*)h, h_stride,        \
-                       (const T_*)Wgu, ids, table, vocab, top, E, (T_*)act, F, W, P, pair_scale, gated, limit,        \
-                       identity);                                                                                     \
+    if (gated) MOE_GATE_UP_FEW(T_, true); else MOE_GATE_UP_FEW(T_, false);                                            \
     hipLaunchKernelGGL((moe_down_few_kernel<T_>), f2, dim3(MOE_THREADS), 0, stream, (const T_*)act, (const T_*)Wd,    \
                        ids, table, vocab, top, E, weight, (const T_*)base, base_stride, (T_*)out, out_stride, F, W,   \
-                       base_scale, out_scale, identity, (const T_*)h, h_stride, pair_scale);                          \
+                       base_scale, out_scale, identity, (const T_*)h, h_stride, pair_scale, n_tokens);                \
   } while (0)
     if (dtype == LMSF_F32) MOE_FEW(float); else MOE_FEW(bf16_t);
 #undef MOE_FEW
+#undef MOE_GATE_UP_FEW
     LMSF_LAUNCH_CHECK("table_moe (few)");
     return 0;
   }
