@@ -58,8 +58,11 @@ __global__ __launch_bounds__(256) void gemm_plain_kernel(const TA* __restrict__ 
       } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          av[e] = k0 + lk + e < K ? to_f32<TA>(arow[k0 + e]) : 0.f;
-          wv[e] = k0 + lk + e < K ? to_f32<TW>(wrow[k0 + e]) : 0.f;
+          // (all loads are made, beyond K of the last entry: behind a test each they would be waited for one by one)
+          const int at = min(k0 + e, K - 1 - lk);
+          const float a1 = to_f32<TA>(arow[at]), w1 = to_f32<TW>(wrow[at]);
+          av[e] = k0 + lk + e < K ? a1 : 0.f;
+          wv[e] = k0 + lk + e < K ? w1 : 0.f;
         }
       }
 #pragma unroll
@@ -314,19 +317,31 @@ static void launch_gemm_plain_split(const void* A, long lda, const void* W, long
 #undef SPLIT
 }
 
-// Whether the split form runs. It takes rows in pieces of 32 x 16 outputs, which fill the chip where 64x64 tiles leave compute
-// units without one, and K in eight parts, of which a K of one or two steps leaves most waves without work: the tiles are
-// ahead from a number of pieces a compute unit on that falls with K and with rows that are read entry by entry. Split form
-// -> tiles in us by the number of pieces on 256 units (2,048 are 2^20 outputs), float32: K = 16 with 1,024 5.9 -> 5.1, with
-// 2,048 10.0 -> 6.7; K = 64 with 2,048 11.2 -> 9.6; K = 128 with 4,096 22.7 -> 15.4; K = 512 with 2,048 25.3 -> 35.2, with
-// 4,096 47.4 -> 41.5, with 8,192 89.1 -> 67.7; rows of 33 entries with 1,024 8.0 -> 8.5; of 1,001 with 2,048 79.5 -> 77.1,
-// with 4,096 149.8 -> 86.5. Up to 32 rows tiles of 64 would be half empty.
-static bool gp_split(int M, int N, int K, bool wide) {
-  const long rows = ((long)M + 31) / 32, pieces = rows * (((long)N + 15) / 16), cus = lmsf_compute_units();
+// Whether the split form runs (``wide``: rows that allow wide loads; ``half``: an operand of 16 bits). It takes rows in
+// pieces of 32 x 16 outputs (8 or 16 rows where there are no more, for which a piece costs a quarter or half as much),
+// which fill the chip where 64x64 tiles leave compute units without one, and K in eight parts, of which a K of one or two
+// steps leaves most waves without work. The tiles are ahead from a number of pieces a compute unit on that falls with K (two
+// workgroups run on a unit at once: up to K = 32 a second round already costs more than a tile's whole K) and that is
+// lower for rows read entry by entry, of 16-bit entries above all. Split form -> tiles in us by the number of pieces on 256
+// units: wide float32, K = 16: 512 3.2 -> 4.1, 875 4.9 -> 4.2; K = 64: 1,008 5.7 -> 7.0, 1,712 9.8 -> 8.0; K = 128: 1,712
+// 11.1 -> 11.5, 2,512 14.2 -> 12.9; K = 256: 2,520 16.5 -> 19.9, 3,969 25.3 -> 21.7. Entry by entry in float32, K = 33:
+// 512 4.1 -> 6.0, 1,250 9.0 -> 6.6; K = 65: 1,008 7.5 -> 8.2, 1,712 12.0 -> 9.1; K = 333: 1,250 19.7 -> 24.0, 1,827 28.1
+// -> 25.0; in bfloat16, K = 15: 441 5.3 -> 4.4, 1,008 9.2 -> 4.6; K = 33: 512 5.3 -> 6.3, 875 8.6 -> 6.4; K = 333: 912
+// 21.2 -> 24.9, 1,200 27.0 -> 24.8. Few rows: 8 of 50,000 columns, K = 16 6.5 -> 5.4, K = 64 6.7 -> 10.4, K = 333 20 -> 41; 16
+// rows 8.0 -> 5.6, 8.6 -> 10.7, 27 -> 41; 32 rows, K = 16 13.4 -> 6.4, K = 128 17.9 -> 18.8, K = 256 21 -> 33.
+static bool gp_split(int M, int N, int K, bool wide, bool half) {
+  const long rows = ((long)M + 31) / 32, pieces = rows * (((long)N + 15) / 16);
   if (rows > 65535 || N > 1 << 26) return false;      // beyond what a grid takes
-  if (M <= 32) return true;
-  if (wide) return 2 * pieces < (K <= 32 ? 8 : K <= 128 ? 15 : 30) * cus;
-  return 2 * pieces < (K <= 64 ? 7 : 15) * cus;
+  if (wide ? (M <= 16 && K > 32) || (M <= 32 && K > 128) : !half && M <= 16 && K > 128) return true;
+  long most;                                          // twice the pieces of a compute unit
+  if (wide)
+    most = K <= 32 ? 4 : K <= 64 ? 9 : K <= 128 ? 14 : 26;
+  else if (half)
+    most = K <= 16 ? 0 : K <= 128 ? 4 : 8;
+  else
+    most = K <= 64 ? 4 : K <= 128 ? 8 : 12;
+  const int eighths = M <= 8 ? 2 : M <= 16 ? 4 : M <= 32 ? 6 : 8;       // what a piece costs
+  return pieces * eighths <= 4 * most * lmsf_compute_units();
 }
 
 template <typename TA, typename TW, typename TO>
@@ -334,7 +349,7 @@ static void launch_gemm_plain(const void* A, long lda, const void* W, long ldw, 
                               int M, int N, int K, hipStream_t stream) {
   const bool wide = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && (size_t)A % (4 * sizeof(TA)) == 0 &&
                     (size_t)W % (4 * sizeof(TW)) == 0;
-  if (!gp_split(M, N, K, wide)) {
+  if (!gp_split(M, N, K, wide, sizeof(TA) == 2 || sizeof(TW) == 2)) {
     const dim3 grid((N + GP_TILE - 1) / GP_TILE, (M + GP_TILE - 1) / GP_TILE), block(256);
     hipLaunchKernelGGL((gemm_plain_kernel<TA, TW, TO>), grid, block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw,
                        (const TW*)bias, (TO*)C, ldc, M, N, K);

@@ -46,8 +46,8 @@ def test_product_of_few_outputs(ops, M, N, K, types, shift):
 
 
 # few rows and many, in both forms of the product: K of one step of 32, of fewer steps than parts, of uneven parts, odd rows
-@pytest.mark.parametrize("M,N,K", [(1100, 1001, 21), (1100, 1001, 333), (2100, 1001, 1030), (9000, 65, 33), (4200, 260, 20),
-                                   (4200, 260, 36), (4200, 260, 132), (4100, 600, 260), (2100, 2050, 800)])
+@pytest.mark.parametrize("M,N,K", [(1100, 1001, 21), (1100, 1001, 333), (2100, 1001, 1030), (33, 4100, 15), (24, 9000, 40),
+                                   (300, 1000, 16), (9000, 65, 33), (4200, 260, 20), (4200, 260, 36), (4200, 260, 132), (4100, 600, 260), (2100, 2050, 800)])
 @pytest.mark.parametrize("types", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32)])
 def test_a_row_does_not_hang_on_the_number_of_rows(ops, M, N, K, types):
     g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
