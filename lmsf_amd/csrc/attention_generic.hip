@@ -37,9 +37,10 @@ __device__ __forceinline__ void gen_load4(const bf16_t* p, float* x) {
 }
 
 // VEC: the key pages start on a boundary of four elements (every row does then: d is a multiple of 4), and a key is read
-// four elements a load.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
+// four elements a load. WAVES: waves a SIMD that registers are kept for: 1 (about 110 registers, so that as many loads as
+// possible are on their way together; four workgroups run on a compute unit) or 5 (72 registers, seven workgroups).
+template <typename T, bool VEC, int WAVES>
+__global__ __launch_bounds__(GEN_THREADS, WAVES) void paged_attention_generic_kernel(
     const T* __restrict__ q, long q_stride, T* __restrict__ out, long out_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ block_tables, int bt_width, const int* __restrict__ seg,
     const int* __restrict__ pos, int nh, int nkv, int d, int ps, float scale, int window, float softcap,
@@ -111,18 +112,18 @@ __global__ __launch_bounds__(GEN_THREADS) void paged_attention_generic_kernel(
     if (pv_active) {
       const int n = min(GEN_THREADS, p - j0 + 1);
       int jj = og;
-      // (up to 256 output dims: eight values of a group's keys are asked for at a time; one by one every value waits for
-      // the one before it, 300 keys of 32 dims in float32 14.0 -> 12.2 us)
+      // (up to 256 output dims: four values of a group's keys are asked for at a time; one by one every value waits for
+      // the one before it)
       if (d <= GEN_THREADS)
-        for (; jj + 7 * ngroups < n; jj += 8 * ngroups) {
-          float v[8];
+        for (; jj + 3 * ngroups < n; jj += 4 * ngroups) {
+          float v[4];
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
+          for (int u = 0; u < 4; ++u) {
             const int key = jj + u * ngroups;
             v[u] = to_f32<T>(v_pages[((long)shead[key] * d + oi) * ps + soff[key]]);
           }
 #pragma unroll
-          for (int u = 0; u < 8; ++u) acc += sp[jj + u * ngroups] * v[u];
+          for (int u = 0; u < 4; ++u) acc += sp[jj + u * ngroups] * v[u];
         }
       for (; jj < n; jj += ngroups) {
         const int head_base = shead[jj], off = soff[jj];
@@ -175,17 +176,28 @@ extern "C" int lmsf_paged_attention_generic_biased(const void* q, long q_stride,
   if (n_tokens == 0) return 0;
   const size_t smem = (size_t)(d + 4 * GEN_THREADS) * 4;
   dim3 grid(n_tokens, nh), block(GEN_THREADS);
+#define GENERIC_W(T_, VEC_, WAVES_)                                                                                     \
+  hipLaunchKernelGGL((paged_attention_generic_kernel<T_, VEC_, WAVES_>), grid, block, smem, stream, (const T_*)q,       \
+                     q_stride, (T_*)out, out_stride, (const T_*)k_pages, (const T_*)v_pages, block_tables, bt_width,    \
+                     seg, pos, nh, nkv, d, ps, scale, window, softcap, bias, sink)
 #define GENERIC(T_, VEC_)                                                                                               \
-  hipLaunchKernelGGL((paged_attention_generic_kernel<T_, VEC_>), grid, block, smem, stream, (const T_*)q, q_stride,     \
-                     (T_*)out, out_stride, (const T_*)k_pages, (const T_*)v_pages, block_tables, bt_width, seg, pos,    \
-                     nh, nkv, d, ps, scale, window, softcap, bias, sink)
+  do {                                                                                                                  \
+    if (many) GENERIC_W(T_, VEC_, 5); else GENERIC_W(T_, VEC_, 1);                                                      \
+  } while (0)
   const bool vec = (size_t)k_pages % (4 * lmsf_elem_size(dtype)) == 0;
+  // More workgroups than the chip takes at once with four on a compute unit: fewer registers, seven on a unit. Both sides
+  // in float32 with 8 heads of 32 / 128, four -> seven a unit: 64 tokens of a prompt 7.6 / 13.8 -> 8.0 / 15.2 us, 100
+  // tokens 9.3 / 22.5 -> 9.7 / 23.3, 140 tokens 14.2 / 38.8 -> 12.4 / 34.6, 200 tokens 22.1 / 61.4 -> 19.5 / 59.3, 256
+  // tokens 32.9 / 105.0 -> 30.5 / 107.2. (Keys read entry by entry and values one by one took 15.1 / 37.9 us for 8
+  // tokens of 300 keys, now 12.1 / 27.7.)
+  const bool many = (long)n_tokens * nh > 4L * lmsf_compute_units();
   if (dtype == LMSF_F32) {
     if (vec) GENERIC(float, true); else GENERIC(float, false);
   } else {
     if (vec) GENERIC(bf16_t, true); else GENERIC(bf16_t, false);
   }
 #undef GENERIC
+#undef GENERIC_W
   LMSF_LAUNCH_CHECK("paged_attention_generic");
   return 0;
 }

@@ -102,3 +102,24 @@ def test_general_attention(ops, d, ps, context, dtype, shift):
             assert ((got[t, h * d:(h + 1) * d] - want).abs() <= tol).all()
 
 
+# as many workgroups as the chip takes at once with four on a compute unit, and more
+@pytest.mark.parametrize("d", [32, 96, 260])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_general_attention_of_many_tokens_gives_the_bits_of_few(ops, d, dtype, shift):
+    nh, nkv, ps = 8, 2, 16
+    T = torch.cuda.get_device_properties(0).multi_processor_count * 4 // nh + 3
+    g = torch.Generator(device="cuda:0").manual_seed(d)
+    pages = -(-T // ps) + 2
+
+    def cache(*shape):
+        n = pages * nkv * ps * d
+        return torch.randn(n + 8, generator=g, device="cuda:0").to(dtype)[shift:shift + n].view(pages, nkv, *shape)
+    k, v = cache(ps, d), cache(d, ps)
+    q = torch.randn(T, nh * d, generator=g, device="cuda:0").to(dtype)
+    table = torch.randperm(pages, generator=g, device="cuda:0")[:-(-T // ps)].to(torch.int32).view(1, -1)
+    seg, pos = torch.zeros(T, dtype=torch.int32, device="cuda:0"), torch.arange(T, dtype=torch.int32, device="cuda:0")
+
+    def run(a, b):
+        return ops.paged_attention(q[a:b], k, v, table, seg[a:b], pos[a:b], nh, nkv, d, d ** -0.5, kernel="generic")
+    assert torch.equal(run(0, T), torch.cat([run(0, T - 20), run(T - 20, T)]))
