@@ -2,8 +2,6 @@
 import pytest
 import torch
 
-from torch_ops import TorchOps
-
 pytestmark = pytest.mark.gpu
 
 
