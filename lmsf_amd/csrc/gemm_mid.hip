@@ -290,7 +290,8 @@ static int launch_mid(dim3 grid, int U, hipStream_t stream, const bf16_t* x, lon
 // Splits of K proposed for these sizes (1: no partial sums, no second kernel). The time of the product is
 // that of the compute unit with the most workgroups, so the number of workgroups should fill the last round
 // over the 256 compute units; against that stand the partial sums, which are written and read once. The
-// proposal minimises bytes / (share of the last round that is filled) + bytes of the partial sums.
+// proposal minimises bytes / (share of the last round that is filled) + bytes of the partial sums. It counts workgroups of
+// 64 outputs on 256 compute units whatever mid_outputs below makes of them: how K is cut decides the bits of the result.
 extern "C" int lmsf_gemm_mid_splits(int M, int N, int K, int act) {
   const int wt = act ? 2 : 1;
   const long blocks = (N + 63) / 64, chunks = K / 64;
@@ -337,9 +338,11 @@ static int mid_check(const void* x, long ldx, const void* W, long ldw, int M, in
 }
 
 // Outputs a workgroup owns: 64, or, where such workgroups leave compute units without one, as few (in steps of 8, at
-// least 32) as the chip still takes at once. QKV of 6,144 x 4,096 in 2 parts at 64 rows: 192 workgroups of 64 outputs
-// 18.1 us, 256 of 48 14.7; gate_up of 28,672 x 4,096: 224 of 64 42.6, 256 of 56 41.5. The gated product after a norm (up to
-// 16 rows), whose x is small, stays at 64 (37.5 against 37.8 at 8 rows).
+// least 32) as the chip still takes at once. 64 outputs a workgroup -> fewer, with the reduction where K is split: QKV of
+// 6,144 x 4,096 in 2 parts at 64 rows (192 workgroups -> 256) 18.4 -> 18.1 us, 12,288 x 4,096 at 32 rows (192 -> 256) 22.0
+// -> 20.5, gated 8,192 x 2,048 at 64 rows (128 -> 256) 21.9 -> 19.6, gated 11,008 x 4,096 (172 -> 230) 41.7 -> 39.9, gated
+// 14,336 x 4,096 (224 -> 256) level; nothing from 1,024 to 32,000 columns and 17 to 128 rows more than 2 % slower. The gated
+// product after a norm (up to 16 rows), whose x is small, stays at 64 (37.5 against 37.8 at 8 rows).
 static int mid_outputs(int N, int n_split, bool after_norm) {
   const int cus = lmsf_compute_units();
   if (after_norm || (long)((N + 63) / 64) * n_split >= cus) return 64;

@@ -2,8 +2,8 @@
 //
 // This is the true 32-bit matrix product of the float32 path (no matrix-core instruction, no
 // reduced-precision input mode), and the fallback of the bfloat16 path for shapes the fast kernels
-// refuse. Inputs may be float32 or bfloat16; products and sums are float32. The reference calls cuBLASLt with float32 compute
-// (tops/csrc/tops/tensorrt_llm/common/cublasMMWrapper.cpp:182-210) and adds the bias afterwards
+// refuse. Inputs may be float32 or bfloat16; products and sums are float32. The reference calls cuBLASLt with
+// float32 compute (tops/csrc/tops/tensorrt_llm/common/cublasMMWrapper.cpp:182-210) and adds the bias afterwards
 // (core/src/model_executor/layers/linear.rs:101-104).
 //
 // Two forms: K split over the waves of a workgroup (further down), or a 64x64 tile per workgroup of 256 threads, 4x4
@@ -211,8 +211,9 @@ static void launch_gemm_plain_few(const void* A, long lda, const void* W, long l
 // while this one is multiplied, and go through an area of LDS that belongs to the wave, from which lane (r, c) takes rows
 // r, r + 8, ... and columns c, c + 8 for the outputs it holds: no barrier inside the loop. The waves' sums are added in
 // wave order at the end. (Without LDS, every lane fetching the rows it multiplies, a row's 16 bytes go to eight lanes of
-// every wave and each line is asked for by all eight waves: 7.9 us where this form took 4.3.) What bounds it is the trip
-// to memory with few outputs; with many the tiles are ahead.
+// every wave and each line is asked for by all eight waves: nearly twice as long for 8 rows of 128 outputs.) What bounds
+// it is the trip to memory with few outputs (8 x 128 x 352 2.9 us where the tiles took 34, 8 x 4,096 x 4,096 13.5 where
+// they took 398); with many the tiles are ahead, which read 2 bytes of LDS a multiply-add where 32 rows here read 3.
 #define GP_ROW (GP_STEP + 4)      // floats a row takes in LDS: eight rows at a time lie on distinct banks
 
 // four neighbouring entries; VEC: in one load (K is a multiple of 4 then), else one by one, those from K on as zeros

@@ -6,7 +6,8 @@
 // The reference leaves these products to cuBLASLt with an offline-tuned algorithm per shape
 // (tops/src/cublas.rs:29-114, tops/csrc/tops/tensorrt_llm/c_api/gemm.cc:43-150).
 //
-// Decomposition. One workgroup owns 16 rows of W (16 outputs per token) over the whole K. Its NW
+// Decomposition. One workgroup owns 16 rows of W (16 outputs per token), or 8 where such workgroups all
+// fit on the chip at once (skinny_narrow), over the whole K. Its NW
 // waves split K in chunks of KC elements, wave w taking chunks w, w + NW, ...: at any moment the
 // workgroup reads NW * KC contiguous elements of each of its rows. Partial sums of the waves are
 // added in a fixed order through LDS, so the result does not depend on timing.
@@ -381,8 +382,9 @@ static int launch_skinny_x(const void* x, long ldx, const void* W, long ldw, con
 
 // Whether a product of M rows with so many outputs (pairs of outputs in the rotary form) runs with tiles of 8 rows of W:
 // where such tiles all fit on the chip at once, tiles of 16 leave half of its compute units or more without a workgroup.
-// Measured at 8 rows, tiles of 16 -> 8: 2,048 x 1,024 to 4,096 (128 -> 256 workgroups) 6.8 -> 6.0 us, 2,048 x 8,192 10.4 ->
-// 8.7, QKV of 3,072 x 2,048 with rotation (96 -> 192) 7.7 -> 7.0; but of 6,144 x 4,096 (192 -> 384) 12.4 -> 13.2.
+// Measured at 8 / 16 rows, tiles of 16 -> 8: 512 x 512 3.0 / 3.2 -> 2.9 / 3.0 us, 2,048 x 2,048 (128 -> 256 workgroups) 5.0 /
+// 5.5 -> 4.8 / 5.1, 2,048 x 8,192 10.5 / 12.3 -> 9.0 / 10.1, gated 2,048 x 4,096 11.9 / 11.9 -> 10.7 / 10.5, QKV of 3,072 x
+// 2,048 with rotation (96 -> 192) 6.9 / 7.4 -> 6.1 / 6.4; but of 6,144 x 4,096 (192 -> 384) 12.4 -> 13.2 at 8 rows.
 static bool skinny_narrow(int M, int outputs) { return M <= 16 && (outputs + 7) / 8 <= lmsf_compute_units(); }
 
 template <int MT, int KC, int NW, typename TOut, int ACT, int DEPTH = 1, bool SCALED = false>

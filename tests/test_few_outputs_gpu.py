@@ -1,4 +1,4 @@
-"""The float32 product split over the waves of a workgroup, and general attention's values read eight keys at a time."""
+"""The float32 product split over the waves of a workgroup, and general attention's values read four keys at a time."""
 import pytest
 import torch
 
@@ -12,7 +12,7 @@ def ops():
 
 
 # the edges of its row forms (8, 16, 32 rows a workgroup) and columns (16), K below, at and beyond a step of 32 and a step
-# for every wave, K that is no multiple of 4, and both sides of the line to the 64x64 tiles (2^20 outputs)
+# for every wave, K that is no multiple of 4, and many outputs (short K in the 64x64 tiles)
 @pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 16, 4), (8, 17, 31), (9, 15, 32), (16, 33, 36), (17, 64, 127), (32, 16, 128),
                                    (33, 70, 132), (65, 130, 260), (7, 128, 352), (5, 20, 256), (5, 20, 257), (5, 20, 515), (1024, 1024, 21), (1025, 1024, 21), (1025, 1024, 20),
                                    (2, 20000, 12)])
@@ -66,9 +66,9 @@ def test_product_of_very_many_rows(ops, M):
     assert ((ops.linear(x, w).double() - exact).abs() <= 5 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
 
 
-# keys just below, at and beyond eight a group (256 / d groups), a second round of 256 keys, pages of odd sizes
+# keys just below, at and beyond four and eight a group (256 / d groups), a second round of 256 keys, pages of odd sizes
 @pytest.mark.parametrize("d,ps", [(32, 16), (4, 3), (96, 16), (256, 8), (260, 16)])
-@pytest.mark.parametrize("context", [1, 7, 8, 63, 64, 65, 256, 257, 300])
+@pytest.mark.parametrize("context", [1, 7, 8, 31, 32, 33, 63, 64, 65, 256, 257, 300])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_general_attention(ops, d, ps, context, dtype, shift):

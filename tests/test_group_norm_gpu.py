@@ -17,7 +17,7 @@ def gn(v, w, groups, eps):
 
 
 # widths below, at and beyond a wave's 256 columns, groups of whole parts of 256 and others, 1, 2 and 4 groups of four a
-# thread, the widest row that is kept in registers and one beyond it (6,144 in three rows of LDS: 12 * W bytes)
+# thread, nearly the widest row that is taken (13,632: three rows of LDS, 12 * W bytes)
 @pytest.mark.parametrize("W,groups", [(4, 1), (252, 1), (256, 1), (260, 1), (512, 2), (768, 3), (768, 2), (1023, 1),
                                       (2048, 2), (2048, 8), (4096, 4), (4100, 1), (8192, 2), (13312, 4)])
 @pytest.mark.parametrize("rows", [1, 3, 513])
