@@ -307,6 +307,17 @@ __global__ __launch_bounds__(512, 4) void gemm_plain_split_kernel(const TA* __re
   }
 }
 
+// Rows of a workgroup of the split form, in eights. A workgroup of 8 rows is done soonest (its chains of multiply-adds and
+// reads of LDS are a quarter of those of 32 rows), one of 32 reads W a quarter as often: 8 rows while such workgroups have
+// a compute unit each (64 x 704 x 128: 32 rows 3.3 us, 16 2.8, 8 2.6; 32 x 1,024 x 2,816 15.4, 10.2, 8.2), 16 rows while
+// there are two of 8 to a unit (64 x 1,024 x 2,816 15.6, 10.9, 13.8; with a short K four: 128 x 1,000 x 128 3.5, 3.1, 4.2),
+// else 32 (96 x 1,024 x 2,816 16.1, 18.5, 19.5).
+static int gp_rows(int M, int N, int K) {
+  const long eights = ((long)M + 7) / 8 * (((long)N + 15) / 16), units = lmsf_compute_units();
+  if (M <= 8 || eights <= units) return 1;
+  return M <= 16 || eights <= (K <= 128 ? 4 : 2) * units ? 2 : 4;
+}
+
 template <typename TA, typename TW, typename TO, bool VEC>
 static void launch_gemm_plain_split(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, long ldc,
                                     int M, int N, int K, hipStream_t stream) {
@@ -314,12 +325,14 @@ static void launch_gemm_plain_split(const void* A, long lda, const void* W, long
 #define SPLIT(MR_)                                                                                                     \
   hipLaunchKernelGGL((gemm_plain_split_kernel<TA, TW, TO, MR_, VEC>), dim3((N + 15) / 16, (M + 8 * MR_ - 1) / (8 * MR_)), \
                      block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw, (const TW*)bias, (TO*)C, ldc, M, N, K)
-  if (M <= 8) SPLIT(1); else if (M <= 16) SPLIT(2); else SPLIT(4);
+  const int rows = gp_rows(M, N, K);
+  if (rows == 1) SPLIT(1); else if (rows == 2) SPLIT(2); else SPLIT(4);
 #undef SPLIT
 }
 
 // Whether the split form runs (``wide``: rows that allow wide loads; ``half``: an operand of 16 bits). It takes rows in
-// pieces of 32 x 16 outputs (8 or 16 rows where there are no more, for which a piece costs a quarter or half as much),
+// pieces of 32 x 16 outputs (8 or 16 rows where there are no more, for which a piece costs a quarter or half as much, or
+// where those run side by side: gp_rows),
 // which fill the chip where 64x64 tiles leave compute units without one, and K in eight parts, of which a K of one or two
 // steps leaves most waves without work. The tiles are ahead from a number of pieces a compute unit on that falls with K (two
 // workgroups run on a unit at once: up to K = 32 a second round already costs more than a tile's whole K) and that is

@@ -56,6 +56,19 @@ def test_a_row_does_not_hang_on_the_number_of_rows(ops, M, N, K, types):
     assert torch.equal(ops.linear(x[-33:], w, out_dtype=torch.float32), y[-33:])
 
 
+# each number of rows a workgroup (8, 16, 32) with more rows than one workgroup's, on either side of where it changes
+@pytest.mark.parametrize("M,N", [(17, 16 * 85), (17, 16 * 86), (33, 16 * 102), (33, 16 * 103), (65, 16 * 113), (65, 16 * 114)])
+@pytest.mark.parametrize("K", [128, 131, 260])
+def test_rows_of_a_workgroup_change_no_bit(ops, M, N, K):
+    g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
+    x, w = (torch.randn(n, K, generator=g, device="cuda:0") for n in (M, N))
+    y = ops.linear(x, w)
+    assert torch.equal(torch.cat([ops.linear(x[i:i + 8], w) for i in range(0, M, 8)]), y)
+    exact = x.double() @ w.double().T
+    bound = (x.double().abs() @ w.double().abs().T) * (16 * -(-K // 256) + 10) * 2.0 ** -24
+    assert ((y - exact).abs() <= bound).all()
+
+
 # as many rows as the grid of the split form takes (32 a workgroup), and one more
 @pytest.mark.parametrize("M", [65535 * 32, 65535 * 32 + 1])
 def test_product_of_very_many_rows(ops, M):
