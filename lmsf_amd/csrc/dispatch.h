@@ -52,7 +52,10 @@ enum {
   // a product that a norm finds unstarted
   LMSF_ROUTE_GEMV_ADD_NORM,   // adds into the stream, leaves stream * w and sums of squares (one or two rows)
   LMSF_ROUTE_SKINNY_ADD_NORM, // the same from the few-rows kernel
-  LMSF_ROUTE_GEMV_ADD         // adds into the stream; the norm kernel follows
+  LMSF_ROUTE_GEMV_ADD,        // adds into the stream; the norm kernel follows
+  // the float32 product's forms around a norm, a rotation and a gated activation (gemm_plain.hip: GpFused)
+  LMSF_ROUTE_PLAIN_ADD_NORM,  // adds into the stream; the product that reads the norm normalises the stream's rows itself
+  LMSF_ROUTE_PLAIN_FUSED      // gated or QKV product with its epilogue, of a tensor or of the stream with its norm to come
 };
 
 typedef struct {
@@ -70,18 +73,24 @@ typedef struct {
 // y = x W^T (+ bias). ``pending_ok``: the caller takes an unfinished product.
 void lmsf_route_linear(const LmsfTunables* t, const LmsfProductShape* s, int pending_ok, LmsfRoute* out);
 // act(x Wg^T) * (x Wu^T). ``scaled_rows_per_tile`` 0: x is a tensor; else x lacks its norm factor, with sums of
-// squares in ``scaled_tiles`` tiles of that many rows.
+// squares in ``scaled_tiles`` tiles of that many rows; LMSF_STREAM_ROWS: x is the float32 stream, its norm to come.
+#define LMSF_STREAM_ROWS (-1)
 void lmsf_route_linear_gated(const LmsfTunables* t, const LmsfProductShape* s, int scaled_rows_per_tile,
                              int scaled_tiles, LmsfRoute* out);
 // The QKV product with rotation and cache write. ``fused_shape``: the epilogue forms apply (a table and slots
 // are given, NeoX pairing over the whole head, a head size that is a multiple of 32, bfloat16 weight and pages,
-// the weight has (nh + 2 nkv) d rows of K columns).
+// the weight has (nh + 2 nkv) d rows of K columns; for float32 operands likewise, pages of float32 and a head size that
+// is a multiple of 16).
 void lmsf_route_qkv(const LmsfTunables* t, const LmsfProductShape* s, int fused_shape, int scaled_rows_per_tile,
                     LmsfRoute* out);
 // A norm whose branch is a product not yet started (M rows, N columns over K). ``fits``: the product has the
 // stream's shape and no rows are selected; ``prepares``: moreover the caller takes rows without their factor and
-// the norm's output and weight are bfloat16.
+// the norm's output and weight are bfloat16. ``fits`` 2: the same of float32 operands; then ``prepares`` says that the
+// caller takes the stream with its norm to come and that output and weight are float32.
 void lmsf_route_deferred_norm(const LmsfTunables* t, int M, int N, int K, int fits, int prepares, LmsfRoute* out);
+// A norm over the float32 stream [M, N] alone, nothing to add and no rows selected, output and weight float32: whether
+// the product that reads it should normalise the rows itself.
+int lmsf_route_stream_norm(const LmsfTunables* t, int M, int N);
 // How the decode attention kernel splits the keys of a step of ``n_single`` single tokens whose longest context
 // is ``max_context``: keys a split (a multiple of 128) and the number of splits.
 void lmsf_route_decode_attention(const LmsfTunables* t, int n_single, int nh, int nkv, int max_context, int* chunk,

@@ -20,6 +20,20 @@ inline bool mid_ok(const LmsfProductShape& s) {
 // the one-or-two-rows kernel keeps x in LDS
 inline bool gemv_ok(int M, int K) { return (long)M * K * 2 <= 128 * 1024; }
 
+inline bool all_f32(const LmsfProductShape& s) {
+  return s.x_dtype == LMSF_F32 && s.w_dtype == LMSF_F32 && s.out_dtype == LMSF_F32;
+}
+// what the float32 product's fused forms ask: rows read wide, and sizes at which the form with K over the waves runs
+inline bool plain_fused_ok(const LmsfTunables* t, const LmsfProductShape& s, bool normed) {
+  return t->fuse_norm_rows > 0 && all_f32(s) && s.K % 4 == 0 && s.ldx % 4 == 0 && s.ldw % 4 == 0 && s.x_ok16 && s.w_ok16 &&
+         lmsf_gemm_plain_fused_fits(s.M, s.N, s.K, normed);
+}
+// Whether the norm over [M, N] is left to the product that reads it, of which only K = N is known here: as if it had as
+// many outputs. (One with more that does not take it runs the norm's kernel first, as without all this.)
+inline bool stream_norm_ok(const LmsfTunables* t, int M, int N) {
+  return t->fuse_norm_rows > 0 && lmsf_gemm_plain_fused_fits(M, N, N, 1);
+}
+
 inline LmsfRoute route(int r) {
   LmsfRoute o;
   o.route = r;
@@ -61,6 +75,10 @@ extern "C" void lmsf_route_linear(const LmsfTunables* t, const LmsfProductShape*
     *out = route(LMSF_ROUTE_DEFERRED);
     return;
   }
+  if (pending_ok && plain_fused_ok(t, s, false) && stream_norm_ok(t, M, N)) {
+    *out = route(LMSF_ROUTE_DEFERRED);
+    return;
+  }
   // one row: a pure stream of W (with two rows only the fused forms gain; the LM head's matrix is large enough for
   // the few-rows kernel to reach the same rate, so it stays there)
   if (bf && 0 < M && M <= std::min(1, t->gemv_max_rows) && s_ok && gemv_ok(M, K) && (long)N * K <= (1L << 28)) {
@@ -92,6 +110,11 @@ extern "C" void lmsf_route_linear_gated(const LmsfTunables* t, const LmsfProduct
                                         int scaled_tiles, LmsfRoute* out) {
   const LmsfProductShape& s = *sp;
   const int M = s.M, I = s.N / 2, K = s.K;
+  const bool normed = scaled_rows_per_tile == LMSF_STREAM_ROWS;
+  if (normed || (scaled_rows_per_tile == 0 && plain_fused_ok(t, s, false))) {
+    *out = route(!normed || plain_fused_ok(t, s, true) ? LMSF_ROUTE_PLAIN_FUSED : LMSF_ROUTE_MATERIALIZE);
+    return;
+  }
   if (scaled_rows_per_tile != 0) {
     if (!(s.w_dtype == LMSF_BF16 && skinny_ok(s) && (scaled_rows_per_tile == 16 || gemv_ok(M, K)))) {
       *out = route(LMSF_ROUTE_MATERIALIZE);
@@ -129,14 +152,19 @@ extern "C" void lmsf_route_qkv(const LmsfTunables* t, const LmsfProductShape* sp
                                int scaled_rows_per_tile, LmsfRoute* out) {
   const LmsfProductShape& s = *sp;
   const int M = s.M, K = s.K;
+  const bool normed = scaled_rows_per_tile == LMSF_STREAM_ROWS, plain_fused = fused_shape && plain_fused_ok(t, s, normed);
+  if (normed || (scaled_rows_per_tile == 0 && plain_fused)) {
+    *out = route(plain_fused ? LMSF_ROUTE_PLAIN_FUSED : LMSF_ROUTE_MATERIALIZE);
+    return;
+  }
   if (scaled_rows_per_tile != 0) {
-    if (fused_shape && skinny_ok(s) && (scaled_rows_per_tile == 16 || gemv_ok(M, K)))
+    if (fused_shape && s.w_dtype == LMSF_BF16 && skinny_ok(s) && (scaled_rows_per_tile == 16 || gemv_ok(M, K)))
       *out = route(scaled_rows_per_tile != 16 ? LMSF_ROUTE_GEMV_SCALED : LMSF_ROUTE_SKINNY_SCALED);
     else
       *out = route(LMSF_ROUTE_MATERIALIZE);
     return;
   }
-  if (fused_shape && s.x_dtype == LMSF_BF16 && 0 < M && M <= std::min(64, std::max(t->skinny_max_rows, t->qkv_fused_max_rows)) &&
+  if (fused_shape && both_bf16(s) && 0 < M && M <= std::min(64, std::max(t->skinny_max_rows, t->qkv_fused_max_rows)) &&
       skinny_ok(s)) {
     *out = route(M <= t->gemv_max_rows && gemv_ok(M, K) ? LMSF_ROUTE_GEMV : LMSF_ROUTE_SKINNY);
     return;
@@ -144,11 +172,15 @@ extern "C" void lmsf_route_qkv(const LmsfTunables* t, const LmsfProductShape* sp
   // the plain product, unfinished where it splits K (the rotation and the cache write then add up the partial sums),
   // but never as a product not yet started
   *out = route(LMSF_ROUTE_SEPARATE);
-  out->pending = M > std::max(std::max(t->fuse_stream_rows, t->fuse_norm_rows), t->skinny_max_rows);
+  out->pending = both_bf16(s) && M > std::max(std::max(t->fuse_stream_rows, t->fuse_norm_rows), t->skinny_max_rows);
 }
 
 extern "C" void lmsf_route_deferred_norm(const LmsfTunables* t, int M, int N, int K, int fits, int prepares,
                                          LmsfRoute* out) {
+  if (fits == 2) {      // (with the norm's kernel to follow all the same, that kernel adds as fast)
+    *out = route(prepares && stream_norm_ok(t, M, N) ? LMSF_ROUTE_PLAIN_ADD_NORM : LMSF_ROUTE_MATERIALIZE);
+    return;
+  }
   const bool one_or_two = fits && M <= std::min(t->fuse_stream_rows, t->gemv_max_rows) && gemv_ok(M, K);
   if (prepares && one_or_two && gemv_ok(M, N))
     *out = route(LMSF_ROUTE_GEMV_ADD_NORM);
@@ -159,6 +191,8 @@ extern "C" void lmsf_route_deferred_norm(const LmsfTunables* t, int M, int N, in
   else
     *out = route(LMSF_ROUTE_MATERIALIZE);
 }
+
+extern "C" int lmsf_route_stream_norm(const LmsfTunables* t, int M, int N) { return stream_norm_ok(t, M, N) ? 1 : 0; }
 
 // Measured: about 512 workgroups fill the chip; beyond that a split only adds partial results, and with two short
 // halves the reduction kernel costs more than the second half saves. With contexts of tens of thousands of keys

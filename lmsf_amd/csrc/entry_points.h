@@ -191,6 +191,15 @@ int lmsf_gemm_mid_reduce(const float* scratch, const void* bias, void* y, int ou
 // gemm_plain.hip
 int lmsf_gemm_plain(const void* A, int a_dtype, long lda, const void* W, int w_dtype, long ldw, const void* bias,
     void* C, int c_dtype, long ldc, int M, int N, int K, hipStream_t stream);
+int lmsf_gemm_plain_fused_fits(int M, int N, int K, int normed);
+int lmsf_gemm_plain_add(const float* x, long ldx, const float* W, long ldw, const float* bias, float* stream_out, long
+    ldy, int M, int N, int K, hipStream_t stream);
+int lmsf_gemm_plain_gated(const float* x, long ldx, const float* W, long ldw, const float* bias, float* y, long ldy, int
+    M, int I, int K, int act, const float* norm_weight, float eps, float weight_offset, hipStream_t stream);
+int lmsf_gemm_plain_qkv(const float* x, long ldx, const float* W, long ldw, const float* bias, float* y, long ldy, int
+    M, int K, const int* positions, const float* table, int max_pos, const int* slots, float* k_pages, float* v_pages,
+    long num_pages, int nh, int nkv, int d, int ps, const float* norm_weight, float eps, float weight_offset,
+    hipStream_t stream);
 
 // gemm_skinny.hip
 int lmsf_gemm_skinny(const void* x, long ldx, const void* W, long ldw, const void* bias, void* y, int out_dtype, long

@@ -233,41 +233,106 @@ __device__ __forceinline__ float4 gp_load4(const bf16_t* p, int k, int K) {
                      k + 2 < K ? bf16_to_f32(p[k + 2]) : 0.f, k + 3 < K ? bf16_to_f32(p[k + 3]) : 0.f);
 }
 
-template <typename TA, typename TW, typename TO, int MR, bool VEC>
+// What a product of the split form does beside multiplying (GP_PLAIN: nothing), float32 operands read wide only. With few
+// rows a kernel between two products costs its start and end and little else (3.5 us in a captured step), so a decoder
+// block's products do the work around them, to the bits of the kernels they replace:
+//   GP_ADD    the product is added to C, the float32 residual stream;
+//   GP_GATED  act(gate) * up of W's two halves of I rows: a workgroup's two times eight rows of W are the gate's and the up
+//             projection's of eight outputs;
+//   GP_QKV    the fused QKV projection: the two times eight rows are those of eight rotation pairs (i, i + d / 2) of a
+//             head, which the epilogue rotates and stores, in the cache too.
+// NORM: A is the residual stream and its rows are normalised on the way in, x * inv * (w + offset); every workgroup makes
+// the factors of its own rows, adding up squares in the order of the norm's kernel (a wave's 64 lanes hold four
+// neighbours each, the parts of 256 columns are added in turn), while its first rows of W are on their way.
+enum { GP_PLAIN = 0, GP_ADD, GP_GATED, GP_QKV };
+
+struct GpFused {
+  const float* norm_weight;         // NORM: [K]
+  float eps, weight_offset;
+  int act;                          // GP_GATED: 1 SiLU, 2 GELU
+  // GP_QKV, pages of float32 (common.h: RopeCacheArgs)
+  const int* positions;
+  const float* table;
+  const int* slots;
+  float *k_pages, *v_pages;
+  int nh, nkv, d, ps;
+};
+
+template <typename TA, typename TW, typename TO, int MR, bool VEC, int FORM = GP_PLAIN, bool NORM = false>
 __global__ __launch_bounds__(512, 4) void gemm_plain_split_kernel(const TA* __restrict__ A, long lda,
                                                                const TW* __restrict__ W, long ldw,
                                                                const TW* __restrict__ bias, TO* __restrict__ C,
-                                                               long ldc, int M, int N, int K) {
+                                                               long ldc, int M, int N, int K, GpFused fu) {
   constexpr int ROWS = 8 * MR + 16;                 // of A, then of W
+  constexpr bool PAIRS = FORM == GP_GATED || FORM == GP_QKV;
   static_assert(ROWS * GP_ROW >= MR * 128, "the waves' sums lie where their steps lay");
+  static_assert(FORM == GP_PLAIN ? !NORM : (VEC && sizeof(TA) == 4 && sizeof(TW) == 4 && sizeof(TO) == 4), "float32 forms");
   __shared__ __align__(16) float area[8][ROWS * GP_ROW];
+  __shared__ float factor[NORM ? 8 * MR : 1];
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r = lane >> 3, c = lane & 7;
   const int m0 = blockIdx.y * (8 * MR), n0 = blockIdx.x * 16;
   float* mine = area[wave];
+  // rows of W: ``first`` + 0..7 and ``second`` + 0..7 (PAIRS: outputs o0 .. o0 + 7 of either half; o0 is within one head)
+  const int half = FORM == GP_QKV ? fu.d / 2 : FORM == GP_GATED ? N / 2 : 8;
+  const int o0 = n0 / 2, first = FORM == GP_QKV ? o0 / half * fu.d + o0 % half : PAIRS ? o0 : n0, second = first + half;
   const TA* a[MR];
   const TW* w[2];
 #pragma unroll
   for (int i = 0; i < MR; ++i) a[i] = A + (long)min(m0 + r + 8 * i, M - 1) * lda;   // rows beyond M: not written
 #pragma unroll
-  for (int j = 0; j < 2; ++j) w[j] = W + (long)min(n0 + r + 8 * j, N - 1) * ldw;
+  for (int j = 0; j < 2; ++j) {
+    const int row = FORM == GP_GATED ? min(first + r, half - 1) + j * half : min((j ? second : first) + r, N - 1);
+    w[j] = W + (long)row * ldw;
+  }
   float acc[MR][2][2];        // of the even and of the odd k: two short chains instead of one
 #pragma unroll
   for (int i = 0; i < MR; ++i)
 #pragma unroll
     for (int e = 0; e < 2; ++e) acc[i][0][e] = acc[i][1][e] = 0.f;
-  float4 x[MR], y[2];
+  float4 x[MR], y[2], g;
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < MR; ++i) x[i] = gp_load4<VEC>(a[i], k0 + 4 * c, K);
 #pragma unroll
     for (int j = 0; j < 2; ++j) y[j] = gp_load4<VEC>(w[j], k0 + 4 * c, K);
+    if (NORM) g = gp_load4<VEC>(fu.norm_weight, k0 + 4 * c, K);
   };
   int k0 = gp_part(wave, K);
   const int end = gp_part(wave + 1, K);
   if (k0 < end) fetch(k0);
+  float inv[MR];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < MR; ++i) {
+      const float* row = reinterpret_cast<const float*>(A) + (long)min(m0 + wave * MR + i, M - 1) * lda;
+      float total = 0.f;
+#pragma unroll 4
+      for (int k = 0; k < K; k += 256) {
+        const float4 v = gp_load4<true>(row, k + 4 * lane, K);
+        float ss = 0.f;
+        ss += v.x * v.x;
+        ss += v.y * v.y;
+        ss += v.z * v.z;
+        ss += v.w * v.w;
+        total += wave_sum(ss);
+      }
+      if (lane == 0) factor[wave * MR + i] = rsqrtf(total / (float)K + fu.eps);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MR; ++i) inv[i] = factor[r + 8 * i];
+  }
   for (; k0 < end; k0 += GP_STEP) {
 #pragma unroll
-    for (int i = 0; i < MR; ++i) *reinterpret_cast<float4*>(mine + (r + 8 * i) * GP_ROW + 4 * c) = x[i];
+    for (int i = 0; i < MR; ++i) {
+      if (NORM) {
+        x[i].x = x[i].x * inv[i] * (g.x + fu.weight_offset);
+        x[i].y = x[i].y * inv[i] * (g.y + fu.weight_offset);
+        x[i].z = x[i].z * inv[i] * (g.z + fu.weight_offset);
+        x[i].w = x[i].w * inv[i] * (g.w + fu.weight_offset);
+      }
+      *reinterpret_cast<float4*>(mine + (r + 8 * i) * GP_ROW + 4 * c) = x[i];
+    }
 #pragma unroll
     for (int j = 0; j < 2; ++j) *reinterpret_cast<float4*>(mine + (8 * MR + r + 8 * j) * GP_ROW + 4 * c) = y[j];
     if (k0 + GP_STEP < end) fetch(k0 + GP_STEP);
@@ -295,15 +360,54 @@ __global__ __launch_bounds__(512, 4) void gemm_plain_split_kernel(const TA* __re
 #pragma unroll
     for (int j = 0; j < 2; ++j) mine[(i * 2 + j) * 64 + lane] = acc[i][j][0] + acc[i][j][1];
   __syncthreads();
-  for (int e = tid; e < MR * 128; e += 512) {
-    const int l = e & 63, j = (e >> 6) & 1, i = e >> 7;
-    const int m = m0 + l / 8 + 8 * i, n = n0 + l % 8 + 8 * j;
-    if (m >= M || n >= N) continue;
+  auto finished = [&](int e, int n) {      // the waves' sums of entry e, and column n's bias
     float s = 0.f;
 #pragma unroll
     for (int v = 0; v < GP_PARTS; ++v) s += area[v][e];
     if (bias) s += to_f32<TW>(bias[n]);
-    C[(long)m * ldc + n] = from_f32<TO>(s);
+    return s;
+  };
+  if constexpr (!PAIRS) {
+    for (int e = tid; e < MR * 128; e += 512) {
+      const int l = e & 63, j = (e >> 6) & 1, i = e >> 7;
+      const int m = m0 + l / 8 + 8 * i, n = n0 + l % 8 + 8 * j;
+      if (m >= M || n >= N) continue;
+      const float s = finished(e, n);
+      TO* to = C + (long)m * ldc + n;
+      if constexpr (FORM == GP_ADD) *to = s + *to; else *to = from_f32<TO>(s);
+    }
+  } else {
+    for (int e = tid; e < MR * 64; e += 512) {
+      const int l = e & 63, i = e >> 6, at = i * 128 + l;
+      const int m = m0 + l / 8 + 8 * i, o = first + l % 8;
+      if (m >= M || (FORM == GP_GATED && o >= half)) continue;
+      const float u = finished(at, o), v = finished(at + 64, o + half);
+      if constexpr (FORM == GP_GATED) {
+        C[(long)m * ldc + o] = (fu.act == 1 ? gated_product_activation<1>(u) : gated_product_activation<2>(u)) * v;
+      } else {
+        const int head = o / fu.d, at_d = o - head * fu.d;
+        float lo = u, hi = v;
+        if (head < fu.nh + fu.nkv) {
+          const float* cs = fu.table + (long)fu.positions[m] * fu.d;
+          rope_rotate(u, v, cs[at_d], cs[half + at_d], &lo, &hi);
+        }
+        C[(long)m * ldc + o] = lo;
+        C[(long)m * ldc + o + half] = hi;
+        const int slot = head >= fu.nh ? fu.slots[m] : -1;
+        if (slot >= 0) {
+          const int page = slot / fu.ps, off = slot - page * fu.ps;
+          if (head < fu.nh + fu.nkv) {
+            float* dst = fu.k_pages + (((long)page * fu.nkv + (head - fu.nh)) * fu.ps + off) * fu.d + at_d;
+            dst[0] = lo;
+            dst[half] = hi;
+          } else {
+            float* dst = fu.v_pages + (((long)page * fu.nkv + (head - fu.nh - fu.nkv)) * fu.d + at_d) * fu.ps + off;
+            dst[0] = lo;
+            dst[(long)half * fu.ps] = hi;
+          }
+        }
+      }
+    }
   }
 }
 
@@ -324,10 +428,24 @@ static void launch_gemm_plain_split(const void* A, long lda, const void* W, long
   const dim3 block(512);
 #define SPLIT(MR_)                                                                                                     \
   hipLaunchKernelGGL((gemm_plain_split_kernel<TA, TW, TO, MR_, VEC>), dim3((N + 15) / 16, (M + 8 * MR_ - 1) / (8 * MR_)), \
-                     block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw, (const TW*)bias, (TO*)C, ldc, M, N, K)
+                     block, 0, stream, (const TA*)A, lda, (const TW*)W, ldw, (const TW*)bias, (TO*)C, ldc, M, N, K, GpFused())
   const int rows = gp_rows(M, N, K);
   if (rows == 1) SPLIT(1); else if (rows == 2) SPLIT(2); else SPLIT(4);
 #undef SPLIT
+}
+
+template <int FORM, bool NORM>
+static void launch_gemm_plain_fused(const float* A, long lda, const float* W, long ldw, const float* bias, float* C,
+                                    long ldc, int M, int N, int K, const GpFused& fu, hipStream_t stream) {
+  const dim3 block(512);
+  constexpr int MOST = NORM ? 2 : 4;      // (many rows leave the norm to its kernel)
+#define FUSED(MR_)                                                                                                     \
+  hipLaunchKernelGGL((gemm_plain_split_kernel<float, float, float, MR_, true, FORM, NORM>),                            \
+                     dim3((N + 15) / 16, (M + 8 * MR_ - 1) / (8 * MR_)), block, 0, stream, A, lda, W, ldw, bias, C, ldc, \
+                     M, N, K, fu)
+  const int rows = gp_rows(M, N, K);
+  if (rows == 1) FUSED(1); else if (rows == 2) FUSED(2); else FUSED(MOST);
+#undef FUSED
 }
 
 // Whether the split form runs (``wide``: rows that allow wide loads; ``half``: an operand of 16 bits). It takes rows in
@@ -405,5 +523,88 @@ extern "C" int lmsf_gemm_plain(const void* A, int a_dtype, long lda, const void*
       return 1;
   }
   LMSF_LAUNCH_CHECK("gemm_plain");
+  return 0;
+}
+
+// The split form's fused products (float32 throughout; see GpFused): whether a product of these sizes runs in the split
+// form at all, and (``normed``) whether it should normalise its rows itself. N: rows of W. K and the row strides a multiple
+// of 4, 16-byte aligned operands. Every workgroup makes its rows' factors anew, which pays for itself while there are two
+// workgroups of 8 rows to a compute unit, one beyond K = 512 (norm, gated product with its activation -> all in one:
+// 8 x 704 x 128 4.6 -> 3.2 us, 64 x 704 x 128 4.7 -> 3.8, 128 x 1,000 x 128 5.1 -> 4.9, 32 x 1,408 x 256 5.0 -> 4.0, 96 rows
+// 6.3 -> 6.7; 16 x 704 x 1,024 6.3 -> 6.0, 48 rows 7.4 -> 8.6; 8 x 5,632 x 1,024 9.0 -> 8.2, x 11,264 x 2,048 20.3 -> 20.9).
+extern "C" int lmsf_gemm_plain_fused_fits(int M, int N, int K, int normed) {
+  if (M <= 0 || K % 4 != 0 || !gp_split(M, N, K, true, false)) return 0;
+  const long eights = ((long)M + 7) / 8 * (((long)N + 15) / 16);
+  return !normed || (K <= 1024 && eights <= (K <= 512 || M <= 8 ? 2 : 1) * lmsf_compute_units()) ? 1 : 0;
+}
+
+static int fused_check(const char* who, const float* x, long ldx, const float* W, long ldw, const float* y, long ldy, int M,
+                       int N, int K, long width) {
+  LMSF_CHECK(x && W && y, "%s: null pointer", who);
+  LMSF_CHECK(M >= 0 && N > 0 && K > 0 && K % 4 == 0, "%s: bad sizes M=%d N=%d K=%d", who, M, N, K);
+  LMSF_CHECK(N <= 1 << 26 && (M + 7) / 8 <= 65535, "%s: M=%d N=%d too large", who, M, N);
+  LMSF_CHECK(ldx >= K && ldw >= K && ldy >= width && ldx % 4 == 0 && ldw % 4 == 0, "%s: bad row strides", who);
+  LMSF_CHECK(lmsf_aligned16(x) && lmsf_aligned16(W), "%s: x and W must be 16-byte aligned", who);
+  return 0;
+}
+static int norm_check(const char* who, const float* norm_weight, int K, float eps) {
+  // (the norm's kernel adds up squares in another order beyond)
+  LMSF_CHECK(norm_weight == nullptr || (lmsf_aligned16(norm_weight) && K <= 4096 && eps > 0.f),
+             "%s: rows of up to 4,096 columns are normalised, by an aligned weight", who);
+  return 0;
+}
+
+// stream += x W^T + bias; stream [M, N] float32 with row stride ldy.
+extern "C" int lmsf_gemm_plain_add(const float* x, long ldx, const float* W, long ldw, const float* bias, float* stream_out,
+                                   long ldy, int M, int N, int K, hipStream_t stream) {
+  if (int rc = fused_check("gemm_plain_add", x, ldx, W, ldw, stream_out, ldy, M, N, K, N)) return rc;
+  if (M == 0) return 0;
+  launch_gemm_plain_fused<GP_ADD, false>(x, ldx, W, ldw, bias, stream_out, ldy, M, N, K, GpFused(), stream);
+  LMSF_LAUNCH_CHECK("gemm_plain_add");
+  return 0;
+}
+
+// act(x Wg^T + bg) * (x Wu^T + bu) for W [2 I, K] = [Wg; Wu]; y [M, I]; act 1 SiLU, 2 GELU. With ``norm_weight`` [K] x is
+// the residual stream and its rows are normalised first, x * rsqrt(mean(x^2) + eps) * (norm_weight + weight_offset).
+extern "C" int lmsf_gemm_plain_gated(const float* x, long ldx, const float* W, long ldw, const float* bias, float* y, long ldy,
+                                     int M, int I, int K, int act, const float* norm_weight, float eps, float weight_offset,
+                                     hipStream_t stream) {
+  if (int rc = fused_check("gemm_plain_gated", x, ldx, W, ldw, y, ldy, M, 2 * I, K, I)) return rc;
+  if (int rc = norm_check("gemm_plain_gated", norm_weight, K, eps)) return rc;
+  LMSF_CHECK(act == 1 || act == 2, "gemm_plain_gated: activation %d (1 silu, 2 gelu)", act);
+  if (M == 0) return 0;
+  GpFused fu = GpFused();
+  fu.norm_weight = norm_weight; fu.eps = eps; fu.weight_offset = weight_offset; fu.act = act;
+  if (norm_weight)
+    launch_gemm_plain_fused<GP_GATED, true>(x, ldx, W, ldw, bias, y, ldy, M, 2 * I, K, fu, stream);
+  else
+    launch_gemm_plain_fused<GP_GATED, false>(x, ldx, W, ldw, bias, y, ldy, M, 2 * I, K, fu, stream);
+  LMSF_LAUNCH_CHECK("gemm_plain_gated");
+  return 0;
+}
+
+// The fused QKV projection, the rotation of its q and k heads over the whole head (NeoX pairing, d a multiple of 16) and
+// the write of k and v into float32 pages; arguments as lmsf_gemm_qkv_rope_cache, ``norm_weight`` as above.
+extern "C" int lmsf_gemm_plain_qkv(const float* x, long ldx, const float* W, long ldw, const float* bias, float* y, long ldy,
+                                   int M, int K, const int* positions, const float* table, int max_pos, const int* slots,
+                                   float* k_pages, float* v_pages, long num_pages, int nh, int nkv, int d, int ps,
+                                   const float* norm_weight, float eps, float weight_offset, hipStream_t stream) {
+  LMSF_CHECK(positions && table && slots && k_pages && v_pages, "gemm_plain_qkv: null pointer");
+  LMSF_CHECK(nh > 0 && nkv > 0 && d > 0 && d % 16 == 0, "gemm_plain_qkv: head size %d must be a multiple of 16", d);
+  LMSF_CHECK(ps > 0 && num_pages > 0 && max_pos > 0, "gemm_plain_qkv: bad page geometry or empty table");
+  const long N = (long)(nh + 2 * nkv) * d;
+  LMSF_CHECK(N <= 1 << 26, "gemm_plain_qkv: %ld columns", N);
+  if (int rc = fused_check("gemm_plain_qkv", x, ldx, W, ldw, y, ldy, M, (int)N, K, N)) return rc;
+  if (int rc = norm_check("gemm_plain_qkv", norm_weight, K, eps)) return rc;
+  if (M == 0) return 0;
+  GpFused fu = GpFused();
+  fu.norm_weight = norm_weight; fu.eps = eps; fu.weight_offset = weight_offset;
+  fu.positions = positions; fu.table = table; fu.slots = slots; fu.k_pages = k_pages; fu.v_pages = v_pages;
+  fu.nh = nh; fu.nkv = nkv; fu.d = d; fu.ps = ps;
+  if (norm_weight)
+    launch_gemm_plain_fused<GP_QKV, true>(x, ldx, W, ldw, bias, y, ldy, M, (int)N, K, fu, stream);
+  else
+    launch_gemm_plain_fused<GP_QKV, false>(x, ldx, W, ldw, bias, y, ldy, M, (int)N, K, fu, stream);
+  LMSF_LAUNCH_CHECK("gemm_plain_qkv");
   return 0;
 }

@@ -119,7 +119,7 @@ typedef int (*LmsfCallbackFn)(const LmsfCallbackArgs* args);
 // What the last step that ran launched, by kind (lmsf_program_stats): the routes of dispatch.h for the products
 // (plain, gated and QKV alike), then the kernels that take an unfinished product, then attention and callbacks.
 enum {
-  LMSF_STAT_NORM_OVER_PARTIALS = 16,
+  LMSF_STAT_NORM_OVER_PARTIALS = 18,
   LMSF_STAT_ROPE_OVER_PARTIALS,
   LMSF_STAT_REDUCE_PARTIALS,
   LMSF_STAT_PREFILL_ATTENTION,

@@ -48,7 +48,8 @@ struct Value {
   int K = 0;
   const void* W = nullptr;
   long ldw = 0;
-  // scaled rows: sums of squares [tiles][rows_per_tile] and what the norm kernel would need instead
+  // scaled rows: sums of squares [tiles][rows_per_tile] and what the norm kernel would need instead; LMSF_STREAM_ROWS: no
+  // sums, p is the float32 stream itself, which the product that reads it normalises
   float* sumsq = nullptr;
   int tiles = 0, rows_per_tile = 0;
   float eps = 0.f, weight_offset = 0.f;
@@ -327,11 +328,11 @@ int materialize(Run& r, const Value& v, Value* res) {
     *res = v;
     return 0;
   }
-  if (v.kind == V_DEFERRED) {
-    const Value x = tensor(const_cast<void*>(v.x), LMSF_BF16, v.M, v.K);
+  if (v.kind == V_DEFERRED) {      // (operands and result of one type)
+    const Value x = tensor(const_cast<void*>(v.x), v.dtype, v.M, v.K);
     Value xs = x;
     xs.ld = v.ldx;
-    return op_linear(r, xs, v.W, LMSF_BF16, v.ldw, v.N, v.bias, v.dtype, false, nullptr, res);
+    return op_linear(r, xs, v.W, v.dtype, v.ldw, v.N, v.bias, v.dtype, false, nullptr, res);
   }
   if (v.kind == V_SCALED) {
     Value none;
@@ -347,6 +348,19 @@ int materialize(Run& r, const Value& v, Value* res) {
   }
   lmsf_set_error("program: an operation reads a register that holds nothing");
   return 1;
+}
+
+// The norm over the float32 stream, left to the product that reads it
+Value stream_rows(float* stream, int M, int H, const void* weight, float eps, float weight_offset) {
+  Value v = tensor(stream, LMSF_F32, M, H);
+  v.kind = V_SCALED;
+  v.rows_per_tile = LMSF_STREAM_ROWS;
+  v.eps = eps;
+  v.weight_offset = weight_offset;
+  v.norm_weight = weight;
+  v.norm_wdtype = LMSF_F32;
+  v.stream = stream;
+  return v;
 }
 
 // HipOps.add_rms_norm, with _run_deferred and _add_rms_norm_pending. M: rows of the operands; rows/n_rows select
@@ -374,10 +388,17 @@ int op_add_rms_norm(Run& r, const Value& branch_in, float* residual, int M, int 
   if (branch.kind == V_DEFERRED) {
     const int Mb = branch.M, N = branch.N, K = branch.K;
     const bool fits = rows == nullptr && residual != nullptr && Mb == M && N == H;
-    const bool prepares = fits && defer_ok && out_dtype == LMSF_BF16 && wdtype == LMSF_BF16;
+    const bool prepares = fits && defer_ok && out_dtype == branch.dtype && wdtype == branch.dtype &&
+                          (branch.dtype == LMSF_BF16 || lmsf_aligned16(weight));
     LmsfRoute rt;
-    lmsf_route_deferred_norm(&t, Mb, N, K, fits ? 1 : 0, prepares ? 1 : 0, &rt);
+    lmsf_route_deferred_norm(&t, Mb, N, K, !fits ? 0 : branch.dtype == LMSF_F32 ? 2 : 1, prepares ? 1 : 0, &rt);
     if (rt.route != LMSF_ROUTE_MATERIALIZE) r.count(rt.route);
+    if (rt.route == LMSF_ROUTE_PLAIN_ADD_NORM) {
+      LAUNCH(lmsf_gemm_plain_add((const float*)branch.x, branch.ldx, (const float*)branch.W, branch.ldw,
+                                 (const float*)branch.bias, residual, H, Mb, N, K, r.stream));
+      *res = stream_rows(residual, M, H, weight, eps, weight_offset);
+      return 0;
+    }
     if (rt.route == LMSF_ROUTE_GEMV_ADD_NORM || rt.route == LMSF_ROUTE_SKINNY_ADD_NORM) {
       const bool one_or_two = rt.route == LMSF_ROUTE_GEMV_ADD_NORM;
       const int tiles = one_or_two ? lmsf_gemv_partials(N) : (N + 15) / 16;
@@ -417,6 +438,11 @@ int op_add_rms_norm(Run& r, const Value& branch_in, float* residual, int M, int 
     RC(materialize(r, branch, &m));
     branch = m;
   }
+  if (branch_in.kind == V_NONE && residual != nullptr && rows == nullptr && defer_ok && out_dtype == LMSF_F32 &&
+      wdtype == LMSF_F32 && lmsf_aligned16(weight) && lmsf_route_stream_norm(&t, M, H)) {
+    *res = stream_rows(residual, M, H, weight, eps, weight_offset);
+    return 0;
+  }
   if (branch.kind == V_NONE && residual == nullptr) {
     lmsf_set_error("program: a norm without operands");
     return 1;
@@ -432,6 +458,17 @@ int op_add_rms_norm(Run& r, const Value& branch_in, float* residual, int M, int 
   return 0;
 }
 
+// the float32 gated product, of a tensor or of the stream with its norm to come
+int gated_plain(Run& r, const Value& x, const void* W, long ldw, int I, const void* bias, int kind, Value* res) {
+  const float* norm = x.kind == V_SCALED ? (const float*)x.norm_weight : nullptr;
+  r.count(LMSF_ROUTE_PLAIN_FUSED);
+  TAKE(y, float*, (size_t)x.M * I * 4);
+  LAUNCH(lmsf_gemm_plain_gated((const float*)x.p, x.ld, (const float*)W, ldw, (const float*)bias, y, I, x.M, I, x.N, kind,
+                               norm, x.eps, x.weight_offset, r.stream));
+  *res = tensor(y, LMSF_F32, x.M, I);
+  return 0;
+}
+
 // act(x Wg^T) * (x Wu^T); kind 1: SiLU, 2: GELU (HipOps.linear_gated launches the same kernels for the same routes)
 int op_linear_gated(Run& r, const Value& x_in, const void* W, int wdtype, long ldw, int w_rows, const void* bias,
                     int kind, Value* res) {
@@ -440,8 +477,9 @@ int op_linear_gated(Run& r, const Value& x_in, const void* W, int wdtype, long l
   const int I = w_rows / 2;
   LmsfRoute rt;
   if (x.kind == V_SCALED) {
-    const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, x.M, x.N, W, wdtype, ldw, w_rows, LMSF_BF16);
+    const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, x.M, x.N, W, wdtype, ldw, w_rows, x.dtype);
     lmsf_route_linear_gated(&t, &shape, x.rows_per_tile, x.tiles, &rt);
+    if (rt.route == LMSF_ROUTE_PLAIN_FUSED) return gated_plain(r, x, W, ldw, I, bias, kind, res);
     if (rt.route != LMSF_ROUTE_MATERIALIZE) {
       r.count(rt.route);
       const int M = x.M, K = x.N;
@@ -465,6 +503,7 @@ int op_linear_gated(Run& r, const Value& x_in, const void* W, int wdtype, long l
   const int M = x.M, K = x.N;
   const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, W, wdtype, ldw, w_rows, x.dtype);
   lmsf_route_linear_gated(&t, &shape, 0, 0, &rt);
+  if (rt.route == LMSF_ROUTE_PLAIN_FUSED) return gated_plain(r, x, W, ldw, I, bias, kind, res);
   if (rt.route != LMSF_ROUTE_SEPARATE) r.count(rt.route);
   if (rt.route == LMSF_ROUTE_GEMV || rt.route == LMSF_ROUTE_SKINNY) {
     TAKE(y, void*, (size_t)M * I * 2);
@@ -505,14 +544,26 @@ int op_qkv_rope_cache(Run& r, const Value& x_in, const LmsfOpDesc& op, const int
   const int N = (op.nh + 2 * op.nkv) * op.d;
   const float* table = (const float*)op.table;
   const auto fused_shape = [&](int K) {
-    return table != nullptr && slots != nullptr && op.neox && op.rot == op.d && op.d % 32 == 0 &&
-           op.wdtype == LMSF_BF16 && op.N == N && op.K == K && op.k_pages != nullptr && op.cache_dtype == LMSF_BF16;
+    return table != nullptr && slots != nullptr && op.neox && op.rot == op.d &&
+           op.d % (op.wdtype == LMSF_F32 ? 16 : 32) == 0 && op.N == N && op.K == K && op.k_pages != nullptr &&
+           op.cache_dtype == op.wdtype;
+  };
+  const auto plain = [&](const Value& v) -> int {      // the float32 product, of a tensor or of the stream with its norm to come
+    const float* norm = v.kind == V_SCALED ? (const float*)v.norm_weight : nullptr;
+    r.count(LMSF_ROUTE_PLAIN_FUSED);
+    TAKE(y, float*, (size_t)v.M * N * 4);
+    LAUNCH(lmsf_gemm_plain_qkv((const float*)v.p, v.ld, (const float*)op.w, op.ldw, (const float*)op.bias, y, N, v.M, v.N,
+                               positions, table, op.max_pos, slots, (float*)op.k_pages, (float*)op.v_pages, op.num_pages,
+                               op.nh, op.nkv, op.d, op.ps, norm, v.eps, v.weight_offset, r.stream));
+    *res = tensor(y, LMSF_F32, v.M, N);
+    return 0;
   };
   LmsfRoute rt;
   if (x.kind == V_SCALED) {
     const int M = x.M, K = x.N;
-    const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, op.w, op.wdtype, op.ldw, op.N, LMSF_BF16);
+    const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, op.w, op.wdtype, op.ldw, op.N, x.dtype);
     lmsf_route_qkv(&t, &shape, fused_shape(K) ? 1 : 0, x.rows_per_tile, &rt);
+    if (rt.route == LMSF_ROUTE_PLAIN_FUSED) return plain(x);
     if (rt.route != LMSF_ROUTE_MATERIALIZE) {
       r.count(rt.route);
       TAKE(y, void*, (size_t)M * N * 2);
@@ -536,6 +587,7 @@ int op_qkv_rope_cache(Run& r, const Value& x_in, const LmsfOpDesc& op, const int
   const int M = x.M, K = x.N;
   const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, op.w, op.wdtype, op.ldw, op.N, x.dtype);
   lmsf_route_qkv(&t, &shape, fused_shape(K) ? 1 : 0, 0, &rt);
+  if (rt.route == LMSF_ROUTE_PLAIN_FUSED) return plain(x);
   if (rt.route != LMSF_ROUTE_SEPARATE) r.count(rt.route);
   if (rt.route == LMSF_ROUTE_GEMV || rt.route == LMSF_ROUTE_SKINNY) {
     TAKE(y, void*, (size_t)M * N * 2);

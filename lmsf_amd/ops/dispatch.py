@@ -29,4 +29,5 @@ class ProductShape(Structure):
 
 
 (PLAIN, MID, LARGE, DEFERRED, GEMV, CHUNKS, SKINNY, BLAS, MATERIALIZE, MID_SCALED, GEMV_SCALED, SKINNY_SCALED, SEPARATE,
- GEMV_ADD_NORM, SKINNY_ADD_NORM, GEMV_ADD) = range(16)
+ GEMV_ADD_NORM, SKINNY_ADD_NORM, GEMV_ADD, PLAIN_ADD_NORM, PLAIN_FUSED) = range(18)
+STREAM_ROWS = -1        # LMSF_STREAM_ROWS

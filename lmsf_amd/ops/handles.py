@@ -31,8 +31,8 @@ class PendingProduct:
 
 
 class DeferredLinear:
-    """A bfloat16 product x weight^T + bias [M, N] of one or two rows that has not been started: the norm
-    that takes it as its branch runs it as a product that adds its result, rounded to bfloat16, straight
+    """A product x weight^T + bias [M, N] of few rows, operands and result of one type, that has not been started: the norm
+    that takes it as its branch runs it as a product that adds its result, rounded to its type, straight
     into the float32 residual stream, so that the addition is no kernel of its own. Made and taken by the
     same operations as ``PendingProduct``."""
 
@@ -61,12 +61,13 @@ class ScaledRows:
     the norm
     (``HipOps.add_rms_norm(DeferredLinear, ..., defer_ok=True)``). The product that takes it
     (``HipOps.qkv_rope_cache``, ``HipOps.linear_gated``) multiplies its rows by rsqrt(sum / H + eps), which
-    is the same product as with the normalised rows up to where the rounding falls. ``HipOps.materialize``
-    runs the norm kernel on the stream instead."""
+    is the same product as with the normalised rows up to where the rounding falls. Of float32 products ``xw`` is
+    the stream itself, without sums (``rows_per_tile`` -1): the product that takes it normalises its rows, to the bits
+    of the norm kernel. ``HipOps.materialize`` runs that kernel on the stream instead."""
 
     __slots__ = ("xw", "sumsq", "tiles", "rows_per_tile", "stream", "weight", "eps", "weight_offset", "dtype")
 
-    def __init__(self, xw: torch.Tensor, sumsq: torch.Tensor, tiles: int, rows_per_tile: int, stream: torch.Tensor,
+    def __init__(self, xw: torch.Tensor, sumsq: Optional[torch.Tensor], tiles: int, rows_per_tile: int, stream: torch.Tensor,
                  weight: torch.Tensor, eps: float, weight_offset: float, dtype: torch.dtype):
         self.xw = xw
         self.sumsq = sumsq

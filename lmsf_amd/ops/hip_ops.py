@@ -202,6 +202,9 @@ class HipOps:
         if weight.shape != (H,) or not weight.is_contiguous():
             raise ValueError("norm weight must be [%d], got %s" % (H, tuple(weight.shape)))
         self._i32(rows, "rows")
+        if (branch is None and rows is None and defer_ok and self._norms_stream(weight, out_dtype)
+                and self.lib.lmsf_route_stream_norm(ctypes.byref(self._tun), N, H)):
+            return ScaledRows(residual, None, 0, D.STREAM_ROWS, residual, weight, float(eps), float(weight_offset), out_dtype)
         n_out = N if rows is None else rows.numel()
         out = torch.empty((n_out, H), dtype=out_dtype, device=ref.device)
         self._check(self.lib.lmsf_add_rms_norm(
@@ -209,6 +212,12 @@ class HipOps:
             _code(weight.dtype), _ptr(out), _code(out_dtype), _ptr(rows), n_out, H, float(eps),
             float(weight_offset), self._stream()))
         return out
+
+    @staticmethod
+    def _norms_stream(weight: torch.Tensor, out_dtype: torch.dtype) -> bool:
+        """A float32 product can normalise the stream's rows by this weight itself."""
+        return (out_dtype == torch.float32 and weight.dtype == torch.float32 and weight.is_contiguous()
+                and weight.data_ptr() % 16 == 0)
 
     def _run_deferred(self, branch: DeferredLinear, residual: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
                       out_dtype: torch.dtype, rows: Optional[torch.Tensor], weight_offset: float, defer_ok: bool):
@@ -220,12 +229,20 @@ class HipOps:
         K = branch.x.shape[1]
         fits = (rows is None and residual is not None and residual.dtype == torch.float32
                 and residual.is_contiguous() and tuple(residual.shape) == branch.shape)
-        prepares = (fits and defer_ok and out_dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-                    and weight.is_contiguous() and weight.shape == (N,))
+        f32 = branch.dtype == torch.float32
+        prepares = (fits and defer_ok and weight.shape == (N,)
+                    and (self._norms_stream(weight, out_dtype) if f32 else
+                         out_dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and weight.is_contiguous()))
         rt = D.Route()
-        self.lib.lmsf_route_deferred_norm(ctypes.byref(self._tun), M, N, K, 1 if fits else 0, 1 if prepares else 0,
-                                          ctypes.byref(rt))
+        self.lib.lmsf_route_deferred_norm(ctypes.byref(self._tun), M, N, K, 0 if not fits else 2 if f32 else 1,
+                                          1 if prepares else 0, ctypes.byref(rt))
         operands = (_ptr(branch.x), branch.x.stride(0), _ptr(branch.weight), branch.weight.stride(0), _ptr(branch.bias))
+        if rt.route == D.PLAIN_ADD_NORM:
+            # adds into the stream; the norm is left to the product that reads it
+            self._dev(branch.x, branch.weight, branch.bias, residual, weight)
+            self._check(self.lib.lmsf_gemm_plain_add(*operands, _ptr(residual), residual.stride(0), M, N, K, self._stream()))
+            return ScaledRows(residual, None, 0, D.STREAM_ROWS, residual, weight, float(eps), float(weight_offset),
+                              out_dtype), None
         if rt.route == D.GEMV_ADD_NORM:
             # adds into the stream, leaves stream * w and its workgroups' sums of squares
             self._dev(branch.x, branch.weight, branch.bias, residual, weight)
@@ -330,7 +347,7 @@ class HipOps:
             max_pos, _ptr(slots), _ptr(k_pages), _ptr(v_pages), num_pages, nh, nkv, d, ps, self._stream()))
 
     def _check_qkv_fused(self, bias, weight, N, table, d, positions, slots, M, k_pages, v_pages, nkv):
-        """Operand checks of the fused QKV forms; returns (pages, page size)."""
+        """Operand checks of the fused QKV forms, pages of the weight's type; returns (pages, page size)."""
         if bias is not None and (bias.shape != (N,) or bias.dtype != weight.dtype or not bias.is_contiguous()):
             raise ValueError("qkv_rope_cache: bias must be [%d] of the weight's dtype" % N)
         if table.dtype != torch.float32 or table.dim() != 2 or table.shape[1] != d or not table.is_contiguous():
@@ -341,25 +358,31 @@ class HipOps:
             raise ValueError("k_pages must be contiguous [pages, %d, page_size, %d]" % (nkv, d))
         num_pages, ps = k_pages.shape[0], k_pages.shape[2]
         if v_pages is None or tuple(v_pages.shape) != (num_pages, nkv, d, ps) or not v_pages.is_contiguous() \
-                or v_pages.dtype != torch.bfloat16:
-            raise ValueError("v_pages must be contiguous bfloat16 [%d, %d, %d, %d]" % (num_pages, nkv, d, ps))
+                or v_pages.dtype != weight.dtype:
+            raise ValueError("v_pages must be contiguous %s [%d, %d, %d, %d]" % (weight.dtype, num_pages, nkv, d, ps))
         return num_pages, ps
+
+    @staticmethod
+    def _norm_of(x) -> tuple:
+        """The norm that a float32 product carries out on its rows: weight, eps and offset, or none."""
+        return (_ptr(x.weight), x.eps, x.weight_offset) if isinstance(x, ScaledRows) else (None, 0.0, 0.0)
 
     def qkv_rope_cache(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], nh: int, nkv: int,
                        d: int, positions: torch.Tensor, table: Optional[torch.Tensor], rot_dim: int, neox: bool,
                        slots: Optional[torch.Tensor], k_pages: Optional[torch.Tensor],
                        v_pages: Optional[torch.Tensor]) -> torch.Tensor:
         """The fused QKV projection, the rotation of its q and k heads and the write of k and v into the
-        pages: ``linear`` followed by ``rope_cache_write``, with the same results. With few bfloat16 rows and
+        pages: ``linear`` followed by ``rope_cache_write``, with the same results. With few rows and
         a NeoX rotation over the whole head, the rotation and the write are the product's epilogue. ``x`` may
         be a ``ScaledRows``."""
         M, K = x.shape
         N = (nh + 2 * nkv) * d
         scaled = isinstance(x, ScaledRows)
         xt = x.xw if scaled else x
-        fused_shape = (table is not None and slots is not None and neox and rot_dim == d and d % 32 == 0
-                       and weight.dtype == torch.bfloat16 and tuple(weight.shape) == (N, K) and xt.stride(1) == 1
-                       and weight.stride(1) == 1 and k_pages is not None and k_pages.dtype == torch.bfloat16)
+        fused_shape = (table is not None and slots is not None and neox and rot_dim == d
+                       and d % (16 if weight.dtype == torch.float32 else 32) == 0 and tuple(weight.shape) == (N, K)
+                       and xt.stride(1) == 1 and weight.stride(1) == 1 and k_pages is not None
+                       and k_pages.dtype == weight.dtype)
         rt = D.Route()
         self.lib.lmsf_route_qkv(ctypes.byref(self._tun), ctypes.byref(self._shape(xt, weight, xt.dtype)),
                                 1 if fused_shape else 0, x.rows_per_tile if scaled else 0, ctypes.byref(rt))
@@ -369,11 +392,13 @@ class HipOps:
         if rt.route != D.SEPARATE:
             self._dev(xt, weight, bias, positions, table, slots, k_pages, v_pages)
             num_pages, ps = self._check_qkv_fused(bias, weight, N, table, d, positions, slots, M, k_pages, v_pages, nkv)
-            y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+            y = torch.empty((M, N), dtype=weight.dtype, device=x.device)
             head = (_ptr(xt), xt.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(y), y.stride(0), M, K,
                     _ptr(positions), _ptr(table), table.shape[0], _ptr(slots), _ptr(k_pages), _ptr(v_pages), num_pages,
                     nh, nkv, d, ps)
-            if rt.route == D.GEMV_SCALED:
+            if rt.route == D.PLAIN_FUSED:
+                self._check(self.lib.lmsf_gemm_plain_qkv(*head, *self._norm_of(x), self._stream()))
+            elif rt.route == D.GEMV_SCALED:
                 self._dev(x.sumsq)
                 self._check(self.lib.lmsf_gemv_scaled_qkv_rope_cache(*head, _ptr(x.sumsq), x.tiles, x.eps, self._stream()))
             elif rt.route == D.SKINNY_SCALED:
@@ -1819,7 +1844,7 @@ class HipOps:
         if (kind == "bounded") != (limit > 0):
             raise ValueError("a limit > 0 goes with the activation 'bounded'")
         if rt.route == D.SEPARATE or (kind == "gelu_tanh" and rt.route not in (D.GEMV, D.SKINNY)) \
-                or (kind == "bounded" and scaled):
+                or (kind == "bounded" and (scaled or rt.route == D.PLAIN_FUSED)):
             # (the tanh form of GELU is an epilogue of the one-row and the few-rows product only)
             return self.gated_act(self.linear(self.materialize(x), weight, bias), kind, limit)
         self._dev(xt, weight, bias)
@@ -1829,9 +1854,12 @@ class HipOps:
             return self._linear_mid(x, weight, bias, kinds[kind], torch.bfloat16, rt, limit=limit)
         if rt.route == D.LARGE:
             return self._linear_large(x, weight, bias, kinds[kind], plan=rt.plan, limit=limit)
-        y = torch.empty((M, I), dtype=torch.bfloat16, device=x.device)
+        y = torch.empty((M, I), dtype=xt.dtype, device=x.device)
         head = (_ptr(xt), xt.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(y))
-        if rt.route == D.MID_SCALED:
+        if rt.route == D.PLAIN_FUSED:
+            self._check(self.lib.lmsf_gemm_plain_gated(*head, y.stride(0), M, I, K, kinds[kind], *self._norm_of(x),
+                                                       self._stream()))
+        elif rt.route == D.MID_SCALED:
             self._check(self.lib.lmsf_gemm_mid_scaled(*head, y.stride(0), M, I, K, kinds[kind], _ptr(x.sumsq), x.tiles,
                                                       x.eps, self._stream()))
         elif rt.route == D.GEMV_SCALED:

@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 36
+ABI_VERSION = 37
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None
@@ -133,6 +133,12 @@ _SIGNATURES = {
     "lmsf_gated_act_limit": (c_int, [_P, _P, c_int, c_int, c_int, c_long, c_int, c_float, _P]),
     "lmsf_gated_act": (c_int, [_P, _P, c_int, c_int, c_int, c_long, c_int, _P]),
     "lmsf_gemm_plain": (c_int, [_P, c_int, c_long, _P, c_int, c_long, _P, _P, c_int, c_long, c_int, c_int, c_int, _P]),
+    "lmsf_gemm_plain_fused_fits": (c_int, [c_int, c_int, c_int, c_int]),
+    "lmsf_gemm_plain_add": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, c_int, c_int, c_int, _P]),
+    "lmsf_gemm_plain_gated": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, c_int, c_int, c_int, c_int, _P, c_float,
+                                      c_float, _P]),
+    "lmsf_gemm_plain_qkv": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, c_int, c_int, _P, _P, c_int, _P, _P, _P, c_long,
+                                    c_int, c_int, c_int, c_int, _P, c_float, c_float, _P]),
     "lmsf_gemm_skinny_limit": (c_int, [_P, c_long, _P, c_long, _P, _P, c_int, c_long, c_int, c_int, c_int, c_int, c_int,
                                        c_float, _P]),
     "lmsf_gemm_skinny": (c_int, [_P, c_long, _P, c_long, _P, _P, c_int, c_long, c_int, c_int, c_int, c_int, c_int, _P]),
@@ -190,6 +196,7 @@ _SIGNATURES = {
     "lmsf_route_linear_gated": (None, [POINTER(Tunables), POINTER(ProductShape), c_int, c_int, POINTER(Route)]),
     "lmsf_route_qkv": (None, [POINTER(Tunables), POINTER(ProductShape), c_int, c_int, POINTER(Route)]),
     "lmsf_route_deferred_norm": (None, [POINTER(Tunables), c_int, c_int, c_int, c_int, c_int, POINTER(Route)]),
+    "lmsf_route_stream_norm": (c_int, [POINTER(Tunables), c_int, c_int]),
     "lmsf_route_decode_attention": (None, [POINTER(Tunables), c_int, c_int, c_int, c_int, POINTER(c_int),
                                            POINTER(c_int)]),
 }

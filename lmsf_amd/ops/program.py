@@ -449,7 +449,7 @@ class StepProgram:
 
     STAT_NAMES = ("plain", "mid", "large", "deferred", "gemv", "chunks", "skinny", "blas", "materialize", "mid_scaled",
                   "gemv_scaled", "skinny_scaled", "separate", "gemv_add_norm", "skinny_add_norm", "gemv_add",
-                  "norm_over_partials", "rope_over_partials", "reduce_partials", "prefill_attention",
+                  "plain_add_norm", "plain_fused", "norm_over_partials", "rope_over_partials", "reduce_partials", "prefill_attention",
                   "decode_attention", "generic_attention", "callback")
 
     def last_step_stats(self) -> dict:
