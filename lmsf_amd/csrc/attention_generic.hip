@@ -15,10 +15,10 @@
 //   s_j = scale * <q, k_j>;  p = softmax_j(s);  out = sum_j p_j v_j
 // with an exact softmax (the reference's decode kernel divides by sum + 1e-6, :279).
 //
-// One workgroup of 256 threads per (token, head): keys are taken 256 at a time, one key per
-// thread for the scores, an online softmax across chunks, and the P V product with the threads
-// arranged as (key group, output dim); a head wider than 256 has one key group and up to four output
-// dims a thread.
+// Two kernels. Heads of up to 256 in pages of a multiple of 4 keys, both on boundaries of four elements, run with a tile of
+// keys a wave (paged_attention_waves_kernel). Anything else: one workgroup of 256 threads per (token, head), keys taken
+// 256 at a time, one key per thread for the scores, an online softmax across chunks, and the P V product with the threads
+// arranged as (key group, output dim); a head wider than 256 has one key group and up to four output dims a thread.
 #include "common.h"
 
 #include <math.h>
@@ -34,6 +34,155 @@ __device__ __forceinline__ void gen_load4(const bf16_t* p, float* x) {
   const uint2 v = *reinterpret_cast<const uint2*>(p);
   x[0] = __uint_as_float(v.x << 16); x[1] = __uint_as_float(v.x & 0xffff0000u);
   x[2] = __uint_as_float(v.y << 16); x[3] = __uint_as_float(v.y & 0xffff0000u);
+}
+
+// Keys in tiles, a wave a tile. What bounds these calls is the number of trips to memory in a row, not the bytes: a tiny
+// model's tokens have 40 kB of keys and values each, and every trip costs 0.5 to 1 us. So a wave asks for a tile's keys
+// AND values at once (8 loads of four elements of each a lane, 8 kB of each in float32), before it knows any score:
+// position -> block table -> keys and values are three trips up to 8 tiles of keys, where the form below makes one for
+// every four keys a thread. Both forms, that one -> this one, 8 heads on one kv head in float32, 32 / 128 wide: 8 tokens of
+// 300 keys 11.0 / 26.6 -> 5.7 / 7.1 us, 1 token of 16 keys 4.6 / 5.8 -> 4.3 / 4.3, of 8,000 keys 187 / 619 -> 40 / 115, a
+// prompt of 140 tokens 11.2 / 33.5 -> 10.6 / 17.4, its 256 tokens behind 768 others 151 / 541 -> 43 / 98; in bfloat16 alike. LPK lanes share a key (d up to 32 LPK; a tile is 64 / LPK keys), every wave keeps an
+// online softmax of its own over its tiles (w, w + 8, ...) with no barrier, and the waves' results are added up in their
+// order at the end, so a token's bits hang on its own position and window alone.
+// Values: lane = (dim, quad of keys in the page), so that consecutive lanes read consecutive 16 bytes of a page.
+#define TILE_WAVES 8
+// what a wave's lanes left in LDS is there for its other lanes (LDS serves a wave's accesses in order)
+__device__ __forceinline__ void gen_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+template <typename T, int LPK>
+__global__ __launch_bounds__(TILE_WAVES * 64) void paged_attention_waves_kernel(
+    const T* __restrict__ q, long q_stride, T* __restrict__ out, long out_stride, const T* __restrict__ k_pages,
+    const T* __restrict__ v_pages, const int* __restrict__ block_tables, int bt_width, const int* __restrict__ seg,
+    const int* __restrict__ pos, int nh, int nkv, int d, int ps, int ps_shift, float scale, int window, float softcap,
+    const float* __restrict__ bias, const float* __restrict__ sink) {
+  constexpr int DMAX = 32 * LPK, KEYS = 64 / LPK, QUADS = KEYS / 4;
+  constexpr int G = QUADS < 4 ? QUADS : 4;          // lanes side by side on the quads of a dim
+  constexpr int DSTEP = 64 / G, DPL = DMAX / DSTEP; // dims a load covers, dims a lane owns: lane / G + DSTEP e
+  constexpr int QPL = QUADS / G;                    // quads a lane takes: lane % G + G i
+  static_assert(DPL * QPL == 8, "eight loads of values a lane");
+  __shared__ __align__(16) float sq[TILE_WAVES][DMAX];   // the query, scaled (a copy a wave: no barrier), then the waves' outputs
+  __shared__ __align__(16) float sp[TILE_WAVES][KEYS];   // a tile's probabilities
+  __shared__ float sm[TILE_WAVES], sl[TILE_WAVES];
+
+  const int t = blockIdx.x, h = blockIdx.y;
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
+  const int s = seg[t], p = pos[t];
+  const int lo = first_visible_key(p, window);
+  const int g = h / (nh / nkv);
+  const int* bt = block_tables + (long)s * bt_width;
+  const float r1 = bias ? bias[h] : 0.f, r2 = bias ? bias[nh + h] : 0.f;
+  const auto page_of = [&](int j) { return ps_shift >= 0 ? j >> ps_shift : j / ps; };
+
+  for (int i = lane; i < DMAX; i += 64) sq[w][i] = i < d ? to_f32<T>(q[(long)t * q_stride + h * d + i]) * scale : 0.f;
+  gen_wave_sync();
+
+  float m = -INFINITY, l = 0.f, acc[DPL];
+#pragma unroll
+  for (int e = 0; e < DPL; ++e) acc[e] = 0.f;
+
+  const int part = lane % LPK;
+  // (tiles begin at a multiple of 4, in the page of the first visible key: a quad never crosses a page)
+  for (int j0 = (lo & ~3) + w * KEYS; j0 <= p; j0 += TILE_WAVES * KEYS) {
+    const int j = j0 + lane / LPK, jc = min(j, p);   // keys beyond the token's own are read as its own and masked
+    const int block = page_of(jc), off = jc - block * ps;
+    int vblock[QPL], voff[QPL];
+#pragma unroll
+    for (int i = 0; i < QPL; ++i) {
+      const int jq = min(j0 + 4 * (lane % G + G * i), p & ~3);
+      vblock[i] = page_of(jq);
+      voff[i] = jq - vblock[i] * ps;
+    }
+    const T* kr = k_pages + (((long)bt[block] * nkv + g) * ps + off) * d;
+    const T* vr[QPL];
+#pragma unroll
+    for (int i = 0; i < QPL; ++i) vr[i] = v_pages + ((long)bt[vblock[i]] * nkv + g) * d * ps + voff[i];
+    float k4[8][4], v4[8][4];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int o = (i * LPK + part) * 4;
+      gen_load4(kr + (o < d ? o : 0), k4[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < QPL; ++i)
+#pragma unroll
+      for (int e = 0; e < DPL; ++e) gen_load4(vr[i] + (long)min(lane / G + DSTEP * e, d - 1) * ps, v4[i * DPL + e]);
+
+    float dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int o = (i * LPK + part) * 4;
+      const float4 q4 = *reinterpret_cast<const float4*>(&sq[w][o]);
+      const float x = q4.x * k4[i][0] + q4.y * k4[i][1] + q4.z * k4[i][2] + q4.w * k4[i][3];
+      dot += o < d ? x : 0.f;
+    }
+#pragma unroll
+    for (int o = 1; o < LPK; o <<= 1) dot += __shfl_xor(dot, o, 64);
+    float sc = softcap > 0.f ? softcap * tanhf(dot / softcap) : dot;   // scores bounded by cap tanh(s / cap)
+    if (bias) sc -= r1 * log1pf(r2 * (float)(p - j));                  // what the distance takes off
+    const bool visible = j >= lo && j <= p;
+    if (!visible) sc = -INFINITY;
+    float tile_max = sc;
+#pragma unroll
+    for (int o = LPK; o < 64; o <<= 1) tile_max = fmaxf(tile_max, __shfl_xor(tile_max, o, 64));
+    const float m_new = fmaxf(m, tile_max);
+    // (a tile whose scores are all -inf adds nothing)
+    const float pr = !visible || m_new == -INFINITY ? 0.f : expf(sc - m_new);
+    const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
+    float tile_sum = pr;
+#pragma unroll
+    for (int o = LPK; o < 64; o <<= 1) tile_sum += __shfl_xor(tile_sum, o, 64);
+    l = l * corr + tile_sum;
+    m = m_new;
+    gen_wave_sync();
+    if (part == 0) sp[w][lane / LPK] = pr;
+    gen_wave_sync();
+#pragma unroll
+    for (int e = 0; e < DPL; ++e) acc[e] *= corr;
+#pragma unroll
+    for (int i = 0; i < QPL; ++i) {
+      const int quad = lane % G + G * i;
+      const float4 p4 = *reinterpret_cast<const float4*>(&sp[w][4 * quad]);
+      const float pq[4] = {p4.x, p4.y, p4.z, p4.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int ju = j0 + 4 * quad + u;
+        const bool in = ju >= lo && ju <= p;       // what lies in a page outside these was never written
+#pragma unroll
+        for (int e = 0; e < DPL; ++e) acc[e] += pq[u] * (in ? v4[i * DPL + e][u] : 0.f);
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < DPL; ++e)
+#pragma unroll
+    for (int o = 1; o < G; o <<= 1) acc[e] += __shfl_xor(acc[e], o, 64);
+  gen_wave_sync();
+  if (lane % G == 0) {
+#pragma unroll
+    for (int e = 0; e < DPL; ++e) sq[w][lane / G + DSTEP * e] = acc[e];
+  }
+  if (lane == 0) {
+    sm[w] = m;
+    sl[w] = l;
+  }
+  __syncthreads();
+  if (tid < d) {
+    // (a sink: exp(sink_h) stands in the denominator beside the keys' exponentials)
+    float top = sink ? sink[h] : -INFINITY;
+#pragma unroll
+    for (int i = 0; i < TILE_WAVES; ++i) top = fmaxf(top, sm[i]);
+    float den = sink ? expf(sink[h] - top) : 0.f, o = 0.f;
+#pragma unroll
+    for (int i = 0; i < TILE_WAVES; ++i) {
+      const float f = sm[i] == -INFINITY ? 0.f : expf(sm[i] - top);
+      den += f * sl[i];
+      o += f * sq[i][tid];
+    }
+    out[(long)t * out_stride + h * d + tid] = from_f32<T>(o / den);
+  }
 }
 
 // VEC: the key pages start on a boundary of four elements (every row does then: d is a multiple of 4), and a key is read
@@ -184,8 +333,25 @@ extern "C" int lmsf_paged_attention_generic_biased(const void* q, long q_stride,
   do {                                                                                                                  \
     if (many) GENERIC_W(T_, VEC_, 5); else GENERIC_W(T_, VEC_, 1);                                                      \
   } while (0)
+  const size_t quad = 4 * lmsf_elem_size(dtype);
+  if (d <= 256 && ps % 4 == 0 && (size_t)k_pages % quad == 0 && (size_t)v_pages % quad == 0) {
+    const int shift = (ps & (ps - 1)) == 0 ? __builtin_ctz((unsigned)ps) : -1;
+#define TILES_OF(T_, LPK_)                                                                                              \
+  hipLaunchKernelGGL((paged_attention_waves_kernel<T_, LPK_>), grid, dim3(TILE_WAVES * 64), 0, stream, (const T_*)q, q_stride, \
+                     (T_*)out, out_stride, (const T_*)k_pages, (const T_*)v_pages, block_tables, bt_width, seg, pos, nh, \
+                     nkv, d, ps, shift, scale, window, softcap, bias, sink)
+#define TILES(T_)                                                                                                       \
+  do {                                                                                                                  \
+    if (d <= 32) TILES_OF(T_, 1); else if (d <= 64) TILES_OF(T_, 2); else if (d <= 128) TILES_OF(T_, 4); else TILES_OF(T_, 8); \
+  } while (0)
+    if (dtype == LMSF_F32) TILES(float); else TILES(bf16_t);
+#undef TILES
+#undef TILES_OF
+    LMSF_LAUNCH_CHECK("paged_attention_generic");
+    return 0;
+  }
   const bool vec = (size_t)k_pages % (4 * lmsf_elem_size(dtype)) == 0;
-  // More workgroups than the chip takes at once with four on a compute unit: fewer registers, seven on a unit. Both sides
+  // What is left: wider heads, pages of other sizes, unaligned ones. More workgroups than the chip takes at once with four on a compute unit: fewer registers, seven on a unit. Both sides
   // in float32 with 8 heads of 32 / 128, four -> seven a unit: 64 tokens of a prompt 7.6 / 13.8 -> 8.0 / 15.2 us, 100
   // tokens 9.3 / 22.5 -> 9.7 / 23.3, 140 tokens 14.2 / 38.8 -> 12.4 / 34.6, 200 tokens 22.1 / 61.4 -> 19.5 / 59.3, 256
   // tokens 32.9 / 105.0 -> 30.5 / 107.2. (Keys read entry by entry and values one by one took 15.1 / 37.9 us for 8

@@ -134,3 +134,39 @@ def test_general_attention_of_many_tokens_gives_the_bits_of_few(ops, d, dtype, s
     def run(a, b):
         return ops.paged_attention(q[a:b], k, v, table, seg[a:b], pos[a:b], nh, nkv, d, d ** -0.5, kernel="generic")
     assert torch.equal(run(0, T), torch.cat([run(0, T - 20), run(T - 20, T)]))
+
+
+# tiles of 64, 32, 16 and 8 keys, eight of them side by side: windows and chunks that begin inside a quad of keys, pages of
+# any multiple of 4, and pages whose unwritten places hold NaN
+@pytest.mark.parametrize("d,ps", [(4, 4), (32, 12), (36, 16), (64, 8), (100, 16), (128, 20), (256, 16)])
+@pytest.mark.parametrize("context", [2, 9, 65, 130, 513, 700])
+@pytest.mark.parametrize("mask", [{}, {"window": 1}, {"window": 70}, {"chunk": 50}])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_general_attention_reads_visible_keys_only(ops, d, ps, context, mask, dtype):
+    nh, nkv, scale, cap = 4, 2, d ** -0.5, 3.0
+    g = torch.Generator().manual_seed(d + context)
+    blocks = -(-context // ps)
+    keys, vals = (torch.randn(nkv, context, d, generator=g).to(dtype) for _ in range(2))
+    k, v = torch.full((blocks + 2, nkv, ps, d), float("nan"), dtype=dtype), torch.full((blocks + 2, nkv, d, ps), float("nan"), dtype=dtype)
+    table = torch.randperm(blocks + 2, generator=g)[:blocks].to(torch.int32)
+    for j in range(context):
+        k[table[j // ps], :, j % ps] = keys[:, j]
+        v[table[j // ps], :, :, j % ps] = vals[:, j]
+    q = torch.randn(2, nh * d, generator=g).to(dtype)
+    pos = torch.tensor([context - 1, context // 2], dtype=torch.int32)
+    bias, sink = torch.rand(2, nh, generator=g), torch.randn(nh, generator=g)
+    got = ops.paged_attention(q.cuda(), k.cuda(), v.cuda(), table.view(1, -1).cuda(), torch.zeros(2, dtype=torch.int32, device="cuda:0"),
+                              pos.cuda(), nh, nkv, d, scale, softcap=cap, distance_bias=bias.cuda(), sink=sink.cuda(),
+                              kernel="generic", **mask).double().cpu()
+    for t in range(2):
+        p = int(pos[t])
+        lo = max(0, p - mask["window"] + 1) if "window" in mask else p // mask["chunk"] * mask["chunk"] if "chunk" in mask else 0
+        j = torch.arange(lo, p + 1)
+        for h in range(nh):
+            s = cap * torch.tanh(keys[h // 2, j].double() @ q[t, h * d:(h + 1) * d].double() * scale / cap)
+            s = s - bias[0, h].double() * torch.log1p(bias[1, h].double() * (p - j))
+            w = torch.softmax(torch.cat([s, sink[h:h + 1].double()]), 0)[:-1]
+            want = w @ vals[h // 2, j].double()
+            # scores of a few units to 2^-21, weights that add up to at most one over values of up to 5 units
+            tol = 2e-5 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
+            assert ((got[t, h * d:(h + 1) * d] - want).abs() <= tol).all()
