@@ -58,3 +58,26 @@ def test_qkv_product_with_rotation(ops, M, d, heads):
     (a, ka, va), (b, kb, vb) = run(heads), run(many)
     assert torch.equal(a[:, :heads * d], b[:, :heads * d]) and torch.equal(ka, kb) and torch.equal(va, vb)
     assert ka.abs().sum() > 0
+
+
+# the first and last widths whose sums of squares come from two workgroups a tile, and one beyond either; 8 rows and 9
+@pytest.mark.parametrize("N", [1008, 1024, 1040, 2048, 2064])
+@pytest.mark.parametrize("M", [3, 8, 9])
+@pytest.mark.parametrize("K,bias", [(64, False), (4104, True)])
+def test_product_before_a_norm(ops, M, N, K, bias):
+    g = torch.Generator().manual_seed(N + M + K)
+    w, x, b = rnd(g, N, K), rnd(g, M, K), rnd(g, N) if bias else None
+    nw = torch.randn(N, generator=g).bfloat16().to("cuda:0")
+    before = torch.randn(M, N, generator=g).to("cuda:0") * 3
+    stream = before.clone()
+    h = ops.add_rms_norm(ops.linear(x, w, b, pending_ok=True), stream, nw, 1e-5, torch.bfloat16, defer_ok=True)
+    assert torch.equal(stream, before + ops.linear(x, w, b).float()) and torch.equal(h.xw, (stream * nw.float()).bfloat16())
+    # the products that take the norm: their factor rsqrt(sum / N + eps) to the roundings of sums of N squares, the
+    # products' own sums of N terms in float32, three roundings to bfloat16 (gate, up, result; silu's slope is below 1.1)
+    normed = h.xw.double() * torch.rsqrt(stream.double().pow(2).mean(1, keepdim=True) + 1e-5)
+    wg = rnd(g, 2 * 1024, N)
+    got = ops.linear_gated(h, wg, None, "silu").double()
+    a, u = (normed @ wg.double().T).split(1024, 1)
+    want = torch.nn.functional.silu(a) * u
+    err = 2.0 ** -8 * (1.1 * a.abs() * u.abs() + want.abs() * 2) + 1e-5
+    assert ((got - want).abs() <= err * 1.05).all()
