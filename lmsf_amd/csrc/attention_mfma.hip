@@ -799,8 +799,8 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     const bf16_t* __restrict__ q, long q_stride, const bf16_t* __restrict__ k_pages,
     const bf16_t* __restrict__ v_pages, const int* __restrict__ block_tables, int btw,
     const int* __restrict__ tok_idx, const int* __restrict__ seg, const int* __restrict__ pos, int nh, int nkv, int d,
-    int ps, float scale_log2, float cap_raw, int window, int HB, int n_hb, int chunk, int n_splits, float* __restrict__ part_o,
-    float* __restrict__ part_ml, bf16_t* __restrict__ out, long out_stride, int heads_first,
+    int ps, unsigned ps_inv, float scale_log2, float cap_raw, int window, int HB, int n_hb, int chunk, int n_splits,
+    float* __restrict__ part_o, float* __restrict__ part_ml, bf16_t* __restrict__ out, long out_stride, int heads_first,
     const float* __restrict__ bias, const float* __restrict__ sink) {
   constexpr int DS = DPAD / 32, DV = DPAD / 16;
   extern __shared__ float lds_f[];
@@ -814,19 +814,23 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
   const int split = blockIdx.z;
   const int n_rep = nh / nkv;
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, c = l & 15, g = l >> 4;
-  const int p = pos[tok];
-  const int lo = first_visible_key(p, window);
-  const int c0 = max(split * chunk, (lo / 32) * 32), c1 = min((split + 1) * chunk, p + 1);   // keys [c0, c1)
-  if (c0 >= c1) return;
   KvView G;
   G.k = k_pages; G.v = v_pages; G.btw = btw; G.nkv = nkv; G.d = d; G.ps = ps; G.kvh = kvh;
   G.bt = block_tables + (long)(seg ? seg[tok] : tok) * btw;   // (no seg: token i is request i, one trip to memory fewer)
+  // key / ps without a division: the product with ceil(2^32 / ps) is the quotient or one more
+  const auto block_of = [&](int key) {
+    const int b = (int)__umulhi((unsigned)key, ps_inv);
+    return b - (b * G.ps > key ? 1 : 0);
+  };
 
+  // Queries, the first step's table entries and the position are asked for together: what bounds a step of few tokens is
+  // the trips to memory in a row (position, table, keys and values), not the bytes. With that, with no integer division (about
+  // 30 instructions each, eight a step) and with four outputs a thread in the merge, with the reduction: 16 heads on one of
+  // 256, 8 tokens of 90 / 400 keys 11.8 / 15.6 -> 8.8 / 12.3 us, 64 of 600 keys 30 -> 23.5; 32 heads on 8 of 128, 8 tokens of
+  // 90 / 8,000 keys 5.7 / 49.4 -> 5.5 / 48.5, 64 of 90 keys 9.1 -> 8.5; of 64, 64 of 90 keys 6.8 -> 6.3; 32 on 32 level.
   const int hin = hb * HB + c;
   const bool valid = c < HB && hin < n_rep;
   const int head = kvh * n_rep + (valid ? hin : 0);
-  DistanceBias db;
-  if constexpr (BIAS) db.load(bias, nh, head, scale_log2);
   Frag8 qf[DS];
 #pragma unroll
   for (int s = 0; s < DS; ++s) {
@@ -836,24 +840,12 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     else
       qf[s].q = make_uint4(0, 0, 0, 0);
   }
-  f32x4_t acc[DV];
-#pragma unroll
-  for (int v = 0; v < DV; ++v) acc[v] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  // (of a token's splits and waves one takes the sink: the first wave of the split that ends with the token's own key)
-  const bool takes_sink = sink && w == 0 && c1 == p + 1;
-  float m = takes_sink ? sink_start(sink, head) : -INFINITY, lsum = takes_sink && g == 0 ? 1.f : 0.f;
-
   // The pages of a step's keys are looked up one step ahead (four entries of the block table a lane: the two
   // blocks of 16 keys whose rows it fetches, the two groups of four keys whose values it fetches), so that the
-  // keys' addresses do not wait for a trip to the table.
-  const int klast = c1 - 1;
-  auto page_of = [&](int key) {
-    // keys beyond the range are masked below; their addresses stay inside the pages that the range has
-    return G.bt[min(key, klast) / G.ps];
-  };
-  auto k_at = [&](int page, int key) { return ((long)(page * G.nkv + G.kvh) * G.ps + (key - (key / G.ps) * G.ps)) * G.d; };
-  auto v_at = [&](int page, int key) { return (long)(page * G.nkv + G.kvh) * G.d * G.ps + (key - (key / G.ps) * G.ps); };
-  auto lookup = [&](int kb, int* out) {
+  // keys' addresses do not wait for a trip to the table. Keys beyond ``last`` are masked below; they are looked up as
+  // ``last``, so that their addresses stay inside the pages that the range has.
+  auto lookup = [&](int kb, int last, int* out) {
+    auto page_of = [&](int key) { return G.bt[block_of(min(key, last))]; };
     if (ROW8) {
       // a group of eight keys lies in one page (pages of a multiple of 8 tokens): one entry for both blocks' rows,
       // one for the values
@@ -863,6 +855,35 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       out[0] = page_of(kb + c); out[1] = page_of(kb + 16 + c); out[2] = page_of(kb + 4 * g); out[3] = page_of(kb + 16 + 4 * g);
     }
   };
+  int pg[4];
+  // (before the position is known: anywhere in the table's row; what lies beyond the range is replaced below)
+  if (window == 0) lookup(split * chunk + w * 32, btw * ps - 1, pg);
+  const int p = pos[tok];
+  const int lo = first_visible_key(p, window);
+  const int c0 = max(split * chunk, (lo / 32) * 32), c1 = min((split + 1) * chunk, p + 1);   // keys [c0, c1)
+  if (c0 >= c1) return;
+  if (window != 0) {
+    lookup(c0 + w * 32, c1 - 1, pg);
+  } else {
+    const int kb = c0 + w * 32, first = __builtin_amdgcn_readfirstlane(pg[0]);   // the page of the step's first key
+    if ((ROW8 ? kb + 8 * (c >> 2) + (c & 3) : kb + c) >= c1) pg[0] = first;
+    if ((ROW8 ? kb + 8 * (c >> 2) + (c & 3) : kb + 16 + c) >= c1) pg[1] = first;
+    if ((ROW8 ? kb + 8 * g : kb + 4 * g) >= c1) pg[2] = first;
+    if ((ROW8 ? kb + 8 * g : kb + 16 + 4 * g) >= c1) pg[3] = first;
+  }
+  DistanceBias db;
+  if constexpr (BIAS) db.load(bias, nh, head, scale_log2);
+  f32x4_t acc[DV];
+#pragma unroll
+  for (int v = 0; v < DV; ++v) acc[v] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  // (of a token's splits and waves one takes the sink: the first wave of the split that ends with the token's own key)
+  const bool takes_sink = sink && w == 0 && c1 == p + 1;
+  float m = takes_sink ? sink_start(sink, head) : -INFINITY, lsum = takes_sink && g == 0 ? 1.f : 0.f;
+
+  auto k_at = [&](int page, int key) {
+    return ((long)(page * G.nkv + G.kvh) * G.ps + (key - block_of(key) * G.ps)) * G.d;
+  };
+  auto v_at = [&](int page, int key) { return (long)(page * G.nkv + G.kvh) * G.d * G.ps + (key - block_of(key) * G.ps); };
   // the keys and values of one step of 32 keys, as the matrix instructions take them
   auto fetch = [&](Frag8 (&kf)[2][DS], Frag8 (&vf)[DV], const int* pg, int kbase) {
 #pragma unroll
@@ -878,10 +899,14 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       }
     }
     const long vo0 = v_at(pg[2], ROW8 ? kbase + 8 * g : kbase + 4 * g), vo1 = v_at(pg[3], kbase + 16 + 4 * g);
+    // (the rows' distance is kept from the compiler, which would otherwise hold every row's offset across the loop: 179
+    // registers instead of 150 at a head size of 128, two waves a SIMD instead of three)
+    int step = 16 * ps;
+    asm volatile("" : "+s"(step));
 #pragma unroll
     for (int v = 0; v < DV; ++v) {
       if (FULL || v * 16 < d) {
-        const long dvo = (long)(v * 16 + c) * ps;
+        const long dvo = (long)v * step + c * ps;
         if (ROW8) {
           vf[v].v = __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(v_pages + vo0 + dvo));
           continue;
@@ -946,11 +971,9 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
       }
     }
   };
-  int pg[4];
-  lookup(c0 + w * 32, pg);
   for (int kbase = c0 + w * 32; kbase < c1; kbase += 128) {
     int pg_next[4] = {pg[0], pg[1], pg[2], pg[3]};
-    if (kbase + 128 < c1) lookup(kbase + 128, pg_next);
+    if (kbase + 128 < c1) lookup(kbase + 128, c1 - 1, pg_next);
     Frag8 kf[2][DS], vf[DV];
     fetch(kf, vf, pg, kbase);
     compute(kf, vf, kbase);
@@ -972,27 +995,34 @@ __global__ __launch_bounds__(256) void attn_decode_mfma_kernel(
     lds_l[w * 16 + c] = lsum;
   }
   __syncthreads();
-  const int rows = min(HB, n_rep - hb * HB);
-  for (int e = tid; e < rows * d; e += 256) {
-    const int r = e / d, dv = e - r * d;
+  // four outputs of a row a thread at a time
+  const int rows = min(HB, n_rep - hb * HB), quads = (FULL ? DPAD : d) / 4;
+  for (int e = tid; e < rows * quads; e += 256) {
+    const int r = e / quads, dv = (e - r * quads) * 4;
     float M = lds_m[r];
 #pragma unroll
     for (int ww = 1; ww < 4; ++ww) M = fmaxf(M, lds_m[ww * 16 + r]);
-    float o = 0.f, ls = 0.f;
+    float ls = 0.f;
+    f32x4_t o = (f32x4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int ww = 0; ww < 4; ++ww) {
       const float mw = lds_m[ww * 16 + r];
       const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
-      o += f * lds_o[(ww * 16 + r) * (DPAD + 4) + dv];
+      const f32x4_t ow = *reinterpret_cast<const f32x4_t*>(lds_o + (ww * 16 + r) * (DPAD + 4) + dv);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] += f * ow[i];
       ls += f * lds_l[ww * 16 + r];
     }
     const int hd = kvh * n_rep + hb * HB + r;
     if (n_splits == 1) {
-      out[(long)tok * out_stride + (long)hd * d + dv] = f32_to_bf16(o / ls);
+      uint2 packed;
+      packed.x = pack2_bf16(o[0] / ls, o[1] / ls);
+      packed.y = pack2_bf16(o[2] / ls, o[3] / ls);
+      *reinterpret_cast<uint2*>(out + (long)tok * out_stride + (long)hd * d + dv) = packed;
       continue;
     }
     const long slot = ((long)i_tok * nh + hd) * n_splits + split;
-    part_o[slot * d + dv] = o;
+    *reinterpret_cast<f32x4_t*>(part_o + slot * d + dv) = o;
     if (dv == 0) {
       part_ml[slot * 2] = M;
       part_ml[slot * 2 + 1] = ls;
@@ -1226,8 +1256,8 @@ static int launch_decode(dim3 grid, hipStream_t stream, const bf16_t* q, long q_
     configured = true;
   }
   hipLaunchKernelGGL(kernel, grid, dim3(256), smem, stream, q, q_stride, k_pages, v_pages, block_tables, btw, tok_idx,
-                     seg, pos, nh, nkv, d, ps, scale_log2, cap_raw, window, HB, n_hb, chunk, n_splits, part_o, part_ml, out,
-                     out_stride, heads_first, bias, sink);
+                     seg, pos, nh, nkv, d, ps, (unsigned)(((1ull << 32) + ps - 1) / ps), scale_log2, cap_raw,
+                     window, HB, n_hb, chunk, n_splits, part_o, part_ml, out, out_stride, heads_first, bias, sink);
   return 0;
 }
 
