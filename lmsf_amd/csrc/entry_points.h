@@ -207,6 +207,9 @@ int lmsf_gemm_skinny(const void* x, long ldx, const void* W, long ldw, const voi
 int lmsf_gemm_qkv_rope_cache(const void* x, long ldx, const void* W, long ldw, const void* bias, void* y, long ldy,
     int M, int K, const int* positions, const float* table, int max_pos, const int* slots, void* k_pages, void*
     v_pages, long num_pages, int nh, int nkv, int d, int ps, int variant, hipStream_t stream);
+int lmsf_gemm_skinny_add_dyt(const void* x, long ldx, const void* W, long ldw, const void* bias, float* stream_f32,
+    long ld_stream, const float* w, const float* b, const float* alpha, void* y, long ldy, int M, int N, int K, int
+    variant, hipStream_t stream);
 int lmsf_gemm_skinny_add_norm(const void* x, long ldx, const void* W, long ldw, const void* bias, void* stream_f32,
     long ld_stream, const void* norm_weight, float weight_offset, void* xw, long ld_xw, float* sumsq, int M, int N,
     int K, int variant, hipStream_t stream);

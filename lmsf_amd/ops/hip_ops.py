@@ -1364,7 +1364,25 @@ class HipOps:
                  rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         """tanh(alpha * r) * weight + bias with r = residual + branch (either may be missing). ``residual``
         (float32 [N, H]) becomes the sum in place when both are given and ``rows`` is None; ``rows`` (int32 [R])
-        selects rows, the output then has R. ``alpha`` is a float32 tensor of one element."""
+        selects rows, the output then has R. ``alpha`` is a float32 tensor of one element. ``branch`` may be an
+        unfinished product (``linear(..., pending_ok=True)``): of few rows it is then made, added and followed by the
+        tanh in one kernel."""
+        if isinstance(branch, DeferredLinear) and rows is None and residual is not None and out_dtype == branch.dtype \
+                and branch.dtype == torch.bfloat16 and branch.shape[0] <= 16 and residual.dtype == torch.float32 \
+                and residual.is_contiguous() and tuple(residual.shape) == branch.shape:
+            M, H = branch.shape
+            self._dev(branch.x, branch.weight, branch.bias, residual, weight, bias, alpha)
+            self._f32_vec(weight, H, "dyt_norm: weight")
+            self._f32_vec(bias, H, "dyt_norm: bias")
+            self._f32_vec(alpha, 1, "dyt_norm: alpha")
+            out = torch.empty((M, H), dtype=out_dtype, device=residual.device)
+            self._check(self.lib.lmsf_gemm_skinny_add_dyt(
+                _ptr(branch.x), branch.x.stride(0), _ptr(branch.weight), branch.weight.stride(0), _ptr(branch.bias),
+                _ptr(residual), residual.stride(0), _ptr(weight), _ptr(bias), _ptr(alpha), _ptr(out), out.stride(0), M, H,
+                branch.x.shape[1], self.skinny_variant, self._stream()))
+            return out
+        if isinstance(branch, (DeferredLinear, PendingProduct)):
+            branch = self.materialize(branch)
         self._dev(branch, residual, weight, bias, alpha, rows)
         ref = branch if branch is not None else residual
         if ref is None or ref.dim() != 2 or not ref.is_contiguous():

@@ -144,6 +144,8 @@ _SIGNATURES = {
     "lmsf_gemm_skinny": (c_int, [_P, c_long, _P, c_long, _P, _P, c_int, c_long, c_int, c_int, c_int, c_int, c_int, _P]),
     "lmsf_gemm_qkv_rope_cache": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, c_int, c_int, _P, _P, c_int, _P, _P, _P,
                                          c_long, c_int, c_int, c_int, c_int, c_int, _P]),
+    "lmsf_gemm_skinny_add_dyt": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, _P, _P, _P, _P, c_long, c_int, c_int,
+                                         c_int, c_int, _P]),
     "lmsf_gemm_skinny_add_norm": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, _P, c_float, _P, c_long, _P, c_int,
                                           c_int, c_int, c_int, _P]),
     "lmsf_gemm_skinny_scaled": (c_int, [_P, c_long, _P, c_long, _P, _P, c_long, c_int, c_int, c_int, c_int, _P, c_int,

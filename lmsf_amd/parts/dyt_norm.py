@@ -19,6 +19,7 @@ class DynamicTanh(Norm):
 
     graph_safe = True
     recordable = False
+    accepts_pending = True
 
     def __init__(self, prefix: str, rt: Runtime, size: int, weight_name: str = "weight", bias_name: str = "bias",
                  alpha_name: str = "alpha", alpha_init: float = 0.5):

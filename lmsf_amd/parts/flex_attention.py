@@ -38,6 +38,7 @@ from .recurrent import ShortConv
 class FlexAttention(Mixer):
     graph_safe = True
     recordable = False
+    may_return_pending = True
 
     def __init__(self, prefix: str, rt: Runtime, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int,
                  v_head_dim: int, scale: float, position: Optional[PartSpec] = None, qkv_bias: bool = False,
@@ -133,7 +134,7 @@ class FlexAttention(Mixer):
             return None
         return StateSpec((self.conv.state_floats,), torch.float32)
 
-    def forward(self, h: torch.Tensor, ctx, binding: CacheBinding) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, ctx, binding: CacheBinding, pending_ok: bool = False):
         ops = self.rt.ops
         H, G, dim, vdim, D = self.H, self.G, self.dim, self.vdim, self.D
         group = ctx.groups[binding.group]
@@ -159,4 +160,4 @@ class FlexAttention(Mixer):
             a = ops.attn_finish(a, D, H, vdim, ctx.positions, gate=p[:, self.n_qkv:self.n_qkv + H])
         elif self.has_gate or D != vdim:
             a = ops.head_gate(a, D, H, vdim, gate=p[:, self.n_qkv:] if self.has_gate else None)
-        return self.o.forward(a)
+        return self.o.forward(a, pending_ok=pending_ok)

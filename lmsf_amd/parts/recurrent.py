@@ -87,6 +87,7 @@ class SelectiveScan(Mixer):
 
     graph_safe = True
     recordable = False
+    may_return_pending = True
 
     def __init__(self, prefix: str, rt: Runtime, hidden_size: int, inner: int, state: int, dt_rank: int, conv: int,
                  names: Optional[Dict[str, str]] = None):
@@ -112,7 +113,7 @@ class SelectiveScan(Mixer):
     def state_spec(self) -> Optional[StateSpec]:
         return StateSpec((self.scan_floats + self.conv.state_floats,), torch.float32)
 
-    def forward(self, h: torch.Tensor, ctx, binding: CacheBinding) -> torch.Tensor:
+    def forward(self, h: torch.Tensor, ctx, binding: CacheBinding, pending_ok: bool = False):
         ops = self.rt.ops
         st = binding.state
         xz = self.in_proj.forward(h)                                            # [N, 2 inner]
@@ -121,7 +122,7 @@ class SelectiveScan(Mixer):
         dt = ops.linear_wide(low[:, :self.rank], self.dt_proj.weight, self.dt_proj.bias)   # float32: a step size
         y = ops.selective_scan(x, dt, low, self.rank, self.rank + self.n, xz[:, self.inner:], self.a_log.weight,
                                self.d.weight, st, ctx)
-        return self.o.forward(y)
+        return self.o.forward(y, pending_ok=pending_ok)
 
 
 @register_part("mixer", "matrix_memory")

@@ -81,3 +81,24 @@ def test_product_before_a_norm(ops, M, N, K, bias):
     want = torch.nn.functional.silu(a) * u
     err = 2.0 ** -8 * (1.1 * a.abs() * u.abs() + want.abs() * 2) + 1e-5
     assert ((got - want).abs() <= err * 1.05).all()
+
+
+@pytest.mark.parametrize("N", [1, 9, 1000, 2048, 2056, 4096])
+@pytest.mark.parametrize("M", [1, 2, 8, 9, 16])
+@pytest.mark.parametrize("K,bias", [(64, False), (4104, True)])
+def test_product_before_dynamic_tanh(ops, M, N, K, bias):
+    """One kernel to the bits of the product and the kernel after it (rows of the few-rows product hang on nothing else, so
+    the separate product of one row is taken from two)."""
+    from lmsf_amd.ops.handles import DeferredLinear
+    g = torch.Generator().manual_seed(N + M + K)
+    w, x, b = rnd(g, N, K), rnd(g, max(M, 2), K), rnd(g, N) if bias else None
+    tw, tb, alpha = (torch.randn(n, generator=g).to("cuda:0") for n in (N, N, 1))
+    before = torch.randn(M, N, generator=g).to("cuda:0") * 2
+    s1, s2 = before.clone(), before.clone()
+    p = ops.linear(x[:M], w, b, pending_ok=True)
+    assert isinstance(p, DeferredLinear)
+    got = ops.dyt_norm(p, s1, tw, tb, alpha, torch.bfloat16)
+    want = ops.dyt_norm(ops.linear(x, w, b)[:M].contiguous(), s2, tw, tb, alpha, torch.bfloat16)
+    assert torch.equal(s1, s2) and torch.equal(got, want) and not torch.equal(s1, before)
+    rows = torch.tensor([M - 1], dtype=torch.int32, device="cuda:0")          # wanted rows alone: the kernels one by one
+    assert torch.equal(ops.dyt_norm(p, before.clone(), tw, tb, alpha, torch.bfloat16, rows=rows), want[M - 1:])
