@@ -1298,7 +1298,8 @@ extern "C" int lmsf_paged_attention_decode_mfma_biased(const void* q, long q_str
   // together and the longest contexts first (32 kv heads: 214 against 176); equal contexts: the same from 16
   // tokens on, and 1 us in 12 the other way round at 8 tokens.
   const bool wp3 = (order & LMSF_ATTENTION_WEIGHTS_F32) != 0;       // softmax weights in full float32
-  order &= ~LMSF_ATTENTION_WEIGHTS_F32;
+  const bool keep_parts = (order & LMSF_ATTENTION_KEEP_PARTS) != 0;
+  order &= ~(LMSF_ATTENTION_WEIGHTS_F32 | LMSF_ATTENTION_KEEP_PARTS);
   const int heads_first = order == 2 || (order == 0 && n >= 16);
   const float scale_log2 = scale * 1.44269504088896340736f;
   const int dpad = (d + 31) / 32 * 32;
@@ -1336,7 +1337,7 @@ extern "C" int lmsf_paged_attention_decode_mfma_biased(const void* q, long q_str
 #undef DECODE_ARGS
   if (rc) return rc;
   LMSF_LAUNCH_CHECK("paged_attention_decode");
-  if (n_splits == 1) return 0;
+  if (n_splits == 1 || keep_parts) return 0;
   if (n_splits <= REDUCE_SERIAL_SPLITS)
     hipLaunchKernelGGL(attn_decode_reduce_serial_kernel, dim3(n, nh), dim3((d + 63) / 64 * 64), 0, stream, part_o,
                        part_ml, (bf16_t*)out, out_stride, tok_idx, pos, nh, d, window, chunk, n_splits);

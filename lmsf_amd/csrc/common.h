@@ -17,6 +17,9 @@ enum { LMSF_F32 = 0, LMSF_BF16 = 1 };
 // enter the product with the values in full float32 (three bfloat16 parts, three matrix instructions) instead of
 // rounded to bfloat16.
 #define LMSF_ATTENTION_WEIGHTS_F32 256
+// Added to ``order`` of a decode attention with several splits: the partial results stay in the scratch memory for the
+// kernel that takes them (lmsf_head_linear_parts); ``out`` is not written.
+#define LMSF_ATTENTION_KEEP_PARTS 512
 
 typedef uint16_t bf16_t;  // raw bfloat16 bits
 

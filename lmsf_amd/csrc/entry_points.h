@@ -101,6 +101,9 @@ int lmsf_latent_cache_write(const void* x, int dtype, long x_stride, const float
 int lmsf_head_linear(const void* x, int dtype, long x_stride, int x_head, const void* W, void* y, long y_stride,
     int y_head, const void* gate, long gate_stride, int n_tokens, int H, int O, int K, const int* positions,
     const float* table, int rot, int max_pos, int x_at, int y_at, int dr, int gate_wide, hipStream_t stream);
+int lmsf_head_linear_parts(const float* scratch, const int* tok_idx, const int* pos, int window, int chunk, int n_splits,
+    int D, const void* W, void* y, long y_stride, int y_head, const void* gate, long gate_stride, int n_tokens, int H, int O,
+    int K, int gate_wide, hipStream_t stream);
 int lmsf_rope_tail(const void* x, int dtype, long x_stride, int x_head, int x_at, void* y, long y_stride, int y_head,
     int y_at, const int* positions, const float* table, int rot, int max_pos, int n_tokens, int H, int dr,
     hipStream_t stream);

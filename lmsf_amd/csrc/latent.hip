@@ -32,8 +32,9 @@ __global__ __launch_bounds__(LAT_THREADS) void latent_cache_write_kernel(
     T* __restrict__ q_out, long q_out_stride, int Q) {
   __shared__ float red[16];
   const int n = blockIdx.x;
-  if (qx) {
-    // the other latent of the same row of the product: q_out = rms_norm(qx) * qw
+  if (blockIdx.y == 1) {
+    // the other latent of the same row of the product: q_out = rms_norm(qx) * qw (a workgroup of its own: one after the
+    // other the two norms are twice the trips to memory and barriers)
     const T* qr = qx + (long)n * x_stride;
     float qs = 0.f;
     for (int i = threadIdx.x; i < Q; i += LAT_THREADS) {
@@ -44,6 +45,7 @@ __global__ __launch_bounds__(LAT_THREADS) void latent_cache_write_kernel(
     const float qrms = sqrtf(qs / (float)Q + eps);
     for (int i = threadIdx.x; i < Q; i += LAT_THREADS)
       q_out[(long)n * q_out_stride + i] = from_f32<T>(to_f32<T>(qr[i]) / qrms * qw[i]);
+    return;
   }
   const int slot = slots[n];
   if (slot < 0) return;                     // a padding token stores nothing
@@ -98,11 +100,11 @@ extern "C" int lmsf_latent_cache_write(const void* x, int dtype, long x_stride, 
   LMSF_CHECK(ps > 0 && num_pages > 0, "latent_cache_write: bad page geometry");
   if (n_tokens <= 0) return 0;
   if (dtype == LMSF_F32)
-    hipLaunchKernelGGL((latent_cache_write_kernel<float>), dim3(n_tokens), dim3(LAT_THREADS), 0, stream,
+    hipLaunchKernelGGL((latent_cache_write_kernel<float>), dim3(n_tokens, qx ? 2 : 1), dim3(LAT_THREADS), 0, stream,
                        (const float*)x, x_stride, w, eps, positions, table, rot, max_pos, slots, (float*)k_pages,
                        (float*)v_pages, R, dr, D, ps, (const float*)qx, qw, (float*)q_out, q_out_stride, Q);
   else
-    hipLaunchKernelGGL((latent_cache_write_kernel<bf16_t>), dim3(n_tokens), dim3(LAT_THREADS), 0, stream,
+    hipLaunchKernelGGL((latent_cache_write_kernel<bf16_t>), dim3(n_tokens, qx ? 2 : 1), dim3(LAT_THREADS), 0, stream,
                        (const bf16_t*)x, x_stride, w, eps, positions, table, rot, max_pos, slots, (bf16_t*)k_pages,
                        (bf16_t*)v_pages, R, dr, D, ps, (const bf16_t*)qx, qw, (bf16_t*)q_out, q_out_stride, Q);
   LMSF_LAUNCH_CHECK("latent_cache_write");
@@ -115,6 +117,7 @@ extern "C" int lmsf_latent_cache_write(const void* x, int dtype, long x_stride, 
 // A workgroup takes HL_TOKENS tokens of one head: their inputs lie in LDS, a thread owns outputs o, o + 256, ...
 // and reads each row of W once for all of them.
 #define HL_TOKENS 8
+#define HLP_MAX_K 256     // the widest head of split decode attention
 
 template <typename T>
 __global__ __launch_bounds__(LAT_THREADS) void head_linear_kernel(
@@ -312,6 +315,108 @@ extern "C" int lmsf_head_linear(const void* x, int dtype, long x_stride, int x_h
                          x_stride, x_head, x_at, (bf16_t*)y, y_stride, y_head, y_at, positions, table, rot, max_pos, H, dr);
   }
   LMSF_LAUNCH_CHECK("head_linear");
+  return 0;
+}
+
+// The same product of what split decode attention leaves (attention_mfma.hip: part_o [i, head, split, D] not normalised,
+// part_ml [.., 2] maximum and sum): a workgroup adds up the splits of up to 16 tokens of one head in LDS, rounded as the
+// attention's own reduction stores them, and multiplies them with 64 outputs' rows on the matrix cores in
+// head_linear_mfma_kernel's order, to the same bits. What bounds it is its launch and one trip to memory: the rows of W, the
+// gates and the partial results are asked for together. Takosun, 8 requests (8 layers), reduction and product apart -> this,
+// with the latents' norms side by side: 20.98 -> 19.89 ms.
+template <int SPLITS>
+__global__ __launch_bounds__(256) void head_linear_parts_kernel(
+    const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ tok_idx,
+    const int* __restrict__ pos, int window, int chunk, int n_splits, int D, const bf16_t* __restrict__ W,
+    bf16_t* __restrict__ y, long y_stride, int y_head, const bf16_t* __restrict__ gate, long gate_stride, int n_tokens, int H,
+    int O, int K, int gate_wide) {
+  constexpr int STEPS = HLP_MAX_K / 32, ROW = HLP_MAX_K + 8;
+  __shared__ __align__(16) bf16_t xs[16 * ROW];      // (rows padded by 16 bytes: operand reads on distinct banks)
+  const int h = blockIdx.y, n0 = blockIdx.x * 16, tid = threadIdx.x;
+  const int wave = tid / LMSF_WAVE, lane = tid % LMSF_WAVE, fr = lane % 16, fg = lane / 16;
+  const int o0 = blockIdx.z * 64 + wave * 16, i_tok = min(n0 + fr, n_tokens - 1);
+  const bf16_t* wa = W + ((long)h * O + min(o0 + fr, O - 1)) * K + fg * 8;
+  bf16x8_t fa[STEPS];
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s)
+    if (s * 32 < K) fa[s] = *reinterpret_cast<const bf16x8_t*>(wa + s * 32);
+  const int tok = tok_idx ? tok_idx[i_tok] : i_tok;
+  bf16_t gates[4] = {0, 0, 0, 0};
+  if (gate) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      gates[j] = gate[(long)tok * gate_stride + (gate_wide ? (long)h * O + min(o0 + fg * 4 + j, O - 1) : h)];
+  }
+  const int quads = K / 4;
+  for (int e = tid; e < min(16, n_tokens - n0) * quads; e += 256) {
+    const int r = e / quads, k = (e - r * quads) * 4, i = n0 + r;
+    const long base = ((long)i * H + h) * n_splits;
+    float2 ml[SPLITS];
+    float4 po[SPLITS];
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s)
+      if (s < n_splits) {
+        ml[s] = *reinterpret_cast<const float2*>(part_ml + (base + s) * 2);
+        po[s] = *reinterpret_cast<const float4*>(part_o + (base + s) * D + k);
+      }
+    const int p = pos[tok_idx ? tok_idx[i] : i];
+    const int s0 = (first_visible_key(p, window) / 32 * 32) / chunk, s1 = min(n_splits - 1, p / chunk);   // these have keys
+    float M = -INFINITY, ls = 0.f;
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s)
+      if (s >= s0 && s <= s1) M = fmaxf(M, ml[s].x);
+    float o[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < SPLITS; ++s)
+      if (s >= s0 && s <= s1) {
+        const float f = exp2f(ml[s].x - M);
+        ls += f * ml[s].y;
+        o[0] += f * po[s].x; o[1] += f * po[s].y; o[2] += f * po[s].z; o[3] += f * po[s].w;
+      }
+    const float inv = 1.0f / ls;
+    uint2 packed;
+    packed.x = pack2_bf16(o[0] * inv, o[1] * inv);
+    packed.y = pack2_bf16(o[2] * inv, o[3] * inv);
+    *reinterpret_cast<uint2*>(xs + r * ROW + k) = packed;
+  }
+  __syncthreads();
+  if (o0 >= O) return;
+  // (rows of tokens that are not there hold what LDS held; their column of the result is not stored)
+  f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < STEPS; ++s)
+    if (s * 32 < K)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[s], *reinterpret_cast<const bf16x8_t*>(xs + fr * ROW + s * 32 + fg * 8), acc, 0, 0, 0);
+  if (n0 + fr >= n_tokens) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int o = o0 + fg * 4 + j;
+    const float g = gate ? 1.f / (1.f + expf(-bf16_to_f32(gates[j]))) : 1.f;
+    if (o < O) y[(long)tok * y_stride + (long)h * y_head + o] = f32_to_bf16(acc[j] * g);
+  }
+}
+
+// Partial results of ``n_splits`` (2 to 16) splits in the layout of lmsf_paged_attention_decode_mfma with
+// LMSF_ATTENTION_KEEP_PARTS (``scratch`` is that call's, as are tok_idx, n_tokens, pos, window, chunk and D); y, gate and W as
+// for lmsf_head_linear, bfloat16. K a multiple of 32, at most D <= 256; W 16-byte aligned.
+extern "C" int lmsf_head_linear_parts(const float* scratch, const int* tok_idx, const int* pos, int window, int chunk,
+                                      int n_splits, int D, const void* W, void* y, long y_stride, int y_head, const void* gate,
+                                      long gate_stride, int n_tokens, int H, int O, int K, int gate_wide, hipStream_t stream) {
+  LMSF_CHECK(scratch && pos && W && y && lmsf_aligned16(scratch) && lmsf_aligned16(W), "head_linear_parts: null or unaligned pointer");
+  LMSF_CHECK(H > 0 && H <= 65535 && O > 0 && K > 0 && K % 32 == 0 && K <= D && D % 4 == 0 && D <= HLP_MAX_K,
+             "head_linear_parts: bad sizes");
+  LMSF_CHECK(y_head >= O && y_stride >= (long)(H - 1) * y_head + O, "head_linear_parts: heads or rows overlap");
+  LMSF_CHECK(n_splits >= 2 && n_splits <= 16 && chunk > 0 && chunk % 32 == 0, "head_linear_parts: bad splits");
+  if (n_tokens <= 0) return 0;
+  const float* part_ml = scratch + (long)n_tokens * H * n_splits * D;
+  const dim3 grid((n_tokens + 15) / 16, H, (O + 63) / 64);
+#define PARTS(S_)                                                                                                      \
+  hipLaunchKernelGGL(head_linear_parts_kernel<S_>, grid, dim3(256), 0, stream, scratch, part_ml, tok_idx, pos, window, chunk, \
+                     n_splits, D, (const bf16_t*)W, (bf16_t*)y, y_stride, y_head, (const bf16_t*)gate, gate_stride,    \
+                     n_tokens, H, O, K, gate_wide)
+  if (n_splits <= 4) PARTS(4); else if (n_splits <= 8) PARTS(8); else PARTS(16);
+#undef PARTS
+  LMSF_LAUNCH_CHECK("head_linear_parts");
   return 0;
 }
 

@@ -116,6 +116,34 @@ class NormedPair:
         return self.a.device
 
 
+class SplitAttention:
+    """Decode attention whose splits of the context are not added up yet: ``scratch`` is what the split kernel left
+    (csrc/attention_mfma.hip), ``tokens`` the token of each of its rows (None: in order), ``pos`` the tokens' positions,
+    ``window`` the kernels' encoding of the mask. Only ``HipOps.paged_attention(..., keep_parts=True)`` makes one, for
+    ``HipOps.head_linear``."""
+
+    __slots__ = ("scratch", "tokens", "pos", "window", "chunk", "splits", "heads", "dim")
+
+    def __init__(self, scratch: torch.Tensor, tokens: Optional[torch.Tensor], pos: torch.Tensor, window: int, chunk: int,
+                 splits: int, heads: int, dim: int):
+        self.scratch = scratch
+        self.tokens = tokens
+        self.pos = pos
+        self.window = window
+        self.chunk = chunk
+        self.splits = splits
+        self.heads = heads
+        self.dim = dim
+
+    @property
+    def shape(self) -> Tuple[int, int]:
+        return (self.pos.shape[0], self.heads * self.dim)
+
+    @property
+    def device(self) -> torch.device:
+        return self.scratch.device
+
+
 class StreamUpdate:
     """A sublayer's result that a residual of several streams X [N, s, W] has not taken yet: the streams become
     X_t = sum_u mix[u, t] X_u + add_t y. ``y`` [N, W] in the run's type, ``mix`` float32 [s, s] (from row to column),

@@ -12,7 +12,7 @@ import torch
 
 from . import dispatch as D
 from . import library
-from .handles import DeferredLinear, NormedPair, PendingProduct, ScaledRows, StreamUpdate
+from .handles import DeferredLinear, NormedPair, PendingProduct, ScaledRows, SplitAttention, StreamUpdate
 
 F32 = 0
 BF16 = 1
@@ -468,7 +468,7 @@ class HipOps:
                         scale: float, window: int = 0, batch=None, kernel: Optional[str] = None,
                         chunk: int = 0, weights_f32: bool = False, softcap: float = 0.0,
                         distance_bias: Optional[torch.Tensor] = None,
-                        sink: Optional[torch.Tensor] = None) -> torch.Tensor:
+                        sink: Optional[torch.Tensor] = None, keep_parts: bool = False):
         """Attention of every query token over the cached keys of its request: those at positions up to its own,
         within the last ``window`` positions if a window is given, or within its own chunk of ``chunk`` positions
         (chunks counted from position 0 of the request) if a chunk size is given. ``weights_f32``: in a bfloat16 run
@@ -483,7 +483,8 @@ class HipOps:
         [pages, nkv, d, page_size]. ``block_tables`` int32 [S, W]; ``seg``, ``pos`` int32 [N].
         ``batch`` (engine.batch.StepContext) carries host-side facts about the step for the choice of
         kernel; without it they are read back from ``seg`` and ``pos``. ``kernel`` forces "generic" or
-        "mfma" (tests). Returns [N, nh*d] in q's dtype.
+        "mfma" (tests). Returns [N, nh*d] in q's dtype; with ``keep_parts`` a ``SplitAttention`` where all tokens are
+        single ones and their contexts were split 2 to 16 ways.
         """
         self._dev(q, k_pages, v_pages, block_tables, seg, pos)
         if q.dim() != 2 or q.stride(1) != 1 or q.shape[1] < nh * d:
@@ -540,14 +541,18 @@ class HipOps:
             chunk, n_splits = c_chunk.value, c_splits.value
             floats = self.lib.lmsf_attention_decode_scratch_floats(plan.n_single, nh, d, n_splits)
             scratch = torch.empty(floats if n_splits > 1 else 1, dtype=torch.float32, device=q.device)
+            keep = keep_parts and plan.tiles is None and plan.n_single == N and 2 <= n_splits <= 16
             self._check(self.lib.lmsf_paged_attention_decode_mfma_biased(
                 _ptr(q), q.stride(0), _ptr(out), out.stride(0), *common, _ptr(plan.single_tokens), plan.n_single,
                 None if plan.token_is_request else _ptr(seg), _ptr(pos), nh, nkv, d, ps, float(scale),
-                int(window or 0), float(softcap), bias, _ptr(sink), chunk, n_splits, _ptr(scratch), self.decode_attention_order + exact,
-                self._stream()))
+                int(window or 0), float(softcap), bias, _ptr(sink), chunk, n_splits, _ptr(scratch), self.decode_attention_order
+                + exact + (self.ATTENTION_KEEP_PARTS if keep else 0), self._stream()))
+            if keep:
+                return SplitAttention(scratch, plan.single_tokens, pos, int(window or 0), chunk, n_splits, nh, d)
         return out
 
-    ATTENTION_WEIGHTS_F32 = 256     # csrc/entry_points.h: LMSF_ATTENTION_WEIGHTS_F32
+    ATTENTION_WEIGHTS_F32 = 256     # csrc/common.h: LMSF_ATTENTION_WEIGHTS_F32
+    ATTENTION_KEEP_PARTS = 512      # csrc/common.h: LMSF_ATTENTION_KEEP_PARTS
 
     def _attention_plan(self, batch, seg: torch.Tensor, pos: torch.Tensor, nh: int, nkv: int) -> "_AttentionPlan":
         """How a step's tokens are split between the two matrix-core kernels: requests with one token go
@@ -749,13 +754,42 @@ class HipOps:
             also_norm.shape[1] if also_norm is not None else 0, self._stream()))
         return q_out
 
+    def takes_attention_parts(self, weight: torch.Tensor) -> bool:
+        """Whether ``head_linear`` with this weight takes a ``SplitAttention``."""
+        return weight.dtype == torch.bfloat16 and weight.shape[2] % 32 == 0 and weight.shape[2] <= 256 \
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
+
+    def _head_linear_parts(self, x: SplitAttention, x_head: int, weight: torch.Tensor, out: torch.Tensor, out_head: int,
+                           gate: Optional[torch.Tensor], gate_wide: bool) -> torch.Tensor:
+        self._dev(x.scratch, weight, out, gate)
+        H, O, K = weight.shape
+        N = x.shape[0]
+        if not self.takes_attention_parts(weight) or out.dtype != weight.dtype or x_head != x.dim or H != x.heads or K > x.dim:
+            raise ValueError("head_linear: this weight does not take split attention of %d heads of %d" % (x.heads, x.dim))
+        if out.stride(1) != 1 or out.shape[1] < (H - 1) * out_head + O or out.shape[0] != N:
+            raise ValueError("head_linear: operands too narrow for %d heads" % H)
+        need = H * O if gate_wide else H
+        if gate is not None and (gate.dtype != out.dtype or gate.stride(1) != 1 or gate.shape[1] < need or gate.shape[0] != N):
+            raise ValueError("head_linear: gate must be [N, >= %d] of the output's dtype" % need)
+        self._check(self.lib.lmsf_head_linear_parts(
+            _ptr(x.scratch), _ptr(x.tokens), _ptr(x.pos), x.window, x.chunk, x.splits, x.dim, _ptr(weight), _ptr(out),
+            out.stride(0), int(out_head), _ptr(gate), gate.stride(0) if gate is not None else 0, N, H, O, K,
+            1 if (gate_wide and gate is not None) else 0, self._stream()))
+        return out
+
     def head_linear(self, x: torch.Tensor, x_head: int, weight: torch.Tensor, out: torch.Tensor, out_head: int,
                     gate: Optional[torch.Tensor] = None, rope_tail=None, gate_wide: bool = False) -> torch.Tensor:
         """Per-head products: out[n, h * out_head + o] = sum_k weight[h, o, k] x[n, h * x_head + k], times
         sigmoid(gate[n, h]) if a gate is given (``gate_wide``: a gate per output, sigmoid(gate[n, h * O + o])).
         ``weight`` contiguous [H, O, K]; x, out and gate are views with
         unit column stride whose first column is head 0's first entry. ``rope_tail`` = (x_at, out_at, width,
-        positions, table): also what ``rope_tail`` does with these arguments, from the same launch where it can be."""
+        positions, table): also what ``rope_tail`` does with these arguments, from the same launch where it can be.
+        ``x`` may be a ``SplitAttention`` (``takes_attention_parts``; no ``rope_tail`` then): its splits are added up in the
+        same launch."""
+        if isinstance(x, SplitAttention):
+            if rope_tail is not None:
+                raise ValueError("head_linear: split attention has no part to rotate")
+            return self._head_linear_parts(x, x_head, weight, out, out_head, gate, gate_wide)
         self._dev(x, weight, out, gate)
         x_at = out_at = width = rot = max_pos = 0
         positions = table = None

@@ -93,6 +93,8 @@ _SIGNATURES = {
                                         c_int, c_int, c_int, c_int, _P, _P, _P, c_long, c_int, _P]),
     "lmsf_head_linear": (c_int, [_P, c_int, c_long, c_int, _P, _P, c_long, c_int, _P, c_long, c_int, c_int, c_int, c_int,
                                  _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P]),
+    "lmsf_head_linear_parts": (c_int, [_P, _P, _P, c_int, c_int, c_int, c_int, _P, _P, c_long, c_int, _P, c_long, c_int, c_int,
+                                       c_int, c_int, c_int, _P]),
     "lmsf_rope_tail": (c_int, [_P, c_int, c_long, c_int, c_int, _P, c_long, c_int, c_int, _P, _P, c_int, c_int, c_int,
                                c_int, c_int, _P]),
     "lmsf_table_moe": (c_int, [_P, c_int, c_long, _P, _P, _P, _P, c_int, c_int, c_int, c_float, _P, c_long, _P, _P, _P, _P,

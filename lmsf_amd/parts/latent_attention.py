@@ -134,6 +134,9 @@ class LatentAttention(Mixer):
         ops.head_linear(q, self.dn + self.dr, self.uk_t.weight, qa, self.D,
                         rope_tail=(self.dn, self.R, self.dr, ctx.positions, table))
         more = {"weights_f32": True} if self.weights_f32 else {}
+        takes_parts = getattr(ops, "takes_attention_parts", None)
+        if takes_parts is not None and takes_parts(self.uv.weight):
+            more["keep_parts"] = True                                        # (the product that follows adds up the splits)
         a = ops.paged_attention(qa, binding.k_pages, binding.v_pages, group.block_tables, ctx.seg_of_token,
                                 ctx.positions, self.H, 1, self.D, self.scale, self.window or 0, batch=ctx, **more)
         out = torch.empty((N, self.H * self.dv), dtype=q.dtype, device=q.device)

@@ -32,3 +32,34 @@ def test_against_the_general_kernel(ops, ps, nh, nkv, d, mask):
     got, want = run("mfma"), run("generic")
     # weights rounded to bfloat16 (2^-9 of values of up to 5 units, averaged) and both results rounded to it
     assert not torch.isnan(got).any() and float((got - want).abs().max()) <= 5 * 2.0 ** -8
+
+
+# 2, 3, 4, 5 and 16 splits, tokens in order and in order of their contexts (16 and more), a last tile of one token, windows
+# that leave the first splits without keys
+@pytest.mark.parametrize("n,longest,splits", [(1, 256, 2), (8, 300, 3), (8, 512, 4), (17, 600, 5), (3, 2000, 16)])
+@pytest.mark.parametrize("H,R,D,O", [(4, 32, 48, 5), (16, 224, 256, 64), (3, 160, 176, 80)])
+@pytest.mark.parametrize("window", [0, 150])
+@pytest.mark.parametrize("wide", [False, True])
+def test_product_that_adds_up_the_splits(ops, n, longest, splits, H, R, D, O, window, wide):
+    from lmsf_amd.ops.handles import SplitAttention
+    g = torch.Generator().manual_seed(n * D + longest)
+    ps, width = 16, longest // 16 + 1
+    pages = n * width
+    k, v = (torch.randn(pages, 1, *s, generator=g).bfloat16().cuda() for s in ((ps, D), (D, ps)))
+    table = torch.randperm(pages, generator=g).to(torch.int32).view(n, width).cuda()
+    pos = torch.randint(0, longest, (n,), generator=g, dtype=torch.int32)
+    pos[0] = longest - 1
+    q, w = torch.randn(n, H * D, generator=g).bfloat16().cuda(), torch.randn(H, O, R, generator=g).bfloat16().cuda()
+    gate = torch.randn(n, (H * O if wide else H) + 3, generator=g).bfloat16().cuda()
+    before = ops.decode_attention_splits
+    ops.decode_attention_splits = splits
+    try:
+        args = (q, k, v, table, torch.arange(n, dtype=torch.int32).cuda(), pos.cuda(), H, 1, D, D ** -0.5, window)
+        kept, whole = ops.paged_attention(*args, keep_parts=True), ops.paged_attention(*args)
+    finally:
+        ops.decode_attention_splits = before
+    assert isinstance(kept, SplitAttention) and kept.shape == whole.shape and kept.splits > 1
+    outs = [torch.zeros(n, H * O, dtype=torch.bfloat16, device="cuda:0") for _ in range(2)]
+    for x, out in zip((kept, whole), outs):
+        ops.head_linear(x, D, w, out, O, gate=gate, gate_wide=wide)
+    assert torch.equal(*outs) and outs[0].abs().sum() > 0
