@@ -167,6 +167,7 @@ class LMHead(Part):
             raise ValueError("lm_head: softcap must be >= 0")
         self.vocab_size, self.hidden_size = int(vocab_size), int(hidden_size)
         self.weight_name = weight_name or "%s.weight" % prefix
+        self.shares_table = not self.weight_name.startswith(prefix)
         self.bias_name = "%s.bias" % prefix if bias else None
         self.weight: Optional[torch.Tensor] = None
         self.bias: Optional[torch.Tensor] = None
@@ -178,7 +179,17 @@ class LMHead(Part):
         return out
 
     def load_weights(self, fetch: Callable[[str], torch.Tensor]) -> None:
-        self.weight = fetch(self.weight_name).contiguous()
+        # a matrix of its own is laid out as linear layers' are, its rows a little apart (``ops.weight_row_pad``; 128,256 x
+        # 8,192 at 4 rows 342 -> 298 us, x 4,096 at 1 and 64 rows 159 and 231 -> 149 and 227); the embedding's table stays as the loader shares it
+        pad_of = getattr(self.rt.ops, "weight_row_pad", None)
+        pad = int(pad_of(self.hidden_size, self.rt.dtype)) if pad_of is not None and not self.shares_table else 0
+        apart = torch.empty((self.vocab_size, self.hidden_size + pad), dtype=self.rt.dtype, device=self.rt.device) if pad else None
+        weight = fetch(self.weight_name)
+        if apart is not None and weight.dtype == apart.dtype and weight.device == apart.device:
+            self.weight = apart[:, :self.hidden_size]
+            self.weight.copy_(weight)
+        else:
+            self.weight = weight.contiguous()
         if self.bias_name:
             self.bias = fetch(self.bias_name).to(self.weight.dtype).contiguous()
 

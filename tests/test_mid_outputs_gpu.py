@@ -58,3 +58,22 @@ def test_float32_output_of_many_columns(ops, N, M):
     exact = x.double() @ w.double().T
     # 64 products and their sums in float32
     assert ((wide.double() - exact).abs() <= 66 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
+
+
+# one round of workgroups, several well filled ones, one nearly empty; at and beyond the line of 12,288 outputs; an output
+# that is not aligned
+@pytest.mark.parametrize("N,K", [(12224, 128), (12288, 128), (16388, 2048), (32000, 128), (20000, 4096), (128256, 64)])
+@pytest.mark.parametrize("M", [1, 4, 8, 16])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_few_rows_and_many_outputs(ops, M, N, K, out, shift):
+    from lmsf_amd.ops.hip_ops import _ptr
+    g = torch.Generator().manual_seed(N + M)
+    w, x, b = rnd(g, N, K), rnd(g, M, K), rnd(g, N)
+    y = torch.full((M * N + 8,), float("nan"), dtype=out, device="cuda:0")[shift:shift + M * N].view(M, N)
+    ops._check(ops.lib.lmsf_gemm_skinny(_ptr(x), K, _ptr(w), K, _ptr(b), _ptr(y), 0 if out == torch.float32 else 1, N, M, N, K,
+                                        0, 0, ops._stream()))
+    exact = x.double() @ w.double().T + b.double()
+    # K products of float32 sums in any order, and one rounding where the output is bfloat16
+    bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * (K + 2) * 2.0 ** -24
+    assert ((y.double() - exact).abs() <= bound + (exact.abs() * 2.0 ** -8 if out == torch.bfloat16 else 0)).all()
