@@ -60,7 +60,9 @@ __device__ __forceinline__ void mid_store4(float* p, const float* o) {
   *reinterpret_cast<float4*>(p) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
-#define MID_STAGES_OF(TW) ((TW) == 2 ? 4 : 5)   // stages of the ring: what fits into the 160 KB of LDS
+// stages of the ring: what fits into the 160 KB of LDS; three for the plain product of two tiles a wave and up to 64 rows, of
+// which two workgroups then share a compute unit
+#define MID_STAGES_OF(TW, ACT, MT) ((TW) == 2 ? ((ACT) == 0 && (MT) <= 4 ? 3 : 4) : 5)
 #define MID_TILE 2048
 
 // MT: tiles of 16 rows of x (2, 4, 6 or 8). ACT: 0 none, 1 silu-gated, 2 gelu-gated, 6 gated with both operands
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
                                                        int n_split, int U, MidRowScale rs) {
   constexpr int WP = ACT ? 2 : 1;      // projections: gate and up, or the only one
   constexpr int WT = WP * TW;          // tiles of 16 rows of W per wave: TW of each projection
-  constexpr int STAGES = MID_STAGES_OF(TW);
+  constexpr int STAGES = MID_STAGES_OF(TW, ACT, MT);
   constexpr int STAGE = (4 * WT + MT) * MID_TILE;
   constexpr int XL = MT / 2;           // halves of x tiles this wave moves per step (2 MT halves over 4 waves)
   constexpr int LPW = 2 * WT + XL;     // transfers per wave and step
@@ -275,7 +277,7 @@ static int launch_mid(dim3 grid, int U, hipStream_t stream, const bf16_t* x, lon
                       MidRowScale rs) {
   static_assert(TW == 1 || TW == 2, "one or two tiles of each projection per wave");
   constexpr int WT = (ACT ? 2 : 1) * TW;
-  const size_t smem = (size_t)MID_STAGES_OF(TW) * (4 * WT + MT) * MID_TILE;
+  const size_t smem = (size_t)MID_STAGES_OF(TW, ACT, MT) * (4 * WT + MT) * MID_TILE;
   auto kernel = gemm_mid_kernel<MT, ACT, PARTIAL, TOut, TW>;
   static bool configured = false;   // per instantiation
   if (!configured) {
@@ -372,10 +374,17 @@ static int mid_product(const bf16_t* xb, long ldx, const bf16_t* Wb, long ldw, c
   // empty) 93 / 105 -> 90 / 95. Up to 64 rows there is too little to share and 64 is ahead, by 2 to 23 %
   // from 65,536 to 110,000 columns of 2,048 to 8,192 (only beyond 128,000 columns of 4,096 are 64 rows 4 % faster with
   // 128).
-  if (out_dtype == LMSF_F32 && n_split == 1 && M > 64 && (N + 127) / 128 >= 2 * lmsf_compute_units()) {
+  // With W's rows apart (not a multiple of 4 KB) and three stages, two workgroups to a compute unit, that holds from 33 rows
+  // on and from one round of workgroups: at 48 / 64 rows 128,256 x 4,096 210 / 226 -> 189 / 200 us, 128,256 x 8,192 406 / 435
+  // -> 365 / 382, 32,000 x 2,048 28.5 / 30.4 -> 26.1 / 27.0, 100,352 x 5,120 220 / 239 -> 207 / 222; at 17 and 32 rows within 3
+  // % of each other either way.
+  const int cus = lmsf_compute_units();
+  const bool apart = ldw * 2 % 4096 != 0;
+  if (out_dtype == LMSF_F32 && n_split == 1 &&
+      ((M > 64 && (N + 127) / 128 >= 2 * cus) || (M > 32 && M <= 64 && apart && (long)((N + 127) / 128) * 100 >= 95L * cus))) {
     const dim3 wide((N + 127) / 128, 1);
 #define WIDE(MT_) rc = launch_mid<MT_, 0, false, float, 2>(wide, 128, stream, xb, ldx, Wb, ldw, bb, (float*)y, ldy, scratch, M, N, K, 1, rs)
-    if (M <= 96) WIDE(6); else WIDE(8);
+    if (M <= 64) WIDE(4); else if (M <= 96) WIDE(6); else WIDE(8);
 #undef WIDE
   } else if (out_dtype == LMSF_F32) {
     if (M <= 32) MID(2, 0, float); else if (M <= 64) MID(4, 0, float); else if (M <= 96) MID(6, 0, float); else MID(8, 0, float);

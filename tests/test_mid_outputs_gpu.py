@@ -77,3 +77,16 @@ def test_few_rows_and_many_outputs(ops, M, N, K, out, shift):
     # K products of float32 sums in any order, and one rounding where the output is bfloat16
     bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * (K + 2) * 2.0 ** -24
     assert ((y.double() - exact).abs() <= bound + (exact.abs() * 2.0 ** -8 if out == torch.bfloat16 else 0)).all()
+
+
+# 128 outputs a workgroup from 33 rows on where W's rows lie apart: the last widths before the line and the first beyond it
+# (243 workgroups on 256 units), remainders; to the bits of fewer rows, which run 64 outputs a workgroup
+@pytest.mark.parametrize("N", [30976, 31104, 31108, 65540])
+@pytest.mark.parametrize("M", [33, 48, 64])
+@pytest.mark.parametrize("K", [64, 448, 2048])
+def test_rows_apart(ops, N, M, K):
+    g = torch.Generator().manual_seed(N + M + K)
+    w, x, b = rnd(g, N, K + 256)[:, :K], rnd(g, M, K), rnd(g, N)
+    many = product(ops, x, w, b, torch.float32, 1, False)
+    assert torch.equal(many[:32], product(ops, x[:32], w, b, torch.float32, 1, False))
+    assert torch.equal(many[M - 32:], product(ops, x[M - 32:], w, b, torch.float32, 1, False))
