@@ -183,9 +183,9 @@ class LMHead(Part):
         # 8,192 at 4 rows 342 -> 298 us, x 4,096 at 1 and 64 rows 159 and 231 -> 149 and 227); the embedding's table stays as the loader shares it
         pad_of = getattr(self.rt.ops, "weight_row_pad", None)
         pad = int(pad_of(self.hidden_size, self.rt.dtype)) if pad_of is not None and not self.shares_table else 0
-        apart = torch.empty((self.vocab_size, self.hidden_size + pad), dtype=self.rt.dtype, device=self.rt.device) if pad else None
         weight = fetch(self.weight_name)
-        if apart is not None and weight.dtype == apart.dtype and weight.device == apart.device:
+        if pad:
+            apart = torch.empty((self.vocab_size, self.hidden_size + pad), dtype=weight.dtype, device=weight.device)
             self.weight = apart[:, :self.hidden_size]
             self.weight.copy_(weight)
         else:
