@@ -74,7 +74,7 @@ __device__ __forceinline__ void mid_store4(float* p, const float* o) {
 // transfers non-temporal it is behind at every number of rows, 42.3 against 40.5 us at 17 rows and 50.1 against 42.7
 // at 48, and is gone.)
 // What the gated product takes when it stands after a norm whose row factor it applies itself (up to 16 rows): x is
-// then bf16(stream * w), sumsq [tiles][16] the sums of stream^2 over 16 columns per row (rows >= M: 0, or the other 8 columns), and the rows
+// then bf16(stream * w), sumsq [tiles][16] the sums of stream^2 over 16 columns per row (rows >= M: 0), and the rows
 // of both products are multiplied by rsqrt(sum / H + eps) before bias and activation, as the few-rows product does
 // (gemm_skinny.hip). sumsq null: no factor.
 struct MidRowScale {
@@ -205,10 +205,6 @@ __global__ __launch_bounds__(256) void gemm_mid_kernel(const bf16_t* __restrict_
     float total = 0.f;
 #pragma unroll
     for (int k = 0; k < 16; ++k) total += red[k * 16 + r];   // in a fixed order
-    if (M <= 8) {                      // places 8 .. 15: the other 8 columns of a tile, or zeros (gemm_skinny.hip)
-#pragma unroll
-      for (int k = 0; k < 16; ++k) total += red[k * 16 + (r ^ 8)];
-    }
     inv = rsqrtf(total / (float)rs.H + rs.eps);
   }
   // this lane holds, for token m = mt * 16 + r, the outputs n = n0 + 16 (w TW + tw) + 4 g .. + 3

@@ -68,8 +68,7 @@ struct NormAroundArgs {
   long ld_stream;
   const bf16_t* norm_weight;  // [N] of the norm that follows
   float weight_offset;
-  float* sumsq_out;           // [ceil(N / 16)][16]: sums of stream^2 over 16 columns, per row (rows >= M: 0); with WROWS 8
-                              // (up to 8 rows) over the first 8 of these columns in places 0 .. 7, the others in 8 .. 15
+  float* sumsq_out;           // [ceil(N / 16)][16]: sums of stream^2 over 16 columns, per row (rows >= M: 0)
   // SCALED: the product after the norm (its x is the bf16(stream * w) written above)
   const float* sumsq_in;      // [in_tiles][16]
   int in_tiles;
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   constexpr int XLOADS = (XROWS + T::ROWS_PER_LOAD - 1) / T::ROWS_PER_LOAD;   // load instructions per tile of x
   constexpr int WLOADS = (WROWS + T::ROWS_PER_LOAD - 1) / T::ROWS_PER_LOAD;   // of a tile of W
   static_assert(WROWS == 16 || (WROWS == 8 && MT == 1 && WLOADS < T::LOADS), "8 rows of W: one row tile, and a whole load fewer");
-  static_assert(WROWS == 16 || ACT != 4 || XROWS == 8, "two workgroups share the 16 sums of squares of 16 columns: 8 rows each");
+  static_assert(WROWS == 16 || ACT != 4, "the sums of squares before a norm are over 16 columns");
   static_assert(XROWS == 16 || (XROWS == 8 && MT == 1 && XLOADS < T::LOADS), "8 rows of x: one row tile, and a whole load fewer");
   static_assert(!(SCALED || ACT == 4 || ACT == 7) || MT == 1, "the forms around a norm take up to 16 rows");
   static_assert((ACT != 4 && ACT != 7) || NW >= 4, "the epilogue of the product before a norm has a thread for each of the tile's 256 elements");
@@ -261,10 +260,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   __syncthreads();
   for (int e = tid; e < MT * 256; e += NW * 64) {
     const int mt = e / 256, l = (e % 256) / 4, j = e % 4;
-    if (WROWS < 16 && (l / 16) * 4 + j >= WROWS) {               // the half that was not fetched
-      if (ACT == 4) extra[e] = 0.f;
-      continue;
-    }
+    if (WROWS < 16 && (l / 16) * 4 + j >= WROWS) continue;       // the half that was not fetched
     float sum[WT];
 #pragma unroll
     for (int wt = 0; wt < WT; ++wt) {
@@ -277,10 +273,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
       float total = 0.f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) total += extra[w * 16 + (l % 16)];
-      if (M <= 8) {            // places 8 .. 15: the other 8 columns of a tile, or zeros
-#pragma unroll
-        for (int w = 0; w < NW; ++w) total += extra[w * 16 + (l % 16 ^ 8)];
-      }
       const float inv = rsqrtf(total / (float)na.H + na.eps);
 #pragma unroll
       for (int wt = 0; wt < WT; ++wt) sum[wt] *= inv;
@@ -373,13 +365,13 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
   if (ACT == 4) {
     // the tile's sum of squares per row, in a fixed order: element e = 4 l + j is row l % 16
     __syncthreads();
-    if (tid < WROWS) {
+    if (tid < 16) {
       float t = 0.f;
 #pragma unroll
       for (int g = 0; g < 4; ++g)
 #pragma unroll
         for (int j = 0; j < 4; ++j) t += extra[(g * 16 + tid) * 4 + j];
-      na.sumsq_out[(long)blockIdx.x * WROWS + tid] = t;
+      na.sumsq_out[(long)blockIdx.x * 16 + tid] = t;
     }
   }
 }
@@ -425,12 +417,9 @@ static int launch_skinny(const void* x, long ldx, const void* W, long ldw, const
   if constexpr (MT == 1 && SkinnyTile<KC>::ROWS_PER_LOAD <= 8) {
 #define GO(X_, W_) \
   return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, X_, W_>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na)
-    if constexpr (ACT == 4) {
-      // Sums of squares of two workgroups share a tile's 16 places, so whole tiles and up to 8 rows. Tiles of 16 -> 8 at 8
-      // rows: 2,048 x 2,048 / 4,096 / 8,192 5.5 / 7.1 / 12.0 -> 4.8 / 6.7 / 10.4 us, 1,536 x 6,144 9.1 -> 7.7, 1,024 x
-      // 4,096 6.7 -> 5.8; below 1,024 columns 768 x 768 and 512 x 2,048 are level (3.6, 4.8).
-      if (M <= 8 && N % 16 == 0 && N >= 1024 && skinny_narrow(M, N)) GO(8, 8);
-    } else {
+    // (Before a norm tiles of 8 would be faster too, 2,048 x 2,048 / 8,192 at 8 rows 5.5 / 12.0 -> 4.8 / 10.4 us, but the sums
+    // of squares would be over 8 columns: another order, another factor, other roundings in every layer behind it.)
+    if constexpr (ACT != 4) {
       if (skinny_narrow(M, ACT == 3 ? N / 2 : N)) {
         if (M <= 8) GO(8, 8);
         GO(16, 8);

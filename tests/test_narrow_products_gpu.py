@@ -60,7 +60,7 @@ def test_qkv_product_with_rotation(ops, M, d, heads):
     assert ka.abs().sum() > 0
 
 
-# the first and last widths whose sums of squares come from two workgroups a tile, and one beyond either; 8 rows and 9
+# the widths at which tiles of 8 outputs would fit on the chip, and one beyond; 8 rows and 9
 @pytest.mark.parametrize("N", [1008, 1024, 1040, 2048, 2064])
 @pytest.mark.parametrize("M", [3, 8, 9])
 @pytest.mark.parametrize("K,bias", [(64, False), (4104, True)])
@@ -81,6 +81,26 @@ def test_product_before_a_norm(ops, M, N, K, bias):
     want = torch.nn.functional.silu(a) * u
     err = 2.0 ** -8 * (1.1 * a.abs() * u.abs() + want.abs() * 2) + 1e-5
     assert ((got - want).abs() <= err * 1.05).all()
+
+
+# whole tiles and a last one of 8 columns, widths on both sides of what tiles of 8 outputs would take at once
+@pytest.mark.parametrize("N", [1000, 1024, 2048, 2064])
+@pytest.mark.parametrize("M", [3, 8, 9, 16])
+def test_sums_of_squares_before_a_norm(ops, M, N):
+    """A row's sums are those of 16 columns one after the other, whatever the number of rows and the width: the factor, and
+    with it every rounding of the layers behind it, hangs on their order."""
+    g = torch.Generator().manual_seed(N + M)
+    w, x = rnd(g, N, 512), rnd(g, M, 512)
+    nw = torch.randn(N, generator=g).bfloat16().to("cuda:0")
+    stream = torch.randn(M, N, generator=g).to("cuda:0")
+    h = ops.add_rms_norm(ops.linear(x, w, pending_ok=True), stream, nw, 1e-5, torch.bfloat16, defer_ok=True)
+    assert h.rows_per_tile == 16 and h.tiles == -(-N // 16)
+    squares = torch.zeros(M, 16 * h.tiles)
+    squares[:, :N] = stream.cpu() * stream.cpu()
+    want = torch.zeros(h.tiles, 16)
+    for i in range(16):
+        want[:, :M] += squares.view(M, h.tiles, 16)[:, :, i].T
+    assert torch.equal(h.sumsq.view(h.tiles, 16).cpu(), want)
 
 
 @pytest.mark.parametrize("N", [1, 9, 1000, 2048, 2056, 4096])
