@@ -128,8 +128,8 @@ __global__ __launch_bounds__(TILE_WAVES * 64) void paged_attention_waves_kernel(
 #pragma unroll
     for (int o = LPK; o < 64; o <<= 1) tile_max = fmaxf(tile_max, __shfl_xor(tile_max, o, 64));
     const float m_new = fmaxf(m, tile_max);
-    // (a tile whose scores are all -inf adds nothing)
-    const float pr = !visible || m_new == -INFINITY ? 0.f : expf(sc - m_new);
+    // (a score of -inf, or an unseen key's, adds nothing, also where nothing stands beside it; one that is no number stays one)
+    const float pr = sc == -INFINITY ? 0.f : expf(sc - m_new);
     const float corr = m == -INFINITY ? 0.f : expf(m - m_new);
     float tile_sum = pr;
 #pragma unroll

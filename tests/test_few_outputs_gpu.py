@@ -170,3 +170,30 @@ def test_general_attention_reads_visible_keys_only(ops, d, ps, context, mask, dt
             # scores of a few units to 2^-21, weights that add up to at most one over values of up to 5 units
             tol = 2e-5 + (want.abs() * 2.0 ** -8 if dtype == torch.bfloat16 else 0)
             assert ((got[t, h * d:(h + 1) * d] - want).abs() <= tol).all()
+
+
+# one NaN key: alone in the first tile of a wave (every other key of that tile beyond the token), among the keys of a full
+# tile, and every key of a tile; a query of NaN beside a sink
+@pytest.mark.parametrize("d", [32, 64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("context,bad", [(1, [0]), (300, [299]), (300, [5]), (300, list(range(64))), (300, list(range(192, 256)))])
+def test_general_attention_keeps_what_is_no_number(ops, d, dtype, context, bad):
+    nh, ps, pages = 2, 16, -(-context // 16)
+    g = torch.Generator().manual_seed(d + context)
+    k, v = torch.randn(pages, 1, ps, d, generator=g).to(dtype), torch.randn(pages, 1, d, ps, generator=g).to(dtype)
+    q = torch.randn(2, nh * d, generator=g).to(dtype)
+    q[1, :d] = float("nan")                           # the second token: head 0 has no number, head 1 all of them
+    table = torch.arange(pages, dtype=torch.int32).view(1, -1).cuda()
+    pos = torch.full((2,), context - 1, dtype=torch.int32, device="cuda:0")
+    sink = torch.zeros(nh, device="cuda:0")
+
+    def run(keys):
+        return ops.paged_attention(q.cuda(), keys.cuda(), v.cuda(), table, torch.zeros(2, dtype=torch.int32, device="cuda:0"), pos,
+                                   nh, 1, d, d ** -0.5, kernel="generic", sink=sink).float()
+    clean = run(k)
+    assert torch.isnan(clean[1, :d]).all() and not torch.isnan(clean[0]).any() and not torch.isnan(clean[1, d:]).any()
+    for j in bad:
+        k[j // ps, :, j % ps] = float("nan")
+    assert torch.isnan(run(k)).all()
+    k[k.isnan()] = float("-inf")                      # scores of +-inf and NaN by the query's signs: no number either
+    assert torch.isnan(run(k)).all()
