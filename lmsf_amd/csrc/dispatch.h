@@ -67,7 +67,7 @@ typedef struct {
   int M, N, K;             // rows of x, rows of W (for a gated product: both halves, 2 I), columns of both
   int x_dtype, w_dtype, out_dtype;
   long ldx, ldw;
-  int x_ok16, w_ok16;
+  int x_ok16, w_ok16, y_ok16;   // x, W and the result (a new one is) 16-byte aligned
 } LmsfProductShape;
 
 // y = x W^T (+ bias). ``pending_ok``: the caller takes an unfinished product.

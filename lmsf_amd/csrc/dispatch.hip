@@ -80,7 +80,7 @@ extern "C" void lmsf_route_linear(const LmsfTunables* t, const LmsfProductShape*
     return;
   }
   // one row: a pure stream of W (with two rows only the fused forms gain; the LM head's matrix is large enough for
-  // the few-rows kernel to reach the same rate, so it stays there)
+  // the kernels below to reach the same rate, so it goes on to them)
   if (bf && 0 < M && M <= std::min(1, t->gemv_max_rows) && s_ok && gemv_ok(M, K) && (long)N * K <= (1L << 28)) {
     *out = route(LMSF_ROUTE_GEMV);
     return;
@@ -94,7 +94,9 @@ extern "C" void lmsf_route_linear(const LmsfTunables* t, const LmsfProductShape*
   // few rows: the weight-streaming kernel; it also serves float32 output where the kernels above do not take the
   // operands, for any number of rows
   if (bf && s_ok && (M <= (out_bf ? t->skinny_max_rows : 64) || !out_bf)) {
-    *out = route(LMSF_ROUTE_SKINNY);
+    // (few rows and many outputs, an LM head: the 17-and-more-rows kernel, unless a variant of the other one is asked for)
+    const bool many = t->skinny_variant == 0 && M <= t->mid_max_rows && s.y_ok16 && lmsf_gemm_mid_many_outputs(M, N, K, s.ldw);
+    *out = route(many ? LMSF_ROUTE_MID : LMSF_ROUTE_SKINNY);
     return;
   }
   // (float32 output that no kernel above takes, a K that is no multiple of 8, goes to the plain kernel: the library

@@ -186,6 +186,7 @@ int lmsf_gemm_mid(const void* x, long ldx, const void* W, long ldw, const void* 
 int lmsf_gemm_mid_scaled_fits(int M, int N, int K, int in_tiles);
 int lmsf_gemm_mid_scaled(const void* x, long ldx, const void* W, long ldw, const void* bias, void* y, long ldy, int M,
     int N, int K, int act, const float* sumsq, int in_tiles, float eps, hipStream_t stream);
+int lmsf_gemm_mid_many_outputs(int M, int N, int K, long ldw);
 int lmsf_gemm_mid_partial(const void* x, long ldx, const void* W, long ldw, int M, int N, int K, int n_split, float*
     scratch, hipStream_t stream);
 int lmsf_gemm_mid_reduce(const float* scratch, const void* bias, void* y, int out_dtype, long ldy, int M, int N, int

@@ -438,6 +438,28 @@ extern "C" int lmsf_gemm_mid(const void* x, long ldx, const void* W, long ldw, c
   return lmsf_gemm_mid_limit(x, ldx, W, ldw, bias, y, out_dtype, ldy, M, N, K, act, 0.f, n_split, scratch, stream);
 }
 
+// Whether a plain product of up to 16 rows has so many outputs (an LM head) that it runs here, where x is read once for 64
+// outputs, instead of in the few-rows kernel, which reads it once for 16. This kernel's time is that of its rounds over the
+// compute units (about the time of reading W over the share of the rounds that is filled), that one's grows with the rows (1.03
+// times that of reading W at 4 rows, 1.09 at 8, 1.37 at 16), so the line is a filled share that falls with the rows. float32
+// output, few-rows kernel -> here, at 4 / 8 / 16 rows: 128,256 x 2,048 83 / 93 / 118 -> 79 / 81 / 86 us, x 4,096 154 / 173 / 223
+// -> 153 / 157 / 165, 32,000 x 2,048 25 / 26 / 32 -> 24 / 24 / 24, 16,384 x 2,048 (one round) 14.4 / 15.1 / 16.5 -> 13.6 / 13.6 /
+// 12.9; with a round nearly empty, 20,000 x 4,096, 28 / 29.5 / 36 against 36 / 36 / 36, or 100,352 x 5,120 (0.875 filled) 153 /
+// 168 / 215 against 164 / 165 / 170; at one row of 4,096 columns and more that kernel is ahead (128,256 x 4,096 155 against 160,
+// 100,352 x 5,120 157 against 170). Below 12,288 outputs its tiles are ahead (8,192 x 2,048 8.8 against 11.6), and so they are
+// where W's rows lie a multiple of 4 KB apart, all on the same memory channels (128,256 x 4,096 at 8 rows 160 against 185): there
+// 64 rows side by side hurt more than 16. (The two kernels add up K in different orders, so from here on the last bits of a row's
+// logits hang on the number of rows beside it, as they do at 1 and at 17 rows: at 4,096 columns between 4 and 8 of them. One line
+// for all rows would cost 3 to 20 % on one side of it.)
+extern "C" int lmsf_gemm_mid_many_outputs(int M, int N, int K, long ldw) {
+  if (M < 1 || M > 16 || N <= 0 || N % 4 != 0 || K <= 0 || K % 64 != 0 || ldw * 2 % 4096 == 0) return 0;
+  const long cus = lmsf_compute_units(), blocks = ((long)N + 63) / 64;
+  if (cus <= 0 || blocks * 4 < cus * 3 || (M == 1 && K > 2048)) return 0;
+  const long rounds = (blocks + cus - 1) / cus, filled = 100 * blocks / (rounds * cus);
+  // (within one round the outputs are shared out evenly)
+  return rounds == 1 || (K <= 2048 && filled >= 95) || 2 * filled >= 236 - 7 * M ? 1 : 0;
+}
+
 // The two halves of a product without activation whose K is split (n_split >= 2): the partial sums alone,
 // scratch[(s * M + m) * N + n], for a kernel that reduces them while it loads its operand (LmsfPartialSum);
 // and the reduction alone, y = sum over s + bias, for a caller that turns out to need the plain result.

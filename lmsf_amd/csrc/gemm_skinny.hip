@@ -47,7 +47,6 @@
 // MFMA: v_mfma_f32_16x16x32_bf16, A = W tile (16 rows x 32 k), B = x tile (32 k x 16 tokens), D[n][m]:
 // lane l holds token m = l % 16 and the four outputs n = (l / 16) * 4 .. + 3.
 #include "common.h"
-#include "entry_points.h"
 
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));   // a 16-byte piece in flight
 
@@ -431,25 +430,6 @@ static int launch_skinny(const void* x, long ldx, const void* W, long ldw, const
   return launch_skinny_x<MT, KC, NW, TOut, ACT, DEPTH, SCALED, 16, 16>(x, ldx, W, ldw, bias, y, ldy, M, N, K, stream, rc, na);
 }
 
-// Whether a plain product of up to 16 rows has so many outputs (an LM head) that it runs in the 17-and-more-rows kernel, which
-// reads x once for 64 outputs where this one reads it once for 16. That kernel's time is that of its rounds over the compute
-// units (about the time of reading W over the share of the rounds that is filled), this one's grows with the rows (1.03 times
-// that of reading W at 4 rows, 1.09 at 8, 1.37 at 16), so the line is a filled share that falls with the rows. float32 output,
-// here -> there, at 4 / 8 / 16 rows: 128,256 x 2,048 82 / 88 / 113 -> 79 / 81 / 87 us, x 4,096 151 / 163 / 210 -> 152 / 157 /
-// 167, 32,000 x 2,048 24.5 / 25.6 / 31.4 -> 23.3 / 23.6 / 22.8, 16,384 x 2,048 (one round) 14.5 / 15.0 / 17.9 -> 13.5 / 13.6 /
-// 13.9; with a round nearly empty, 20,000 x 4,096, 28 / 29.5 / 36 against 36 / 36 / 36, or 100,352 x 5,120 (0.875 filled) 151 /
-// 160 / 201 against 163 / 165 / 170. Below 12,288 outputs the tiles here are ahead (8,192 x 2,048 8.8 against 11.6), and so
-// they are where W's rows lie a multiple of 4 KB apart, all on the same memory channels (128,256 x 4,096 at 8 rows 160
-// against 185): there 64 rows side by side hurt more than 16.
-static bool many_outputs(int M, int N, int K, long ldw) {
-  if (ldw * 2 % 4096 == 0) return false;
-  const long cus = lmsf_compute_units(), blocks = ((long)N + 63) / 64;
-  if (M > 16 || cus <= 0 || blocks * 4 < cus * 3 || (M == 1 && K > 2048)) return false;
-  const long rounds = (blocks + cus - 1) / cus, filled = 100 * blocks / (rounds * cus);
-  // (within one round the outputs are shared out evenly)
-  return rounds == 1 || (K <= 2048 && filled >= 95) || 2 * filled >= 236 - 7 * M;
-}
-
 // x [M, K] bfloat16 (row stride ldx), W [N, K] bfloat16 (row stride ldw), bias [N] bfloat16 or null,
 // y [M, N] of out_dtype. Needs M <= 64, K a multiple of 8, 16-byte aligned x and W and row strides
 // that are multiples of 8 elements; anything else is refused. ``variant`` picks the tiling (0: default).
@@ -469,8 +449,6 @@ extern "C" int lmsf_gemm_skinny_limit(const void* x, long ldx, const void* W, lo
   LMSF_CHECK((act >= 0 && act <= 2) || act == 5 || act == 6, "gemm_skinny: unknown activation %d", act);
   LMSF_CHECK(act == 0 || out_dtype == LMSF_BF16, "gemm_skinny: the gated form writes bfloat16 only");
   if (M == 0) return 0;
-  if (act == 0 && variant == 0 && K % 64 == 0 && N % 4 == 0 && ldy % 4 == 0 && lmsf_aligned16(y) && many_outputs(M, N, K, ldw))
-    return lmsf_gemm_mid(x, ldx, W, ldw, bias, y, out_dtype, ldy, M, N, K, 0, 1, nullptr, stream);
   const int mt = (M + 15) / 16;
   int rc = 0;
   NormAroundArgs bound = NormAroundArgs();

@@ -160,7 +160,7 @@ inline int esize(int dtype) { return dtype == LMSF_F32 ? 4 : 2; }
 
 // what the functions of dispatch.h want to know of a product x W^T, W of ``w_rows`` rows
 LmsfProductShape shape_of(const void* x, int x_dtype, long ldx, int M, int K, const void* W, int wdtype, long ldw,
-                          int w_rows, int out_dtype) {
+                          int w_rows, int out_dtype, const void* out = nullptr) {
   LmsfProductShape s;
   s.M = M;
   s.N = w_rows;
@@ -172,6 +172,7 @@ LmsfProductShape shape_of(const void* x, int x_dtype, long ldx, int M, int K, co
   s.ldw = ldw;
   s.x_ok16 = lmsf_aligned16(x);
   s.w_ok16 = lmsf_aligned16(W);
+  s.y_ok16 = lmsf_aligned16(out);     // (null: a new one)
   return s;
 }
 
@@ -262,7 +263,7 @@ int op_linear(Run& r, const Value& x, const void* W, int wdtype, long ldw, int N
     return 1;
   }
   const int M = x.M, K = x.N;
-  const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, W, wdtype, ldw, N, out_dtype);
+  const LmsfProductShape shape = shape_of(x.p, x.dtype, x.ld, M, K, W, wdtype, ldw, N, out_dtype, out);
   LmsfRoute rt;
   lmsf_route_linear(&t, &shape, pending_ok ? 1 : 0, &rt);
   if (rt.route != LMSF_ROUTE_CHUNKS) r.count(rt.route);

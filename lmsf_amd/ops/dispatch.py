@@ -25,7 +25,8 @@ class Route(Structure):
 
 class ProductShape(Structure):
     _fields_ = ([(n, c_int) for n in ("M", "N", "K", "x_dtype", "w_dtype", "out_dtype")]
-                + [("ldx", c_long), ("ldw", c_long), ("x_ok16", c_int), ("w_ok16", c_int)])
+                + [("ldx", c_long), ("ldw", c_long), ("x_ok16", c_int), ("w_ok16", c_int),
+                   ("y_ok16", c_int)])
 
 
 (PLAIN, MID, LARGE, DEFERRED, GEMV, CHUNKS, SKINNY, BLAS, MATERIALIZE, MID_SCALED, GEMV_SCALED, SKINNY_SCALED, SEPARATE,

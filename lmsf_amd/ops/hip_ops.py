@@ -99,11 +99,13 @@ class HipOps:
         """The switch points as they are now, in the order of ``dispatch.TUNABLE_NAMES``."""
         return self._tun.as_tuple()
 
-    def _shape(self, x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype) -> D.ProductShape:
+    def _shape(self, x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype,
+               out: Optional[torch.Tensor] = None) -> D.ProductShape:
         """What the C++ side wants to know of a product x weight^T before it names the kernel."""
         return D.ProductShape(x.shape[0], weight.shape[0], x.shape[1], _code(x.dtype), _code(weight.dtype),
                               _code(out_dtype), x.stride(0), weight.stride(0), 1 if x.data_ptr() % 16 == 0 else 0,
-                              1 if weight.data_ptr() % 16 == 0 else 0)
+                              1 if weight.data_ptr() % 16 == 0 else 0,
+                              1 if out is None or out.data_ptr() % 16 == 0 else 0)
 
     # ------------------------------------------------------------------ helpers
 
@@ -1793,7 +1795,7 @@ class HipOps:
                     or out.device != x.device:
                 raise ValueError("linear: out must be a contiguous [%d, %d] %s tensor on x's device" % (M, N, out_dtype))
         rt = D.Route()
-        self.lib.lmsf_route_linear(ctypes.byref(self._tun), ctypes.byref(self._shape(x, weight, out_dtype)),
+        self.lib.lmsf_route_linear(ctypes.byref(self._tun), ctypes.byref(self._shape(x, weight, out_dtype, out)),
                                    1 if pending_ok else 0, ctypes.byref(rt))
         if rt.route == D.MID:
             return self._linear_mid(x, weight, bias, 0, out_dtype, rt, out=out)

@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 38      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
+ABI_VERSION = 39      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None

@@ -60,23 +60,50 @@ def test_float32_output_of_many_columns(ops, N, M):
     assert ((wide.double() - exact).abs() <= 66 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all()
 
 
-# one round of workgroups, several well filled ones, one nearly empty; at and beyond the line of 12,288 outputs; an output
-# that is not aligned
-@pytest.mark.parametrize("N,K", [(12224, 128), (12288, 128), (16388, 2048), (32000, 128), (20000, 4096), (128256, 64)])
-@pytest.mark.parametrize("M", [1, 4, 8, 16])
+# Which kernel a product of up to 16 rows and so many outputs runs in, on 256 compute units: the numbers of rows (of 1, 2, 4, 8,
+# 16) that run 64 outputs a workgroup. 191 workgroups of 64 outputs and 192 (the line of 12,288 outputs); a second round nearly
+# empty; two rounds 0.98 and 0.88 filled, at short and long rows; one row, of a long K and of a short one, of matrices too large
+# for the one-row kernel; rows back to back, 4 KB apart.
+MANY = [(12224, 128, 256, ()), (12288, 128, 256, (2, 4, 8, 16)), (16388, 2048, 256, ()), (32000, 2048, 256, (2, 4, 8, 16)),
+        (20000, 4096, 256, ()), (32000, 4160, 256, (8, 16)), (28672, 4160, 256, (16,)), (16384, 16448, 256, (2, 4, 8, 16)),
+        (32000, 2048, 0, ()), (147456, 2048, 256, (1, 2, 4, 8, 16))]
+
+
+@pytest.mark.parametrize("N,K,pad,here", MANY)
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("shift", [0, 1])
-def test_few_rows_and_many_outputs(ops, M, N, K, out, shift):
+def test_few_rows_and_many_outputs(ops, N, K, pad, here, out):
+    from lmsf_amd.ops import dispatch as D
     from lmsf_amd.ops.hip_ops import _ptr
-    g = torch.Generator().manual_seed(N + M)
-    w, x, b = rnd(g, N, K), rnd(g, M, K), rnd(g, N)
-    y = torch.full((M * N + 8,), float("nan"), dtype=out, device="cuda:0")[shift:shift + M * N].view(M, N)
-    ops._check(ops.lib.lmsf_gemm_skinny(_ptr(x), K, _ptr(w), K, _ptr(b), _ptr(y), 0 if out == torch.float32 else 1, N, M, N, K,
-                                        0, 0, ops._stream()))
-    exact = x.double() @ w.double().T + b.double()
-    # K products of float32 sums in any order, and one rounding where the output is bfloat16
-    bound = (x.double().abs() @ w.double().abs().T + b.double().abs()) * (K + 2) * 2.0 ** -24
-    assert ((y.double() - exact).abs() <= bound + (exact.abs() * 2.0 ** -8 if out == torch.bfloat16 else 0)).all()
+    import ctypes
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are for 256 compute units")
+    g = torch.Generator().manual_seed(N + K)
+    w, b, xs = rnd(g, N, K + pad)[:, :K], rnd(g, N), rnd(g, 16, K)
+    code = 0 if out == torch.float32 else 1
+    for M in (1, 2, 4, 8, 16):
+        x = xs[:M]
+        exact, size = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+        for shift in (0, 1):                     # an output that is not aligned stays in the few-rows kernel
+            buf = torch.full((M * N + 16,), float("nan"), dtype=out, device="cuda:0")
+            y = ops.linear(x, w, b, out_dtype=out, out=buf[shift:shift + M * N].view(M, N))
+            assert torch.isnan(buf[:shift]).all() and torch.isnan(buf[shift + M * N:]).all()
+            # K products and their sums in float32 in any order, and one rounding where the output is bfloat16
+            assert ((y.double() - exact).abs() <= size * (K + 2) * 2.0 ** -24
+                    + (exact.abs() * 2.0 ** -8 if out == torch.bfloat16 else 0)).all()
+            r = D.Route()
+            ops.lib.lmsf_route_linear(ctypes.byref(ops._tun), ctypes.byref(ops._shape(x, w, out, y)), 0, ctypes.byref(r))
+            if M == 1 and N * K <= 1 << 28:
+                assert r.route == D.GEMV
+                continue
+            want = torch.empty(M, N, dtype=out, device="cuda:0")
+            args = (_ptr(x), K, _ptr(w), w.stride(0), _ptr(b), _ptr(want), code, N, M, N, K)
+            if M in here and shift == 0:
+                assert r.route == D.MID and r.splits == 1
+                ops._check(ops.lib.lmsf_gemm_mid(*args, 0, 1, None, ops._stream()))
+            else:
+                assert r.route == D.SKINNY
+                ops._check(ops.lib.lmsf_gemm_skinny(*args, 0, 0, ops._stream()))
+            assert torch.equal(y, want)
 
 
 # 128 outputs a workgroup from 33 rows on where W's rows lie apart: the last widths before the line and the first beyond it
