@@ -91,6 +91,9 @@ void lmsf_route_deferred_norm(const LmsfTunables* t, int M, int N, int K, int fi
 // A norm over the float32 stream [M, N] alone, nothing to add and no rows selected, output and weight float32: whether
 // the product that reads it should normalise the rows itself.
 int lmsf_route_stream_norm(const LmsfTunables* t, int M, int N);
+// A Dynamic Tanh whose branch is a product not yet started, of the stream's shape, no rows selected, output bfloat16:
+// whether the few-rows product does the addition and the tanh as well. Else the product runs first.
+int lmsf_route_deferred_tanh(const LmsfTunables* t, int M);
 // How the decode attention kernel splits the keys of a step of ``n_single`` single tokens whose longest context
 // is ``max_context``: keys a split (a multiple of 128) and the number of splits.
 void lmsf_route_decode_attention(const LmsfTunables* t, int n_single, int nh, int nkv, int max_context, int* chunk,

@@ -578,8 +578,8 @@ extern "C" int lmsf_gemm_skinny_add_norm(const void* x, long ldx, const void* W,
 }
 
 // The product before Dynamic Tanh, up to 16 rows: stream [M, N] float32 += bf16(x W^T + bias) in place; y [M, N] =
-// bf16(tanh(alpha stream) w + b), to the bits of the product and the kernel after it (dyt_norm.hip). 8 rows, the two kernels
-// -> this one: a decode step of eight layers with nine such pairs about 26 us less (Niresun, 8 requests: 15.14 -> 14.50 ms).
+// bf16(tanh(alpha stream) w + b), to the bits of the few-rows product and the kernel after it (dyt_norm.hip; a product of one
+// row by itself runs in the one-row kernel, which adds up K in another order). 8 rows, the two kernels -> this one: a decode step of eight layers with nine such pairs about 26 us less (Niresun, 8 requests: 15.14 -> 14.50 ms).
 extern "C" int lmsf_gemm_skinny_add_dyt(const void* x, long ldx, const void* W, long ldw, const void* bias, float* stream_f32,
                                         long ld_stream, const float* w, const float* b, const float* alpha, void* y, long ldy,
                                         int M, int N, int K, int variant, hipStream_t stream) {

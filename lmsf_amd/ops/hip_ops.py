@@ -1404,8 +1404,9 @@ class HipOps:
         unfinished product (``linear(..., pending_ok=True)``): of few rows it is then made, added and followed by the
         tanh in one kernel."""
         if isinstance(branch, DeferredLinear) and rows is None and residual is not None and out_dtype == branch.dtype \
-                and branch.dtype == torch.bfloat16 and branch.shape[0] <= 16 and residual.dtype == torch.float32 \
-                and residual.is_contiguous() and tuple(residual.shape) == branch.shape:
+                and branch.dtype == torch.bfloat16 and residual.dtype == torch.float32 and residual.is_contiguous() \
+                and tuple(residual.shape) == branch.shape \
+                and self.lib.lmsf_route_deferred_tanh(ctypes.byref(self._tun), branch.shape[0]):
             M, H = branch.shape
             self._dev(branch.x, branch.weight, branch.bias, residual, weight, bias, alpha)
             self._f32_vec(weight, H, "dyt_norm: weight")

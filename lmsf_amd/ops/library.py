@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 39      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
+ABI_VERSION = 40      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None
@@ -201,6 +201,7 @@ _SIGNATURES = {
     "lmsf_route_qkv": (None, [POINTER(Tunables), POINTER(ProductShape), c_int, c_int, POINTER(Route)]),
     "lmsf_route_deferred_norm": (None, [POINTER(Tunables), c_int, c_int, c_int, c_int, c_int, POINTER(Route)]),
     "lmsf_route_stream_norm": (c_int, [POINTER(Tunables), c_int, c_int]),
+    "lmsf_route_deferred_tanh": (c_int, [POINTER(Tunables), c_int]),
     "lmsf_route_decode_attention": (None, [POINTER(Tunables), c_int, c_int, c_int, c_int, POINTER(c_int),
                                            POINTER(c_int)]),
 }

@@ -119,6 +119,13 @@ def test_a_norm_that_finds_its_branch_unstarted(lib):
     assert norm(1, fits=0, prepares=0) == D.MATERIALIZE               # rows are selected: the product runs first
 
 
+def test_a_dynamic_tanh_that_finds_its_branch_unstarted(lib):
+    t = defaults()
+    assert [lib.lmsf_route_deferred_tanh(ctypes.byref(t), M) for M in (1, 2, 16, 17)] == [1, 1, 1, 0]
+    t.skinny_max_rows = 0                             # without the few-rows kernel
+    assert lib.lmsf_route_deferred_tanh(ctypes.byref(t), 1) == 0
+
+
 def test_decode_attention_splits(lib):
     t = defaults()
 

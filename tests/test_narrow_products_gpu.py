@@ -107,8 +107,8 @@ def test_sums_of_squares_before_a_norm(ops, M, N):
 @pytest.mark.parametrize("M", [1, 2, 8, 9, 16])
 @pytest.mark.parametrize("K,bias", [(64, False), (4104, True)])
 def test_product_before_dynamic_tanh(ops, M, N, K, bias):
-    """One kernel to the bits of the product and the kernel after it (rows of the few-rows product hang on nothing else, so
-    the separate product of one row is taken from two)."""
+    """One kernel to the bits of the few-rows product and the kernel after it (a separate product of one row would run in the
+    one-row kernel, so it is taken from two: rows of the few-rows product hang on nothing else)."""
     from lmsf_amd.ops.handles import DeferredLinear
     g = torch.Generator().manual_seed(N + M + K)
     w, x, b = rnd(g, N, K), rnd(g, max(M, 2), K), rnd(g, N) if bias else None
@@ -122,3 +122,26 @@ def test_product_before_dynamic_tanh(ops, M, N, K, bias):
     assert torch.equal(s1, s2) and torch.equal(got, want) and not torch.equal(s1, before)
     rows = torch.tensor([M - 1], dtype=torch.int32, device="cuda:0")          # wanted rows alone: the kernels one by one
     assert torch.equal(ops.dyt_norm(p, before.clone(), tw, tb, alpha, torch.bfloat16, rows=rows), want[M - 1:])
+
+
+def test_one_row_before_dynamic_tanh_without_the_few_rows_kernel(ops):
+    """With the few-rows kernel switched off the one-row product and the tanh's kernel run one after the other."""
+    from lmsf_amd.ops.handles import DeferredLinear
+    g = torch.Generator().manual_seed(5)
+    N, K = 32768, 8192                                # (so many that a few would round otherwise)
+    w, x = rnd(g, N, K), rnd(g, 1, K)
+    tw, tb, alpha = (torch.randn(n, generator=g).to("cuda:0") for n in (N, N, 1))
+    s1 = torch.randn(1, N, generator=g).to("cuda:0")
+    names = ("skinny_max_rows", "mid_max_rows", "large_max_rows")
+    s2, before = s1.clone(), [getattr(ops, n) for n in names]
+    for n in names:
+        setattr(ops, n, 0)
+    try:
+        p = ops.linear(x, w, pending_ok=True)
+        assert isinstance(p, DeferredLinear)
+        got = ops.dyt_norm(p, s1, tw, tb, alpha, torch.bfloat16)
+        want = ops.dyt_norm(ops.linear(x, w), s2, tw, tb, alpha, torch.bfloat16)
+    finally:
+        for n, v in zip(names, before):
+            setattr(ops, n, v)
+    assert torch.equal(s1, s2) and torch.equal(got, want)
