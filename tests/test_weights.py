@@ -2,6 +2,7 @@
 import json
 import os
 import struct
+import weakref
 
 import pytest
 import torch
@@ -310,6 +311,41 @@ def test_weight_rows_lie_as_far_apart_as_the_kernels_ask(tmp_path):
 def _is_model_tensor(model, t):
     return any(getattr(p, a, None) is not None and getattr(p, a).data_ptr() == t.data_ptr()
                for p in model.parts() for a in ("weight", "bias"))
+
+
+@pytest.mark.parametrize("stored", [torch.bfloat16, torch.float32])
+def test_head_of_its_own_is_read_into_memory_made_before_it(monkeypatch, stored):
+    """As linear layers are loaded: the rows' memory first (made after the source it would be cut out of the block that the
+    source's conversion has freed), then the source, which nothing holds afterwards; a shared table stays as it is."""
+    from lmsf_amd.parts import PartSpec, build_part
+
+    class Ops:
+        def weight_row_pad(self, in_features, dtype):
+            return 8 if dtype == torch.bfloat16 else 4
+
+    rt = Runtime(ops=Ops(), device=torch.device("cpu"), dtype=torch.bfloat16, max_positions=8)
+    source, events, made = torch.randn(6, 16).to(stored), [], torch.empty
+
+    def fetch(name):
+        events.append("read")
+        t = source.clone()
+        read.append(weakref.ref(t))
+        return t
+
+    def empty(*args, **kw):
+        events.append("made")
+        return made(*args, **kw)
+
+    read = []
+    monkeypatch.setattr(torch, "empty", empty)
+    head = build_part("head", PartSpec("lm_head", {"vocab_size": 6, "hidden_size": 16}), "lm_head", rt)
+    head.load_weights(fetch)
+    assert events[:2] == ["made", "read"] and read[0]() is None
+    assert head.weight.stride() == (24 if stored == torch.bfloat16 else 20, 1) and head.weight.dtype == stored and torch.equal(head.weight, source)
+    events.clear()
+    tied = build_part("head", PartSpec("lm_head", {"vocab_size": 6, "hidden_size": 16, "weight_name": "e.weight"}), "lm_head", rt)
+    tied.load_weights(lambda name: source)
+    assert events == [] and tied.weight.data_ptr() == source.data_ptr()
 
 
 def test_matrices_stored_in_32_bits_are_cast_to_the_run_type_at_load(tmp_path):
