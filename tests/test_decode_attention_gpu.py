@@ -1,5 +1,7 @@
 """Decode attention: the first step's pages are looked up before the position is known, and a key's page is found without a
 division. Page sizes that are no power of two, contexts around the ends of pages, steps and splits, stale table entries."""
+from types import SimpleNamespace
+
 import pytest
 import torch
 
@@ -34,9 +36,9 @@ def test_against_the_general_kernel(ops, ps, nh, nkv, d, mask):
     assert not torch.isnan(got).any() and float((got - want).abs().max()) <= 5 * 2.0 ** -8
 
 
-# 2, 3, 4, 5 and 16 splits, tokens in order and in order of their contexts (16 and more), a last tile of one token, windows
-# that leave the first splits without keys
-@pytest.mark.parametrize("n,longest,splits", [(1, 256, 2), (8, 300, 3), (8, 512, 4), (17, 600, 5), (3, 2000, 16)])
+# 2, 3, 4, 5 and 16 splits, tokens in order and (16 and more) in order of their contexts as a step lists them, last tiles of one
+# token, windows that leave the first splits without keys
+@pytest.mark.parametrize("n,longest,splits", [(1, 256, 2), (8, 300, 3), (8, 512, 4), (17, 600, 5), (33, 300, 3), (3, 2000, 16)])
 @pytest.mark.parametrize("H,R,D,O", [(4, 32, 48, 5), (16, 224, 256, 64), (3, 160, 176, 80)])
 @pytest.mark.parametrize("window", [0, 150])
 @pytest.mark.parametrize("wide", [False, True])
@@ -55,10 +57,15 @@ def test_product_that_adds_up_the_splits(ops, n, longest, splits, H, R, D, O, wi
     ops.decode_attention_splits = splits
     try:
         args = (q, k, v, table, torch.arange(n, dtype=torch.int32).cuda(), pos.cuda(), H, 1, D, D ** -0.5, window)
-        kept, whole = ops.paged_attention(*args, keep_parts=True), ops.paged_attention(*args)
+        batch = SimpleNamespace(aux={}, host_seg_lens=[1] * n, host_seg_starts=list(range(n + 1)), host_seg_first_pos=pos.tolist(),
+                                max_context=longest, replayed=False, all_single=True, n_tokens=n,
+                                longest_first=torch.argsort(pos, descending=True, stable=True).to(torch.int32).cuda())
+        kept, whole = ops.paged_attention(*args, batch=batch, keep_parts=True), ops.paged_attention(*args, batch=batch)
+        assert torch.equal(whole, ops.paged_attention(*args))
     finally:
         ops.decode_attention_splits = before
     assert isinstance(kept, SplitAttention) and kept.shape == whole.shape and kept.splits > 1
+    assert (kept.tokens is not None) == (n >= 16)
     outs = [torch.zeros(n, H * O, dtype=torch.bfloat16, device="cuda:0") for _ in range(2)]
     for x, out in zip((kept, whole), outs):
         ops.head_linear(x, D, w, out, O, gate=gate, gate_wide=wide)
