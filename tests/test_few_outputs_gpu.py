@@ -113,12 +113,14 @@ def test_general_attention(ops, d, ps, context, dtype, shift):
             assert ((got[t, h * d:(h + 1) * d] - want).abs() <= tol).all()
 
 
-# as many workgroups as the chip takes at once with four on a compute unit, and more
+# as many workgroups as the chip takes at once with four on a compute unit, and more: the two register budgets of the form
+# without tiles, which pages of 18 tokens, wider heads and unaligned pages run in, and the tiles
 @pytest.mark.parametrize("d", [32, 96, 260])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shift", [0, 1])
-def test_general_attention_of_many_tokens_gives_the_bits_of_few(ops, d, dtype, shift):
-    nh, nkv, ps = 8, 2, 16
+@pytest.mark.parametrize("ps", [16, 18])
+def test_general_attention_of_many_tokens_gives_the_bits_of_few(ops, d, dtype, shift, ps):
+    nh, nkv = 8, 2
     T = torch.cuda.get_device_properties(0).multi_processor_count * 4 // nh + 3
     g = torch.Generator(device="cuda:0").manual_seed(d)
     pages = -(-T // ps) + 2
