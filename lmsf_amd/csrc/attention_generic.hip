@@ -40,11 +40,14 @@ __device__ __forceinline__ void gen_load4(const bf16_t* p, float* x) {
 // model's tokens have 40 kB of keys and values each, and every trip costs 0.5 to 1 us. So a wave asks for a tile's keys
 // AND values at once (8 loads of four elements of each a lane, 8 kB of each in float32), before it knows any score:
 // position -> block table -> keys and values are three trips up to 8 tiles of keys, where the form below makes one for
-// every four keys a thread. Both forms, that one -> this one, 8 heads on one kv head in float32, 32 / 128 wide: 8 tokens of
-// 300 keys 11.0 / 26.6 -> 5.7 / 7.1 us, 1 token of 16 keys 4.6 / 5.8 -> 4.3 / 4.3, of 8,000 keys 187 / 619 -> 40 / 115, a
-// prompt of 140 tokens 11.2 / 33.5 -> 10.6 / 17.4, its 256 tokens behind 768 others 151 / 541 -> 43 / 98; in bfloat16 alike. LPK lanes share a key (d up to 32 LPK; a tile is 64 / LPK keys), every wave keeps an
-// online softmax of its own over its tiles (w, w + 8, ...) with no barrier, and the waves' results are added up in their
-// order at the end, so a token's bits hang on its own position and window alone.
+// every four keys a thread. Both forms, that one -> this one, 8 heads on one kv head in float32, 32 / 128 / 256 wide: 8
+// tokens of 300 keys 11.0 / 27 / 48 -> 5.7 / 8.0 / 11.7 us, 1 token of 16 keys 4.6 / 6.7 / 8.3 -> 4.3 / 5.7 / 5.4, of 8,000
+// keys 187 / 620 / 1,179 -> 40 / 115 / 212, a prompt of 140 tokens 11.2 / 34 / 65 -> 10.6 / 18.6 / 24, 256 tokens behind
+// 768 others 151 / 536 / 1,072 -> 43 / 104 / 188, a prompt of 2,048 tokens (128 / 256 wide) 4,610 / 9,164 -> 813 / 1,557,
+// heads of 160 and 192 in between; in bfloat16 alike (2,048 tokens 4,176 / 8,318 -> 581 / 1,082). LPK lanes share a key (d
+// up to 32 LPK; a tile is 64 / LPK keys), every wave keeps an online softmax of its own over its tiles (w, w + 8, ...) with
+// no barrier, and the waves' results are added up in their order at the end, so a token's bits hang on its own position and
+// window alone.
 // Values: lane = (dim, quad of keys in the page), so that consecutive lanes read consecutive 16 bytes of a page.
 #define TILE_WAVES 8
 // what a wave's lanes left in LDS is there for its other lanes (LDS serves a wave's accesses in order)
@@ -351,11 +354,12 @@ extern "C" int lmsf_paged_attention_generic_biased(const void* q, long q_stride,
     return 0;
   }
   const bool vec = (size_t)k_pages % (4 * lmsf_elem_size(dtype)) == 0;
-  // What is left: wider heads, pages of other sizes, unaligned ones. More workgroups than the chip takes at once with four on a compute unit: fewer registers, seven on a unit. Both sides
-  // in float32 with 8 heads of 32 / 128, four -> seven a unit: 64 tokens of a prompt 7.6 / 13.8 -> 8.0 / 15.2 us, 100
-  // tokens 9.3 / 22.5 -> 9.7 / 23.3, 140 tokens 14.2 / 38.8 -> 12.4 / 34.6, 200 tokens 22.1 / 61.4 -> 19.5 / 59.3, 256
-  // tokens 32.9 / 105.0 -> 30.5 / 107.2. (Keys read entry by entry and values one by one took 15.1 / 37.9 us for 8
-  // tokens of 300 keys, now 12.1 / 27.7.)
+  // What is left: wider heads, pages of other sizes, unaligned ones. More workgroups than the chip takes at once with four
+  // on a compute unit: fewer registers, seven on a unit. Both sides in float32, 8 heads on one kv head, of 32 / 256 in
+  // pages of 18 and of 512 in pages of 16, four -> seven a unit: 64 tokens of a prompt 6.4 / 15.9 / 40 -> 6.9 / 18.5 / 45
+  // us, 100 tokens 8.0 / 27 / 77 -> 8.0 / 28 / 78, 140 tokens (beyond the line) 11.3 / 44 / 131 -> 9.4 / 42 / 126, 200
+  // tokens 14.8 / 73 / 238 -> 14.1 / 74 / 226, 512 tokens 56 / 376 / 1,344 -> 53 / 429 / 1,406: ahead while seven a unit
+  // hold all that four do not, and with narrow heads; wide heads of many tokens lose 5 to 14 %.
   const bool many = (long)n_tokens * nh > 4L * lmsf_compute_units();
   if (dtype == LMSF_F32) {
     if (vec) GENERIC(float, true); else GENERIC(float, false);

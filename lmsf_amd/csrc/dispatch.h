@@ -1,7 +1,7 @@
 // Which kernel runs an operation: the one table of switch points of this library.
 //
 // The matrix products change kernels with the number of rows (one row: a pure stream of W; up to 16: the
-// few-rows kernel with its fused epilogues; 17 to 128: the 17-and-more-rows kernel; up to 256, or 1,024 for deep
+// few-rows kernel with its fused epilogues, or for an LM head the next one; 17 to 128: the 17-and-more-rows kernel; up to 256, or 1,024 for deep
 // products: the many-rows kernel; beyond: the BLAS library), and so do the forms in which a norm, a rotation or
 // a gated activation is folded into them. Both callers of the kernels, the step program (program.hip) and the
 // Python face (ops/hip_ops.py), ask the functions below and launch what they are told; neither decides anything

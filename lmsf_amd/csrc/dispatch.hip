@@ -196,9 +196,9 @@ extern "C" void lmsf_route_deferred_norm(const LmsfTunables* t, int M, int N, in
 
 extern "C" int lmsf_route_stream_norm(const LmsfTunables* t, int M, int N) { return stream_norm_ok(t, M, N) ? 1 : 0; }
 
-// One and two rows too, which would otherwise run in the one-row kernel and the tanh's: product and tanh -> one kernel at 1 / 2 /
-// 8 / 16 rows 2,048 x 2,048 7.0 / 7.5 / 7.7 / 8.0 -> 5.0 / 4.7 / 5.2 / 5.4 us, 4,096 x 14,336 24.0 / 22.8 / 23.6 / 26.9 -> 21.5 / 20.4 /
-// 20.8 / 24.1, 512 x 512 5.6 -> 3.5 at any. 16 rows is what that form takes.
+// One and two rows too, which would otherwise run in the one-row kernel and the tanh's: product and tanh -> one kernel at 1
+// / 2 / 8 / 16 rows 2,048 x 2,048 7.0 / 7.5 / 7.7 / 8.0 -> 5.0 / 4.7 / 5.2 / 5.4 us, 4,096 x 14,336 24.0 / 22.8 / 23.6 /
+// 26.9 -> 21.5 / 20.4 / 20.8 / 24.1, 512 x 512 5.6 -> 3.5 at any. 16 rows is what that form takes.
 extern "C" int lmsf_route_deferred_tanh(const LmsfTunables* t, int M) { return M <= std::min(t->skinny_max_rows, 16) ? 1 : 0; }
 
 // Measured: about 512 workgroups fill the chip; beyond that a split only adds partial results, and with two short

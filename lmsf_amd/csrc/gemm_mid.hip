@@ -367,11 +367,10 @@ static int mid_product(const bf16_t* xb, long ldx, const bf16_t* Wb, long ldw, c
   // Beyond 64 rows and many more outputs than the chip has workgroups for (an LM head): 128 a workgroup, so that x, which
   // every workgroup reads whole from the caches, is read half as often. 64 -> 128 outputs a workgroup in float32: 128,256 x
   // 4,096 at 96 / 128 rows 293 / 325 -> 247 / 265 us, 66,560 x 2,048 (520 workgroups of 128, a last round that is nearly
-  // empty) 93 / 105 -> 90 / 95. Up to 64 rows there is too little to share and 64 is ahead, by 2 to 23 %
-  // from 65,536 to 110,000 columns of 2,048 to 8,192 (only beyond 128,000 columns of 4,096 are 64 rows 4 % faster with
-  // 128).
-  // With W's rows apart (not a multiple of 4 KB) and three stages, two workgroups to a compute unit, that holds from 33 rows
-  // on and from one round of workgroups: at 48 / 64 rows 128,256 x 4,096 210 / 226 -> 189 / 200 us, 128,256 x 8,192 406 / 435
+  // empty) 93 / 105 -> 90 / 95. Up to 64 rows that depends on the distance between W's rows. A multiple of 4 KB, back to back:
+  // 64 outputs stay ahead, by 2 to 23 % from 65,536 to 110,000 columns of 2,048 to 8,192 (only beyond 128,000 columns of 4,096
+  // are 64 rows 4 % faster with 128). Any other, rows apart: with three stages, so that two workgroups share a compute unit, 128
+  // are ahead from 33 rows on and from one round of workgroups: at 48 / 64 rows 128,256 x 4,096 210 / 226 -> 189 / 200 us, 128,256 x 8,192 406 / 435
   // -> 365 / 382, 32,000 x 2,048 28.5 / 30.4 -> 26.1 / 27.0, 100,352 x 5,120 220 / 239 -> 207 / 222; at 17 and 32 rows within 3
   // % of each other either way.
   const int cus = lmsf_compute_units();

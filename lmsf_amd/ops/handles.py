@@ -63,7 +63,8 @@ class ScaledRows:
     (``HipOps.qkv_rope_cache``, ``HipOps.linear_gated``) multiplies its rows by rsqrt(sum / H + eps), which
     is the same product as with the normalised rows up to where the rounding falls. Of float32 products ``xw`` is
     the stream itself, without sums (``rows_per_tile`` -1): the product that takes it normalises its rows, to the bits
-    of the norm kernel. ``HipOps.materialize`` runs that kernel on the stream instead."""
+    of the norm kernel. ``HipOps.materialize`` runs that kernel on the stream instead. Either way the stream is read when
+    the handle is consumed, which must be before anything is added to it."""
 
     __slots__ = ("xw", "sumsq", "tiles", "rows_per_tile", "stream", "weight", "eps", "weight_offset", "dtype")
 
@@ -138,10 +139,6 @@ class SplitAttention:
     @property
     def shape(self) -> Tuple[int, int]:
         return (self.pos.shape[0], self.heads * self.dim)
-
-    @property
-    def device(self) -> torch.device:
-        return self.scratch.device
 
 
 class StreamUpdate:

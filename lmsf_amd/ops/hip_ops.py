@@ -182,7 +182,9 @@ class HipOps:
         and ``rows`` is None. ``rows`` (int32 [R]) selects input rows; the output then has R rows.
         ``branch`` may be a ``PendingProduct``: its partial sums are added up on the way in; or a
         ``DeferredLinear``, which then runs as a product that adds into ``residual``. With ``defer_ok``
-        the caller takes a ``ScaledRows`` as well (up to 16 rows, after a ``DeferredLinear``).
+        the caller takes a ``ScaledRows`` as well: in bfloat16 of up to 16 rows after a ``DeferredLinear``, in float32 of
+        as many rows as the product that reads them normalises itself (``lmsf_route_stream_norm``), with or without a
+        branch. It must be consumed before anything is added to ``residual``, which may be what it reads.
         """
         if isinstance(branch, PendingProduct):
             return self._add_rms_norm_pending(branch, residual, weight, eps, out_dtype, rows, weight_offset)

@@ -160,7 +160,8 @@ class Part:
     # A norm whose ``forward_add`` takes ``defer_ok=True`` and may then return the norm not yet computed
     # (ops.handles.ScaledRows) sets ``may_defer``; a mixer or feed-forward whose ``forward`` takes such an
     # ``h`` (it hands it to ``rt.ops.qkv_rope_cache`` or ``rt.ops.linear_gated``, or calls ``rt.ops.materialize``
-    # first) sets ``accepts_normed``. A block asks for a deferred norm only where both say so.
+    # first) sets ``accepts_normed``. A block asks for a deferred norm only where both say so, and adds nothing to the
+    # residual stream before that part has read it: in float32 the handle is the stream itself, not a copy.
     may_defer = False
     accepts_normed = False
 
