@@ -88,12 +88,21 @@ class TensorDecl:
     reference casts everything (core/src/model_executor/models/model_factory.rs:124-139). ``init`` says how
     the random-weights mode fills it: "normal" (mean 0, the mode's standard deviation), "ones", "zeros", "last_one"
     (zeros and a final 1), "const:x" (every entry x), "normal:s" (standard deviation s whatever the mode's) or, for an
-    integer table, "choices:E" (every row distinct numbers below E)."""
+    integer table, "choices:E" (every row distinct numbers below E). ``row_gap_bytes``: a matrix that the part keeps as it
+    is fetched, with this much memory left between two rows (``ops.weight_row_pad``); one that several parts share has none."""
 
     shape: Tuple[int, ...]
     kind: str = "float"
     init: str = "normal"
     keeps_float32: bool = False
+    row_gap_bytes: int = 0
+
+    def memory(self, dtype: torch.dtype, device) -> torch.Tensor:
+        """Memory for the tensor, its rows as far apart as declared."""
+        if not self.row_gap_bytes:
+            return torch.empty(self.shape, dtype=dtype, device=device)
+        rows, cols = self.shape
+        return torch.empty((rows, cols + self.row_gap_bytes // dtype.itemsize), dtype=dtype, device=device)[:, :cols]
 
 
 @dataclass(frozen=True)

@@ -167,37 +167,22 @@ class LMHead(Part):
             raise ValueError("lm_head: softcap must be >= 0")
         self.vocab_size, self.hidden_size = int(vocab_size), int(hidden_size)
         self.weight_name = weight_name or "%s.weight" % prefix
-        self.shares_table = not self.weight_name.startswith(prefix)
         self.bias_name = "%s.bias" % prefix if bias else None
         self.weight: Optional[torch.Tensor] = None
         self.bias: Optional[torch.Tensor] = None
 
     def checkpoint_tensors(self) -> Dict[str, TensorDecl]:
-        out = {self.weight_name: TensorDecl((self.vocab_size, self.hidden_size))}
+        # A matrix of its own is laid out as linear layers' are, its rows a little apart (128,256 x 8,192 at 4 rows 342 -> 298
+        # us, x 4,096 at 1 and 64 rows 159 and 231 -> 149 and 227); the embedding's table stays as the loader shares it.
+        pad_of = getattr(self.rt.ops, "weight_row_pad", None)
+        gap = int(pad_of(self.hidden_size, self.rt.dtype)) * self.rt.dtype.itemsize if pad_of is not None else 0
+        out = {self.weight_name: TensorDecl((self.vocab_size, self.hidden_size), row_gap_bytes=gap)}
         if self.bias_name:
             out[self.bias_name] = TensorDecl((self.vocab_size,))
         return out
 
     def load_weights(self, fetch: Callable[[str], torch.Tensor]) -> None:
-        # A matrix of its own is laid out as linear layers' are, its rows a little apart (``ops.weight_row_pad``; 128,256 x
-        # 8,192 at 4 rows 342 -> 298 us, x 4,096 at 1 and 64 rows 159 and 231 -> 149 and 227); the embedding's table stays
-        # as the loader shares it. As there the memory is made before the matrix is read: made after it, torch would cut it
-        # out of what the source's conversion has just freed. The matrix as it was read stands beside it until it is copied.
-        pad_of = getattr(self.rt.ops, "weight_row_pad", None)
-        if pad_of is None or self.shares_table:
-            self.weight = fetch(self.weight_name).contiguous()
-        else:
-            def apart(dtype, device):
-                row = self.hidden_size + int(pad_of(self.hidden_size, dtype))
-                return torch.empty((self.vocab_size, row), dtype=dtype, device=device)[:, :self.hidden_size]
-
-            self.weight = apart(self.rt.dtype, self.rt.device)
-            weight = fetch(self.weight_name)
-            if weight.dtype != self.weight.dtype or weight.device != self.weight.device:   # kept in 32 bits, or elsewhere
-                self.weight = None
-                self.weight = apart(weight.dtype, weight.device)
-            self.weight.copy_(weight)
-            del weight
+        self.weight = fetch(self.weight_name)
         if self.bias_name:
             self.bias = fetch(self.bias_name).to(self.weight.dtype).contiguous()
 

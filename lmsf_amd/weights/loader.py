@@ -14,6 +14,7 @@ norms' weights) or where the caller asks for it for all of them (``keep_float32`
 then run in float32 arithmetic, at twice the memory). A tensor declared "int" becomes int32.
 """
 import warnings
+from dataclasses import replace
 from typing import Callable, Dict, Iterable, List, Optional, Sequence, Tuple
 
 import torch
@@ -58,6 +59,7 @@ def collect_declarations(parts: Iterable[Part], shared: Optional[set] = None) ->
                                      % (name, decls[name].shape, decl.shape))
                 if shared is not None:
                     shared.add(name)
+                decl = replace(decl, row_gap_bytes=0)      # every part takes a shared one
             decls[name] = decl
     return decls
 
@@ -96,6 +98,20 @@ def _convert(t: torch.Tensor, decl: TensorDecl, run_dtype: torch.dtype, keep_flo
     if t.dtype in (torch.float32, torch.float64) and (decl.keeps_float32 or keep_float32):
         return t.to(torch.float32)          # stored in 32 bits (or more) and meant to stay so
     return t.to(run_dtype)
+
+
+PIECE_BYTES = 64 << 20
+
+
+def _read_rows_apart(stored: torch.Tensor, decl: TensorDecl, device, run_dtype: torch.dtype, keep_float32: bool) -> torch.Tensor:
+    """The matrix ``stored`` (over the mapped file) with the declared distance between its rows, copied in pieces: beside
+    the memory that stays only one piece is alive, where a copy of the whole matrix would double it (2.1 GB for an LM
+    head of 128,256 x 8,192)."""
+    out = decl.memory(_convert(stored[:0], decl, run_dtype, keep_float32).dtype, device)
+    step = max(1, PIECE_BYTES // max(1, stored.shape[1] * stored.element_size()))
+    for r in range(0, stored.shape[0], step):
+        out[r:r + step].copy_(_convert(stored[r:r + step].to(device), decl, run_dtype, keep_float32))
+    return out
 
 
 def _return_freed_memory(device) -> None:
@@ -141,7 +157,9 @@ def load_weights(parts: Sequence[Part], folder: str, device: torch.device, run_d
                 return cache[name]
             f, _ = entries[name]
             try:
-                if torch.device(device).type == "cuda":
+                if decls[name].row_gap_bytes:
+                    t = _read_rows_apart(f.read(name, copy=False), decls[name], device, run_dtype, keep_float32)
+                elif torch.device(device).type == "cuda":
                     # from the mapped file to the device as stored, converted there: the bytes are passed over once
                     # on the host, and a 32-bit checkpoint is cast by the GPU
                     t = _convert(f.read(name, copy=False).to(device), decls[name], run_dtype, keep_float32)
@@ -185,6 +203,8 @@ def load_weights_from_generator(parts: Sequence[Part], make: Callable[[str, Tens
         if tuple(t.shape) != tuple(decls[name].shape):
             raise WeightsError("generated tensor %r has shape %s, declared %s"
                                % (name, list(t.shape), list(decls[name].shape)))
+        if decls[name].row_gap_bytes and t.is_contiguous():       # (made back to back)
+            t = decls[name].memory(t.dtype, t.device).copy_(t)
         if name in shared:
             cache[name] = t
         return t

@@ -60,7 +60,7 @@ def random_tensor(name: str, decl: TensorDecl, seed: int, std: float, dtype: tor
     gen.manual_seed(tensor_seed(seed, name))
     t = torch.empty(decl.shape, dtype=torch.float32, device=device)
     t.normal_(0.0, std, generator=gen)
-    return t.to(dtype)
+    return decl.memory(dtype, device).copy_(t) if decl.row_gap_bytes else t.to(dtype)
 
 
 def declared_tensors(arch: Architecture, config: ArchConfig) -> Dict[str, TensorDecl]:

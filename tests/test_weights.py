@@ -2,7 +2,6 @@
 import json
 import os
 import struct
-import weakref
 
 import pytest
 import torch
@@ -313,39 +312,43 @@ def _is_model_tensor(model, t):
                for p in model.parts() for a in ("weight", "bias"))
 
 
-@pytest.mark.parametrize("stored", [torch.bfloat16, torch.float32])
-def test_head_of_its_own_is_read_into_memory_made_before_it(monkeypatch, stored):
-    """As linear layers are loaded: the rows' memory first (made after the source it would be cut out of the block that the
-    source's conversion has freed), then the source, which nothing holds afterwards; a shared table stays as it is."""
-    from lmsf_amd.parts import PartSpec, build_part
+@pytest.mark.parametrize("tied", [False, True])
+@pytest.mark.parametrize("stored", ["bfloat16", "float32"])
+@pytest.mark.parametrize("keep", [False, True])
+def test_head_of_its_own_is_read_in_pieces_into_rows_apart(tmp_path, monkeypatch, tied, stored, keep):
+    """An LM head's matrix lies as linear layers' do, and beside the memory that stays only a piece of it is alive while it is
+    read; a table that the embedding shares is read whole and stays back to back."""
+    from types import SimpleNamespace
+    from lmsf_amd.weights import loader
+    folder, cfg = make_model_folder(tmp_path, "A" if tied else "B", dtype=stored)
+    raw = load_file(os.path.join(folder, "model.safetensors"))
+    name = "model.embed_tokens.weight" if "lm_head.weight" not in raw else "lm_head.weight"
+    assert (name == "lm_head.weight") != tied
+    ops = SimpleNamespace(weight_row_pad=lambda in_features, dtype: 24 if dtype == torch.bfloat16 else 12)
+    rt = Runtime(ops=ops, device=torch.device("cpu"), dtype=torch.bfloat16, max_positions=cfg.max_position_embeddings)
+    model = DecoderModel(get_architecture(cfg.architecture).build_spec(cfg), rt)
+    monkeypatch.setattr(loader, "PIECE_BYTES", 5 * raw[name].shape[1] * raw[name].element_size())
+    most, convert = [0], loader._convert
 
-    class Ops:
-        def weight_row_pad(self, in_features, dtype):
-            return 8 if dtype == torch.bfloat16 else 4
+    def watched(t, decl, *args):
+        if decl.row_gap_bytes:
+            most[0] = max(most[0], t.shape[0])
+        return convert(t, decl, *args)
+    monkeypatch.setattr(loader, "_convert", watched)
+    load_weights(model.parts(), folder, torch.device("cpu"), torch.bfloat16, keep_float32=keep)
+    w, dtype = model.head.weight, torch.float32 if keep and stored == "float32" else torch.bfloat16
+    assert w.dtype == dtype and torch.equal(w, raw[name].to(dtype))
+    assert w.stride() == (w.shape[1] + (0 if tied else 48 // dtype.itemsize), 1)
+    assert most[0] == (0 if tied else 5) and (model.embedding.weight.data_ptr() == w.data_ptr()) == tied
 
-    rt = Runtime(ops=Ops(), device=torch.device("cpu"), dtype=torch.bfloat16, max_positions=8)
-    source, events, made = torch.randn(6, 16).to(stored), [], torch.empty
 
-    def fetch(name):
-        events.append("read")
-        t = source.clone()
-        read.append(weakref.ref(t))
-        return t
-
-    def empty(*args, **kw):
-        events.append("made")
-        return made(*args, **kw)
-
-    read = []
-    monkeypatch.setattr(torch, "empty", empty)
-    head = build_part("head", PartSpec("lm_head", {"vocab_size": 6, "hidden_size": 16}), "lm_head", rt)
-    head.load_weights(fetch)
-    assert events[:2] == ["made", "read"] and read[0]() is None
-    assert head.weight.stride() == (24 if stored == torch.bfloat16 else 20, 1) and head.weight.dtype == stored and torch.equal(head.weight, source)
-    events.clear()
-    tied = build_part("head", PartSpec("lm_head", {"vocab_size": 6, "hidden_size": 16, "weight_name": "e.weight"}), "lm_head", rt)
-    tied.load_weights(lambda name: source)
-    assert events == [] and tied.weight.data_ptr() == source.data_ptr()
+def test_random_head_is_made_in_rows_apart():
+    """The same values as back to back, rounded straight into the memory that stays."""
+    from lmsf_amd.parts.base import TensorDecl
+    from lmsf_amd.weights import random_tensor
+    for dtype in (torch.bfloat16, torch.float32):
+        a, b = (random_tensor("w", TensorDecl((7, 16), row_gap_bytes=gap), 3, 0.02, dtype, torch.device("cpu")) for gap in (0, 32))
+        assert torch.equal(a, b) and a.is_contiguous() and b.stride() == (16 + 32 // dtype.itemsize, 1)
 
 
 def test_matrices_stored_in_32_bits_are_cast_to_the_run_type_at_load(tmp_path):
