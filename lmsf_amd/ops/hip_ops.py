@@ -1770,6 +1770,14 @@ class HipOps:
         argument."""
         return self.weight_row_pad_bytes // torch.empty((), dtype=dtype).element_size()
 
+    def head_row_pad(self, in_features: int, dtype: torch.dtype) -> int:
+        """The same for an LM head's matrix: only where its rows are a multiple of 4 KB. Back to back -> 512 bytes apart, at 8 /
+        16 / 64 rows: 128,256 x 4,096 162 / 198 / 231 -> 156 / 164 / 200 us, 65,536 x 6,144 2 / 24 / 30 % faster; of other lengths there
+        is nothing to gain at few rows and it goes either way beyond: rows of 2 KB (32,000 and 128,256 x 1,024) 0 to 5 / 2 to 6 /
+        5 to 8 % slower, of 6 and 7 KB (3,072 and 3,584 columns) level to 4 % slower, of 5 and 10 KB (2,560 and 5,120) level at 8
+        rows and 2 to 8 % faster from 17 on."""
+        return self.weight_row_pad(in_features, dtype) if in_features * dtype.itemsize % 4096 == 0 else 0
+
     def linear(self, x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                out_dtype: Optional[torch.dtype] = None, pending_ok: bool = False,
                out: Optional[torch.Tensor] = None):

@@ -89,7 +89,7 @@ class TensorDecl:
     the random-weights mode fills it: "normal" (mean 0, the mode's standard deviation), "ones", "zeros", "last_one"
     (zeros and a final 1), "const:x" (every entry x), "normal:s" (standard deviation s whatever the mode's) or, for an
     integer table, "choices:E" (every row distinct numbers below E). ``row_gap_bytes``: a matrix that the part keeps as it
-    is fetched, with this much memory left between two rows (``ops.weight_row_pad``); one that several parts share has none."""
+    is fetched, with this much memory left between two rows (``ops.head_row_pad``); one that several parts share has none."""
 
     shape: Tuple[int, ...]
     kind: str = "float"

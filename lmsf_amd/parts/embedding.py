@@ -172,9 +172,9 @@ class LMHead(Part):
         self.bias: Optional[torch.Tensor] = None
 
     def checkpoint_tensors(self) -> Dict[str, TensorDecl]:
-        # A matrix of its own is laid out as linear layers' are, its rows a little apart (128,256 x 8,192 at 4 rows 342 -> 298
-        # us, x 4,096 at 1 and 64 rows 159 and 231 -> 149 and 227); the embedding's table stays as the loader shares it.
-        pad_of = getattr(self.rt.ops, "weight_row_pad", None)
+        # a matrix of its own may have its rows a little apart, as linear layers' are; the embedding's table stays as the
+        # loader shares it
+        pad_of = getattr(self.rt.ops, "head_row_pad", None)
         gap = int(pad_of(self.hidden_size, self.rt.dtype)) * self.rt.dtype.itemsize if pad_of is not None else 0
         out = {self.weight_name: TensorDecl((self.vocab_size, self.hidden_size), row_gap_bytes=gap)}
         if self.bias_name:

@@ -312,6 +312,7 @@ def _is_model_tensor(model, t):
                for p in model.parts() for a in ("weight", "bias"))
 
 
+@pytest.mark.filterwarnings("ignore:.*stored in 32 bits")
 @pytest.mark.parametrize("tied", [False, True])
 @pytest.mark.parametrize("stored", ["bfloat16", "float32"])
 @pytest.mark.parametrize("keep", [False, True])
@@ -324,7 +325,7 @@ def test_head_of_its_own_is_read_in_pieces_into_rows_apart(tmp_path, monkeypatch
     raw = load_file(os.path.join(folder, "model.safetensors"))
     name = "model.embed_tokens.weight" if "lm_head.weight" not in raw else "lm_head.weight"
     assert (name == "lm_head.weight") != tied
-    ops = SimpleNamespace(weight_row_pad=lambda in_features, dtype: 24 if dtype == torch.bfloat16 else 12)
+    ops = SimpleNamespace(head_row_pad=lambda in_features, dtype: 24 if dtype == torch.bfloat16 else 12)
     rt = Runtime(ops=ops, device=torch.device("cpu"), dtype=torch.bfloat16, max_positions=cfg.max_position_embeddings)
     model = DecoderModel(get_architecture(cfg.architecture).build_spec(cfg), rt)
     monkeypatch.setattr(loader, "PIECE_BYTES", 5 * raw[name].shape[1] * raw[name].element_size())
@@ -340,6 +341,17 @@ def test_head_of_its_own_is_read_in_pieces_into_rows_apart(tmp_path, monkeypatch
     assert w.dtype == dtype and torch.equal(w, raw[name].to(dtype))
     assert w.stride() == (w.shape[1] + (0 if tied else 48 // dtype.itemsize), 1)
     assert most[0] == (0 if tied else 5) and (model.embedding.weight.data_ptr() == w.data_ptr()) == tied
+
+
+def test_heads_rows_lie_apart_only_where_they_share_memory_channels():
+    """Rows of a multiple of 4 KB; any other length is back to back."""
+    from types import SimpleNamespace
+    from lmsf_amd.ops.hip_ops import HipOps
+    ops = SimpleNamespace(weight_row_pad=lambda in_features, dtype: 512 // dtype.itemsize)
+    pad = lambda n, dtype: HipOps.head_row_pad(ops, n, dtype)          # noqa: E731
+    assert [pad(n, torch.bfloat16) for n in (2048, 4096, 8192, 6144)] == [256] * 4
+    assert [pad(n, torch.bfloat16) for n in (128, 512, 1024, 2560, 3072, 3584, 5120)] == [0] * 7
+    assert pad(1024, torch.float32) == 128 and pad(128, torch.float32) == 0
 
 
 def test_random_head_is_made_in_rows_apart():
