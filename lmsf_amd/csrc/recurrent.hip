@@ -15,12 +15,31 @@
 
 #include <math.h>
 
-__device__ __forceinline__ float rc_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// log(1 + e) for 0 <= e <= 1 as 2 atanh(s), s = e / (2 + e) <= 1/3: the series of atanh up to s^15 (the next term is below 2e-9 of
+// the sum), s from the hardware's reciprocal and one correction, with what s still lacks (rest) added to the small terms.
+// 20 instructions where log1pf takes 90 in one chain; against 64 bits over 4 million arguments between exp(-87) and 1 at most 1.0 last
+// place off, as log1pf is.
+__device__ __forceinline__ float rc_log1p(float e) {
+  const float b = 2.f + e, inv = __builtin_amdgcn_rcpf(b);
+  float s = e * inv;
+  s = fmaf(fmaf(-s, b, e), inv, s);
+  const float rest = (fmaf(-s, b, e) - s * (e - (b - 2.f))) * inv;
+  const float q = s * s;
+  float p = 2.f / 15.f;
+  p = fmaf(p, q, 2.f / 13.f);
+  p = fmaf(p, q, 2.f / 11.f);
+  p = fmaf(p, q, 2.f / 9.f);
+  p = fmaf(p, q, 2.f / 7.f);
+  p = fmaf(p, q, 2.f / 5.f);
+  p = fmaf(p, q, 2.f / 3.f);
+  return fmaf(2.f, s, fmaf(p * q, s, 2.f * rest));
+}
+__device__ __forceinline__ float rc_softplus(float z) { return fmaxf(z, 0.f) + rc_log1p(expf(-fabsf(z))); }
 __device__ __forceinline__ float rc_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
 // exp of a decay's exponent, in the recurrences' inner loops: one multiplication and the hardware's 2^x (relative error
 // about |x| 2^-24 beside the instruction's own last bit; an exponent that large forgets within a token)
 __device__ __forceinline__ float rc_decay(float x) { return __expf(x); }
-__device__ __forceinline__ float rc_logsigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
+__device__ __forceinline__ float rc_logsigmoid(float z) { return fminf(z, 0.f) - rc_log1p(expf(-fabsf(z))); }
 
 // ---------------------------------------------------------------- short causal convolution
 // out[t, c] = act(bias[c] + sum_j w[c, j] u[t - taps + 1 + j, c]); an input before the segment's first token is
@@ -600,19 +619,18 @@ extern "C" long lmsf_mlstm_state_floats(int H, int d, int dv) {
 // column, by the first block); chunks one after the other, a thread an entry of each product.
 #define MLC_THREADS 1024
 
-// MODE 0: a segment's chunks one after the other in one workgroup, the state from the slot and back to it.
-// Steps with long segments run the chunks side by side instead, in three launches:
-// MODE 1: every chunk leaves U = K^T (w [V | 1]) with w_u = exp(g_u - G), G = max_u g_u, and (F_last, G) in scratch;
+// A segment's chunks one after the other in one workgroup, the state from the slot and back to it. Steps with segments of 32
+// and more tokens run the chunks side by side instead, in three launches:
+// summaries: every chunk leaves U = K^T (w [V | 1]) with w_u = exp(g_u - G), G = max_u g_u, and (F_last, G) in scratch;
 // mlstm_fold_kernel turns them, chunk after chunk, into every chunk's S_0 (in U's place) and m_0 and writes the slot's S;
-// MODE 2: every chunk computes its outputs from its S_0 and m_0 (and the last one writes the slot's m).
+// outputs: every chunk computes its outputs from its S_0 and m_0 (and the last one writes the slot's m).
 // Chunk j of segment s is entry chunk_base[s] + j of the scratch: U as [H, d, dv + 1], fg as [H, 2], m0 as [H].
-template <typename T, int MODE>
+template <typename T>
 __global__ __launch_bounds__(MLC_THREADS) void mlstm_chunk_kernel(
     const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, long qkv_stride,
     const float* __restrict__ gates, long gates_stride, float* __restrict__ state, long state_stride,
     const int* __restrict__ seg_starts, const int* __restrict__ state_slots, float* __restrict__ o_raw, long o_stride,
-    int H, int d, int dv, int L, int DVB, float qscale, float cap, int n_vb, const int* __restrict__ chunk_base,
-    float* __restrict__ sc_U, float* __restrict__ sc_fg, float* __restrict__ sc_m0, float* __restrict__ den) {
+    int H, int d, int dv, int L, int DVB, float qscale, float cap, float* __restrict__ den) {
   extern __shared__ float lds[];
   // row lengths in LDS are odd, so that threads that walk down neighbouring rows meet different banks
   const int dp = d | 1, NCp = (DVB + 1) | 1, Lp = L | 1;
@@ -627,35 +645,27 @@ __global__ __launch_bounds__(MLC_THREADS) void mlstm_chunk_kernel(
   float* sM = sg + L;
   float* sw = sM + L;
   const int tid = threadIdx.x;
-  const int h = blockIdx.x, s = blockIdx.y;
-  const int vb = MODE == 0 ? blockIdx.z : blockIdx.z % n_vb, j = MODE == 0 ? 0 : blockIdx.z / n_vb;
+  const int h = blockIdx.x, s = blockIdx.y, vb = blockIdx.z;
   const int e0 = vb * DVB;
   // (n is carried by the first block of columns alone: it is that block's to read and to write, and the other blocks
   // need nothing of it, because the division by max(|n . q|, exp(-m)) + 1e-6 is left to the kernel that follows)
   const int nb = min(DVB, dv - e0), cols = dv + 1, NC = nb + (vb == 0 ? 1 : 0);
-  const int seg_start = seg_starts[s], seg_end = seg_starts[s + 1];
-  if (MODE != 0 && j * L >= seg_end - seg_start) return;
-  const int start = MODE == 0 ? seg_start : seg_start + j * L;
-  const int end = MODE == 0 ? seg_end : min(seg_end, start + L);
-  const long ent = MODE == 0 ? 0 : (long)chunk_base[s] + j;
+  const int start = seg_starts[s], end = seg_starts[s + 1];
   float* st = state + (long)state_slots[s] * state_stride;
-  // where S_0 comes from (and, MODE 0, goes back to) and where m_0 lies
-  float* gS = MODE == 0 ? st + (long)h * d * cols : sc_U + (ent * H + h) * d * cols;
-  float* gm = MODE == 0 ? st + (long)H * d * cols + (long)h * mls_m_copies(dv) + vb : sc_m0 + ent * H + h;
-  if (MODE != 1) {
-    for (int i = tid; i < d * NC; i += MLC_THREADS) {
-      const int dd = i / NC, c = i % NC;
-      sS[dd * NCp + c] = c < nb ? gS[(long)dd * cols + e0 + c] : gS[(long)dd * cols + dv];
-    }
+  float* gS = st + (long)h * d * cols;
+  float* gm = st + (long)H * d * cols + (long)h * mls_m_copies(dv) + vb;
+  for (int i = tid; i < d * NC; i += MLC_THREADS) {
+    const int dd = i / NC, c = i % NC;
+    sS[dd * NCp + c] = c < nb ? gS[(long)dd * cols + e0 + c] : gS[(long)dd * cols + dv];
   }
-  float m = MODE == 1 ? -INFINITY : gm[0];
+  float m = gm[0];
   for (int t0 = start; t0 < end; t0 += L) {
     const int nt = min(L, end - t0);
     __syncthreads();
     for (int i = tid; i < nt * d; i += MLC_THREADS) {
       const int tt = i / d, dd = i % d;
       const long at = (long)(t0 + tt) * qkv_stride + h * d + dd;
-      if (MODE != 1) sq[tt * dp + dd] = to_f32<T>(q[at]) * qscale;
+      sq[tt * dp + dd] = to_f32<T>(q[at]) * qscale;
       sk[tt * dp + dd] = to_f32<T>(k[at]);
     }
     for (int i = tid; i < nt * NC; i += MLC_THREADS) {
@@ -690,83 +700,334 @@ __global__ __launch_bounds__(MLC_THREADS) void mlstm_chunk_kernel(
     __syncthreads();
     const float M_last = sM[nt - 1];
     if (tid < nt) sw[tid] = expf(sg[tid] - M_last);
-    if (MODE != 1) {
-      // P[t][u] = (q_t . k_u) exp(g_u - M_t) for u <= t
-      for (int i = tid; i < nt * nt; i += MLC_THREADS) {
-        const int t = i / nt, u = i % nt;
-        float acc = 0.f;
-        if (u <= t) {
-          const float* qr = sq + t * dp;
-          const float* kr = sk + u * dp;
-#pragma unroll 8
-          for (int dd = 0; dd < d; ++dd) acc += qr[dd] * kr[dd];
-          acc *= expf(sg[u] - sM[t]);
-        }
-        sP[t * Lp + u] = acc;
-      }
-      __syncthreads();
-      // [O | n.q][t][c] = w_0(t) q_t [S_0 | n_0] + P[t] [V | 1]
-      for (int i = tid; i < nt * NC; i += MLC_THREADS) {
-        const int t = i / NC, c = i % NC;
-        float acc = 0.f;
+    // P[t][u] = (q_t . k_u) exp(g_u - M_t) for u <= t
+    for (int i = tid; i < nt * nt; i += MLC_THREADS) {
+      const int t = i / nt, u = i % nt;
+      float acc = 0.f;
+      if (u <= t) {
         const float* qr = sq + t * dp;
+        const float* kr = sk + u * dp;
 #pragma unroll 8
-        for (int dd = 0; dd < d; ++dd) acc += qr[dd] * sS[dd * NCp + c];
-        acc *= expf(m - sM[t]);
-        const float* pr = sP + t * Lp;
-#pragma unroll 4
-        for (int u = 0; u <= t; ++u) acc += pr[u] * sv[u * NCp + c];
-        so[t * NCp + c] = acc;
+        for (int dd = 0; dd < d; ++dd) acc += qr[dd] * kr[dd];
+        acc *= expf(sg[u] - sM[t]);
       }
-      __syncthreads();
-      for (int i = tid; i < nt * nb; i += MLC_THREADS) {
-        const int t = i / nb, c = i % nb;
-        o_raw[(long)(t0 + t) * o_stride + h * dv + e0 + c] = so[t * NCp + c];
-      }
-      if (vb == 0 && tid < nt)
-        den[(long)(t0 + tid) * H + h] = fmaxf(fabsf(so[tid * NCp + nb]), expf(-(sF[tid] + sM[tid]))) + 1e-6f;
-    } else {
-      __syncthreads();
+      sP[t * Lp + u] = acc;
     }
-    if (MODE == 0) {
-      // [S | n] <- exp(m_0 - M_last) [S_0 | n_0] + K^T (w [V | 1])
-      const float wl = expf(m - M_last);
-      for (int i = tid; i < d * NC; i += MLC_THREADS) {
-        const int dd = i / NC, c = i % NC;
-        float r = sS[dd * NCp + c] * wl;
-#pragma unroll 8
-        for (int u = 0; u < nt; ++u) r += sk[u * dp + dd] * sw[u] * sv[u * NCp + c];
-        sS[dd * NCp + c] = r;
-      }
-      m = sF[nt - 1] + M_last;
-    }
-    if (MODE == 2 && end == seg_end && tid == 0)
-      st[(long)H * d * cols + (long)h * mls_m_copies(dv) + vb] = sF[nt - 1] + M_last;      // this block's copy of m
-    if (MODE == 1) {
-      // U = K^T (w [V | 1]) straight to the scratch; (F_last, G) beside it
-      for (int i = tid; i < d * NC; i += MLC_THREADS) {
-        const int dd = i / NC, c = i % NC;
-        float r = 0.f;
-#pragma unroll 8
-        for (int u = 0; u < nt; ++u) r += sk[u * dp + dd] * sw[u] * sv[u * NCp + c];
-        if (c < nb) gS[(long)dd * cols + e0 + c] = r;
-        else if (vb == 0) gS[(long)dd * cols + dv] = r;
-      }
-      if (tid == 0 && vb == 0) {
-        sc_fg[(ent * H + h) * 2] = sF[nt - 1];
-        sc_fg[(ent * H + h) * 2 + 1] = M_last;
-      }
-    }
-  }
-  if (MODE == 0) {
     __syncthreads();
+    // [O | n.q][t][c] = w_0(t) q_t [S_0 | n_0] + P[t] [V | 1]
+    for (int i = tid; i < nt * NC; i += MLC_THREADS) {
+      const int t = i / NC, c = i % NC;
+      float acc = 0.f;
+      const float* qr = sq + t * dp;
+#pragma unroll 8
+      for (int dd = 0; dd < d; ++dd) acc += qr[dd] * sS[dd * NCp + c];
+      acc *= expf(m - sM[t]);
+      const float* pr = sP + t * Lp;
+#pragma unroll 4
+      for (int u = 0; u <= t; ++u) acc += pr[u] * sv[u * NCp + c];
+      so[t * NCp + c] = acc;
+    }
+    __syncthreads();
+    for (int i = tid; i < nt * nb; i += MLC_THREADS) {
+      const int t = i / nb, c = i % nb;
+      o_raw[(long)(t0 + t) * o_stride + h * dv + e0 + c] = so[t * NCp + c];
+    }
+    if (vb == 0 && tid < nt)
+      den[(long)(t0 + tid) * H + h] = fmaxf(fabsf(so[tid * NCp + nb]), expf(-(sF[tid] + sM[tid]))) + 1e-6f;
+    // [S | n] <- exp(m_0 - M_last) [S_0 | n_0] + K^T (w [V | 1])
+    const float wl = expf(m - M_last);
     for (int i = tid; i < d * NC; i += MLC_THREADS) {
       const int dd = i / NC, c = i % NC;
-      if (c < nb) gS[(long)dd * cols + e0 + c] = sS[dd * NCp + c];
-      else if (vb == 0) gS[(long)dd * cols + dv] = sS[dd * NCp + c];
+      float r = sS[dd * NCp + c] * wl;
+#pragma unroll 8
+      for (int u = 0; u < nt; ++u) r += sk[u * dp + dd] * sw[u] * sv[u * NCp + c];
+      sS[dd * NCp + c] = r;
     }
-    if (tid == 0) gm[0] = m;                     // this block's copy
+    m = sF[nt - 1] + M_last;
   }
+  __syncthreads();
+  for (int i = tid; i < d * NC; i += MLC_THREADS) {
+    const int dd = i / NC, c = i % NC;
+    if (c < nb) gS[(long)dd * cols + e0 + c] = sS[dd * NCp + c];
+    else if (vb == 0) gS[(long)dd * cols + dv] = sS[dd * NCp + c];
+  }
+  if (tid == 0) gm[0] = m;                       // this block's copy
+}
+
+// The chunks of long segments side by side, on the matrix cores in float32 (v_mfma_f32_16x16x4_f32: every product and sum
+// stays 32 bits wide). A workgroup of four waves: one head of one chunk and 64 value columns, a wave 16 of them for all of the
+// chunk's tokens. SUMMARY: U = K^T (w [V | 1]) and (F_last, G) to the scratch; otherwise the outputs from S_0 and m_0.
+// Operands come from LDS in the model's type (two workgroups a compute unit at heads of 128) but S_0's, of which a wave
+// reads 16 columns of its own straight into registers, asked for before anything else. The k index of four instructions in
+// a row is dealt as 16 S + 4 g + j (j the instruction, g the lane's group), so that an operand row is one read for all four.
+// n, the column of ones, is one dot product a token or row beside it.
+// 1,997 tokens of 8 requests, 8 heads of 128 by 128: an entry of each product a thread with both factors read from LDS for every
+// multiplication 187 (outputs) and 104 us (summaries) -> 40 and 21.
+#define MLX_THREADS 256
+#define MLX_COLS 64
+#define MLX_PIECE 128            // entries of d whose rows of S_0 a wave holds at a time
+#define MLX_MOST 64              // tokens of a chunk at most
+
+template <typename T> __device__ __forceinline__ void mlx_four(const T* p, float* o);
+template <> __device__ __forceinline__ void mlx_four<float>(const float* p, float* o) {
+  const float4 v = *reinterpret_cast<const float4*>(p);
+  o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+}
+template <> __device__ __forceinline__ void mlx_four<bf16_t>(const bf16_t* p, float* o) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  o[0] = __uint_as_float(v.x << 16); o[1] = __uint_as_float(v.x & 0xffff0000u);
+  o[2] = __uint_as_float(v.y << 16); o[3] = __uint_as_float(v.y & 0xffff0000u);
+}
+__host__ __device__ static inline int mlx_rows(int d) { return (d + 31) / 32 * 32; }
+template <typename T> __host__ __device__ static inline int mlx_pitch(int d) { return mlx_rows(d) + 16 / (int)sizeof(T); }
+template <typename T> static size_t mlx_lds(int L, int d, bool summary) {
+  const size_t L16 = (L + 15) / 16 * 16;
+  return ((summary ? 1 : 2) * L16 * mlx_pitch<T>(d) + L16 * (MLX_COLS + 16 / sizeof(T))) * sizeof(T) +
+         ((summary ? 0 : L16 * (L16 + 4) + mlx_rows(d)) + 4 * MLX_MOST) * sizeof(float);
+}
+
+template <typename T, bool SUMMARY>
+__global__ __launch_bounds__(MLX_THREADS) void mlstm_chunk_mfma_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, long qkv_stride,
+    const float* __restrict__ gates, long gates_stride, float* __restrict__ state, long state_stride,
+    const int* __restrict__ seg_starts, const int* __restrict__ state_slots, float* __restrict__ o_raw, long o_stride,
+    int H, int d, int dv, int L, float qscale, float cap, int n_vb, const int* __restrict__ chunk_base,
+    float* __restrict__ sc_U, float* __restrict__ sc_fg, const float* __restrict__ sc_m0, float* __restrict__ den, int vec) {
+  constexpr int VEC = 16 / (int)sizeof(T), TILES = MLX_MOST / 16, VP = MLX_COLS + VEC;
+  extern __shared__ __align__(16) unsigned char mlx_raw[];
+  const int tid = threadIdx.x, w = tid / LMSF_WAVE, l = tid % LMSF_WAVE, r = l % 16, g = l / 16;
+  const int h = blockIdx.x, s = blockIdx.y, vb = blockIdx.z % n_vb, j = blockIdx.z / n_vb;
+  const int seg_start = seg_starts[s], seg_end = seg_starts[s + 1];
+  if (j * L >= seg_end - seg_start) return;
+  const int t0 = seg_start + j * L, nt = min(L, seg_end - t0);
+  const int e0 = vb * MLX_COLS, nb = min(MLX_COLS, dv - e0), cols = dv + 1;
+  const int L16 = (L + 15) / 16 * 16, n_tiles = (nt + 15) / 16, d16 = mlx_rows(d), dp = mlx_pitch<T>(d), Lp = L16 + 4;
+  float* sF = reinterpret_cast<float*>(mlx_raw);       // [64] F_t;  then [64] g_s;  [64] M_t;  [64] exp(g_s - M_last)
+  float* sg = sF + MLX_MOST;
+  float* sM = sg + MLX_MOST;
+  float* sw = sM + MLX_MOST;
+  T* sk = reinterpret_cast<T*>(sw + MLX_MOST);         // [L16][dp]
+  T* sv = sk + L16 * dp;                               // [L16][VP]
+  T* sq = sv + L16 * VP;                               // [L16][dp]   (from here on: not for the summaries)
+  float* sP = reinterpret_cast<float*>(sq + L16 * dp); // [L16][Lp]
+  float* sn = sP + L16 * Lp;                           // [d16] n_0
+  const long ent = ((long)chunk_base[s] + j) * H + h;
+  float* gS = sc_U + ent * d * cols;
+  const int col = e0 + 16 * w + r;                     // this lane's value column
+  const bool wave_live = 16 * w < nb, col_live = 16 * w + r < nb;
+
+  // S_0's columns of this wave: entry 4 S + i is row 16 S + 4 g + i of the piece
+  float s0[MLX_PIECE / 4];
+  auto load_s0 = [&](int d0) {
+#pragma unroll
+    for (int S = 0; S < MLX_PIECE / 16; ++S)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int dd = d0 + 16 * S + 4 * g + i;
+        s0[4 * S + i] = dd < d && col_live ? gS[(long)dd * cols + col] : 0.f;
+      }
+  };
+  const float m0 = SUMMARY ? -INFINITY : sc_m0[ent];
+  if (!SUMMARY) load_s0(0);
+  // the chunk's gates: i_t and f_t
+  if (tid < MLX_MOST) {
+    float gi = 0.f, gf = 0.f;
+    if (tid < nt) {
+      gi = cap * tanhf(gates[(long)(t0 + tid) * gates_stride + h] / cap);
+      gf = rc_logsigmoid(cap * tanhf(gates[(long)(t0 + tid) * gates_stride + H + h] / cap));
+    }
+    // F_t, g_t = i_t - F_t and M_t = max(m_0, max_{u <= t} g_u): running sums and maxima over the first wave's lanes
+    float F = gf;
+    for (int o = 1; o < LMSF_WAVE; o <<= 1) {
+      const float up = __shfl_up(F, o, LMSF_WAVE);
+      if (tid >= o) F += up;
+    }
+    const float gt = tid < nt ? gi - F : -INFINITY;
+    float G = fmaxf(gt, m0);
+    for (int o = 1; o < LMSF_WAVE; o <<= 1) {
+      const float up = __shfl_up(G, o, LMSF_WAVE);
+      if (tid >= o) G = fmaxf(G, up);
+    }
+    sF[tid] = F;
+    sg[tid] = gt;
+    sM[tid] = G;
+    sw[tid] = tid < nt ? expf(gt - __shfl(G, nt - 1, LMSF_WAVE)) : 0.f;
+  }
+  // keys (and queries) and values, zeros beyond the chunk's tokens and the head's entries; four pieces asked for at a time
+  auto stage = [&](const T* src, T* dst, int pitch, int width, int have) {
+    if (vec) {
+      const int pieces = width / VEC, total = L16 * pieces;
+      for (int i0 = tid; i0 < total; i0 += 4 * MLX_THREADS) {
+        Vec16<T> x[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          const int i = i0 + n * MLX_THREADS, tt = i / pieces, dd = (i - tt * pieces) * VEC;
+          x[n].v = {};
+          if (tt < nt && dd < have) x[n].load(src + (long)(t0 + tt) * qkv_stride + dd);
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          const int i = i0 + n * MLX_THREADS, tt = i / pieces, dd = (i - tt * pieces) * VEC;
+          if (i < total) x[n].store(dst + tt * pitch + dd);
+        }
+      }
+    } else {
+      for (int i = tid; i < L16 * width; i += MLX_THREADS) {
+        const int tt = i / width, dd = i - tt * width;
+        dst[tt * pitch + dd] = tt < nt && dd < have ? src[(long)(t0 + tt) * qkv_stride + dd] : T(0);
+      }
+    }
+  };
+  stage(k + (long)h * d, sk, dp, d16, d);
+  stage(v + (long)h * dv + e0, sv, VP, MLX_COLS, nb);
+  if (!SUMMARY) stage(q + (long)h * d, sq, dp, d16, d);
+  if (!SUMMARY && vb == 0)
+    for (int i = tid; i < d16; i += MLX_THREADS) sn[i] = i < d ? gS[(long)i * cols + dv] : 0.f;
+  __syncthreads();
+
+  if constexpr (SUMMARY) {
+    if (wave_live) {
+      float b[MLX_MOST / 4];       // w_u v_u: entry 4 S + i is token 16 S + 4 g + i
+#pragma unroll
+      for (int S = 0; S < TILES; ++S)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int u = 16 * S + 4 * g + i;
+          b[4 * S + i] = S < n_tiles ? sw[u] * to_f32<T>(sv[u * VP + 16 * w + r]) : 0.f;
+        }
+      for (int d0 = 0; d0 < d16; d0 += 16) {
+        f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int S = 0; S < TILES; ++S)
+          if (S < n_tiles) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              acc = __builtin_amdgcn_mfma_f32_16x16x4f32(to_f32<T>(sk[(16 * S + 4 * g + i) * dp + d0 + r]), b[4 * S + i], acc,
+                                                         0, 0, 0);
+          }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int dd = d0 + 4 * g + e;
+          if (dd < d && col_live) gS[(long)dd * cols + col] = acc[e];
+        }
+      }
+    }
+    if (vb == 0) {
+      for (int dd = tid; dd < d; dd += MLX_THREADS) {
+        float n = 0.f;
+        for (int u = 0; u < nt; ++u) n += to_f32<T>(sk[u * dp + dd]) * sw[u];
+        gS[(long)dd * cols + dv] = n;
+      }
+      if (tid == 0) {
+        sc_fg[ent * 2] = sF[nt - 1];
+        sc_fg[ent * 2 + 1] = sM[nt - 1];
+      }
+    }
+    return;
+  }
+
+  // P[t][u] = (q_t . k_u) exp(g_u - M_t) for u <= t, the tiles on and below the diagonal shared out among the waves
+  for (int at = w, i = 0; i < n_tiles; ++i) {
+    for (; at <= i; at += MLX_THREADS / LMSF_WAVE) {
+      f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+      if constexpr (sizeof(T) == 2) {
+        // (products of two bfloat16 numbers are exact in float32: the bfloat16 instruction's sums are as wide)
+        const T* qr = sq + (16 * i + r) * dp + 8 * g;
+        const T* kr = sk + (16 * at + r) * dp + 8 * g;
+#pragma unroll 4
+        for (int dd = 0; dd < d16; dd += 32)
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(qr + dd),
+                                                        *reinterpret_cast<const bf16x8_t*>(kr + dd), acc, 0, 0, 0);
+      } else {
+        const T* qr = sq + (16 * i + r) * dp + 4 * g;
+        const T* kr = sk + (16 * at + r) * dp + 4 * g;
+#pragma unroll 4
+        for (int dd = 0; dd < d16; dd += 16) {
+          float a[4], b[4];
+          mlx_four<T>(qr + dd, a);
+          mlx_four<T>(kr + dd, b);
+#pragma unroll
+          for (int n = 0; n < 4; ++n) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n], b[n], acc, 0, 0, 0);
+        }
+      }
+      const int u = 16 * at + r;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = 16 * i + 4 * g + e;
+        sP[t * Lp + u] = u <= t && t < nt ? acc[e] * qscale * expf(sg[u] - sM[t]) : 0.f;
+      }
+    }
+    at -= i + 1;      // the next row of tiles begins where this one ended
+  }
+  // q_t S_0
+  f32x4_t acc[TILES];
+#pragma unroll
+  for (int i = 0; i < TILES; ++i) acc[i] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  if (wave_live) {
+    for (int d0 = 0; d0 < d16; d0 += MLX_PIECE) {
+      if (d0 > 0) load_s0(d0);
+#pragma unroll
+      for (int S = 0; S < MLX_PIECE / 16; ++S)
+        if (d0 + 16 * S < d16) {
+#pragma unroll
+          for (int i = 0; i < TILES; ++i)
+            if (i < n_tiles) {
+              float a[4];
+              mlx_four<T>(sq + (16 * i + r) * dp + d0 + 16 * S + 4 * g, a);
+#pragma unroll
+              for (int n = 0; n < 4; ++n) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n], s0[4 * S + n], acc[i], 0, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+      if (i < n_tiles) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] *= qscale * expf(m0 - sM[16 * i + 4 * g + e]);
+      }
+  }
+  __syncthreads();      // P is there
+  if (wave_live) {
+    // + P V
+#pragma unroll
+    for (int S = 0; S < TILES; ++S)
+      if (S < n_tiles) {
+        float b[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) b[n] = to_f32<T>(sv[(16 * S + 4 * g + n) * VP + 16 * w + r]);
+#pragma unroll
+        for (int i = S; i < TILES; ++i)
+          if (i < n_tiles) {
+            float a[4];
+            mlx_four<float>(sP + (16 * i + r) * Lp + 16 * S + 4 * g, a);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[n], b[n], acc[i], 0, 0, 0);
+          }
+      }
+#pragma unroll
+    for (int i = 0; i < TILES; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int t = 16 * i + 4 * g + e;
+        if (t < nt && col_live) o_raw[(long)(t0 + t) * o_stride + (long)h * dv + col] = acc[i][e];
+      }
+  }
+  if (vb == 0) {
+    // max(|n . q|, exp(-m)) + 1e-6: four threads a token
+    const int t = tid / 4, part = tid % 4;
+    float a = 0.f, b = 0.f;
+    if (t < nt) {
+      for (int dd = part; dd < d; dd += 4) a += to_f32<T>(sq[t * dp + dd]) * sn[dd];
+      for (int u = part; u <= t; u += 4) b += sP[t * Lp + u];
+    }
+    a = a * qscale * expf(m0 - sM[t]) + b;
+    a += __shfl_xor(a, 1, LMSF_WAVE);
+    a += __shfl_xor(a, 2, LMSF_WAVE);
+    if (t < nt && part == 0) den[(long)(t0 + t) * H + h] = fmaxf(fabsf(a), expf(-(sF[t] + sM[t]))) + 1e-6f;
+  }
+  if (t0 + nt == seg_end && tid < MLX_COLS / MLS_M_COLS && e0 + tid * MLS_M_COLS < dv)      // these columns' copies of m
+    state[(long)state_slots[s] * state_stride + (long)H * d * cols + (long)h * mls_m_copies(dv) + vb * (MLX_COLS / MLS_M_COLS) + tid] =
+        sF[nt - 1] + sM[nt - 1];
 }
 
 // Chunk after chunk of a segment: the chunk's S_0 and m_0 take U's place and sc_m0, then
@@ -787,9 +1048,12 @@ __global__ __launch_bounds__(256) void mlstm_fold_kernel(float* __restrict__ sta
   float S = st[(long)h * per + i];
   float m = st[(long)H * per + (long)h * mls_m_copies(dv)];      // (copy 0; nobody writes m in this launch)
   const long base = chunk_base[s];
+  // (a chunk's U is asked for before the one ahead of it is written over)
+  float U_next = sc_U[(base * H + h) * per + i];
   for (int j = 0; j < n_chunks; ++j) {
     const long ent = (base + j) * H + h;
-    const float U = sc_U[ent * per + i];
+    const float U = U_next;
+    if (j + 1 < n_chunks) U_next = sc_U[(ent + H) * per + i];
     const float F = sc_fg[ent * 2], G = sc_fg[ent * 2 + 1];
     sc_U[ent * per + i] = S;
     if (i == 0) sc_m0[ent] = m;
@@ -943,48 +1207,61 @@ extern "C" int lmsf_mlstm_chunked(const void* q, const void* k, const void* v, i
   LMSF_CHECK(L > 0, "mlstm_chunked: heads of %d entries do not fit a workgroup's LDS", d);
   const size_t smem = ((size_t)2 * L * dp + (size_t)2 * L * NCp + (size_t)L * (L | 1) + (size_t)d * NCp + 4 * L) * sizeof(float);
   const int n_vb = (dv + DVB - 1) / DVB;
-  LMSF_CHECK(!chunk_base || (long)n_vb * max_chunks <= 65535, "mlstm_chunked: too many chunks");
-#define MLC_RESERVE(T, MODE)                                                                                       \
-  do {                                                                                                             \
-    static size_t reserved = 0;                                                                                    \
-    if (smem > 64 * 1024 && smem > reserved) {                                                                     \
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(mlstm_chunk_kernel<T, MODE>),               \
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);                   \
-      if (e != hipSuccess) {                                                                                       \
-        lmsf_set_error("mlstm_chunked: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));          \
-        return 2;                                                                                                  \
-      }                                                                                                            \
-      reserved = smem;                                                                                             \
-    }                                                                                                              \
+  LMSF_CHECK(!chunk_base || (long)((dv + MLX_COLS - 1) / MLX_COLS) * max_chunks <= 65535, "mlstm_chunked: too many chunks");
+#define MLS_RESERVE(KERNEL, BYTES)                                                                                    \
+  do {                                                                                                               \
+    static size_t reserved = 0;                                                                                      \
+    if ((BYTES) > 64 * 1024 && (BYTES) > reserved) {                                                                 \
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(KERNEL),                                      \
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(BYTES));                  \
+      if (e != hipSuccess) {                                                                                         \
+        lmsf_set_error("mlstm_chunked: cannot reserve %zu bytes of LDS: %s", (size_t)(BYTES), hipGetErrorString(e)); \
+        return 2;                                                                                                    \
+      }                                                                                                              \
+      reserved = (BYTES);                                                                                            \
+    }                                                                                                                \
   } while (0)
-#define MLC_LAUNCH(T, MODE, GRID)                                                                                  \
-  do {                                                                                                             \
-    MLC_RESERVE(T, MODE);                                                                                          \
-    hipLaunchKernelGGL((mlstm_chunk_kernel<T, MODE>), GRID, dim3(MLC_THREADS), smem, stream, (const T*)q,          \
-                       (const T*)k, (const T*)v, qkv_stride, gates, gates_stride, state, state_stride, seg_starts, \
-                       state_slots, o_raw, (long)H * dv, H, d, dv, L, DVB, qscale, cap, n_vb, chunk_base, sc_U,    \
-                       sc_fg, sc_m0, o_raw + (long)n_tokens * H * dv);                                             \
+#define MLC_LAUNCH(T)                                                                                                \
+  do {                                                                                                               \
+    MLS_RESERVE(mlstm_chunk_kernel<T>, smem);                                                                        \
+    hipLaunchKernelGGL((mlstm_chunk_kernel<T>), dim3(H, n_segments, n_vb), dim3(MLC_THREADS), smem, stream,          \
+                       (const T*)q, (const T*)k, (const T*)v, qkv_stride, gates, gates_stride, state, state_stride,  \
+                       seg_starts, state_slots, o_raw, (long)H * dv, H, d, dv, L, DVB, qscale, cap, den);            \
   } while (0)
+  float* den = o_raw + (long)n_tokens * H * dv;
   float* sc_U = entries;
   float* sc_fg = entries ? entries + n_entries * H * d * (dv + 1) : nullptr;
   float* sc_m0 = entries ? sc_fg + n_entries * H * 2 : nullptr;
   if (!chunk_base) {
-    dim3 grid(H, n_segments, n_vb);
-    if (dtype == LMSF_F32) MLC_LAUNCH(float, 0, grid); else MLC_LAUNCH(bf16_t, 0, grid);
+    if (dtype == LMSF_F32) MLC_LAUNCH(float); else MLC_LAUNCH(bf16_t);
     LMSF_LAUNCH_CHECK("mlstm_chunk");
   } else {
-    dim3 grid(H, n_segments, n_vb * max_chunks);
-    if (dtype == LMSF_F32) MLC_LAUNCH(float, 1, grid); else MLC_LAUNCH(bf16_t, 1, grid);
+    const int m_vb = (dv + MLX_COLS - 1) / MLX_COLS;
+    dim3 grid(H, n_segments, m_vb * max_chunks);
+    const int vw = dtype == LMSF_F32 ? 4 : 8;
+    const int vec = d % vw == 0 && dv % vw == 0 && qkv_stride % vw == 0 && lmsf_aligned16(q) && lmsf_aligned16(k) &&
+                    lmsf_aligned16(v);
+#define MLX_LAUNCH(T, SUM)                                                                                            \
+  do {                                                                                                               \
+    const size_t lds = mlx_lds<T>(L, d, SUM);                                                                        \
+    MLS_RESERVE((mlstm_chunk_mfma_kernel<T, SUM>), lds);                                                             \
+    hipLaunchKernelGGL((mlstm_chunk_mfma_kernel<T, SUM>), grid, dim3(MLX_THREADS), lds, stream, (const T*)q,         \
+                       (const T*)k, (const T*)v, qkv_stride, gates, gates_stride, state, state_stride, seg_starts,   \
+                       state_slots, o_raw, (long)H * dv, H, d, dv, L, qscale, cap, m_vb, chunk_base, sc_U, sc_fg,    \
+                       sc_m0, den, vec);                                                                             \
+  } while (0)
+    if (dtype == LMSF_F32) MLX_LAUNCH(float, true); else MLX_LAUNCH(bf16_t, true);
     LMSF_LAUNCH_CHECK("mlstm_chunk (summaries)");
     const long per = (long)d * (dv + 1);
     hipLaunchKernelGGL(mlstm_fold_kernel, dim3(H, n_segments, (unsigned)((per + 255) / 256)), dim3(256), 0, stream, state,
                        state_stride, seg_starts, state_slots, chunk_base, sc_U, sc_fg, sc_m0, H, d, dv, L);
     LMSF_LAUNCH_CHECK("mlstm_chunk (fold)");
-    if (dtype == LMSF_F32) MLC_LAUNCH(float, 2, grid); else MLC_LAUNCH(bf16_t, 2, grid);
+    if (dtype == LMSF_F32) MLX_LAUNCH(float, false); else MLX_LAUNCH(bf16_t, false);
+#undef MLX_LAUNCH
     LMSF_LAUNCH_CHECK("mlstm_chunk (outputs)");
   }
 #undef MLC_LAUNCH
-#undef MLC_RESERVE
+#undef MLS_RESERVE
   const long units = (long)n_tokens * H;
   dim3 ngrid((unsigned)((units + 3) / 4)), block(256);
   if (dtype == LMSF_F32)

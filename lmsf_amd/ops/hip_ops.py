@@ -1523,7 +1523,12 @@ class HipOps:
 
     scan_chunk_tokens = 64         # tokens of a chunk of the selective scan's chunked form
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
-    recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side
+    recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
+    # The matrix memory's chunks run side by side from this many tokens on at heads of 128 and more, from twice as many at
+    # smaller ones. One workgroup a head and 32 columns against side by side, bfloat16: 8 heads of 128, one segment of 24 / 32 /
+    # 48 tokens 26 / 31 / 44 against 29 / 29 / 33 us, 8 of them 28 / 33 / 47 against 36 / 35 / 39, of 100 tokens 84 against 37;
+    # heads of 256 at 24 / 32 tokens 44 / 53 against 40 / 40; heads of 64 at 48 / 100 tokens 28 / 51 against 27 / 30.
+    matrix_memory_parallel_min_tokens = 32
 
     def _chunk_plan(self, batch, chunk: int):
         """(per segment its first entry of scratch or -1, entries in all, the most chunks of a segment) for a step
@@ -1631,7 +1636,7 @@ class HipOps:
             L = self.lib.lmsf_mlstm_chunk_tokens(int(dim))
             bases = entries = None
             n_entries, most = 0, 1
-            if L > 0 and max(lens) >= self.recurrent_parallel_min_chunks * L:
+            if L > 0 and max(lens) >= self.matrix_memory_parallel_min_tokens * (1 if dim >= 128 else 2):
                 key = ("mlstm_chunks", L)
                 plan = batch.aux.get(key)
                 if plan is None:

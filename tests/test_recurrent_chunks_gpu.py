@@ -1,0 +1,79 @@
+"""The recurrences over portions of prompts at the sizes where their chunks and tiles end: the matrix memory's chunks side by
+side on the matrix cores, against the recurrence token by token in 64 bits."""
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def ops():
+    from lmsf_amd.ops.hip_ops import HipOps
+    return HipOps()
+
+
+def batch(lens):
+    starts = [sum(lens[:i]) for i in range(len(lens) + 1)]
+    return types.SimpleNamespace(
+        aux={}, host_seg_lens=list(lens), host_seg_starts=starts, n_tokens=starts[-1], n_segments=len(lens), replayed=False,
+        all_single=False, seg_starts=torch.tensor(starts, dtype=torch.int32, device="cuda"),
+        state_slots=torch.arange(len(lens), dtype=torch.int32, device="cuda").flip(0),
+        seg_of_token=torch.repeat_interleave(torch.arange(len(lens), dtype=torch.int32), torch.tensor(lens)).cuda())
+
+
+def memory_by_tokens(q, k, v, gates, og, w, state, lens, H, d, dv, scale, cap, eps):
+    """[out, state] in float64; state as [slots, H, d, dv + 1] and the running maximum [slots, H]."""
+    S, m = state
+    outs, at = [], 0
+    for s, n in enumerate(lens):
+        slot = len(lens) - 1 - s
+        for t in range(at, at + n):
+            i, f = cap * torch.tanh(gates[t, :H] / cap), torch.nn.functional.logsigmoid(cap * torch.tanh(gates[t, H:] / cap))
+            now = torch.maximum(f + m[slot], i)
+            one = torch.cat([v[t].view(H, dv), torch.ones(H, 1, dtype=torch.float64)], 1)
+            S[slot] = torch.exp(f + m[slot] - now)[:, None, None] * S[slot] + \
+                torch.exp(i - now)[:, None, None] * k[t].view(H, d)[:, :, None] * one[:, None]
+            m[slot] = now
+            o = (S[slot] * (q[t].view(H, d) * scale)[:, :, None]).sum(1)
+            o = o[:, :dv] / (torch.maximum(o[:, dv].abs(), torch.exp(-now)) + 1e-6)[:, None]
+            outs.append((o / torch.sqrt((o * o).mean(1, keepdim=True) + eps)).reshape(-1) * w * torch.sigmoid(og[t]))
+        at += n
+    return torch.stack(outs)
+
+
+# heads of 16 and 32 entries' multiples and not, values that end inside a block of 16 and of 64 columns, segments of a tile's, a
+# chunk's and several chunks' tokens and one more or less, a short one beside them; 200 and 260: more rows of S_0 than a
+# wave holds at a time, and smaller chunks
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d,dv,lens", [(2, 128, 128, (64, 65, 3)), (3, 40, 70, (100, 127)), (1, 17, 5, (65, 192)), (2, 64, 64, (128, 16)),
+                                         (2, 200, 24, (33, 47)), (1, 260, 136, (40,)), (2, 128, 65, (32, 33, 1))])
+def test_matrix_memory_side_by_side(H, d, dv, lens, dtype):
+    o, g = ops(), torch.Generator().manual_seed(d + dv)
+    N, scale, cap, eps = sum(lens), d ** -0.5, 15.0, 1e-5
+    buf = torch.randn(N, H * (2 * d + 2 * dv), generator=g).to(dtype)
+    cut = (H * d, 2 * H * d, 2 * H * d + H * dv)
+    gates, w = torch.randn(N, 2 * H, generator=g) * 2, torch.rand(H * dv, generator=g) + 0.5
+    floats, copies = o.mlstm_state_floats(H, d, dv), (dv + 31) // 32
+    S = torch.randn(len(lens), H, d, dv + 1, generator=g)
+    m = torch.rand(len(lens), H, generator=g)
+    state = torch.cat([S.reshape(len(lens), -1), m.repeat_interleave(copies, 1)], 1)
+    assert state.shape[1] == floats
+    dev, st = buf.cuda(), state.cuda()
+    q, k, v, og = dev[:, :cut[0]], dev[:, cut[0]:cut[1]], dev[:, cut[1]:cut[2]], dev[:, cut[2]:]
+    b = batch(lens)
+    o.matrix_memory_parallel_min_tokens = 1
+    out = o.mlstm(q, k, v, gates.cuda(), og, w.cuda(), st, b, H, d, dv, scale, cap, eps)
+    assert any(key[0] == "mlstm_chunks" for key in b.aux)
+    x = buf.double()
+    S64, m64 = S.double(), m.double()
+    ref = memory_by_tokens(x[:, :cut[0]], x[:, cut[0]:cut[1]], x[:, cut[1]:cut[2]], gates.double(), x[:, cut[2]:], w.double(),
+                           (S64, m64), lens, H, d, dv, scale, cap, eps)
+    # sums of up to 260 float32 products that partly cancel, against the row's root mean square; a bfloat16 result's own
+    # rounding (8 bits) is at most 2^-8 of it
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    err = ((out.cpu().double() - ref).abs() - rel * ref.abs()).amax(1) / ref.pow(2).mean(1).sqrt()
+    assert err.max() < 2e-4, float(err.max())
+    got = st.cpu().double()
+    gs, gm = got[:, :H * d * (dv + 1)].view(S64.shape), got[:, H * d * (dv + 1):].view(len(lens), H, copies)
+    assert (gs - S64).abs().max() < 2e-5 * S64.abs().max() and (gm - m64[:, :, None]).abs().max() < 1e-4
