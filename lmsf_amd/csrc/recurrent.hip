@@ -385,9 +385,14 @@ __global__ __launch_bounds__(256) void selective_scan_fold_kernel(const float* _
 }
 
 // The same for states of up to 32 entries: a lane a channel, its whole state in registers, so that nothing crosses
-// lanes and every instruction works on 64 channels. B and C of a tile of 8 tokens go through LDS (every lane reads the
-// same entry); x, dt and z of the tile are asked for from memory together, a lane its own channel's.
+// lanes and every instruction works on 64 channels. B and C of up to 64 tokens go through LDS at a time (every lane reads the
+// same entry); x, dt and z of 8 tokens are asked for together, a lane its own channel's, while the 8 before are worked on. What
+// bounds a prompt's portions is the instructions of a token, some 200 of which 16 are exponentials at a quarter of the
+// rate: the softplus takes 30 of them (log1pf would take 110 in one chain), the rates are multiplied by log2(e) once.
+// 1,997 tokens of 8 requests, 4,096 channels by 16 entries, chunks of 64: summaries and outputs 68 + 99 -> 48 + 75 us; with
+// states of a chunk read and written 16 bytes at a time and chunks of 32 the whole scan 130 -> 99.
 #define SCANL_TT 8
+#define SCANL_BT 64
 
 template <typename T, int NS, bool SUMMARY>
 __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
@@ -396,7 +401,7 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
     const float* __restrict__ Dw, float* __restrict__ state, long state_stride, const int* __restrict__ seg_starts,
     const int* __restrict__ state_slots, T* __restrict__ y, long y_stride, int inner, int nstate, int chunk,
     const int* __restrict__ scratch_base, float* __restrict__ scratch, int vec) {
-  __shared__ float sB[SCANL_TT * NS], sC[SCANL_TT * NS];
+  __shared__ __align__(16) float sB[SCANL_BT * NS], sC[SUMMARY ? 1 : SCANL_BT * NS];
   const int tid = threadIdx.x;
   const int c = blockIdx.x * 256 + tid;
   const int s = blockIdx.z, j = blockIdx.y;
@@ -412,93 +417,101 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
   const int cc = live ? c : 0;                                 // (a lane beyond the channels computes on channel 0's and stores nothing)
   const long entry = (long)inner * (nstate + 1);
   float* st = state + (long)state_slots[s] * state_stride + (long)cc * nstate;
-  float a[NS], S[NS];
-  if (vec && base < 0) {
+  float a[NS], S[NS];                                          // a: the rates times log2(e)
+  constexpr float LOG2E = 1.4426950408889634f;
+  // where the state comes from: the slot's, or the chunk's as selective_scan_fold_kernel left it; a summary begins from zero
+  // and, the first one, copies the slot's state to the entry before the first chunk
+  const float* from = base < 0 ? st : scratch + (long)(base + j) * entry + (long)cc * nstate;
+  float* copy = SUMMARY && j == 0 && live ? scratch + (long)base * entry + (long)c * nstate : nullptr;
+  if (vec) {
     // a channel's NS rates and state entries, 16 bytes a load (one by one every load asks for 64 cache lines: 8 single
     // tokens of 4,096 channels by 16 entries 10.5 -> 5.3 us)
 #pragma unroll
     for (int n = 0; n + 3 < NS; n += 4) {
-      const float4 s4 = *reinterpret_cast<const float4*>(st + n);
       const float4 a4 = *reinterpret_cast<const float4*>(A_log + (long)cc * NS + n);
-      S[n] = s4.x; S[n + 1] = s4.y; S[n + 2] = s4.z; S[n + 3] = s4.w;
       a[n] = a4.x; a[n + 1] = a4.y; a[n + 2] = a4.z; a[n + 3] = a4.w;
+      float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (!SUMMARY) s4 = *reinterpret_cast<const float4*>(from + n);
+      else if (copy) *reinterpret_cast<float4*>(copy + n) = *reinterpret_cast<const float4*>(st + n);
+      S[n] = s4.x; S[n + 1] = s4.y; S[n + 2] = s4.z; S[n + 3] = s4.w;
     }
 #pragma unroll
-    for (int n = 0; n < NS; ++n) a[n] = -expf(a[n]);
+    for (int n = 0; n < NS; ++n) a[n] = -expf(a[n]) * LOG2E;
   } else {
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const bool ok = n < nstate;
-      a[n] = ok ? -expf(A_log[(long)cc * nstate + n]) : 0.f;
-      S[n] = 0.f;
-      if (ok) {
-        if (base < 0) {
-          S[n] = st[n];
-        } else if (SUMMARY) {
-          if (j == 0 && live) scratch[(long)base * entry + (long)c * nstate + n] = st[n];     // the entry before the first chunk
-        } else {
-          S[n] = scratch[(long)(base + j) * entry + (long)cc * nstate + n];    // folded by selective_scan_fold_kernel
-        }
-      }
+      a[n] = ok ? -expf(A_log[(long)cc * nstate + n]) * LOG2E : 0.f;
+      S[n] = ok && !SUMMARY ? from[n] : 0.f;
+      if (ok && copy) copy[n] = st[n];
     }
   }
   if (SUMMARY && j == n_chunks - 1) return;
   const float dw = Dw[cc];
   float sum_dt = 0.f;
-  for (int t0 = start; t0 < end; t0 += SCANL_TT) {
-    const int nt = min(SCANL_TT, end - t0);
-    float rx[SCANL_TT], rdt[SCANL_TT], rz[SCANL_TT];
+  // 8 tokens of this lane's channel, as they lie in memory (a token beyond ``last`` is ``last``'s again)
+  struct Held {
+    T x[SCANL_TT], z[SUMMARY ? 1 : SCANL_TT];
+    float dt[SCANL_TT];
+  };
+  auto fetch = [&](Held& h, int t0, int last) {
 #pragma unroll
     for (int tt = 0; tt < SCANL_TT; ++tt) {
-      const long t = t0 + (tt < nt ? tt : 0);
-      rx[tt] = to_f32<T>(x[t * x_stride + cc]);
-      rdt[tt] = dt_pre[t * dt_stride + cc];
-      rz[tt] = SUMMARY ? 0.f : to_f32<T>(z[t * z_stride + cc]);
+      const long t = min(t0 + tt, last);
+      h.x[tt] = x[t * x_stride + cc];
+      h.dt[tt] = dt_pre[t * dt_stride + cc];
+      if constexpr (!SUMMARY) h.z[tt] = z[t * z_stride + cc];
     }
-    __syncthreads();
-    for (int i = tid; i < nt * NS; i += 256) {
+  };
+  Held now, next;
+  if (start < end) fetch(now, start, end - 1);
+  for (int tb = start; tb < end; tb += SCANL_BT) {
+    const int nb = min(SCANL_BT, end - tb);
+    if (tb > start) __syncthreads();
+    for (int i = tid; i < nb * NS; i += 256) {
       const int tt = i / NS, n = i % NS;
-      const long t = t0 + tt;
+      const long t = tb + tt;
       sB[i] = n < nstate ? to_f32<T>(bc[t * bc_stride + b_at + n]) : 0.f;
       if (!SUMMARY) sC[i] = n < nstate ? to_f32<T>(bc[t * bc_stride + c_at + n]) : 0.f;
     }
     __syncthreads();
+    for (int u = 0; u < nb; u += SCANL_TT) {
+      if (tb + u + SCANL_TT < end) fetch(next, tb + u + SCANL_TT, end - 1);
 #pragma unroll
-    for (int tt = 0; tt < SCANL_TT; ++tt) {
-      if (tt < nt) {
-        const float dtv = rc_softplus(rdt[tt]), xv = rx[tt];
-        const float dx = dtv * xv;
-        sum_dt += dtv;
-        float acc = 0.f;
+      for (int tt = 0; tt < SCANL_TT; ++tt) {
+        if (u + tt < nb) {
+          const float dtv = rc_softplus(now.dt[tt]), xv = to_f32<T>(now.x[tt]);
+          const float dx = dtv * xv;
+          sum_dt += dtv;
+          float acc = 0.f;
 #pragma unroll
-        for (int n = 0; n < NS; ++n) {
-          S[n] = rc_decay(dtv * a[n]) * S[n] + dx * sB[tt * NS + n];
-          if (!SUMMARY) acc += S[n] * sC[tt * NS + n];
-        }
-        if (!SUMMARY && live) {
-          const float zv = rz[tt];
-          y[(long)(t0 + tt) * y_stride + c] = from_f32<T>((acc + dw * xv) * (zv / (1.f + expf(-zv))));
+          for (int n = 0; n < NS; ++n) {
+            S[n] = __builtin_amdgcn_exp2f(dtv * a[n]) * S[n] + dx * sB[(u + tt) * NS + n];
+            if (!SUMMARY) acc += S[n] * sC[(u + tt) * NS + n];
+          }
+          if constexpr (!SUMMARY) {
+            const float zv = to_f32<T>(now.z[tt]);
+            if (live) y[(long)(tb + u + tt) * y_stride + c] = from_f32<T>((acc + dw * xv) * (zv / (1.f + expf(-zv))));
+          }
         }
       }
+      now = next;
     }
   }
   if (!live) return;
   if (SUMMARY) {
-    float* ent = scratch + (long)(base + j + 1) * entry;
+    scratch[(long)(base + j + 1) * entry + (long)inner * nstate + c] = sum_dt;
+  } else if (j < n_chunks - 1) {
+    return;
+  }
+  float* to = SUMMARY ? scratch + (long)(base + j + 1) * entry + (long)c * nstate : st;
+  if (vec) {
+#pragma unroll
+    for (int n = 0; n + 3 < NS; n += 4) *reinterpret_cast<float4*>(to + n) = make_float4(S[n], S[n + 1], S[n + 2], S[n + 3]);
+  } else {
 #pragma unroll
     for (int n = 0; n < NS; ++n)
-      if (n < nstate) ent[(long)c * nstate + n] = S[n];
-    ent[(long)inner * nstate + c] = sum_dt;
-  } else if (j == n_chunks - 1) {
-    if (vec) {
-#pragma unroll
-      for (int n = 0; n + 3 < NS; n += 4)
-        *reinterpret_cast<float4*>(st + n) = make_float4(S[n], S[n + 1], S[n + 2], S[n + 3]);
-    } else {
-#pragma unroll
-      for (int n = 0; n < NS; ++n)
-        if (n < nstate) st[n] = S[n];
-    }
+      if (n < nstate) to[n] = S[n];
   }
 }
 
@@ -532,7 +545,7 @@ extern "C" int lmsf_selective_scan(const void* x, int dtype, long x_stride, cons
     dim3 lgrid((inner + 255) / 256, chunked ? max_chunks : 1, n_segments), lblock(256);
     // (the kernel holds exactly these numbers of entries, and every channel's lie on a 16-byte boundary)
     const int vec = (nstate == 4 || nstate == 8 || nstate == 16 || nstate == 32) && state_stride % 4 == 0 &&
-                    lmsf_aligned16(state) && lmsf_aligned16(A_log);
+                    lmsf_aligned16(state) && lmsf_aligned16(A_log) && (!chunked || (inner % 4 == 0 && lmsf_aligned16(scratch)));
 #define SCANL(T, NS, SUM)                                                                                              \
   hipLaunchKernelGGL((selective_scan_lane_kernel<T, NS, SUM>), lgrid, lblock, 0, stream, (const T*)x, x_stride, dt_pre, \
                      dt_stride, (const T*)bc, bc_stride, b_at, c_at, (const T*)z, z_stride, A_log, Dw, state,          \

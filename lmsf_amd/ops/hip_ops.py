@@ -1510,6 +1510,10 @@ class HipOps:
         # segments longer than a chunk (portions of prompts) are cut into chunks that run side by side; which
         # segments, and where their chunks' summaries lie, is worked out once a step on the host
         chunk, max_chunks, bases, scratch = self.scan_chunk_tokens, 1, None, None
+        lens = getattr(batch, "host_seg_lens", None)
+        few = N * inner <= self.scan_few_work
+        if lens and max(lens) > (chunk // 2 if few else chunk):
+            chunk = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
         plan = self._chunk_plan(batch, chunk)
         if plan is not None:
             bases, entries, max_chunks = plan
@@ -1521,7 +1525,14 @@ class HipOps:
             _ptr(y), y.stride(0), N, S, inner, n, int(chunk), int(max_chunks), _ptr(bases), _ptr(scratch), self._stream()))
         return y
 
-    scan_chunk_tokens = 64         # tokens of a chunk of the selective scan's chunked form
+    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones into chunks of 32; where the
+    # tokens times the channels are few, so that the chip is far from full, from 33 tokens on and into chunks of 16. Chunks of 16 / 32
+    # / 64, 16 entries: 509 tokens of 4,096 channels 49 / 45 / 80 us, 2,048 of 4,096 132 / 109 / 105, 1,997 of 4,096 in 8 requests
+    # 104 / 99 / 130, of 1,024 53 / 55 / 80; 509 of 1,024 35 / 42 / 78, 8 times 128 of 1,024 31 / 40 / 79, 100 of 4,096 26 / 38 / 76.
+    # In one piece 8 times 64 tokens take 37 us, in chunks of 32 43 (4,096 channels) and of 16 27 (1,024).
+    scan_chunk_tokens = 64
+    scan_cut_tokens = 32
+    scan_few_work = 1 << 20        # tokens times channels
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
     recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
     # The matrix memory's chunks run side by side from this many tokens on at heads of 128 and more, from twice as many at

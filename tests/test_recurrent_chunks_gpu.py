@@ -1,5 +1,5 @@
 """The recurrences over portions of prompts at the sizes where their chunks and tiles end: the matrix memory's chunks side by
-side on the matrix cores, against the recurrence token by token in 64 bits."""
+side on the matrix cores, the selective scan's pieces, against the recurrences token by token in 64 bits."""
 import types
 
 import pytest
@@ -77,3 +77,35 @@ def test_matrix_memory_side_by_side(H, d, dv, lens, dtype):
     got = st.cpu().double()
     gs, gm = got[:, :H * d * (dv + 1)].view(S64.shape), got[:, H * d * (dv + 1):].view(len(lens), H, copies)
     assert (gs - S64).abs().max() < 2e-5 * S64.abs().max() and (gm - m64[:, :, None]).abs().max() < 1e-4
+
+
+# one piece and cuts of 16 and of 32 tokens, pieces of fewer than 8, states that the kernel's number of entries is and is not,
+# channels that end inside a workgroup
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("inner,n,lens,few", [(256, 16, (32,), None), (300, 16, (65, 7, 1), None), (260, 5, (97, 130), None),
+                                              (512, 32, (33,), 0), (256, 4, (200, 33), 0), (256, 16, (129, 64), 0), (302, 8, (70,), 0)])
+def test_selective_scan_in_pieces(inner, n, lens, few, dtype):
+    o, g = ops(), torch.Generator().manual_seed(inner + n)
+    if few is not None:
+        o.scan_few_work = few
+    N = sum(lens)
+    x, z, bc = (torch.randn(N, c, generator=g).to(dtype) for c in (inner, inner, 2 * n))
+    dt, al, D = torch.randn(N, inner, generator=g) * 3 - 1, torch.randn(inner, n, generator=g), torch.randn(inner, generator=g)
+    st0 = torch.randn(len(lens), inner * n, generator=g)
+    st = st0.cuda()
+    y = o.selective_scan(x.cuda(), dt.cuda(), bc.cuda(), 0, n, z.cuda(), al.cuda(), D.cuda(), st, batch(lens))
+    S = st0.double().view(len(lens), inner, n)
+    X, Z, B, C = x.double(), z.double(), bc.double()[:, :n], bc.double()[:, n:]
+    sp, A, ref, at = torch.nn.functional.softplus(dt.double(), threshold=50), -torch.exp(al.double()), [], 0
+    for s, length in enumerate(lens):
+        slot = len(lens) - 1 - s
+        for t in range(at, at + length):
+            S[slot] = torch.exp(sp[t][:, None] * A) * S[slot] + (sp[t] * X[t])[:, None] * B[t]
+            ref.append(((S[slot] * C[t]).sum(1) + D.double() * X[t]) * (Z[t] * torch.sigmoid(Z[t])))
+        at += length
+    ref = torch.stack(ref)
+    scale = ref.abs().amax(1, keepdim=True)
+    # (a state's exponentials are off by their exponents' 2^-24, and sum up over the tokens that a state remembers)
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    assert (((y.cpu().double() - ref).abs() - rel * ref.abs()) / scale).max() < 5e-6
+    assert (st.cpu().double().view(S.shape) - S).abs().max() < 5e-6 * S.abs().max()
