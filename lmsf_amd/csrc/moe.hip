@@ -7,8 +7,8 @@
 // Few tokens (decoding), and float32 at any number: every (token, choice) streams its expert's rows, a wave per
 // output, the token's vector in LDS, 16-byte loads where the rows allow them.
 // Many tokens in bfloat16: the (token, choice) pairs are grouped by expert on the device (one small kernel: counts,
-// offsets, an order, a list of tiles of up to 128 pairs of one expert), and each tile runs on the matrix cores
-// against 128 of its expert's outputs (A = 16 rows of W x 32 k, B = 16 pairs x 32 k; in the gated product the gate
+// offsets, an order, a list of tiles of up to 160 pairs of one expert), and each tile runs on the matrix cores
+// against 256 rows of its expert's matrix (A = 16 rows of W x 32 k, B = 16 pairs x 32 k; in the gated product the gate
 // and the up rows of the same outputs), operands through LDS. The down product leaves float32 rows per pair; a last kernel adds a token's pairs and the shared part. A pair's result
 // does not depend on where in its tile it lies, so the order inside an expert's group (atomic counters) is free.
 // Accumulation in float32 throughout.
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(MOE_THREADS) void moe_down_few_kernel(
 
 // ---------------------------------------------------------------- many tokens: grouped by expert, matrix cores
 
-#define MOE_TILE 128         // pairs a tile holds
+#define MOE_TILE 160         // pairs a tile holds
 
 // Groups the P = N * top pairs by expert. order[i]: the pair at place i of the grouped sequence; tiles: for every
 // tile (of up to ``tile_pairs`` pairs) its expert, its first place and its number of pairs; n_tiles[0]: how many
@@ -354,157 +354,243 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
                                                         int* __restrict__ order, int* __restrict__ tiles,
                                                         int* __restrict__ n_tiles) {
   extern __shared__ int sm[];   // [E] counts, [E] first places, [E] fill counters
+  constexpr int HELD = 8;       // pairs whose experts a thread keeps between the two walks
   int* cnt = sm;
   int* first = sm + E;
   int* fill = sm + 2 * E;
-  for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = fill[e] = 0;
-  __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
+  const int tid = threadIdx.x, step = blockDim.x;
+  const auto expert_of = [&](int p) {
     const int id = min(max(ids ? ids[p / top] : p / top, 0), vocab - 1);
-    const int e = min(max(table[(long)id * top + p % top], 0), E + identity - 1);
+    return min(max(table[(long)id * top + p % top], 0), E + identity - 1);
+  };
+  int held[HELD];
+#pragma unroll
+  for (int i = 0; i < HELD; ++i) held[i] = tid + i * step < P ? expert_of(tid + i * step) : E;
+  for (int e = tid; e < E; e += step) cnt[e] = fill[e] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < HELD; ++i)
+    if (held[i] < E) atomicAdd(&cnt[held[i]], 1);
+  for (int p = tid + HELD * step; p < P; p += step) {
+    const int e = expert_of(p);
     if (e < E) atomicAdd(&cnt[e], 1);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid < LMSF_WAVE) {
+    // places and tiles of 64 experts at a time: running sums over the lanes
     int at = 0, t = 0;
-    for (int e = 0; e < E; ++e) {
-      first[e] = at;
-      for (int s = 0; s < cnt[e]; s += tile_pairs) {
-        tiles[3 * t] = e;
-        tiles[3 * t + 1] = at + s;
-        tiles[3 * t + 2] = min(tile_pairs, cnt[e] - s);
-        ++t;
+    for (int e0 = 0; e0 < E; e0 += LMSF_WAVE) {
+      const int e = e0 + tid, n = e < E ? cnt[e] : 0, mine = (n + tile_pairs - 1) / tile_pairs;
+      int places = n, tl = mine;
+      for (int o = 1; o < LMSF_WAVE; o <<= 1) {
+        const int up = __shfl_up(places, o, LMSF_WAVE), ut = __shfl_up(tl, o, LMSF_WAVE);
+        if (tid >= o) {
+          places += up;
+          tl += ut;
+        }
       }
-      at += cnt[e];
+      const int begin = at + places - n;
+      if (e < E) first[e] = begin;
+      for (int i = 0; i < mine; ++i) {
+        int* to = tiles + 3 * (t + tl - mine + i);
+        to[0] = e;
+        to[1] = begin + i * tile_pairs;
+        to[2] = min(tile_pairs, n - i * tile_pairs);
+      }
+      at += __shfl(places, LMSF_WAVE - 1, LMSF_WAVE);
+      t += __shfl(tl, LMSF_WAVE - 1, LMSF_WAVE);
     }
-    n_tiles[0] = t;
+    if (tid == 0) n_tiles[0] = t;
   }
   __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    const int id = min(max(ids ? ids[p / top] : p / top, 0), vocab - 1);
-    const int e = min(max(table[(long)id * top + p % top], 0), E + identity - 1);
+#pragma unroll
+  for (int i = 0; i < HELD; ++i)
+    if (held[i] < E) order[first[held[i]] + atomicAdd(&fill[held[i]], 1)] = tid + i * step;
+  for (int p = tid + HELD * step; p < P; p += step) {
+    const int e = expert_of(p);
     if (e < E) order[first[e] + atomicAdd(&fill[e], 1)] = p;
   }
 }
 
-// One tile of up to 128 pairs against 128 outputs of its expert, operands through LDS. GATED: x = the tokens' vectors
-// (row of pair p: p / top), Wm = Wgu, K = W, O = F, y = act [P, F] bfloat16 = silu(gate) * up; else x = act (row of pair
-// p: p), Wm = Wd, K = F, O = W, y = float32 rows [P, W]. A step of 32 k: the workgroup copies the rows of W (128, or 128 gate + 128 up) and the 128 pairs' rows, 64 bytes of each, into
-// LDS with 16-byte loads (the next step's while this step is multiplied: two buffers, one barrier a step), and every
-// wave of the 2 x 2 reads the fragments of its 64 pairs and 64 outputs from there (rows of 64 bytes back to back: a
-// fragment's 64 lanes read 1 KB in a row, no bank conflicts). A first form whose waves fetched their fragments
-// themselves, straight from memory in tiles of 64 pairs, did 2.7 times fewer multiplications per byte fetched and lost
-// at every number of pairs: 2,048 tokens (256 pairs an expert) 319 against 194 us for the four kernels, 512 tokens 230
-// against 98, 64 tokens (8 pairs an expert, every tile mostly empty) 101 against 83.
+// One tile of up to 160 pairs against 256 rows of its expert's matrix, operands through LDS: 128 outputs with gate and up (KIND
+// 1: x = the tokens' vectors, row of pair p: p / top, Wm = Wgu, K = W, O = F, y = act [P, F] bfloat16 = silu(gate) * up), or 256
+// outputs (KIND 0: x = act, row of pair p: p, Wm = Wd, K = F, O = W, y = float32 rows [P, W]; KIND 2: one matrix an expert, Wm
+// [E, O, K], with relu(.)^2). In a step of 64 k the 256 rows of W and the 160 pairs' rows, 128 bytes of each (whole cache lines:
+// with 64 every line came to the compute unit twice), travel from memory straight into LDS (global_load_lds_dwordx4), two
+// of MOE_STAGES steps on their way at a time, one barrier a step. The 16-byte piece c of row r lies in slot (c + r) mod 8 of
+// its row, so that the fragments' reads meet distinct banks. Eight waves, two a SIMD, wait for LDS in turn: two rows of them
+// over the pairs, four columns over W; a wave leaves out the 16s of pairs that its tile does not have. The blocks of outputs vary
+// fastest over the workgroups and fall to the dies in turn, so that an expert's rows are read by one die, whose tiles of
+// that expert share them in its L2. What bounds the kernel is these rows' way into the compute units.
+// 3,994 pairs of 16 experts, 2,048 -> 2 x 1,024 -> 2,048, all four kernels, with tiles of 128 pairs by 128 outputs copied through
+// registers 32 k at a time 217 -> 116 us; 66 pairs 77 -> 55; 8,192 pairs of 8, 4,096 -> 2 x 1,536 -> 4,096, 766 -> 583.
+#define MOE_TILE_ROWS 256
+#define MOE_TILE_WAVES 8
+#define MOE_STAGES 3
+#define MOE_STAGE_BYTES ((MOE_TILE_ROWS + MOE_TILE) * 128)
 
-// KIND 0: the down product; 1: gate and up with silu(gate) * up; 2: one matrix an expert (Wm [E, O, K]) with relu(.)^2.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is named as clobbered on purpose
+// (inline assembly: through the compiler's builtin every LDS read that follows would wait for all transfers in flight; the
+// waits are explicit)
+__device__ __forceinline__ void moe_global_to_lds_16(const void* src, unsigned lds_base_uniform) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_base_uniform)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 template <int KIND>
-__global__ __launch_bounds__(256) void moe_tile_lds_kernel(const bf16_t* __restrict__ x, long x_stride, int top,
-                                                           const bf16_t* __restrict__ Wm, const int* __restrict__ order,
-                                                           const int* __restrict__ tiles, const int* __restrict__ n_tiles,
-                                                           void* __restrict__ y, int O, int K,
-                                                           const float* __restrict__ pair_scale, float limit) {
+__global__ __launch_bounds__(MOE_TILE_WAVES * 64) void moe_tile_lds_kernel(
+    const bf16_t* __restrict__ x, long x_stride, int top, const bf16_t* __restrict__ Wm, const int* __restrict__ order,
+    const int* __restrict__ tiles, const int* __restrict__ n_tiles, void* __restrict__ y, int O, int K, int o_blocks,
+    const float* __restrict__ pair_scale, float limit) {
   constexpr bool GATED = KIND == 1, UP = KIND != 0;
-  constexpr int AR = GATED ? 256 : 128;            // rows of W a step
-  constexpr int NLA = AR * 4 / 256;                // 16-byte pieces of W a thread copies a step
-  constexpr int NLB = MOE_TILE * 4 / 256;      // and of the pairs' rows
-  constexpr int NA = GATED ? 8 : 4;                // fragments of W a wave
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  __shared__ __attribute__((aligned(16))) unsigned char lds[2][(AR + MOE_TILE) * 64];
-  const int t = blockIdx.x;
-  if (t >= n_tiles[0]) return;
+  constexpr int OUTS = GATED ? MOE_TILE_ROWS / 2 : MOE_TILE_ROWS;    // outputs a workgroup
+  constexpr int OW = OUTS / (MOE_TILE_WAVES / 2);  // and a wave
+  constexpr int NA = MOE_TILE_ROWS / (MOE_TILE_WAVES / 2) / 16;      // fragments of W a wave
+  constexpr int NB = MOE_TILE / 32;                // and of the pairs
+  constexpr int STAGES = MOE_STAGES, STAGE = MOE_STAGE_BYTES;
+  constexpr int ROWS8 = STAGE / 1024;              // transfers of 8 rows a step
+  constexpr int LOADS = (ROWS8 + MOE_TILE_WAVES - 1) / MOE_TILE_WAVES;   // and those of a wave
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int t = blockIdx.x / o_blocks, o_base = (blockIdx.x - t * o_blocks) * OUTS;
+  if (t >= n_tiles[0] || o_base >= O) return;
   const int e = tiles[3 * t], place = tiles[3 * t + 1], count = tiles[3 * t + 2];
   const int tid = threadIdx.x, wave = tid / LMSF_WAVE, lane = tid % LMSF_WAVE;
   const int fr = lane % 16, fg = lane / 16;
-  const int wr = wave / 2, wc = wave % 2;          // the wave's 64 pairs and 64 outputs
-  const int o_base = blockIdx.y * 128;
-  // what this thread copies: piece (tid % 4) of rows tid / 4, + 64, ...
-  const bf16_t* ga[NLA];
-  const bf16_t* gb[NLB];
+  const int wr = wave / (MOE_TILE_WAVES / 2), wc = wave % (MOE_TILE_WAVES / 2);   // the wave's half of the pairs and OW outputs
+  // what this lane moves: slot lane % 8 of row lane / 8 of a transfer's 8 rows (transfers beyond the last are the last again)
+  const int piece = ((lane & 7) - (lane >> 3)) & 7;
+  const bf16_t* src[LOADS];
 #pragma unroll
-  for (int i = 0; i < NLA; ++i) {
-    const int r = tid / 4 + i * 64;                // 0 .. AR-1; gated: rows 128 .. 255 are the up rows
-    const int o = min(o_base + (r & 127), O - 1);
-    ga[i] = Wm + ((long)e * (GATED ? 2 : 1) * O + (GATED && r >= 128 ? O : 0) + o) * K + (tid % 4) * 8;
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = min(wave * LOADS + i, ROWS8 - 1) * 8 + (lane >> 3);    // W (gated: 128 gate rows, 128 up rows), then the pairs
+    if (r < MOE_TILE_ROWS) {
+      const int o = min(o_base + (r & (OUTS - 1)), O - 1);
+      src[i] = Wm + ((long)e * (GATED ? 2 : 1) * O + (r >= OUTS ? O : 0) + o) * K + piece * 8;
+    } else {
+      const int p = order[place + min(r - MOE_TILE_ROWS, count - 1)];
+      src[i] = x + (long)(UP ? p / top : p) * x_stride + piece * 8;
+    }
   }
-#pragma unroll
-  for (int i = 0; i < NLB; ++i) {
-    const int p = order[place + min(tid / 4 + i * 64, count - 1)];
-    gb[i] = x + (long)(UP ? p / top : p) * x_stride + (tid % 4) * 8;
-  }
-  f32x4_t acc[NA][4];
+  f32x4_t acc[NA][NB];
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[a][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  u32x4 ra[NLA], rb[NLB];
+    for (int mt = 0; mt < NB; ++mt) acc[a][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // 16s of pairs that the wave has: an expert's last tile may be nearly empty
+  const int mine = __builtin_amdgcn_readfirstlane((count - wr * (MOE_TILE / 2) + 15) / 16);
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) const unsigned char*)lds;
+  const int n_steps = (K + 63) / 64;               // K is a multiple of 32: the last step may be half a one
+  auto issue = [&](int step, int stage_byte) {
+    // (the second half of a last half step is fetched from the first half's place and not multiplied)
+    const int k = step * 64 - (step * 64 + 32 >= K && piece >= 4 ? 32 : 0);
 #pragma unroll
-  for (int i = 0; i < NLA; ++i) ra[i] = *reinterpret_cast<const u32x4*>(ga[i]);
+    for (int i = 0; i < LOADS; ++i)
+      moe_global_to_lds_16(src[i] + k, __builtin_amdgcn_readfirstlane(lds0 + stage_byte + min(wave * LOADS + i, ROWS8 - 1) * 1024));
+  };
 #pragma unroll
-  for (int i = 0; i < NLB; ++i) rb[i] = *reinterpret_cast<const u32x4*>(gb[i]);
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < n_steps) issue(s, s * STAGE);
+  int consume = 0, produce = (STAGES - 1) * STAGE;
+  for (int it = 0; it < n_steps; ++it) {
+    // step ``it`` has arrived when at most the transfers of the later steps are outstanding
+    if (it + STAGES - 2 < n_steps)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 2) * LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();      // everybody's part of step ``it`` is there, and everybody is done with step ``it - 1``
+    if (it + STAGES - 1 < n_steps) issue(it + STAGES - 1, produce);
+    produce = produce + STAGE == STAGES * STAGE ? 0 : produce + STAGE;
+    const unsigned char* buf = lds + consume;
 #pragma unroll
-  for (int i = 0; i < NLA; ++i) *reinterpret_cast<u32x4*>(lds[0] + (tid / 4 + i * 64) * 64 + (tid % 4) * 16) = ra[i];
+    for (int s = 0; s < 2; ++s) {
+      if (it * 64 + s * 32 >= K) break;
+      const int at = fr * 128 + (((s * 4 + fg) + fr) & 7) * 16;
+      bf16x8_t fa[NA], fb[NB];
 #pragma unroll
-  for (int i = 0; i < NLB; ++i) *reinterpret_cast<u32x4*>(lds[0] + (AR + tid / 4 + i * 64) * 64 + (tid % 4) * 16) = rb[i];
-  __syncthreads();
-  int cur = 0;
-  for (int k = 0; k < K; k += 32) {
-    const bool more = k + 32 < K;
-    if (more) {
+      for (int a = 0; a < NA; ++a)       // fragment a: outputs wc * OW + (a * 16) mod OW ..; gated: the second half are the up rows of the same outputs
+        fa[a] = *reinterpret_cast<const bf16x8_t*>(buf + ((a * 16 >= OW ? OUTS : 0) + wc * OW + (a * 16) % OW) * 128 + at);
 #pragma unroll
-      for (int i = 0; i < NLA; ++i) ra[i] = *reinterpret_cast<const u32x4*>(ga[i] + k + 32);
+      for (int mt = 0; mt < NB; ++mt)
+        if (mt < mine) fb[mt] = *reinterpret_cast<const bf16x8_t*>(buf + (MOE_TILE_ROWS + wr * (MOE_TILE / 2) + mt * 16) * 128 + at);
 #pragma unroll
-      for (int i = 0; i < NLB; ++i) rb[i] = *reinterpret_cast<const u32x4*>(gb[i] + k + 32);
+      for (int mt = 0; mt < NB; ++mt)
+        if (mt < mine) {
+#pragma unroll
+          for (int a = 0; a < NA; ++a) acc[a][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[mt], acc[a][mt], 0, 0, 0);
+        }
     }
-    const unsigned char* buf = lds[cur];
-    bf16x8_t fa[NA], fb[4];
-#pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      // fragment a: outputs wc * 64 + (a % 4) * 16 ..; gated: a >= 4 are the up rows of the same outputs
-      const int row = (GATED && a >= 4 ? 128 : 0) + wc * 64 + (a & 3) * 16 + fr;
-      fa[a] = *reinterpret_cast<const bf16x8_t*>(buf + row * 64 + fg * 16);
-    }
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-      fb[mt] = *reinterpret_cast<const bf16x8_t*>(buf + (AR + wr * 64 + mt * 16 + fr) * 64 + fg * 16);
-#pragma unroll
-    for (int a = 0; a < NA; ++a)
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt) acc[a][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[a], fb[mt], acc[a][mt], 0, 0, 0);
-    if (more) {
-      unsigned char* nxt = lds[cur ^ 1];
-#pragma unroll
-      for (int i = 0; i < NLA; ++i) *reinterpret_cast<u32x4*>(nxt + (tid / 4 + i * 64) * 64 + (tid % 4) * 16) = ra[i];
-#pragma unroll
-      for (int i = 0; i < NLB; ++i) *reinterpret_cast<u32x4*>(nxt + (AR + tid / 4 + i * 64) * 64 + (tid % 4) * 16) = rb[i];
-    }
-    __syncthreads();
-    cur ^= 1;
+    consume = consume + STAGE == STAGES * STAGE ? 0 : consume + STAGE;
   }
-  // lane: pair wr * 64 + mt * 16 + fr, outputs o_base + wc * 64 + a * 16 + fg * 4 .. + 3
+  // lane: pair wr * (MOE_TILE / 2) + mt * 16 + fr, outputs o_base + wc * OW + a * 16 + fg * 4 .. + 3 (O is a multiple of 32)
+  const bool wide = ((uintptr_t)y & 15) == 0;
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int slot = wr * 64 + mt * 16 + fr;
+  for (int mt = 0; mt < NB; ++mt) {
+    const int slot = wr * (MOE_TILE / 2) + mt * 16 + fr;
     if (slot >= count) continue;
     const int p = order[place + slot];
     const float ps = UP && pair_scale ? pair_scale[p] : 1.f;
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < OW / 16; ++a) {
+      const int o = o_base + wc * OW + a * 16 + fg * 4;
+      if (o >= O) continue;
+      float r[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int o = o_base + wc * 64 + a * 16 + fg * 4 + j;
-        if (o >= O) continue;
         if (GATED) {
-          const float g = bf16_to_f32(f32_to_bf16(ps * acc[a][mt][j])), u = bf16_to_f32(f32_to_bf16(ps * acc[NA - 4 + a][mt][j]));
-          reinterpret_cast<bf16_t*>(y)[(long)p * O + o] = f32_to_bf16(limit > 0.f ? bounded_gate(g, u, limit) : g / (1.f + expf(-g)) * u);
+          const float g = bf16_to_f32(f32_to_bf16(ps * acc[a][mt][j])), u = bf16_to_f32(f32_to_bf16(ps * acc[NA - OW / 16 + a][mt][j]));
+          r[j] = limit > 0.f ? bounded_gate(g, u, limit) : g / (1.f + expf(-g)) * u;
         } else if (UP) {
           const float u = fmaxf(bf16_to_f32(f32_to_bf16(ps * acc[a][mt][j])), 0.f);
-          reinterpret_cast<bf16_t*>(y)[(long)p * O + o] = f32_to_bf16(u * u);
+          r[j] = u * u;
         } else {
-          reinterpret_cast<float*>(y)[(long)p * O + o] = acc[a][mt][j];
+          r[j] = acc[a][mt][j];
         }
       }
+      if (UP) {
+        bf16_t* to = reinterpret_cast<bf16_t*>(y) + (long)p * O + o;
+        if (wide) {
+          *reinterpret_cast<uint2*>(to) = make_uint2(pack2_bf16(r[0], r[1]), pack2_bf16(r[2], r[3]));
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) to[j] = f32_to_bf16(r[j]);
+        }
+      } else {
+        float* to = reinterpret_cast<float*>(y) + (long)p * O + o;
+        if (wide) {
+          *reinterpret_cast<float4*>(to) = make_float4(r[0], r[1], r[2], r[3]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) to[j] = r[j];
+        }
+      }
+    }
   }
+}
+
+template <int KIND>
+static int launch_moe_tiles(int max_tiles, hipStream_t stream, const bf16_t* x, long x_stride, int top, const bf16_t* Wm,
+                            const int* order, const int* tiles, const int* n_tiles, void* y, int O, int K,
+                            const float* pair_scale, float limit) {
+  constexpr int smem = MOE_STAGES * MOE_STAGE_BYTES, OUTS = KIND == 1 ? MOE_TILE_ROWS / 2 : MOE_TILE_ROWS;
+  static bool configured = false;   // per instantiation
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(moe_tile_lds_kernel<KIND>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+    if (e != hipSuccess) {
+      lmsf_set_error("table_moe: cannot reserve %d bytes of LDS: %s", smem, hipGetErrorString(e));
+      return 2;
+    }
+    configured = true;
+  }
+  // (blocks of outputs up to a multiple of 8, one for every die in turn; the surplus ends at once)
+  const int blocks = (O + OUTS - 1) / OUTS, o_blocks = blocks > 4 ? (blocks + 7) / 8 * 8 : blocks;
+  LMSF_CHECK((long)max_tiles * o_blocks < 2147483647L, "table_moe: too many tiles");
+  hipLaunchKernelGGL((moe_tile_lds_kernel<KIND>), dim3((unsigned)(max_tiles * o_blocks)),
+                     dim3(MOE_TILE_WAVES * 64), smem, stream, x, x_stride,
+                     top, Wm, order, tiles, n_tiles, y, O, K, o_blocks, pair_scale, limit);
+  return 0;
 }
 
 // out[n, o] = base[n, o] + weight * sum_k rows[n * top + k, o]; the choices of ``table`` (row ids[n], or n) from E on are
@@ -609,15 +695,14 @@ extern "C" int lmsf_table_moe_act(const void* h, int dtype, long h_stride, const
     int* n_tiles = tiles + 3 * (max_tiles + 1);
     hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), (size_t)3 * E * 4, stream, ids, table, vocab, top, E, identity,
                        P, MOE_TILE, order, tiles, n_tiles);
-    if (gated)
-      hipLaunchKernelGGL((moe_tile_lds_kernel<1>), dim3(max_tiles, (F + 127) / 128), dim3(256), 0, stream,
-                         (const bf16_t*)h, h_stride, top, (const bf16_t*)Wgu, order, tiles, n_tiles, act, F, W, pair_scale, limit);
-    else
-      hipLaunchKernelGGL((moe_tile_lds_kernel<2>), dim3(max_tiles, (F + 127) / 128), dim3(256), 0, stream,
-                         (const bf16_t*)h, h_stride, top, (const bf16_t*)Wgu, order, tiles, n_tiles, act, F, W, pair_scale, limit);
-    hipLaunchKernelGGL((moe_tile_lds_kernel<0>), dim3(max_tiles, (W + 127) / 128), dim3(256), 0, stream,
-                       (const bf16_t*)act, (long)F, top, (const bf16_t*)Wd, order, tiles, n_tiles, (void*)scratch_rows, W,
-                       F, (const float*)nullptr, 0.f);
+    int rc = gated ? launch_moe_tiles<1>(max_tiles, stream, (const bf16_t*)h, h_stride, top, (const bf16_t*)Wgu, order, tiles, n_tiles,
+                                         act, F, W, pair_scale, limit)
+                   : launch_moe_tiles<2>(max_tiles, stream, (const bf16_t*)h, h_stride, top, (const bf16_t*)Wgu, order, tiles, n_tiles,
+                                         act, F, W, pair_scale, limit);
+    if (rc == 0)
+      rc = launch_moe_tiles<0>(max_tiles, stream, (const bf16_t*)act, (long)F, top, (const bf16_t*)Wd, order, tiles, n_tiles,
+                               scratch_rows, W, F, nullptr, 0.f);
+    if (rc) return rc;
     const bool vec = W % 4 == 0 && out_stride % 4 == 0 && h_stride % 4 == 0 && (!base || base_stride % 4 == 0) &&
                      ((uintptr_t)out) % 8 == 0 && ((uintptr_t)base) % 8 == 0 && lmsf_aligned16(scratch_rows);
 #define MOE_COMBINE(V)                                                                                                \
