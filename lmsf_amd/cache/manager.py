@@ -44,7 +44,8 @@ def _raise(lib, status: int, who: str = "") -> None:
 
 
 def _ptr(a: Optional[np.ndarray]):
-    return None if a is None else ctypes.c_void_p(a.ctypes.data)
+    # (``a.ctypes.data`` builds two objects on the way to the same number)
+    return None if a is None else ctypes.c_void_p(a.__array_interface__["data"][0])
 
 
 class PagePool:

@@ -16,7 +16,7 @@ import torch
 from ..cache.manager import CacheError, CacheManager
 from ..cache.storage import CacheStorage
 from ..parts.base import Runtime
-from .batch import GroupView, StepContext, StepEntry
+from .batch import GroupView, StepBuffer, StepContext, StepEntry
 
 
 class StepError(ValueError):
@@ -326,12 +326,9 @@ class ModelExecutor:
         else:
             dev = host.clone()
 
-        def view(name: str) -> torch.Tensor:
-            o, n = offsets[name]
-            return dev[o:o + n]
-
+        buffer = StepBuffer(dev, offsets)
         if static is None and self._prev_tokens is not None:
-            self.rt.ops.patch_tokens(view("token_ids"), dev[src_at:src_at + n_all], self._prev_tokens)
+            self.rt.ops.patch_tokens(buffer.view("token_ids"), dev[src_at:src_at + n_all], self._prev_tokens)
         S_all = Sp if static is not None else S
         if static is None:
             seg_starts = section("seg_starts").tolist()
@@ -339,16 +336,12 @@ class ModelExecutor:
         else:
             # a captured step is told nothing that changes from step to step
             seg_starts, state_slots, lens, starts = list(range(S_all + 1)), [], [1] * S_all, []
-        groups = [GroupView(slots=view("slots%d" % gi),
-                            block_tables=view("tables%d" % gi).view(S_all, widths[gi]),
-                            page_size=mgr.groups[gi].page_size) for gi in range(G)]
+        groups = [GroupView.of_buffer(buffer, gi, S_all, int(widths[gi]), mgr.groups[gi].page_size) for gi in range(G)]
         # (where the plan lies on the device and how it is laid out travel with the step, not with the program)
-        aux = {"program_plan": (dev.data_ptr() + 4 * plan_at, plan_info)} if plan_cap else {}
-        return StepContext(
-            aux=aux, n_tokens=n_all, n_segments=S_all, token_ids=view("token_ids"), positions=view("positions"),
-            seg_of_token=view("seg_of"), seg_starts=view("seg_starts"), seg_first_pos=view("seg_first"),
-            state_slots=view("state_slots"), logit_rows=view("logit_rows"), n_logit_rows=R, groups=groups,
-            longest_first=dev[order_at:order_at + n_all] if single else None,
+        aux = {"program_plan": (buffer.base + 4 * plan_at, plan_info)} if plan_cap else {}
+        return StepContext.of_buffer(
+            buffer, dev[order_at:order_at + n_all] if single else None,
+            aux=aux, n_tokens=n_all, n_segments=S_all, n_logit_rows=R, groups=groups,
             host_seg_starts=seg_starts, host_seg_lens=lens, host_seg_first_pos=list(starts),
             host_state_slots=list(state_slots),
             request_ids=[e.request_id for e in entries] if static is None else [],
@@ -460,6 +453,8 @@ class _Staging:
         self._events: list = [None] * self.PARTS
         self._sent = [False] * self.PARTS
         self._turn = 0
+        self._last: Optional[torch.cuda.Stream] = None       # the stream that the last copy went to
+        self._raw_stream = None
 
     def _wait(self, turn: int) -> None:
         if self._sent[turn]:
@@ -487,8 +482,19 @@ class _Staging:
         if self._events[self._turn] is None:
             self._events[self._turn] = torch.cuda.Event()
         to.copy_(host, non_blocking=True)
-        self._events[self._turn].record(torch.cuda.current_stream(to.device))
+        self._events[self._turn].record(self._stream())
         self._sent[self._turn] = True
+
+    def _stream(self) -> "torch.cuda.Stream":
+        """The device's current stream: the object made for its handle the last time, where it is the same one."""
+        if self._raw_stream is None:
+            from ..ops.hip_ops import _current_device, _raw_stream
+            self._raw_stream = _raw_stream
+            self._index = self._device.index if self._device.index is not None else _current_device()
+        raw = self._raw_stream(self._index)
+        if self._last is None or self._last.cuda_stream != raw:
+            self._last = torch.cuda.current_stream(self._device)
+        return self._last
 
 
 class _StaticBatch:

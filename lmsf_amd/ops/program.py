@@ -419,7 +419,7 @@ class StepProgram:
         _declare(self.lib)
         self.device = device
         self._keep = recorder.keep
-        self.tunables = hip_ops.tunables()
+        self._tunables = bytes(hip_ops._tun)
         self.handle = c_void_p(self.lib.lmsf_program_create(ctypes.byref(hip_ops._tun)))
         for op in recorder.ops:
             if self.lib.lmsf_program_add(self.handle, ctypes.byref(op)) != 0:
@@ -445,7 +445,7 @@ class StepProgram:
 
     def stale(self) -> bool:
         """True once somebody has changed the kernels' switch points since the recording (tests, tuning)."""
-        return self.tunables != self.hip_ops.tunables()
+        return self._tunables != bytes(self.hip_ops._tun)
 
     STAT_NAMES = ("plain", "mid", "large", "deferred", "gemv", "chunks", "skinny", "blas", "materialize", "mid_scaled",
                   "gemv_scaled", "skinny_scaled", "separate", "gemv_add_norm", "skinny_add_norm", "gemv_add",
@@ -523,11 +523,12 @@ class StepProgram:
         st = StepDesc()
         st.n_tokens, st.n_segments, st.n_logit_rows = ctx.n_tokens, ctx.n_segments, ctx.n_logit_rows
         st.max_context, st.all_single, st.n_groups = int(ctx.max_context), 1 if ctx.all_single else 0, len(ctx.groups)
-        st.token_ids, st.positions, st.seg_of = ctx.token_ids.data_ptr(), ctx.positions.data_ptr(), ctx.seg_of_token.data_ptr()
-        st.logit_rows = ctx.logit_rows.data_ptr() if ctx.n_logit_rows else None
-        st.longest_first = ctx.longest_first.data_ptr() if ctx.longest_first is not None else None
+        at = ctx.addresses()
+        st.token_ids, st.positions, st.seg_of = at["token_ids"], at["positions"], at["seg_of"]
+        st.logit_rows = at["logit_rows"] if ctx.n_logit_rows else None
+        st.longest_first = at["longest_first"]
         for gi, g in enumerate(ctx.groups):
-            st.slots[gi], st.tables[gi], st.widths[gi] = g.slots.data_ptr(), g.block_tables.data_ptr(), g.block_tables.shape[1]
+            st.slots[gi], st.tables[gi], st.widths[gi] = g.addresses()
         if plan is not None:
             st.plan, st.plan_info = plan
         st.workspace, st.workspace_bytes = self.workspace.data_ptr(), self.workspace.numel()
