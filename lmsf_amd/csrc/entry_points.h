@@ -143,6 +143,16 @@ int lmsf_selective_scan(const void* x, int dtype, long x_stride, const float* dt
     state, long state_stride, const int* seg_starts, const int* state_slots, void* y, long y_stride, int n_tokens, int
     n_segments, int inner, int nstate, int chunk, int max_chunks, const int* scratch_base, float* scratch,
     hipStream_t stream);
+int lmsf_selective_scan_step_fits(int n_tokens, int inner, int nstate, int rank, int b_at, int c_at, long low_stride, long ldw,
+    long state_stride, const void* low, const void* W, const void* state, const void* A_log);
+int lmsf_selective_scan_step(const void* x, long x_stride, const void* low, long low_stride, const void* W, long ldw,
+    const void* bias, int rank, int b_at, int c_at, const void* z, long z_stride, const float* A_log, const float* Dw,
+    float* state, long state_stride, const int* state_slots, void* y, long y_stride, int n_tokens, int inner, int nstate,
+    hipStream_t stream);
+int lmsf_mlstm_step(const void* q, const void* k, const void* v, int dtype, long qkv_stride, const void* x, long x_stride,
+    const void* gate_w, long ldw, const void* gate_b, int K, const void* og, long og_stride, const float* norm_w, float* state,
+    long state_stride, const int* state_slots, void* out, long out_stride, float* o_raw, int n_tokens, int H, int d, int dv,
+    float qscale, float cap, float eps, hipStream_t stream);
 long lmsf_mlstm_state_floats(int H, int d, int dv);
 long lmsf_mlstm_chunk_scratch_floats(int n_tokens, int H, int dv);
 int lmsf_mlstm_chunk_tokens(int d);

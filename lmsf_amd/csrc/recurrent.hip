@@ -600,6 +600,114 @@ extern "C" int lmsf_selective_scan(const void* x, int dtype, long x_stride, cons
   return 0;
 }
 
+// The scan of a step of single tokens with the product before it inside: dt_pre = low W^T + bias (W [inner, rank] bfloat16, low
+// the first ``rank`` columns of the rows that hold B and C) takes eight matrix instructions of a workgroup, and a launch
+// and a trip of dt through memory are gone. A workgroup: 32 channels of 8 tokens, a thread a (token, channel) with its
+// whole state in registers; everything it needs from memory is asked for at once. What bounds it is that one trip.
+// 8 tokens of 4,096 channels by 16 entries, rank 128: product and scan 4.0 + 5.4 us -> 5.6.
+#define SCAN_STEP_CH 32
+#define SCAN_STEP_TOK 8
+
+template <int NS>
+__global__ __launch_bounds__(256) void selective_scan_step_kernel(
+    const bf16_t* __restrict__ x, long x_stride, const bf16_t* __restrict__ low, long low_stride,
+    const bf16_t* __restrict__ W, long ldw, const bf16_t* __restrict__ bias, int rank, int b_at, int c_at,
+    const bf16_t* __restrict__ z, long z_stride, const float* __restrict__ A_log, const float* __restrict__ Dw,
+    float* __restrict__ state, long state_stride, const int* __restrict__ state_slots, bf16_t* __restrict__ y, long y_stride,
+    int n_tokens, int inner) {
+  __shared__ float sdt[SCAN_STEP_TOK][SCAN_STEP_CH + 1];
+  const int tid = threadIdx.x, wave = tid / LMSF_WAVE, lane = tid % LMSF_WAVE, r = lane % 16, g = lane / 16;
+  const int t0 = blockIdx.y * SCAN_STEP_TOK, c0 = blockIdx.x * SCAN_STEP_CH;
+  const int tok = tid / SCAN_STEP_CH, t = min(t0 + tok, n_tokens - 1), c = c0 + tid % SCAN_STEP_CH;
+  const bool live = t0 + tok < n_tokens;               // (inner is a multiple of the workgroup's channels)
+  float* st = state + (long)state_slots[t] * state_stride + (long)c * NS;
+  float S[NS], a[NS], B[NS], C[NS];
+#pragma unroll
+  for (int n = 0; n < NS; n += 4) {
+    const float4 s4 = *reinterpret_cast<const float4*>(st + n), a4 = *reinterpret_cast<const float4*>(A_log + (long)c * NS + n);
+    S[n] = s4.x; S[n + 1] = s4.y; S[n + 2] = s4.z; S[n + 3] = s4.w;
+    a[n] = a4.x; a[n + 1] = a4.y; a[n + 2] = a4.z; a[n + 3] = a4.w;
+  }
+  const bf16_t* row = low + (long)t * low_stride;
+#pragma unroll
+  for (int n = 0; n < NS; n += 8) {
+    Vec16<bf16_t> vb, vc;
+    vb.load(row + b_at + n);
+    vc.load(row + c_at + n);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      B[n + e] = vb.get(e);
+      C[n + e] = vc.get(e);
+    }
+  }
+  const float xv = bf16_to_f32(x[(long)t * x_stride + c]), zv = bf16_to_f32(z[(long)t * z_stride + c]), dw = Dw[c];
+  const float db = bias ? bf16_to_f32(bias[c]) : 0.f;
+  if (wave < SCAN_STEP_CH / 16) {
+    // 16 channels by 8 tokens (the instruction's other 8 columns repeat them)
+    const bf16_t* wr = W + (long)(c0 + wave * 16 + r) * ldw + g * 8;
+    const bf16_t* lr = low + (long)min(t0 + r % SCAN_STEP_TOK, n_tokens - 1) * low_stride + g * 8;
+    f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = 0; k < rank; k += 32)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8_t*>(wr + k),
+                                                    *reinterpret_cast<const bf16x8_t*>(lr + k), acc, 0, 0, 0);
+    if (r < SCAN_STEP_TOK) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sdt[r][wave * 16 + 4 * g + e] = acc[e];
+    }
+  }
+  __syncthreads();
+  const float dt = rc_softplus(sdt[tok][tid % SCAN_STEP_CH] + db), dx = dt * xv;
+  float acc = 0.f;
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    S[n] = __builtin_amdgcn_exp2f(dt * (-expf(a[n]) * 1.4426950408889634f)) * S[n] + dx * B[n];
+    acc += S[n] * C[n];
+  }
+  if (!live) return;
+  y[(long)t * y_stride + c] = f32_to_bf16((acc + dw * xv) * (zv / (1.f + expf(-zv))));
+#pragma unroll
+  for (int n = 0; n < NS; n += 4) *reinterpret_cast<float4*>(st + n) = make_float4(S[n], S[n + 1], S[n + 2], S[n + 3]);
+}
+
+// 1 where lmsf_selective_scan_step takes these sizes, strides (in elements) and addresses; the scan with its product beside
+// it serves the rest.
+extern "C" int lmsf_selective_scan_step_fits(int n_tokens, int inner, int nstate, int rank, int b_at, int c_at, long low_stride,
+                                             long ldw, long state_stride, const void* low, const void* W, const void* state,
+                                             const void* A_log) {
+  return n_tokens > 0 && inner > 0 && inner % SCAN_STEP_CH == 0 && (nstate == 8 || nstate == 16 || nstate == 32) && rank > 0 &&
+         rank % 32 == 0 && b_at >= 0 && c_at >= 0 && b_at % 8 == 0 && c_at % 8 == 0 && low_stride % 8 == 0 && ldw % 8 == 0 &&
+         state_stride % 4 == 0 && lmsf_aligned16(low) && lmsf_aligned16(W) && lmsf_aligned16(state) && lmsf_aligned16(A_log);
+}
+
+// A step of single tokens (token i is segment i): x, z, y [n_tokens, inner], low [n_tokens, >= rank + ...] with B and C at
+// columns b_at and c_at, W [inner, rank] (row stride ldw), bias [inner] or null, all bfloat16; the rest as in
+// lmsf_selective_scan.
+extern "C" int lmsf_selective_scan_step(const void* x, long x_stride, const void* low, long low_stride, const void* W, long ldw,
+                                        const void* bias, int rank, int b_at, int c_at, const void* z, long z_stride,
+                                        const float* A_log, const float* Dw, float* state, long state_stride,
+                                        const int* state_slots, void* y, long y_stride, int n_tokens, int inner, int nstate,
+                                        hipStream_t stream) {
+  LMSF_CHECK(x && low && W && z && A_log && Dw && state && state_slots && y, "selective_scan_step: null pointer");
+  LMSF_CHECK(lmsf_selective_scan_step_fits(n_tokens, inner, nstate, rank, b_at, c_at, low_stride, ldw, state_stride, low, W, state,
+                                           A_log),
+             "selective_scan_step: sizes that the scan and its product take one after the other");
+  LMSF_CHECK(x_stride >= inner && z_stride >= inner && y_stride >= inner && ldw >= rank && low_stride >= rank &&
+                 low_stride >= b_at + nstate && low_stride >= c_at + nstate && state_stride >= (long)inner * nstate,
+             "selective_scan_step: strides too small");
+  LMSF_CHECK((n_tokens + SCAN_STEP_TOK - 1) / SCAN_STEP_TOK <= 65535, "selective_scan_step: too many tokens");
+  const dim3 grid(inner / SCAN_STEP_CH, (n_tokens + SCAN_STEP_TOK - 1) / SCAN_STEP_TOK), block(256);
+#define SCAN_STEP(NS)                                                                                                 \
+  hipLaunchKernelGGL((selective_scan_step_kernel<NS>), grid, block, 0, stream, (const bf16_t*)x, x_stride,             \
+                     (const bf16_t*)low, low_stride, (const bf16_t*)W, ldw, (const bf16_t*)bias, rank, b_at, c_at,     \
+                     (const bf16_t*)z, z_stride, A_log, Dw, state, state_stride, state_slots, (bf16_t*)y, y_stride,    \
+                     n_tokens, inner)
+  if (nstate == 8) SCAN_STEP(8); else if (nstate == 16) SCAN_STEP(16); else SCAN_STEP(32);
+#undef SCAN_STEP
+  LMSF_LAUNCH_CHECK("selective_scan_step");
+  return 0;
+}
+
 // ---------------------------------------------------------------- matrix memory with exponential gates
 // Per head, with log gates i = cap tanh(ipre / cap), f = logsigmoid(cap tanh(fpre / cap)) and a running maximum m
 // (0 before the first token):
@@ -1176,6 +1284,126 @@ __global__ __launch_bounds__(256) void mlstm_token_kernel(
   if (tid < MLD_COLS / MLS_M_COLS && e0 + tid * MLS_M_COLS < dv) gm[tid] = m;       // this block's copies of m
 }
 
+// A step of single tokens with the product of the gates inside (gates = x W^T + bias, W [2 H, K]: the input gates' rows, then
+// the forget gates'): two rows of W a workgroup, added up by all of its lanes while the memory's rows are on their way, so
+// that the product is no launch and no trip of its own. As mlstm_token_kernel otherwise, with eight waves, of which each asks for
+// 16 rows of the memory at once. What bounds it is the trip to memory behind the slot's number.
+// 8 tokens, 8 heads of 128 by 128, K 2,048: product and memory 4.0 + 10.6 us -> 8.9.
+#define MLT_THREADS 512
+#define MLT_ROWS 16
+
+template <typename T>
+__global__ __launch_bounds__(MLT_THREADS) void mlstm_step_kernel(
+    const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, long qkv_stride, const T* __restrict__ x,
+    long x_stride, const T* __restrict__ W, long ldw, const T* __restrict__ bias, int K, float* __restrict__ state,
+    long state_stride, const int* __restrict__ state_slots, float* __restrict__ o_raw, long o_stride, float* __restrict__ den,
+    int H, int d, int dv, float qscale, float cap) {
+  constexpr int WAVES = MLT_THREADS / LMSF_WAVE, VEC = 16 / (int)sizeof(T);
+  extern __shared__ float lds[];
+  float* sq = lds;                       // [d]
+  float* sk = sq + d;                    // [d]
+  float* so = sk + d;                    // [WAVES][64]
+  float* sgate = so + WAVES * MLD_COLS;  // [WAVES][2]
+  const int tid = threadIdx.x, wave = tid / LMSF_WAVE, lane = tid % LMSF_WAVE;
+  const int h = blockIdx.x, t = blockIdx.y, e0 = blockIdx.z * MLD_COLS;
+  const int cols = dv + 1;
+  const bool col_ok = e0 + lane < dv;
+  float* st = state + (long)state_slots[t] * state_stride;
+  float* gS = st + (long)h * d * cols;
+  float* gm = st + (long)H * d * cols + (long)h * mls_m_copies(dv) + blockIdx.z * (MLD_COLS / MLS_M_COLS);
+  const float m0 = gm[0];
+  float rows[MLT_ROWS];
+  auto ask = [&](int d0) {
+#pragma unroll
+    for (int j = 0; j < MLT_ROWS; ++j) {
+      const int dd = d0 + wave + WAVES * j;
+      rows[j] = dd < d && col_ok ? gS[(long)dd * cols + e0 + lane] : 0.f;
+    }
+  };
+  ask(0);
+  // n's rows: a thread each of the first block of columns
+  float n0 = 0.f;
+  if (blockIdx.z == 0 && tid < d) n0 = gS[(long)tid * cols + dv];
+  float gi = 0.f, gf = 0.f;
+  const T* xr = x + (long)t * x_stride;
+  const T* wi = W + (long)h * ldw;
+  const T* wf = W + (long)(H + h) * ldw;
+  for (int i = tid * VEC; i < K; i += MLT_THREADS * VEC) {
+    Vec16<T> a, b, c;
+    a.load(xr + i);
+    b.load(wi + i);
+    c.load(wf + i);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      gi += a.get(e) * b.get(e);
+      gf += a.get(e) * c.get(e);
+    }
+  }
+  for (int i = tid; i < d; i += MLT_THREADS) {
+    sq[i] = to_f32<T>(q[(long)t * qkv_stride + h * d + i]) * qscale;
+    sk[i] = to_f32<T>(k[(long)t * qkv_stride + h * d + i]);
+  }
+  const float vv = col_ok ? to_f32<T>(v[(long)t * qkv_stride + h * dv + e0 + lane]) : 0.f;
+  gi = wave_sum(gi);
+  gf = wave_sum(gf);
+  if (lane == 0) {
+    sgate[2 * wave] = gi;
+    sgate[2 * wave + 1] = gf;
+  }
+  __syncthreads();
+  gi = bias ? to_f32<T>(bias[h]) : 0.f;
+  gf = bias ? to_f32<T>(bias[H + h]) : 0.f;
+#pragma unroll
+  for (int w = 0; w < WAVES; ++w) {
+    gi += sgate[2 * w];
+    gf += sgate[2 * w + 1];
+  }
+  gi = cap * tanhf(gi / cap);
+  gf = rc_logsigmoid(cap * tanhf(gf / cap));
+  const float m = fmaxf(gf + m0, gi), keep = expf(gf + m0 - m), take = expf(gi - m);
+  float acc = 0.f;
+  for (int d0 = 0; d0 < d; d0 += WAVES * MLT_ROWS) {
+    if (d0 > 0) ask(d0);
+#pragma unroll
+    for (int j = 0; j < MLT_ROWS; ++j) {
+      const int dd = d0 + wave + WAVES * j;
+      if (dd < d && col_ok) {
+        const float s = keep * rows[j] + take * sk[dd] * vv;
+        gS[(long)dd * cols + e0 + lane] = s;
+        acc += s * sq[dd];
+      }
+    }
+  }
+  so[wave * MLD_COLS + lane] = acc;
+  float part = 0.f;
+  if (blockIdx.z == 0) {
+    // n and n . q, by the first block of columns alone: a thread a row
+    for (int dd = tid; dd < d; dd += MLT_THREADS) {
+      const float s = keep * (dd == tid ? n0 : gS[(long)dd * cols + dv]) + take * sk[dd];
+      gS[(long)dd * cols + dv] = s;
+      part += s * sq[dd];
+    }
+    part = wave_sum(part);
+  }
+  __syncthreads();                       // (the gates' sums have been read, the outputs' are there)
+  if (blockIdx.z == 0 && lane == 0) sgate[wave] = part;
+  if (wave == 0 && col_ok) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) o += so[w * MLD_COLS + lane];
+    o_raw[(long)t * o_stride + h * dv + e0 + lane] = o;
+  }
+  if (blockIdx.z == 0) {
+    __syncthreads();
+    if (tid == 0) {
+      float nq = 0.f;
+      for (int w = 0; w < WAVES; ++w) nq += sgate[w];
+      den[(long)t * H + h] = fmaxf(fabsf(nq), expf(-m)) + 1e-6f;
+    }
+  }
+  if (tid < MLD_COLS / MLS_M_COLS && e0 + tid * MLS_M_COLS < dv) gm[tid] = m;       // this block's copies of m
+}
+
 // the temporary of the forms that leave the division to the heads' kernel: numerators float32 [n_tokens, H * dv], then
 // denominators [n_tokens, H]
 extern "C" long lmsf_mlstm_chunk_scratch_floats(int n_tokens, int H, int dv) { return (long)n_tokens * H * (dv + 1); }
@@ -1328,6 +1556,44 @@ extern "C" int lmsf_mlstm_tokens(const void* q, const void* k, const void* v, in
                        o_raw + (long)n_tokens * H * dv, (const bf16_t*)og,
                        og_stride, norm_w, (bf16_t*)out, out_stride, n_tokens, H, dv, eps);
   }
+  LMSF_LAUNCH_CHECK("head_norm_gate");
+  return 0;
+}
+
+// lmsf_mlstm_tokens for a step of single tokens (token i is segment i) that makes its gates itself: x [n_tokens, K] (row stride
+// x_stride) and gate_w [2 H, K] (ldw) with rows on 16-byte boundaries, gate_b [2 H] or null, of the tokens' type.
+extern "C" int lmsf_mlstm_step(const void* q, const void* k, const void* v, int dtype, long qkv_stride, const void* x,
+                               long x_stride, const void* gate_w, long ldw, const void* gate_b, int K, const void* og,
+                               long og_stride, const float* norm_w, float* state, long state_stride, const int* state_slots,
+                               void* out, long out_stride, float* o_raw, int n_tokens, int H, int d, int dv, float qscale,
+                               float cap, float eps, hipStream_t stream) {
+  LMSF_CHECK(q && k && v && x && gate_w && og && norm_w && state && state_slots && out && o_raw, "mlstm_step: null pointer");
+  LMSF_CHECK(dtype == LMSF_F32 || dtype == LMSF_BF16, "mlstm_step: unknown dtype code %d", dtype);
+  LMSF_CHECK(H > 0 && H <= 65535 && d > 0 && d <= 4096 && dv > 0, "mlstm_step: bad sizes H=%d d=%d dv=%d", H, d, dv);
+  LMSF_CHECK(cap > 0.f, "mlstm_step: the gates' cap must be > 0");
+  const int vw = 16 / lmsf_elem_size(dtype);
+  LMSF_CHECK(K > 0 && K % vw == 0 && x_stride >= K && ldw >= K && x_stride % vw == 0 && ldw % vw == 0 && lmsf_aligned16(x) &&
+                 lmsf_aligned16(gate_w),
+             "mlstm_step: rows of %d columns must lie on 16-byte boundaries", K);
+  LMSF_CHECK(og_stride >= (long)H * dv && out_stride >= (long)H * dv && state_stride >= lmsf_mlstm_state_floats(H, d, dv),
+             "mlstm_step: strides too small");
+  LMSF_CHECK(n_tokens >= 0 && n_tokens <= 65535 && (dv + MLD_COLS - 1) / MLD_COLS <= 65535, "mlstm_step: bad counts");
+  if (n_tokens == 0) return 0;
+  const dim3 grid(H, n_tokens, (dv + MLD_COLS - 1) / MLD_COLS);
+  const size_t smem = (size_t)(2 * d + (MLT_THREADS / LMSF_WAVE) * (MLD_COLS + 2)) * sizeof(float);
+  float* den = o_raw + (long)n_tokens * H * dv;
+  const dim3 ngrid((unsigned)(((long)n_tokens * H + 3) / 4));
+#define ML_STEP(T)                                                                                                    \
+  do {                                                                                                               \
+    hipLaunchKernelGGL((mlstm_step_kernel<T>), grid, dim3(MLT_THREADS), smem, stream, (const T*)q, (const T*)k,      \
+                       (const T*)v, qkv_stride, (const T*)x, x_stride, (const T*)gate_w, ldw, (const T*)gate_b, K,   \
+                       state, state_stride, state_slots, o_raw, (long)H * dv, den, H, d, dv, qscale, cap);           \
+    LMSF_LAUNCH_CHECK("mlstm_step");                                                                                 \
+    hipLaunchKernelGGL((head_norm_gate_kernel<T>), ngrid, dim3(256), 0, stream, o_raw, (long)H * dv, den,            \
+                       (const T*)og, og_stride, norm_w, (T*)out, out_stride, n_tokens, H, dv, eps);                  \
+  } while (0)
+  if (dtype == LMSF_F32) ML_STEP(float); else ML_STEP(bf16_t);
+#undef ML_STEP
   LMSF_LAUNCH_CHECK("head_norm_gate");
   return 0;
 }

@@ -1525,6 +1525,35 @@ class HipOps:
             _ptr(y), y.stride(0), N, S, inner, n, int(chunk), int(max_chunks), _ptr(bases), _ptr(scratch), self._stream()))
         return y
 
+    def selective_scan_step(self, x: torch.Tensor, low: torch.Tensor, rank: int, dt_weight: torch.Tensor,
+                            dt_bias: Optional[torch.Tensor], b_at: int, c_at: int, z: torch.Tensor, a_log: torch.Tensor,
+                            d_skip: torch.Tensor, state: torch.Tensor, batch) -> Optional[torch.Tensor]:
+        """``selective_scan`` of a step of single tokens with dt = low[:, :rank] dt_weight^T + dt_bias made inside
+        (bfloat16, ``low`` [N, >= rank + 2 n] holds B and C as well). None where that kernel does not take the operands."""
+        N, inner = x.shape
+        n = a_log.shape[1]
+        ok = all(t.dtype == torch.bfloat16 and t.dim() == 2 and t.stride(1) == 1 for t in (x, low, z, dt_weight)) \
+            and a_log.dtype == torch.float32 and a_log.is_contiguous() and state.dtype == torch.float32 \
+            and tuple(dt_weight.shape) == (inner, rank) and tuple(z.shape) == (N, inner) and a_log.shape[0] == inner \
+            and low.shape[0] == N and low.shape[1] >= max(rank, b_at + n, c_at + n) \
+            and (dt_bias is None or (dt_bias.dtype == torch.bfloat16 and dt_bias.shape == (inner,) and dt_bias.is_contiguous()))
+        if not ok or not self.lib.lmsf_selective_scan_step_fits(N, inner, n, int(rank), int(b_at), int(c_at), low.stride(0),
+                                                                dt_weight.stride(0), state.stride(0), _ptr(low), _ptr(dt_weight),
+                                                                _ptr(state), _ptr(a_log)):
+            return None
+        self._dev(x, low, dt_weight, dt_bias, z, a_log, d_skip)
+        self._f32_vec(d_skip, inner, "selective_scan: D")
+        self._state_view(state, inner * n, "selective_scan")
+        _, _, slots, S = self._segments(batch, N)
+        if S != N:
+            return None
+        y = torch.empty((N, inner), dtype=x.dtype, device=x.device)
+        self._check(self.lib.lmsf_selective_scan_step(
+            _ptr(x), x.stride(0), _ptr(low), low.stride(0), _ptr(dt_weight), dt_weight.stride(0), _ptr(dt_bias), int(rank),
+            int(b_at), int(c_at), _ptr(z), z.stride(0), _ptr(a_log), _ptr(d_skip), _ptr(state), state.stride(0), _ptr(slots),
+            _ptr(y), y.stride(0), N, inner, n, self._stream()))
+        return y
+
     # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones into chunks of 32; where the
     # tokens times the channels are few, so that the chip is far from full, from 33 tokens on and into chunks of 16. Chunks of 16 / 32
     # / 64, 16 entries: 509 tokens of 4,096 channels 49 / 45 / 80 us, 2,048 of 4,096 132 / 109 / 105, 1,997 of 4,096 in 8 requests
@@ -1670,6 +1699,38 @@ class HipOps:
             out_gate.stride(0), _ptr(norm_weight), _ptr(state), state.stride(0), _ptr(seg_starts), _ptr(slots), _ptr(out),
             out.stride(0), _ptr(raw), N, S, int(heads), int(dim), int(vdim), float(q_scale), float(gate_cap), float(eps),
             self._stream()))
+        return out
+
+    def mlstm_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, x: torch.Tensor, gate_weight: torch.Tensor,
+                   gate_bias: Optional[torch.Tensor], out_gate: torch.Tensor, norm_weight: torch.Tensor, state: torch.Tensor,
+                   batch, heads: int, dim: int, vdim: int, q_scale: float, gate_cap: float,
+                   eps: float) -> Optional[torch.Tensor]:
+        """``mlstm`` of a step of single tokens with gates = x gate_weight^T + gate_bias (gate_weight [2 heads, K]) made
+        inside. None where that kernel does not take the operands."""
+        N, K = x.shape
+        vec = 16 // x.element_size()
+        ok = all(t.dtype == x.dtype and t.dim() == 2 and t.stride(1) == 1 for t in (q, k, v, x, gate_weight, out_gate)) \
+            and tuple(gate_weight.shape) == (2 * heads, K) and K % vec == 0 and x.stride(0) % vec == 0 \
+            and gate_weight.stride(0) % vec == 0 and x.data_ptr() % 16 == 0 and gate_weight.data_ptr() % 16 == 0 \
+            and q.stride(0) == k.stride(0) == v.stride(0) and 0 < N <= 65535 and dim <= 4096 \
+            and all(t.shape[0] == N and t.shape[1] >= w for t, w in ((q, heads * dim), (k, heads * dim), (v, heads * vdim),
+                                                                     (out_gate, heads * vdim))) \
+            and (gate_bias is None or (gate_bias.dtype == x.dtype and gate_bias.shape == (2 * heads,) and gate_bias.is_contiguous()))
+        if not ok:
+            return None
+        self._dev(q, k, v, x, gate_weight, gate_bias, out_gate, norm_weight)
+        self._f32_vec(norm_weight, heads * vdim, "mlstm: norm weight")
+        self._state_view(state, self.mlstm_state_floats(heads, dim, vdim), "mlstm")
+        _, _, slots, S = self._segments(batch, N)
+        if S != N:
+            return None
+        out = torch.empty((N, heads * vdim), dtype=q.dtype, device=q.device)
+        raw = torch.empty(self.lib.lmsf_mlstm_chunk_scratch_floats(N, heads, vdim), dtype=torch.float32, device=q.device)
+        self._check(self.lib.lmsf_mlstm_step(
+            _ptr(q), _ptr(k), _ptr(v), _code(q.dtype), q.stride(0), _ptr(x), x.stride(0), _ptr(gate_weight),
+            gate_weight.stride(0), _ptr(gate_bias), K, _ptr(out_gate), out_gate.stride(0), _ptr(norm_weight), _ptr(state),
+            state.stride(0), _ptr(slots), _ptr(out), out.stride(0), _ptr(raw), N, int(heads), int(dim), int(vdim),
+            float(q_scale), float(gate_cap), float(eps), self._stream()))
         return out
 
     # ------------------------------------------------------------------ attention with keys and values of two sizes

@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 40      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
+ABI_VERSION = 41      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None
@@ -118,6 +118,11 @@ _SIGNATURES = {
     "lmsf_selective_scan": (c_int, [_P, c_int, c_long, _P, c_long, _P, c_long, c_int, c_int, _P, c_long, _P, _P, _P,
                                     c_long, _P, _P, _P, c_long, c_int, c_int, c_int, c_int, c_int, c_int, _P, _P, _P]),
     "lmsf_selective_scan_entry_floats": (c_long, [c_int, c_int]),
+    "lmsf_selective_scan_step_fits": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_long, c_long, c_long, _P, _P, _P, _P]),
+    "lmsf_selective_scan_step": (c_int, [_P, c_long, _P, c_long, _P, c_long, _P, c_int, c_int, c_int, _P, c_long, _P, _P, _P,
+                                         c_long, _P, _P, c_long, c_int, c_int, c_int, _P]),
+    "lmsf_mlstm_step": (c_int, [_P, _P, _P, c_int, c_long, _P, c_long, _P, c_long, _P, c_int, _P, c_long, _P, _P, c_long, _P,
+                                _P, c_long, _P, c_int, c_int, c_int, c_int, c_float, c_float, c_float, _P]),
     "lmsf_mlstm_chunk_scratch_floats": (c_long, [c_int, c_int, c_int]),
     "lmsf_mlstm_chunked": (c_int, [_P, _P, _P, c_int, c_long, _P, c_long, _P, c_long, _P, _P, c_long, _P, _P, _P, c_long,
                                    _P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, _P, c_int, c_long,

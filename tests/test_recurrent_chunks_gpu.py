@@ -109,3 +109,51 @@ def test_selective_scan_in_pieces(inner, n, lens, few, dtype):
     rel = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
     assert (((y.cpu().double() - ref).abs() - rel * ref.abs()) / scale).max() < 5e-6
     assert (st.cpu().double().view(S.shape) - S).abs().max() < 5e-6 * S.abs().max()
+
+
+# heads whose rows end inside a wave's 16 and beyond them, values that end inside a block of 64, gates of a row of one piece and
+# of more columns than the workgroup reads at a time
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,H,d,dv,K", [(1, 8, 128, 128, 2048), (9, 3, 40, 70, 8), (2, 1, 200, 24, 4104), (17, 2, 260, 65, 520)])
+def test_matrix_memory_of_single_tokens_makes_its_gates(N, H, d, dv, K, dtype):
+    o, g = ops(), torch.Generator().manual_seed(d + dv)
+    scale, cap, eps = d ** -0.5, 15.0, 1e-5
+    buf = torch.randn(N, H * (2 * d + 2 * dv), generator=g).to(dtype)
+    x, gw = torch.randn(N, K, generator=g).to(dtype), (torch.randn(2 * H, K, generator=g) * K ** -0.5).to(dtype)
+    gb, w = torch.randn(2 * H, generator=g).to(dtype), torch.rand(H * dv, generator=g) + 0.5
+    cut, copies = (H * d, 2 * H * d, 2 * H * d + H * dv), (dv + 31) // 32
+    S, m = torch.randn(N, H, d, dv + 1, generator=g), torch.rand(N, H, generator=g)
+    st = torch.cat([S.reshape(N, -1), m.repeat_interleave(copies, 1)], 1).cuda()
+    dev = buf.cuda()
+    out = o.mlstm_step(dev[:, :cut[0]], dev[:, cut[0]:cut[1]], dev[:, cut[1]:cut[2]], x.cuda(), gw.cuda(), gb.cuda(),
+                       dev[:, cut[2]:], w.cuda(), st, batch([1] * N), H, d, dv, scale, cap, eps)
+    b, S64, m64 = buf.double(), S.double(), m.double()
+    ref = memory_by_tokens(b[:, :cut[0]], b[:, cut[0]:cut[1]], b[:, cut[1]:cut[2]], x.double() @ gw.double().T + gb.double(),
+                           b[:, cut[2]:], w.double(), (S64, m64), [1] * N, H, d, dv, scale, cap, eps)
+    rel = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    err = ((out.cpu().double() - ref).abs() - rel * ref.abs()).amax(1) / ref.pow(2).mean(1).sqrt()
+    assert err.max() < 2e-4, float(err.max())
+    got = st.cpu().double()
+    gs, gm = got[:, :H * d * (dv + 1)].view(S64.shape), got[:, H * d * (dv + 1):].view(N, H, copies)
+    assert (gs - S64).abs().max() < 2e-5 * S64.abs().max() and (gm - m64[:, :, None]).abs().max() < 1e-4
+
+
+@pytest.mark.parametrize("N,inner,n,rank", [(1, 32, 16, 32), (8, 4096, 16, 128), (9, 96, 8, 160), (17, 64, 32, 64)])
+@pytest.mark.parametrize("biased", [True, False])
+def test_selective_scan_of_single_tokens_makes_its_steps(N, inner, n, rank, biased):
+    o, g, bf = ops(), torch.Generator().manual_seed(inner + n), torch.bfloat16
+    x, z, low = (torch.randn(N, c, generator=g).to(bf) for c in (inner, inner, rank + 2 * n))
+    W, bias = (torch.randn(inner, rank, generator=g) * rank ** -0.5).to(bf), torch.randn(inner, generator=g).to(bf)
+    al, D, st0 = torch.randn(inner, n, generator=g), torch.randn(inner, generator=g), torch.randn(N, inner * n, generator=g)
+    st = st0.cuda()
+    y = o.selective_scan_step(x.cuda(), low.cuda(), rank, W.cuda(), bias.cuda() if biased else None, rank, rank + n, z.cuda(),
+                              al.cuda(), D.cuda(), st, batch([1] * N))
+    S = st0.double().view(N, inner, n).flip(0)          # (the slots of ``batch`` run backwards)
+    X, Z, L = x.double(), z.double(), low.double()
+    dt = torch.nn.functional.softplus(L[:, :rank] @ W.double().T + (bias.double() if biased else 0), threshold=50)
+    S = torch.exp(-dt[:, :, None] * torch.exp(al.double())) * S + (dt * X)[:, :, None] * L[:, None, rank:rank + n]
+    ref = ((S * L[:, None, rank + n:]).sum(2) + D.double() * X) * (Z * torch.sigmoid(Z))
+    assert (((y.cpu().double() - ref).abs() - 2.0 ** -8 * ref.abs()) / ref.abs().amax(1, keepdim=True)).max() < 5e-6
+    assert (st.cpu().double().view(S.shape) - S.flip(0)).abs().max() < 5e-6 * S.abs().max()
+    assert o.selective_scan_step(x.cuda()[:, :inner - 8], low.cuda(), rank, W.cuda()[:inner - 8], None, rank, rank + n,
+                                 z.cuda()[:, :inner - 8], al.cuda()[:inner - 8], D.cuda()[:inner - 8], st, batch([1] * N)) is None
