@@ -37,6 +37,60 @@ __global__ __launch_bounds__(256) void dyt_norm_kernel(const TB* __restrict__ br
   for (int e = 0; e < V; ++e) out[(long)row * H + i0 + e] = from_f32<TO>(tanhf(a * r[e]) * w[i0 + e] + b[i0 + e]);
 }
 
+// The same for many rows: a thread takes four neighbouring columns of R rows, asks for all of them at once and reads w and b,
+// which are more bytes than a row of the stream and the branch, once for all of them. Memory-bound: 12 bytes an entry with
+// bfloat16 around it; 2,048 rows of 2,048 22.0 -> 12.5 us (4.0 TB/s), 1,034 rows 13.4 -> 8.5, 8,000 rows 76 -> 36.
+template <typename T> struct Dyt4;
+template <> struct Dyt4<float> {
+  static __device__ __forceinline__ float4 load(const float* p) { return *reinterpret_cast<const float4*>(p); }
+  static __device__ __forceinline__ void store(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
+};
+template <> struct Dyt4<bf16_t> {
+  static __device__ __forceinline__ float4 load(const bf16_t* p) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    return make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                       __uint_as_float(v.y & 0xffff0000u));
+  }
+  static __device__ __forceinline__ void store(bf16_t* p, float4 v) {
+    *reinterpret_cast<uint2*>(p) = make_uint2(pack2_bf16(v.x, v.y), pack2_bf16(v.z, v.w));
+  }
+};
+template <typename TB, typename TO, int R>
+__global__ __launch_bounds__(256) void dyt_norm_rows_kernel(const TB* __restrict__ branch, float* __restrict__ residual,
+                                                            const float* __restrict__ w, const float* __restrict__ b,
+                                                            const float* __restrict__ alpha, TO* __restrict__ out,
+                                                            const int* __restrict__ rows, int n_rows, int H) {
+  const int row0 = blockIdx.x * R, i0 = (blockIdx.y * 256 + threadIdx.x) * 4;
+  if (i0 >= H) return;
+  long src[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int row = min(row0 + q, n_rows - 1);
+    src[q] = (rows ? rows[row] : row) * (long)H + i0;
+  }
+  float4 r[R], y[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) r[q] = residual ? Dyt4<float>::load(residual + src[q]) : make_float4(0.f, 0.f, 0.f, 0.f);
+  if (branch) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) y[q] = Dyt4<TB>::load(branch + src[q]);
+  }
+  const float a = alpha[0];
+  const float4 wv = Dyt4<float>::load(w + i0), bv = Dyt4<float>::load(b + i0);
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    if (branch) {
+      r[q].x += y[q].x; r[q].y += y[q].y; r[q].z += y[q].z; r[q].w += y[q].w;
+    }
+    if (row0 + q < n_rows) {
+      if (branch && residual && !rows) Dyt4<float>::store(residual + src[q], r[q]);
+      Dyt4<TO>::store(out + (long)(row0 + q) * H + i0,
+                      make_float4(tanhf(a * r[q].x) * wv.x + bv.x, tanhf(a * r[q].y) * wv.y + bv.y,
+                                  tanhf(a * r[q].z) * wv.z + bv.z, tanhf(a * r[q].w) * wv.w + bv.w));
+    }
+  }
+}
+
 extern "C" int lmsf_dyt_norm(const void* branch, int branch_dtype, float* residual, const float* w, const float* b,
                              const float* alpha, void* out, int out_dtype, const int* rows, int n_rows, int H,
                              hipStream_t stream) {
@@ -49,6 +103,24 @@ extern "C" int lmsf_dyt_norm(const void* branch, int branch_dtype, float* residu
   const bool v4 = H % 4 == 0;
   const int per = v4 ? 4 : 1;
   dim3 grid(n_rows, (H / per + 255) / 256), block(256);
+  // R rows a thread where that leaves more than a workgroup a compute unit (fewer: level, both wait for one trip to memory),
+  // and every piece is aligned.
+  constexpr int R = 4;
+  const bool many = v4 && (long)((n_rows + R - 1) / R) * ((H / 4 + 255) / 256) > 256 && lmsf_aligned16(residual) &&
+                    lmsf_aligned16(w) && lmsf_aligned16(b) && lmsf_aligned16(branch) && lmsf_aligned16(out);
+  if (many) {
+    grid.x = (n_rows + R - 1) / R;
+#define DYT_ROWS(TB, TO)                                                                                               \
+  hipLaunchKernelGGL((dyt_norm_rows_kernel<TB, TO, R>), grid, block, 0, stream, (const TB*)branch, residual, w, b,     \
+                     alpha, (TO*)out, rows, n_rows, H)
+    if (branch_dtype == LMSF_F32 && out_dtype == LMSF_F32) DYT_ROWS(float, float);
+    else if (branch_dtype == LMSF_F32) DYT_ROWS(float, bf16_t);
+    else if (out_dtype == LMSF_F32) DYT_ROWS(bf16_t, float);
+    else DYT_ROWS(bf16_t, bf16_t);
+#undef DYT_ROWS
+    LMSF_LAUNCH_CHECK("dyt_norm_rows");
+    return 0;
+  }
 #define DYT(TB, TO)                                                                                                    \
   do {                                                                                                                 \
     if (v4)                                                                                                            \

@@ -99,6 +99,36 @@ def test_dynamic_tanh_with_and_without_the_addition(dtype, H):
     close(o.dyt_norm(dev(branch), None, dev(w), dev(b), dev(alpha), dtype), P.dyt(branch.float(), w, b, alpha), dtype)
 
 
+@pytest.mark.parametrize("branch_dtype", DTYPES)
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("N,H", [(1021, 1028), (1024, 2048), (1027, 52), (1028, 52), (1029, 52)])
+def test_dynamic_tanh_of_many_rows_is_that_of_few(N, H, dtype, branch_dtype):
+    """Above 1,024 rows (512 of more than 1,024 columns) a thread takes four rows. The same rows a few at a time, which the
+    other kernel takes, give the same bits."""
+    o = ops()
+    g = torch.Generator().manual_seed(N + H)
+    branch = (torch.randn((N, H), generator=g) * 2).to(branch_dtype).cuda()
+    res = (torch.randn((N, H), generator=g) * 3).cuda()
+    w, b = torch.randn(H, generator=g).cuda(), torch.randn(H, generator=g).cuda()
+    alpha = torch.tensor([0.37]).cuda()
+    rows = torch.randint(0, N, (N + 3,), generator=g, dtype=torch.int32).cuda()
+    cut = lambda f: torch.cat([f(slice(i, min(i + 100, N))) for i in range(0, N, 100)])
+    many, few = res.clone(), res.clone()
+    assert torch.equal(o.dyt_norm(branch, many, w, b, alpha, dtype),
+                       cut(lambda s: o.dyt_norm(branch[s], few[s], w, b, alpha, dtype)))
+    assert torch.equal(many, few) and torch.equal(many, res + branch.float())
+    only_residual = cut(lambda s: o.dyt_norm(None, res[s], w, b, alpha, dtype))
+    only_branch = cut(lambda s: o.dyt_norm(branch[s], None, w, b, alpha, dtype))
+    assert torch.equal(o.dyt_norm(None, res, w, b, alpha, dtype), only_residual)
+    assert torch.equal(o.dyt_norm(branch, None, w, b, alpha, dtype), only_branch)
+    assert torch.equal(o.dyt_norm(None, res, w, b, alpha, dtype, rows=rows), only_residual[rows.long()])
+    both = res.clone()
+    assert torch.equal(o.dyt_norm(branch, both, w, b, alpha, dtype, rows=rows),
+                       o.dyt_norm(None, many, w, b, alpha, dtype)[rows.long()]) and torch.equal(both, res)
+    shifted = torch.empty(N * H + 1, device="cuda")[1:].view(N, H).copy_(res)       # not aligned: the kernel of few rows
+    assert torch.equal(o.dyt_norm(None, shifted, w, b, alpha, dtype), only_residual)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_gated_activation_in_the_tanh_form(dtype):
     g = torch.Generator().manual_seed(1)
