@@ -71,6 +71,35 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ u
   out[(long)t * out_stride + c] = from_f32<T>(acc);
 }
 
+// The same for a step of single tokens with the number of taps known: the state, the filter and the input are asked for at
+// once, where the loop above waits for each of them (it also writes the state, so that no load may pass an earlier store).
+// 4 taps of 4,096 channels, bfloat16: 8 tokens 2.99 -> 2.13 us, 128 tokens 6.84 -> 4.29; other numbers of taps keep the loop.
+template <typename T, int ACT, int TAPS>
+__global__ __launch_bounds__(256) void short_conv_step_kernel(const T* __restrict__ u, long u_stride, const T* __restrict__ w,
+                                                              const T* __restrict__ bias, float* __restrict__ state,
+                                                              long state_stride, const int* __restrict__ seg_of,
+                                                              const int* __restrict__ state_slots, T* __restrict__ out,
+                                                              long out_stride, int C) {
+  const int t = blockIdx.x;
+  const int c = blockIdx.y * 256 + threadIdx.x;
+  if (c >= C) return;
+  const int s = seg_of[t];
+  float wj[TAPS], x[TAPS];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) wj[j] = to_f32<T>(w[(long)c * TAPS + j]);
+  x[TAPS - 1] = to_f32<T>(u[(long)t * u_stride + c]);
+  float acc = bias ? to_f32<T>(bias[c]) : 0.f;
+  float* st = state + (long)state_slots[s] * state_stride + (long)c * (TAPS - 1);
+#pragma unroll
+  for (int j = 0; j < TAPS - 1; ++j) x[j] = st[j];
+#pragma unroll
+  for (int j = 0; j < TAPS; ++j) acc += wj[j] * x[j];
+#pragma unroll
+  for (int j = 1; j < TAPS; ++j) st[j - 1] = x[j];
+  if (ACT == 1) acc = acc / (1.f + expf(-acc));
+  out[(long)t * out_stride + c] = from_f32<T>(acc);
+}
+
 // The same for portions of prompts: a thread takes two neighbouring channels of SC_TT tokens one after the other and keeps
 // their last inputs in registers, so that an input is read once and the filters once a thread. A token that begins a
 // segment takes its history from that segment's state.
@@ -198,11 +227,25 @@ extern "C" int lmsf_short_conv(const void* u, int dtype, long u_stride, const vo
     if (taps == 2) SC_TILE(T, A, 2); else if (taps == 3) SC_TILE(T, A, 3); else if (taps == 4) SC_TILE(T, A, 4);     \
     else SC_TILE(T, A, 5);                                                                                           \
   } while (0)
+#define SC_STEP(T, A, N)                                                                                             \
+  hipLaunchKernelGGL((short_conv_step_kernel<T, A, N>), grid, block, 0, stream, (const T*)u, u_stride, (const T*)w,   \
+                     (const T*)bias, state, state_stride, seg_of, state_slots, (T*)out, out_stride, C)
+#define SC_STEP_TAPS(T, A)                                                                                           \
+  do {                                                                                                               \
+    if (taps == 2) SC_STEP(T, A, 2); else if (taps == 3) SC_STEP(T, A, 3); else if (taps == 4) SC_STEP(T, A, 4);     \
+    else SC_STEP(T, A, 5);                                                                                           \
+  } while (0)
 #define SC(T, A)                                                                                                      \
   hipLaunchKernelGGL((short_conv_kernel<T, A>), grid, block, 0, stream, (const T*)u, u_stride, (const T*)w,           \
                      (const T*)bias, state, state_stride, seg_of, seg_starts, state_slots, (T*)out, out_stride, C, taps, \
                      single)
-  if (pairs) {
+  if (single && taps >= 2 && taps <= 5) {
+    if (dtype == LMSF_F32) {
+      if (act) SC_STEP_TAPS(float, 1); else SC_STEP_TAPS(float, 0);
+    } else {
+      if (act) SC_STEP_TAPS(bf16_t, 1); else SC_STEP_TAPS(bf16_t, 0);
+    }
+  } else if (pairs) {
     if (dtype == LMSF_F32) {
       if (act) SC_TAPS(float, 1); else SC_TAPS(float, 0);
     } else {
@@ -214,6 +257,8 @@ extern "C" int lmsf_short_conv(const void* u, int dtype, long u_stride, const vo
     if (act) SC(bf16_t, 1); else SC(bf16_t, 0);
   }
 #undef SC
+#undef SC_STEP_TAPS
+#undef SC_STEP
 #undef SC_TAPS
 #undef SC_TILE
   LMSF_LAUNCH_CHECK("short_conv");

@@ -183,6 +183,25 @@ def test_short_convolution_over_cut_requests(dtype, C, taps, act, off):
     assert float(state[1].abs().max()) == 0.0 and float(state[:, :3].abs().max()) == 0.0     # nobody else's memory
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("act", [None, "silu"])
+@pytest.mark.parametrize("C,taps", [(1, 1), (255, 2), (257, 3), (1024, 4), (300, 5), (24, 6)])
+def test_short_convolution_of_single_tokens_is_that_of_any_step(dtype, act, C, taps):
+    """A step that is told to be of single tokens has kernels of its own (2 to 5 taps with the number known)."""
+    o = ops()
+    g = torch.Generator().manual_seed(C)
+    slots = [3, 0, 5, 1]
+    u = torch.randn((4, C + 3), generator=g).to(dtype).cuda()[:, 1:C + 1]
+    w, bias = torch.randn((C, taps), generator=g).to(dtype).cuda(), torch.randn(C, generator=g).to(dtype).cuda()
+    state = torch.randn((6, C * (taps - 1) + 1), generator=g).cuda()
+    one, other = state.clone(), state.clone()
+    single, general = Step([1] * 4, slots), Step([1] * 4, slots)
+    single.all_single, general.all_single = True, False
+    view = lambda s: s[:, 1:] if taps > 1 else None
+    assert torch.equal(o.short_conv(u, w, bias, view(one), single, act), o.short_conv(u, w, bias, view(other), general, act))
+    assert torch.equal(one, other)
+
+
 def rotary_table(max_pos, rot, base, scaling=None):
     f = P.rotary_frequencies(rot, base, scaling).to(torch.float32)
     ang = torch.arange(max_pos, dtype=torch.float32)[:, None] * f[None, :]
