@@ -1159,11 +1159,24 @@ __global__ __launch_bounds__(MLX_THREADS) void mlstm_chunk_mfma_kernel(
     for (int S = 0; S < TILES; ++S)
       if (S < n_tiles) {
         float b[4];
+        bool finite = true;
 #pragma unroll
-        for (int n = 0; n < 4; ++n) b[n] = to_f32<T>(sv[(16 * S + 4 * g + n) * VP + 16 * w + r]);
+        for (int n = 0; n < 4; ++n) {
+          b[n] = to_f32<T>(sv[(16 * S + 4 * g + n) * VP + 16 * w + r]);
+          finite = finite && (__float_as_uint(b[n]) & 0x7f800000u) != 0x7f800000u;
+        }
+        // On the diagonal P holds zeros for tokens that come later. A value of theirs that is no finite number would reach the
+        // earlier ones through them, so that such a tile is added entry by entry, what a token sees alone.
+        const bool whole = __all(finite);
+        if (!whole) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            for (int t = 16 * S + 4 * g + e, u = 16 * S; u <= t; ++u)
+              acc[S][e] += sP[t * Lp + u] * to_f32<T>(sv[u * VP + 16 * w + r]);
+        }
 #pragma unroll
         for (int i = S; i < TILES; ++i)
-          if (i < n_tiles) {
+          if (i < n_tiles && (whole || i > S)) {
             float a[4];
             mlx_four<float>(sP + (16 * i + r) * Lp + 16 * S + 4 * g, a);
 #pragma unroll

@@ -79,6 +79,37 @@ def test_matrix_memory_side_by_side(H, d, dv, lens, dtype):
     assert (gs - S64).abs().max() < 2e-5 * S64.abs().max() and (gm - m64[:, :, None]).abs().max() < 1e-4
 
 
+# a token in the middle of a tile of 16, at its last place and in a second chunk; columns of two waves and the last one
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+@pytest.mark.parametrize("token,column", [(5, 0), (47, 37), (70, 69)])
+def test_matrix_memory_keeps_a_value_from_earlier_tokens(token, column, value, dtype):
+    """A value that is no finite number reaches its own token and later ones of its head, no earlier token and no other head."""
+    o, g = ops(), torch.Generator().manual_seed(token)
+    H, d, dv, lens = 2, 40, 70, (90, 33)
+    N, scale = sum(lens), d ** -0.5
+    buf = torch.randn(N, H * (2 * d + 2 * dv), generator=g).to(dtype)
+    gates, w = torch.randn(N, 2 * H, generator=g), torch.ones(H * dv)
+    state = torch.randn(len(lens), o.mlstm_state_floats(H, d, dv), generator=g)
+    cut = (H * d, 2 * H * d, 2 * H * d + H * dv)
+    o.matrix_memory_parallel_min_tokens = 1
+
+    def run(buf):
+        dev, b = buf.cuda(), batch(lens)
+        out = o.mlstm(dev[:, :cut[0]], dev[:, cut[0]:cut[1]], dev[:, cut[1]:cut[2]], gates.cuda(), dev[:, cut[2]:], w.cuda(),
+                      state.cuda(), b, H, d, dv, scale, 15.0, 1e-5)
+        assert any(key[0] == "mlstm_chunks" for key in b.aux)
+        return out.float().cpu()
+    plain, odd = run(buf), buf.clone()
+    odd[token, cut[1] + column] = value
+    out = run(odd)
+    assert not out[token:lens[0], :dv].isfinite().all(1).any()
+    assert torch.equal(out[:, dv:], plain[:, dv:]) and torch.equal(out[lens[0]:], plain[lens[0]:])
+    # (the tile's products are added in another order: 16 float32 sums, and the result's rounding where it has 8 bits)
+    rel = 2.0 ** -7 if dtype == torch.bfloat16 else 1e-5
+    assert ((out - plain)[:token, :dv].abs() <= rel * plain[:token, :dv].abs() + 1e-5).all()
+
+
 # one piece and cuts of 16 and of 32 tokens, pieces of fewer than 8, states that the kernel's number of entries is and is not,
 # channels that end inside a workgroup
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
