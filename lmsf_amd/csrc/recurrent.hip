@@ -39,6 +39,12 @@ __device__ __forceinline__ float rc_sigmoid(float z) { return 1.f / (1.f + expf(
 // exp of a decay's exponent, in the recurrences' inner loops: one multiplication and the hardware's 2^x (relative error
 // about |x| 2^-24 beside the instruction's own last bit; an exponent that large forgets within a token)
 __device__ __forceinline__ float rc_decay(float x) { return __expf(x); }
+// exp(a) log2(e), a rate for 2^x; of an ``a`` whose product (or exponential) is beyond float32 the largest number, so that a step
+// size of zero still keeps the state (infinity times zero would not)
+__device__ __forceinline__ float rc_rate2(float a) {
+  const float r = expf(a) * 1.4426950408889634f;
+  return r > 3.402823466e38f ? 3.402823466e38f : r;
+}
 __device__ __forceinline__ float rc_logsigmoid(float z) { return fminf(z, 0.f) - rc_log1p(expf(-fabsf(z))); }
 
 // ---------------------------------------------------------------- short causal convolution
@@ -463,7 +469,6 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
   const long entry = (long)inner * (nstate + 1);
   float* st = state + (long)state_slots[s] * state_stride + (long)cc * nstate;
   float a[NS], S[NS];                                          // a: the rates times log2(e)
-  constexpr float LOG2E = 1.4426950408889634f;
   // where the state comes from: the slot's, or the chunk's as selective_scan_fold_kernel left it; a summary begins from zero
   // and, the first one, copies the slot's state to the entry before the first chunk
   const float* from = base < 0 ? st : scratch + (long)(base + j) * entry + (long)cc * nstate;
@@ -481,12 +486,12 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
       S[n] = s4.x; S[n + 1] = s4.y; S[n + 2] = s4.z; S[n + 3] = s4.w;
     }
 #pragma unroll
-    for (int n = 0; n < NS; ++n) a[n] = -expf(a[n]) * LOG2E;
+    for (int n = 0; n < NS; ++n) a[n] = -rc_rate2(a[n]);
   } else {
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const bool ok = n < nstate;
-      a[n] = ok ? -expf(A_log[(long)cc * nstate + n]) * LOG2E : 0.f;
+      a[n] = ok ? -rc_rate2(A_log[(long)cc * nstate + n]) : 0.f;
       S[n] = ok && !SUMMARY ? from[n] : 0.f;
       if (ok && copy) copy[n] = st[n];
     }
@@ -706,7 +711,7 @@ __global__ __launch_bounds__(256) void selective_scan_step_kernel(
   float acc = 0.f;
 #pragma unroll
   for (int n = 0; n < NS; ++n) {
-    S[n] = __builtin_amdgcn_exp2f(dt * (-expf(a[n]) * 1.4426950408889634f)) * S[n] + dx * B[n];
+    S[n] = __builtin_amdgcn_exp2f(dt * -rc_rate2(a[n])) * S[n] + dx * B[n];
     acc += S[n] * C[n];
   }
   if (!live) return;

@@ -188,3 +188,22 @@ def test_selective_scan_of_single_tokens_makes_its_steps(N, inner, n, rank, bias
     assert (st.cpu().double().view(S.shape) - S.flip(0)).abs().max() < 5e-6 * S.abs().max()
     assert o.selective_scan_step(x.cuda()[:, :inner - 8], low.cuda(), rank, W.cuda()[:inner - 8], None, rank, rank + n,
                                  z.cuda()[:, :inner - 8], al.cuda()[:inner - 8], D.cuda()[:inner - 8], st, batch([1] * N)) is None
+
+
+# one piece, chunks, a step of single tokens; a number of entries that the kernel holds and one that it does not
+@pytest.mark.parametrize("n", [16, 5])
+@pytest.mark.parametrize("lens", [(3,), (70, 2), (1, 1)])
+def test_selective_scan_keeps_states_at_the_largest_rates(n, lens):
+    """exp(88.5) is a float32 number whose product with log2(e) is none: a step size of zero still leaves the state alone."""
+    o, g, bf = ops(), torch.Generator().manual_seed(n), torch.bfloat16
+    N, inner, rank = sum(lens), 64, 32
+    x, z, low = (torch.randn(N, c, generator=g).to(bf).cuda() for c in (inner, inner, rank + 2 * 16))
+    al, D = torch.full((inner, n), 88.5, device="cuda"), torch.ones(inner, device="cuda")
+    st0 = torch.randn(len(lens), inner * n, generator=g).cuda()
+    st = st0.clone()
+    y = o.selective_scan(x, torch.full((N, inner), -200.0, device="cuda"), low, rank, rank + 16, z, al, D, st, batch(lens))
+    assert torch.equal(st, st0) and y.isfinite().all()
+    if lens == (1, 1) and n == 16:
+        W, bias = torch.zeros(inner, rank, dtype=bf, device="cuda"), torch.full((inner,), -200.0, dtype=bf, device="cuda")
+        y = o.selective_scan_step(x, low, rank, W, bias, rank, rank + 16, z, al, D, st, batch(lens))
+        assert torch.equal(st, st0) and y.isfinite().all()
