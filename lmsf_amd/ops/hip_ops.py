@@ -1509,11 +1509,8 @@ class HipOps:
         y = torch.empty((N, inner), dtype=x.dtype, device=x.device)
         # segments longer than a chunk (portions of prompts) are cut into chunks that run side by side; which
         # segments, and where their chunks' summaries lie, is worked out once a step on the host
-        chunk, max_chunks, bases, scratch = self.scan_chunk_tokens, 1, None, None
-        lens = getattr(batch, "host_seg_lens", None)
-        few = N * inner <= self.scan_few_work
-        if lens and max(lens) > (chunk // 2 if few else chunk):
-            chunk = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
+        chunk = self._scan_chunk(getattr(batch, "host_seg_lens", None), N, inner, n)
+        max_chunks, bases, scratch = 1, None, None
         plan = self._chunk_plan(batch, chunk)
         if plan is not None:
             bases, entries, max_chunks = plan
@@ -1554,14 +1551,30 @@ class HipOps:
             _ptr(y), y.stride(0), N, inner, n, self._stream()))
         return y
 
-    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones into chunks of 32; where the
-    # tokens times the channels are few, so that the chip is far from full, from 33 tokens on and into chunks of 16. Chunks of 16 / 32
-    # / 64, 16 entries: 509 tokens of 4,096 channels 49 / 45 / 80 us, 2,048 of 4,096 132 / 109 / 105, 1,997 of 4,096 in 8 requests
-    # 104 / 99 / 130, of 1,024 53 / 55 / 80; 509 of 1,024 35 / 42 / 78, 8 times 128 of 1,024 31 / 40 / 79, 100 of 4,096 26 / 38 / 76.
-    # In one piece 8 times 64 tokens take 37 us, in chunks of 32 43 (4,096 channels) and of 16 27 (1,024).
+    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 32 entries, which
+    # a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far from full, from 33
+    # tokens on and into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 509 tokens of 4,096 channels 49 / 47 / 67 us, 2,048 of
+    # 4,096 137 / 114 / 108, 8 times 256 of 4,096 105 / 101 / 104, of 1,024 46 / 46 / 68; 509 of 1,024 35 / 42 / 65, 8 times 128 of
+    # 1,024 31 / 41 / 66, 70 of 4,096 26 / 38 / 63. In one piece 8 times 64 tokens take 37 us, in chunks of 32 43 (4,096 channels)
+    # and of 16 27 (1,024). Larger states, 16 lanes a channel, cost more to leave and fold than short chunks save: 2,048 tokens of
+    # 2,048 channels by 64 entries 281 / 247 / 236 us, of 4,096 by 256 1,581 / 1,277 / 1,111, 48 tokens beside 32 single ones of
+    # 4,096 by 256 156 / 167 / 88. They keep chunks of 64.
     scan_chunk_tokens = 64
     scan_cut_tokens = 32
     scan_few_work = 1 << 20        # tokens times channels
+    scan_cut_entries = 32
+
+    def _scan_chunk(self, lens, n_tokens: int, inner: int, n: int) -> int:
+        """Tokens of a chunk of the selective scan of ``n_tokens`` tokens in segments of ``lens``, ``inner`` channels by ``n``
+        entries; segments that are longer are cut."""
+        chunk = self.scan_chunk_tokens
+        if not lens or n > self.scan_cut_entries:
+            return chunk
+        few = n_tokens * inner <= self.scan_few_work
+        if max(lens) > (chunk // 2 if few else chunk):
+            chunk = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
+        return chunk
+
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
     recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
     # The matrix memory's chunks run side by side from this many tokens on at heads of 128 and more, from twice as many at

@@ -353,10 +353,12 @@ def test_long_portions_take_the_forms_that_work_on_chunks(tmp_path, which, index
     cfg = single_layer(which, index)
     core, cfg, w = build(tmp_path, cfg, dtype, seed=7, pages=64, block=16)
     o = ops()
-    keep = o.scan_chunk_tokens
+    keep, plan, chunks = (o.scan_chunk_tokens, o.scan_cut_tokens, o.scan_few_work), o._chunk_plan, set()
     try:
-        if chunk:
-            o.scan_chunk_tokens = chunk
+        if chunk:       # (chunks of that many tokens, however few the step's are)
+            o.scan_chunk_tokens = o.scan_cut_tokens = chunk
+            o.scan_few_work = 0
+        o._chunk_plan = lambda batch, n: (chunks.add(n), plan(batch, n))[1]
         V = cfg["vocab"]
         a, b = tokens(700, V, 5), tokens(60, V, 6)
         steps = [[("a", 301), ("b", 3)], [("a", 1), ("b", 1)], [("b", 40), ("a", 333)], [("a", 1)], [("a", 60), ("b", 16)]] + \
@@ -364,8 +366,10 @@ def test_long_portions_take_the_forms_that_work_on_chunks(tmp_path, which, index
         got = replay(core.executor, StepEntry, {"a": a, "b": b}, steps)
         for k, t in (("a", a), ("b", b)):
             check(got[k], plain_logits(cfg, w, t), dtype, k, (cfg, w, t))
+        assert chunks == ({chunk} if chunk else set())
     finally:
-        o.scan_chunk_tokens = keep
+        o.scan_chunk_tokens, o.scan_cut_tokens, o.scan_few_work = keep
+        del o._chunk_plan
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

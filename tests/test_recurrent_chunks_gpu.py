@@ -111,20 +111,26 @@ def test_matrix_memory_keeps_a_value_from_earlier_tokens(token, column, value, d
 
 
 # one piece and cuts of 16 and of 32 tokens, pieces of fewer than 8, states that the kernel's number of entries is and is not,
-# channels that end inside a workgroup
+# channels that end inside a workgroup; whole segments of more tokens than lie in LDS at a time; states of more entries than a
+# lane holds, whose chunks keep 64 tokens, and several tiles (of 16 and of 8 tokens) in a chunk of 32
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("inner,n,lens,few", [(256, 16, (32,), None), (300, 16, (65, 7, 1), None), (260, 5, (97, 130), None),
-                                              (512, 32, (33,), 0), (256, 4, (200, 33), 0), (256, 16, (129, 64), 0), (302, 8, (70,), 0)])
-def test_selective_scan_in_pieces(inner, n, lens, few, dtype):
+@pytest.mark.parametrize("inner,n,lens,sizes,chunk", [
+    (256, 16, (32,), {}, 64), (300, 16, (65, 7, 1), {}, 16), (260, 5, (97, 130), {}, 16), (512, 32, (33,), {"few_work": 0}, 64),
+    (256, 4, (200, 33), {"few_work": 0}, 32), (256, 16, (129, 64), {"few_work": 0}, 32), (302, 8, (70,), {"few_work": 0}, 32),
+    (300, 16, (65, 128, 129, 200), {"chunk_tokens": 256, "cut_tokens": 256, "few_work": 0}, 256),
+    (48, 33, (65, 33), {}, 64), (40, 72, (150, 31, 1), {"chunk_tokens": 32}, 32), (24, 200, (33, 100), {"chunk_tokens": 32}, 32)])
+def test_selective_scan_in_pieces(inner, n, lens, sizes, chunk, dtype):
     o, g = ops(), torch.Generator().manual_seed(inner + n)
-    if few is not None:
-        o.scan_few_work = few
+    for name, value in sizes.items():
+        setattr(o, "scan_" + name, value)
     N = sum(lens)
     x, z, bc = (torch.randn(N, c, generator=g).to(dtype) for c in (inner, inner, 2 * n))
     dt, al, D = torch.randn(N, inner, generator=g) * 3 - 1, torch.randn(inner, n, generator=g), torch.randn(inner, generator=g)
     st0 = torch.randn(len(lens), inner * n, generator=g)
     st = st0.cuda()
-    y = o.selective_scan(x.cuda(), dt.cuda(), bc.cuda(), 0, n, z.cuda(), al.cuda(), D.cuda(), st, batch(lens))
+    b = batch(lens)
+    y = o.selective_scan(x.cuda(), dt.cuda(), bc.cuda(), 0, n, z.cuda(), al.cuda(), D.cuda(), st, b)
+    assert list(b.aux) == [("chunk_plan", chunk)]
     S = st0.double().view(len(lens), inner, n)
     X, Z, B, C = x.double(), z.double(), bc.double()[:, :n], bc.double()[:, n:]
     sp, A, ref, at = torch.nn.functional.softplus(dt.double(), threshold=50), -torch.exp(al.double()), [], 0
