@@ -1572,7 +1572,9 @@ class HipOps:
             return chunk
         few = n_tokens * inner <= self.scan_few_work
         if max(lens) > (chunk // 2 if few else chunk):
-            chunk = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
+            cut = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
+            if -(-max(lens) // cut) <= 65535:      # the launch's limit; a longer segment keeps the longer chunks
+                return cut
         return chunk
 
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form

@@ -141,3 +141,13 @@ def test_decode_attention_splits(lib):
     assert split(8, 100000) > split(8, 30000)         # long contexts: more workgroups than the chip holds at once
     t.decode_attention_splits = 2
     assert split(8, 8000) == 2
+
+
+@pytest.mark.parametrize("lens,inner,n,chunk", [
+    ((64,) * 8, 4096, 16, 64), ((64,), 4096, 16, 16), ((33,), 1024, 16, 16), ((32,), 1024, 16, 64), ((1, 512), 4096, 16, 32),
+    ((64, 512), 4096, 33, 64), ((65,), 64, 256, 64), ((), 64, 16, 64),
+    # (no more chunks than a launch takes: segments beyond that keep the longer ones)
+    ((16 * 65535,), 1, 16, 16), ((16 * 65535 + 1,), 1, 16, 64), ((32 * 65535,), 64, 16, 32), ((3, 32 * 65535 + 1), 64, 16, 64)])
+def test_chunks_of_the_selective_scan(lens, inner, n, chunk):
+    from lmsf_amd.ops.hip_ops import HipOps
+    assert HipOps.__new__(HipOps)._scan_chunk(lens, sum(lens), inner, n) == chunk
