@@ -790,8 +790,8 @@ extern "C" long lmsf_mlstm_state_floats(int H, int d, int dv) {
 // column, by the first block); chunks one after the other, a thread an entry of each product.
 #define MLC_THREADS 1024
 
-// A segment's chunks one after the other in one workgroup, the state from the slot and back to it. Steps with segments of 32
-// and more tokens run the chunks side by side instead, in three launches:
+// A segment's chunks one after the other in one workgroup, the state from the slot and back to it. Steps with longer
+// segments (from 32 tokens on at heads of 256, from 96 at heads below 64) run the chunks side by side instead, in three launches:
 // summaries: every chunk leaves U = K^T (w [V | 1]) with w_u = exp(g_u - G), G = max_u g_u, and (F_last, G) in scratch;
 // mlstm_fold_kernel turns them, chunk after chunk, into every chunk's S_0 (in U's place) and m_0 and writes the slot's S;
 // outputs: every chunk computes its outputs from its S_0 and m_0 (and the last one writes the slot's m).

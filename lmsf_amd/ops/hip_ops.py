@@ -1579,11 +1579,19 @@ class HipOps:
 
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
     recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
-    # The matrix memory's chunks run side by side from this many tokens on at heads of 128 and more, from twice as many at
-    # smaller ones. One workgroup a head and 32 columns against side by side, bfloat16: 8 heads of 128, one segment of 24 / 32 /
-    # 48 tokens 26 / 31 / 44 against 29 / 29 / 33 us, 8 of them 28 / 33 / 47 against 36 / 35 / 39, of 100 tokens 84 against 37;
-    # heads of 256 at 24 / 32 tokens 44 / 53 against 40 / 40; heads of 64 at 48 / 100 tokens 28 / 51 against 27 / 30.
+    # The matrix memory's chunks run side by side where the step's longest segment has this many tokens at heads of 256 and
+    # more, 1.5 times as many from 128 on, twice from 64 on and three times below. The rule is for the whole step: a single token then has
+    # a chunk of its own, whose memory goes through scratch, where the other form (a workgroup a head and 32 columns) is held up
+    # by its longest segment. Side by side over the other form, bfloat16, states not in cache, 1 / 4 / 8 / 16 segments of that many tokens and
+    # the most of them beside 8 or 24 single tokens: 8 heads of 128, 32 tokens 0.97 / 1.00 / 1.06 / 0.74 and 1.13, 48 tokens 0.77 / 0.81 /
+    # 0.85 / 0.59 and 0.89; 4 heads of 256, 24 tokens 0.93 / 1.02 / 1.10 / 0.79 and 1.17, 32 tokens 0.77 / 0.85 / 0.92 / 0.66 and 0.99;
+    # 16 heads of 64, 48 tokens 1.01 / 1.03 / 1.05 / 0.72 and 1.12, 64 tokens 0.85 / 0.86 / 0.89 / 0.61 and 1.00; 16 heads of 32, 64
+    # tokens 1.08 / 1.09 / 1.08 / 1.09 and 1.17, 100 tokens 0.81 / 0.81 / 0.82 / 0.88 and 1.04. With 256 single tokens beside one
+    # portion of 48 to 300 tokens 0.66 to 0.83 (8 heads of 128) and 0.66 to 0.90 (4 of 256).
     matrix_memory_parallel_min_tokens = 32
+
+    def _memory_side_by_side(self, lens, dim: int) -> bool:
+        return max(lens) >= self.matrix_memory_parallel_min_tokens * (1 if dim >= 256 else 1.5 if dim >= 128 else 2 if dim >= 64 else 3)
 
     def _chunk_plan(self, batch, chunk: int):
         """(per segment its first entry of scratch or -1, entries in all, the most chunks of a segment) for a step
@@ -1691,7 +1699,7 @@ class HipOps:
             L = self.lib.lmsf_mlstm_chunk_tokens(int(dim))
             bases = entries = None
             n_entries, most = 0, 1
-            if L > 0 and max(lens) >= self.matrix_memory_parallel_min_tokens * (1 if dim >= 128 else 2):
+            if L > 0 and self._memory_side_by_side(lens, dim):
                 key = ("mlstm_chunks", L)
                 plan = batch.aux.get(key)
                 if plan is None:

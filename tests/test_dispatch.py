@@ -151,3 +151,12 @@ def test_decode_attention_splits(lib):
 def test_chunks_of_the_selective_scan(lens, inner, n, chunk):
     from lmsf_amd.ops.hip_ops import HipOps
     assert HipOps.__new__(HipOps)._scan_chunk(lens, sum(lens), inner, n) == chunk
+
+
+@pytest.mark.parametrize("dim,tokens", [(512, 32), (256, 32), (255, 48), (128, 48), (127, 64), (64, 64), (63, 96), (16, 96)])
+def test_the_matrix_memory_goes_side_by_side(dim, tokens):
+    """Where every mix of segments that was measured is no slower for it."""
+    from lmsf_amd.ops.hip_ops import HipOps
+    o = HipOps.__new__(HipOps)
+    for beside in ([], [1] * 64, [tokens - 1] * 8):
+        assert not o._memory_side_by_side([tokens - 1] + beside, dim) and o._memory_side_by_side(beside + [tokens], dim)
