@@ -720,14 +720,23 @@ __global__ __launch_bounds__(256) void selective_scan_step_kernel(
   for (int n = 0; n < NS; n += 4) *reinterpret_cast<float4*>(st + n) = make_float4(S[n], S[n + 1], S[n + 2], S[n + 3]);
 }
 
-// 1 where lmsf_selective_scan_step takes these sizes, strides (in elements) and addresses; the scan with its product beside
-// it serves the rest.
-extern "C" int lmsf_selective_scan_step_fits(int n_tokens, int inner, int nstate, int rank, int b_at, int c_at, long low_stride,
-                                             long ldw, long state_stride, const void* low, const void* W, const void* state,
-                                             const void* A_log) {
+static bool scan_step_takes(int n_tokens, int inner, int nstate, int rank, int b_at, int c_at, long low_stride, long ldw,
+                            long state_stride, const void* low, const void* W, const void* state, const void* A_log) {
   return n_tokens > 0 && inner > 0 && inner % SCAN_STEP_CH == 0 && (nstate == 8 || nstate == 16 || nstate == 32) && rank > 0 &&
          rank % 32 == 0 && b_at >= 0 && c_at >= 0 && b_at % 8 == 0 && c_at % 8 == 0 && low_stride % 8 == 0 && ldw % 8 == 0 &&
          state_stride % 4 == 0 && lmsf_aligned16(low) && lmsf_aligned16(W) && lmsf_aligned16(state) && lmsf_aligned16(A_log);
+}
+
+// 1 where a step of these sizes, strides (in elements) and addresses is lmsf_selective_scan_step's; the scan with its product
+// beside it serves the rest. Up to 2^27 multiplications of the product, which every 8 tokens read W for again. Step against product
+// and scan, 16 entries, states not in cache: 4,096 channels, rank 128, 8 / 64 / 256 / 512 tokens 5.5 / 14.0 / 48.5 / 89.4 against 8.3 / 18.5
+// / 54.0 / 90.8 us; 8,192 channels, rank 256, 64 (2^27) / 96 / 256 / 512 tokens 29.9 / 42.3 / 101 / 199 against 31.7 / 41.9 / 92 / 170;
+// 16,384 channels, rank 512, 16 (2^27) / 32 / 128 tokens 18.6 / 35.8 / 123 against 19.4 / 32.2 / 87.
+extern "C" int lmsf_selective_scan_step_fits(int n_tokens, int inner, int nstate, int rank, int b_at, int c_at, long low_stride,
+                                             long ldw, long state_stride, const void* low, const void* W, const void* state,
+                                             const void* A_log) {
+  return scan_step_takes(n_tokens, inner, nstate, rank, b_at, c_at, low_stride, ldw, state_stride, low, W, state, A_log) &&
+         (double)n_tokens * inner * rank <= 134217728.0;
 }
 
 // A step of single tokens (token i is segment i): x, z, y [n_tokens, inner], low [n_tokens, >= rank + ...] with B and C at
@@ -739,8 +748,7 @@ extern "C" int lmsf_selective_scan_step(const void* x, long x_stride, const void
                                         const int* state_slots, void* y, long y_stride, int n_tokens, int inner, int nstate,
                                         hipStream_t stream) {
   LMSF_CHECK(x && low && W && z && A_log && Dw && state && state_slots && y, "selective_scan_step: null pointer");
-  LMSF_CHECK(lmsf_selective_scan_step_fits(n_tokens, inner, nstate, rank, b_at, c_at, low_stride, ldw, state_stride, low, W, state,
-                                           A_log),
+  LMSF_CHECK(scan_step_takes(n_tokens, inner, nstate, rank, b_at, c_at, low_stride, ldw, state_stride, low, W, state, A_log),
              "selective_scan_step: sizes that the scan and its product take one after the other");
   LMSF_CHECK(x_stride >= inner && z_stride >= inner && y_stride >= inner && ldw >= rank && low_stride >= rank &&
                  low_stride >= b_at + nstate && low_stride >= c_at + nstate && state_stride >= (long)inner * nstate,

@@ -160,3 +160,11 @@ def test_the_matrix_memory_goes_side_by_side(dim, tokens):
     o = HipOps.__new__(HipOps)
     for beside in ([], [1] * 64, [tokens - 1] * 8):
         assert not o._memory_side_by_side([tokens - 1] + beside, dim) and o._memory_side_by_side(beside + [tokens], dim)
+
+
+@pytest.mark.parametrize("inner,rank,most", [(4096, 128, 256), (8192, 256, 64), (16384, 512, 16), (1024, 64, 2048)])
+def test_scans_of_single_tokens_with_the_product_inside_end(lib, inner, rank, most):
+    """Every 8 tokens read the product's matrix again: beyond 2^27 multiplications the product is a kernel of its own."""
+    fits = lambda n: lib.lmsf_selective_scan_step_fits(n, inner, 16, rank, rank, rank + 16, rank + 32, rank, inner * 16, 256, 256,   # noqa: E731
+                                                       256, 256)
+    assert [fits(n) for n in (1, most, most + 1, 65535)] == [1, 1, 0, 0]
