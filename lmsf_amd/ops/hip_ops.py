@@ -1724,6 +1724,16 @@ class HipOps:
             self._stream()))
         return out
 
+    @staticmethod
+    def _memory_step(n_tokens: int, heads: int, dim: int, vdim: int) -> bool:
+        """Whether a step of single tokens makes its gates itself: at heads of 128 entries and more at any number of tokens; below,
+        where a workgroup's eight waves find little to read and its gates are much of it, up to 4,096 workgroups (a token, a head, 64 columns),
+        below 64 entries up to 1,536. Step against product and memory, bfloat16, states not in cache: 8 heads of 128, K 2,048, 8 / 64 /
+        512 tokens 11.6 / 32.2 / 177 against 17.6 / 36.8 / 195 us; 4 heads of 256, K 1,024, 16.1 / 50.3 / 331 against 25.4 / 50.0 / 357;
+        16 heads of 64, K 2,048, 256 tokens (4,096 workgroups) / 384 / 512 56.8 / 82.0 / 105 against 63.5 / 79.7 / 96.5; 16 heads of 32,
+        K 1,024, 48 tokens (1,536) / 64 / 256 19.5 / 24.0 / 84 against 21.8 / 23.4 / 61."""
+        return dim >= 128 or n_tokens * heads * -(-vdim // 64) <= (4096 if dim >= 64 else 1536)
+
     def mlstm_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, x: torch.Tensor, gate_weight: torch.Tensor,
                    gate_bias: Optional[torch.Tensor], out_gate: torch.Tensor, norm_weight: torch.Tensor, state: torch.Tensor,
                    batch, heads: int, dim: int, vdim: int, q_scale: float, gate_cap: float,
@@ -1735,7 +1745,7 @@ class HipOps:
         ok = all(t.dtype == x.dtype and t.dim() == 2 and t.stride(1) == 1 for t in (q, k, v, x, gate_weight, out_gate)) \
             and tuple(gate_weight.shape) == (2 * heads, K) and K % vec == 0 and x.stride(0) % vec == 0 \
             and gate_weight.stride(0) % vec == 0 and x.data_ptr() % 16 == 0 and gate_weight.data_ptr() % 16 == 0 \
-            and q.stride(0) == k.stride(0) == v.stride(0) and 0 < N <= 65535 and dim <= 4096 \
+            and q.stride(0) == k.stride(0) == v.stride(0) and 0 < N <= 65535 and dim <= 4096 and self._memory_step(N, heads, dim, vdim) \
             and all(t.shape[0] == N and t.shape[1] >= w for t, w in ((q, heads * dim), (k, heads * dim), (v, heads * vdim),
                                                                      (out_gate, heads * vdim))) \
             and (gate_bias is None or (gate_bias.dtype == x.dtype and gate_bias.shape == (2 * heads,) and gate_bias.is_contiguous()))

@@ -168,3 +168,10 @@ def test_scans_of_single_tokens_with_the_product_inside_end(lib, inner, rank, mo
     fits = lambda n: lib.lmsf_selective_scan_step_fits(n, inner, 16, rank, rank, rank + 16, rank + 32, rank, inner * 16, 256, 256,   # noqa: E731
                                                        256, 256)
     assert [fits(n) for n in (1, most, most + 1, 65535)] == [1, 1, 0, 0]
+
+
+@pytest.mark.parametrize("heads,dim,vdim,most", [(8, 128, 128, 65535), (4, 512, 64, 65535), (16, 64, 64, 256), (32, 127, 65, 64),
+                                                 (32, 32, 32, 48), (16, 63, 64, 96)])
+def test_the_matrix_memory_of_single_tokens_makes_its_gates_up_to(heads, dim, vdim, most):
+    from lmsf_amd.ops.hip_ops import HipOps
+    assert [HipOps._memory_step(n, heads, dim, vdim) for n in (1, most, most + 1)] == [True, True, dim >= 128]
