@@ -91,6 +91,17 @@ __global__ __launch_bounds__(256) void dyt_norm_rows_kernel(const TB* __restrict
   }
 }
 
+// 1 where n_rows rows of H columns are the kernel's of R rows a thread (where every piece is aligned): more than a workgroup a
+// compute unit (fewer: level, both wait for one trip to memory), and 512 columns, or 8,000 rows: fewer columns leave a
+// workgroup's waves idle, and a wave with four rows to itself is slower than four waves until the chip is full. One row a thread against four: 1,030
+// rows of 64 / 256 / 384 / 512 columns 3.2 / 3.6 / 4.2 / 5.0 against 4.5 / 4.1 / 4.5 / 4.9 us, 2,048 rows of 64 / 256 / 384 3.7 / 4.6 / 5.9
+// against 5.2 / 4.9 / 5.4, 8,000 rows of 8 / 64 / 256 6.9 / 6.9 / 11.7 against 5.2 / 5.1 / 7.6.
+#define DYT_ROWS_A_THREAD 4
+extern "C" int lmsf_dyt_norm_many(int n_rows, int H) {
+  const int R = DYT_ROWS_A_THREAD;
+  return H % 4 == 0 && (H >= 512 || n_rows >= 8000) && (long)((n_rows + R - 1) / R) * ((H / 4 + 255) / 256) > 256;
+}
+
 extern "C" int lmsf_dyt_norm(const void* branch, int branch_dtype, float* residual, const float* w, const float* b,
                              const float* alpha, void* out, int out_dtype, const int* rows, int n_rows, int H,
                              hipStream_t stream) {
@@ -103,11 +114,9 @@ extern "C" int lmsf_dyt_norm(const void* branch, int branch_dtype, float* residu
   const bool v4 = H % 4 == 0;
   const int per = v4 ? 4 : 1;
   dim3 grid(n_rows, (H / per + 255) / 256), block(256);
-  // R rows a thread where that leaves more than a workgroup a compute unit (fewer: level, both wait for one trip to memory),
-  // and every piece is aligned.
-  constexpr int R = 4;
-  const bool many = v4 && (long)((n_rows + R - 1) / R) * ((H / 4 + 255) / 256) > 256 && lmsf_aligned16(residual) &&
-                    lmsf_aligned16(w) && lmsf_aligned16(b) && lmsf_aligned16(branch) && lmsf_aligned16(out);
+  constexpr int R = DYT_ROWS_A_THREAD;
+  const bool many = lmsf_dyt_norm_many(n_rows, H) && lmsf_aligned16(residual) && lmsf_aligned16(w) && lmsf_aligned16(b) &&
+                    lmsf_aligned16(branch) && lmsf_aligned16(out);
   if (many) {
     grid.x = (n_rows + R - 1) / R;
 #define DYT_ROWS(TB, TO)                                                                                               \

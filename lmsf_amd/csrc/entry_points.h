@@ -130,6 +130,7 @@ int lmsf_rms_pair(const void* a, long a_stride, const void* b, long b_stride, in
     wb, void* out, int n_rows, int W, float eps, float scale, hipStream_t stream);
 
 // dyt_norm.hip
+int lmsf_dyt_norm_many(int n_rows, int H);
 int lmsf_dyt_norm(const void* branch, int branch_dtype, float* residual, const float* w, const float* b, const float*
     alpha, void* out, int out_dtype, const int* rows, int n_rows, int H, hipStream_t stream);
 

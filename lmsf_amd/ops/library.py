@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 41      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
+ABI_VERSION = 42      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None
@@ -112,6 +112,7 @@ _SIGNATURES = {
     "lmsf_logit_cap": (c_int, [_P, c_long, c_int, c_int, c_float, c_float, _P]),
     "lmsf_table_moe_scratch_ints": (c_long, [c_int, c_int, c_int]),
     "lmsf_table_moe_grouped": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_long]),
+    "lmsf_dyt_norm_many": (c_int, [c_int, c_int]),
     "lmsf_dyt_norm": (c_int, [_P, c_int, _P, _P, _P, _P, _P, c_int, _P, c_int, c_int, _P]),
     "lmsf_short_conv": (c_int, [_P, c_int, c_long, _P, _P, c_int, _P, c_long, _P, _P, _P, _P, c_long, c_int, c_int, c_int,
                                 c_int, c_int, _P]),

@@ -175,3 +175,10 @@ def test_scans_of_single_tokens_with_the_product_inside_end(lib, inner, rank, mo
 def test_the_matrix_memory_of_single_tokens_makes_its_gates_up_to(heads, dim, vdim, most):
     from lmsf_amd.ops.hip_ops import HipOps
     assert [HipOps._memory_step(n, heads, dim, vdim) for n in (1, most, most + 1)] == [True, True, dim >= 128]
+
+
+@pytest.mark.parametrize("H,rows", [(512, 1025), (1024, 1025), (1028, 513), (2048, 513), (2052, 341), (508, 8000), (8, 8000), (64, 8000)])
+def test_dynamic_tanh_takes_four_rows_a_thread_from(lib, H, rows):
+    """Where the chip is full of wide workgroups: narrow rows only once there are very many."""
+    assert [lib.lmsf_dyt_norm_many(n, H) for n in (1, rows - 1, rows, rows + 1)] == [0, 0, 1, 1]
+    assert not lib.lmsf_dyt_norm_many(100000, H + 2)

@@ -101,9 +101,9 @@ def test_dynamic_tanh_with_and_without_the_addition(dtype, H):
 
 @pytest.mark.parametrize("branch_dtype", DTYPES)
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("N,H", [(1021, 1028), (1024, 2048), (1027, 52), (1028, 52), (1029, 52)])
+@pytest.mark.parametrize("N,H", [(1021, 1028), (1024, 2048), (1027, 52), (1028, 52), (1029, 52), (8001, 52), (1025, 512)])
 def test_dynamic_tanh_of_many_rows_is_that_of_few(N, H, dtype, branch_dtype):
-    """Above 1,024 rows (512 of more than 1,024 columns) a thread takes four rows. The same rows a few at a time, which the
+    """Above 1,024 rows (512 of more than 1,024 columns; 7,999 of fewer than 512) a thread takes four rows. The same rows a few at a time, which the
     other kernel takes, give the same bits."""
     o = ops()
     g = torch.Generator().manual_seed(N + H)
