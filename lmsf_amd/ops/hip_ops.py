@@ -1730,14 +1730,23 @@ class HipOps:
         return out
 
     @staticmethod
-    def _memory_step(n_tokens: int, heads: int, dim: int, vdim: int) -> bool:
-        """Whether a step of single tokens makes its gates itself: at heads of 128 entries and more at any number of tokens; below,
-        where a workgroup's eight waves find little to read and its gates are much of it, up to 4,096 workgroups (a token, a head, 64 columns),
-        below 64 entries up to 1,536. Step against product and memory, bfloat16, states not in cache: 8 heads of 128, K 2,048, 8 / 64 /
-        512 tokens 11.6 / 32.2 / 177 against 17.6 / 36.8 / 195 us; 4 heads of 256, K 1,024, 16.1 / 50.3 / 331 against 25.4 / 50.0 / 357;
-        16 heads of 64, K 2,048, 256 tokens (4,096 workgroups) / 384 / 512 56.8 / 82.0 / 105 against 63.5 / 79.7 / 96.5; 16 heads of 32,
-        K 1,024, 48 tokens (1,536) / 64 / 256 19.5 / 24.0 / 84 against 21.8 / 23.4 / 61."""
-        return dim >= 128 or n_tokens * heads * -(-vdim // 64) <= (4096 if dim >= 64 else 1536)
+    def _memory_step(n_tokens: int, heads: int, dim: int, vdim: int, size: int) -> bool:
+        """Whether a step of single tokens of ``size`` bytes an entry makes its gates itself, by the workgroups (a token, a head,
+        64 columns) it takes. At heads of 128 entries and more it does, but with float32, whose product beside it is quicker, just
+        beyond 1,024, where the chip holds all but a few at once; below, where a workgroup's eight waves find little to read and its gates
+        are much of it, up to 4,096 (float32 2,048), below 64 entries up to 1,536 (float32, and below 32 entries, 512). Step against
+        product and memory, states not in cache, bfloat16: 8 heads of 128, K 2,048, 8 / 64 / 512 tokens 10.8 / 30 / 179 against 17.0 / 37 /
+        198 us; 4 heads of 256, K 1,024, 17 / 51 / 160 (256 tokens) against 28 / 53 / 188; 16 heads of 64, K 1,024, 4,096 / 6,144 / 8,192
+        55 / 79 / 103 against 60 / 75 / 93; 16 heads of 32, K 512, 2,048 / 3,072 24.4 / 33.6 against 26.4 / 32.6; 4 of 16, 512 / 768 8.5 /
+        12.2 against 12.4 / 11.1. float32: 4 heads of 256 at 1,024 / 1,152 / 1,280 49 / 57 / 60 against 50 / 55 / 58, 4 of 160 at 1,008 / 1,248 /
+        1,344 34 / 41 / 43 against 33 / 37 / 43; 16 of 64 at 2,048 / 3,072 31.5 / 42.9 against 32.3 / 42.3; 16 of 32 at 512 / 1,024
+        9.2 / 13.6 against 11.7 / 13.0."""
+        groups = n_tokens * heads * -(-vdim // 64)
+        if dim >= 128:
+            return size == 2 or not 1024 < groups <= 1280
+        if dim >= 64:
+            return groups <= 8192 // size
+        return groups <= (1536 if dim >= 32 and size == 2 else 512)
 
     def mlstm_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, x: torch.Tensor, gate_weight: torch.Tensor,
                    gate_bias: Optional[torch.Tensor], out_gate: torch.Tensor, norm_weight: torch.Tensor, state: torch.Tensor,
@@ -1750,7 +1759,7 @@ class HipOps:
         ok = all(t.dtype == x.dtype and t.dim() == 2 and t.stride(1) == 1 for t in (q, k, v, x, gate_weight, out_gate)) \
             and tuple(gate_weight.shape) == (2 * heads, K) and K % vec == 0 and x.stride(0) % vec == 0 \
             and gate_weight.stride(0) % vec == 0 and x.data_ptr() % 16 == 0 and gate_weight.data_ptr() % 16 == 0 \
-            and q.stride(0) == k.stride(0) == v.stride(0) and 0 < N <= 65535 and dim <= 4096 and self._memory_step(N, heads, dim, vdim) \
+            and q.stride(0) == k.stride(0) == v.stride(0) and 0 < N <= 65535 and dim <= 4096 and self._memory_step(N, heads, dim, vdim, x.element_size()) \
             and all(t.shape[0] == N and t.shape[1] >= w for t, w in ((q, heads * dim), (k, heads * dim), (v, heads * vdim),
                                                                      (out_gate, heads * vdim))) \
             and (gate_bias is None or (gate_bias.dtype == x.dtype and gate_bias.shape == (2 * heads,) and gate_bias.is_contiguous()))

@@ -174,11 +174,14 @@ def test_scans_of_single_tokens_with_the_product_inside_end(lib, inner, rank, mo
     assert [fits(n) for n in (1, most, most + 1, 65535)] == [1, 1, 0, 0]
 
 
-@pytest.mark.parametrize("heads,dim,vdim,most", [(8, 128, 128, 65535), (4, 512, 64, 65535), (16, 64, 64, 256), (32, 127, 65, 64),
-                                                 (32, 32, 32, 48), (16, 63, 64, 96)])
-def test_the_matrix_memory_of_single_tokens_makes_its_gates_up_to(heads, dim, vdim, most):
+@pytest.mark.parametrize("heads,dim,vdim,size,most", [
+    (4, 512, 64, 2, 65535), (16, 64, 64, 2, 256), (32, 127, 65, 2, 64), (32, 32, 32, 2, 48), (16, 63, 64, 2, 96), (4, 16, 16, 2, 128),
+    (16, 64, 64, 4, 128), (16, 63, 64, 4, 32), (4, 16, 16, 4, 128)])
+def test_the_matrix_memory_of_single_tokens_makes_its_gates_up_to(heads, dim, vdim, size, most):
     from lmsf_amd.ops.hip_ops import HipOps
-    assert [HipOps._memory_step(n, heads, dim, vdim) for n in (1, most, most + 1)] == [True, True, dim >= 128]
+    assert [HipOps._memory_step(n, heads, dim, vdim, size) for n in (1, most, most + 1)] == [True, True, dim >= 128]
+    # (wide heads: in float32 all but just beyond what the chip holds at once)
+    assert [HipOps._memory_step(n, 8, 128, 128, size) for n in (64, 65, 80, 81, 4096)] == [True, size == 2, size == 2, True, True]
 
 
 @pytest.mark.parametrize("H,rows", [(512, 1025), (1024, 1025), (1028, 513), (2048, 513), (2052, 341), (508, 8000), (8, 8000), (64, 8000)])
