@@ -1051,10 +1051,18 @@ __global__ __launch_bounds__(MLX_THREADS) void mlstm_chunk_mfma_kernel(
         }
       }
     } else {
-      for (int i = tid; i < L16 * width; i += MLX_THREADS) {
-        const int tt = i / width, dd = i - tt * width;
-        dst[tt * pitch + dd] = tt < nt && dd < have ? src[(long)(t0 + tt) * qkv_stride + dd] : T(0);
-      }
+      // (a row a wave, four of its rows asked for at a time)
+      for (int tt = w; tt < L16; tt += 4 * MLX_THREADS / LMSF_WAVE)
+        for (int dd = l; dd < width; dd += LMSF_WAVE) {
+          T x[4];
+#pragma unroll
+          for (int n = 0; n < 4; ++n) {
+            const int t = tt + n * MLX_THREADS / LMSF_WAVE;
+            x[n] = t < nt && dd < have ? src[(long)(t0 + t) * qkv_stride + dd] : T(0);
+          }
+#pragma unroll
+          for (int n = 0; n < 4; ++n) dst[(tt + n * MLX_THREADS / LMSF_WAVE) * pitch + dd] = x[n];
+        }
     }
   };
   stage(k + (long)h * d, sk, dp, d16, d);
