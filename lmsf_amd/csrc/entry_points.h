@@ -157,6 +157,7 @@ int lmsf_mlstm_step(const void* q, const void* k, const void* v, int dtype, long
 long lmsf_mlstm_state_floats(int H, int d, int dv);
 long lmsf_mlstm_chunk_scratch_floats(int n_tokens, int H, int dv);
 int lmsf_mlstm_chunk_tokens(int d);
+int lmsf_mlstm_side_tokens(int d);
 long lmsf_mlstm_chunk_entry_floats(int H, int d, int dv);
 int lmsf_mlstm_chunked(const void* q, const void* k, const void* v, int dtype, long qkv_stride, const float* gates,
     long gates_stride, const void* og, long og_stride, const float* norm_w, float* state, long state_stride, const

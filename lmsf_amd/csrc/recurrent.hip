@@ -799,7 +799,7 @@ extern "C" long lmsf_mlstm_state_floats(int H, int d, int dv) {
 #define MLC_THREADS 1024
 
 // A segment's chunks one after the other in one workgroup, the state from the slot and back to it. Steps with longer
-// segments (from 32 tokens on at heads of 256, from 96 at heads below 64) run the chunks side by side instead, in three launches:
+// segments (from 32 tokens on at heads of 256, from 192 at the latest) run the chunks side by side instead, in three launches:
 // summaries: every chunk leaves U = K^T (w [V | 1]) with w_u = exp(g_u - G), G = max_u g_u, and (F_last, G) in scratch;
 // mlstm_fold_kernel turns them, chunk after chunk, into every chunk's S_0 (in U's place) and m_0 and writes the slot's S;
 // outputs: every chunk computes its outputs from its S_0 and m_0 (and the last one writes the slot's m).
@@ -1497,12 +1497,19 @@ extern "C" int lmsf_mlstm_chunk_tokens(int d) {
   return 0;
 }
 
+// and where the chunks run side by side (0: they do not): at least a tile of the matrix instruction, of which 8 and 4 tokens (heads
+// of 483 and more) would fill a half and a quarter
+extern "C" int lmsf_mlstm_side_tokens(int d) {
+  const int L = lmsf_mlstm_chunk_tokens(d);
+  return L > 0 && L < 16 ? 16 : L;
+}
+
 // floats of scratch a chunk of the side-by-side form takes: U as [H, d, dv + 1], (F_last, G) and m_0 per head
 extern "C" long lmsf_mlstm_chunk_entry_floats(int H, int d, int dv) { return (long)H * d * (dv + 1) + 3L * H; }
 
 // ``chunk_base`` null: every segment's chunks one after the other in a workgroup. Otherwise (steps with long
 // segments) chunk_base[s] is segment s's first entry of ``entries`` (``n_entries`` of them, each
-// lmsf_mlstm_chunk_entry_floats), a segment having ceil(tokens / lmsf_mlstm_chunk_tokens(d)) chunks and the longest
+// lmsf_mlstm_chunk_entry_floats), a segment having ceil(tokens / lmsf_mlstm_side_tokens(d)) chunks and the longest
 // ``max_chunks``; the chunks then run side by side.
 extern "C" int lmsf_mlstm_chunked(const void* q, const void* k, const void* v, int dtype, long qkv_stride,
                                   const float* gates, long gates_stride, const void* og, long og_stride,
@@ -1556,25 +1563,25 @@ extern "C" int lmsf_mlstm_chunked(const void* q, const void* k, const void* v, i
     if (dtype == LMSF_F32) MLC_LAUNCH(float); else MLC_LAUNCH(bf16_t);
     LMSF_LAUNCH_CHECK("mlstm_chunk");
   } else {
-    const int m_vb = (dv + MLX_COLS - 1) / MLX_COLS;
+    const int m_vb = (dv + MLX_COLS - 1) / MLX_COLS, LS = lmsf_mlstm_side_tokens(d);
     dim3 grid(H, n_segments, m_vb * max_chunks);
     const int vw = dtype == LMSF_F32 ? 4 : 8;
     const int vec = d % vw == 0 && dv % vw == 0 && qkv_stride % vw == 0 && lmsf_aligned16(q) && lmsf_aligned16(k) &&
                     lmsf_aligned16(v);
 #define MLX_LAUNCH(T, SUM)                                                                                            \
   do {                                                                                                               \
-    const size_t lds = mlx_lds<T>(L, d, SUM);                                                                        \
+    const size_t lds = mlx_lds<T>(LS, d, SUM);                                                                       \
     MLS_RESERVE((mlstm_chunk_mfma_kernel<T, SUM>), lds);                                                             \
     hipLaunchKernelGGL((mlstm_chunk_mfma_kernel<T, SUM>), grid, dim3(MLX_THREADS), lds, stream, (const T*)q,         \
                        (const T*)k, (const T*)v, qkv_stride, gates, gates_stride, state, state_stride, seg_starts,   \
-                       state_slots, o_raw, (long)H * dv, H, d, dv, L, qscale, cap, m_vb, chunk_base, sc_U, sc_fg,    \
+                       state_slots, o_raw, (long)H * dv, H, d, dv, LS, qscale, cap, m_vb, chunk_base, sc_U, sc_fg,   \
                        sc_m0, den, vec);                                                                             \
   } while (0)
     if (dtype == LMSF_F32) MLX_LAUNCH(float, true); else MLX_LAUNCH(bf16_t, true);
     LMSF_LAUNCH_CHECK("mlstm_chunk (summaries)");
     const long per = (long)d * (dv + 1);
     hipLaunchKernelGGL(mlstm_fold_kernel, dim3(H, n_segments, (unsigned)((per + 255) / 256)), dim3(256), 0, stream, state,
-                       state_stride, seg_starts, state_slots, chunk_base, sc_U, sc_fg, sc_m0, H, d, dv, L);
+                       state_stride, seg_starts, state_slots, chunk_base, sc_U, sc_fg, sc_m0, H, d, dv, LS);
     LMSF_LAUNCH_CHECK("mlstm_chunk (fold)");
     if (dtype == LMSF_F32) MLX_LAUNCH(float, false); else MLX_LAUNCH(bf16_t, false);
 #undef MLX_LAUNCH

@@ -1585,18 +1585,29 @@ class HipOps:
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
     recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
     # The matrix memory's chunks run side by side where the step's longest segment has this many tokens at heads of 256 and
-    # more, 1.5 times as many from 128 on, twice from 64 on and three times below. The rule is for the whole step: a single token then has
+    # more, 1.5 times as many from 128 on, twice from 64 on, where their values are whole blocks of 64 columns; with others twice from 64
+    # on, three times from 32 on and six times below, and six times too in steps of more than 16 segments of which fewer than a quarter are that
+    # long; anywhere from three of the other form's chunks on. The rule is for the whole step: a single token then has
     # a chunk of its own, whose memory goes through scratch, where the other form (a workgroup a head and 32 columns) is held up
-    # by its longest segment. Side by side over the other form, bfloat16, states not in cache, 1 / 4 / 8 / 16 segments of that many tokens and
-    # the most of them beside 8 or 24 single tokens: 8 heads of 128, 32 tokens 0.97 / 1.00 / 1.06 / 0.74 and 1.13, 48 tokens 0.77 / 0.81 /
-    # 0.85 / 0.59 and 0.89; 4 heads of 256, 24 tokens 0.93 / 1.02 / 1.10 / 0.79 and 1.17, 32 tokens 0.77 / 0.85 / 0.92 / 0.66 and 0.99;
-    # 16 heads of 64, 48 tokens 1.01 / 1.03 / 1.05 / 0.72 and 1.12, 64 tokens 0.85 / 0.86 / 0.89 / 0.61 and 1.00; 16 heads of 32, 64
-    # tokens 1.08 / 1.09 / 1.08 / 1.09 and 1.17, 100 tokens 0.81 / 0.81 / 0.82 / 0.88 and 1.04. With 256 single tokens beside one
-    # portion of 48 to 300 tokens 0.66 to 0.83 (8 heads of 128) and 0.66 to 0.90 (4 of 256).
+    # by its longest segment. Side by side over the other form, bfloat16, states not in cache, 1 / 4 / 16 segments of that many tokens and
+    # the most of them beside 8, 24, 64 or 200 single tokens: 8 heads of 128, 32 tokens 0.98 / 1.03 / 0.77 and 1.14, 48 tokens 0.76 / 0.81
+    # / 0.60 and 0.89; 4 heads of 256, 24 tokens 0.93 / 1.02 / 0.79 and 1.18, 32 tokens 0.77 / 0.85 / 0.66 and 0.99; 16 heads of 64,
+    # 48 tokens 1.02 / 1.05 / 0.72 and 1.19, 64 tokens 0.85 / 0.89 / 0.61 and 1.02 (float32 up to 1.01 and 1.02 at the same lines). 8 heads of
+    # 130 by 66, 48 tokens beside 24 1.21 (float32 1.35), 64 beside 24 1.01 (1.05), 96 beside 64 1.06 (1.48); 5 of 99 by 130, 64 beside
+    # 24 1.04 (1.12), beside 200 0.9 (1.26); 16 of 32, 96 tokens 0.82 / 0.84 / 0.90, beside 24 0.9, beside 64 1.32; 4 of 16, 96
+    # tokens 1.29, 128 tokens 1.10, 191 tokens 0.81.
     matrix_memory_parallel_min_tokens = 32
 
-    def _memory_side_by_side(self, lens, dim: int) -> bool:
-        return max(lens) >= self.matrix_memory_parallel_min_tokens * (1 if dim >= 256 else 1.5 if dim >= 128 else 2 if dim >= 64 else 3)
+    def _memory_side_by_side(self, lens, dim: int, vdim: int, chunk: int) -> bool:
+        """``chunk``: the tokens of the other form's chunks."""
+        least = self.matrix_memory_parallel_min_tokens
+        if dim >= 64 and vdim % 64 == 0:
+            tokens = least * (1 if dim >= 256 else 1.5 if dim >= 128 else 2)
+        else:
+            tokens = least * (2 if dim >= 64 else 3 if dim >= 32 else 6)
+            if len(lens) > 16 and 4 * sum(n >= tokens for n in lens) < len(lens):
+                tokens = least * 6
+        return max(lens) >= min(tokens, 3 * chunk)
 
     def _chunk_plan(self, batch, chunk: int):
         """(per segment its first entry of scratch or -1, entries in all, the most chunks of a segment) for a step
@@ -1704,7 +1715,8 @@ class HipOps:
             L = self.lib.lmsf_mlstm_chunk_tokens(int(dim))
             bases = entries = None
             n_entries, most = 0, 1
-            if L > 0 and self._memory_side_by_side(lens, dim):
+            if L > 0 and self._memory_side_by_side(lens, dim, vdim, L):
+                L = self.lib.lmsf_mlstm_side_tokens(int(dim))
                 key = ("mlstm_chunks", L)
                 plan = batch.aux.get(key)
                 if plan is None:

@@ -10,7 +10,7 @@ from typing import Optional
 from ..csrc import build as _build
 from .dispatch import ProductShape, Route, Tunables
 
-ABI_VERSION = 42      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
+ABI_VERSION = 43      # goes up with every change of an entry point, a structure or a flag (tests/test_library.py)
 
 _lib: Optional[ctypes.CDLL] = None
 _lib_path: Optional[str] = None
@@ -125,6 +125,7 @@ _SIGNATURES = {
     "lmsf_mlstm_step": (c_int, [_P, _P, _P, c_int, c_long, _P, c_long, _P, c_long, _P, c_int, _P, c_long, _P, _P, c_long, _P,
                                 _P, c_long, _P, c_int, c_int, c_int, c_int, c_float, c_float, c_float, _P]),
     "lmsf_mlstm_chunk_scratch_floats": (c_long, [c_int, c_int, c_int]),
+    "lmsf_mlstm_side_tokens": (c_int, [c_int]),
     "lmsf_mlstm_chunked": (c_int, [_P, _P, _P, c_int, c_long, _P, c_long, _P, c_long, _P, _P, c_long, _P, _P, _P, c_long,
                                    _P, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_float, _P, c_int, c_long,
                                    _P, _P]),

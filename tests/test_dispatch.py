@@ -157,13 +157,19 @@ def test_chunks_of_the_selective_scan(lens, inner, n, chunk):
     assert HipOps.__new__(HipOps)._scan_chunk(lens, sum(lens), inner, n) == chunk
 
 
-@pytest.mark.parametrize("dim,tokens", [(512, 32), (256, 32), (255, 48), (128, 48), (127, 64), (64, 64), (63, 96), (16, 96)])
-def test_the_matrix_memory_goes_side_by_side(dim, tokens):
-    """Where every mix of segments that was measured is no slower for it."""
+@pytest.mark.parametrize("dim,vdim,tokens,many", [
+    (512, 512, 24, 24), (256, 256, 32, 32), (255, 64, 48, 48), (128, 128, 48, 48), (127, 64, 64, 64), (64, 64, 64, 64),
+    (256, 72, 64, 96), (130, 66, 64, 192), (64, 40, 64, 192), (63, 64, 96, 192), (32, 32, 96, 192), (31, 64, 192, 192)])
+def test_the_matrix_memory_goes_side_by_side(lib, dim, vdim, tokens, many):
+    """Where every mix of segments that was measured is no slower for it: heads of whole blocks of 64 values beside any
+    number of single tokens, others (``many``) later beside many; never later than three of the other form's chunks."""
     from lmsf_amd.ops.hip_ops import HipOps
-    o = HipOps.__new__(HipOps)
-    for beside in ([], [1] * 64, [tokens - 1] * 8):
-        assert not o._memory_side_by_side([tokens - 1] + beside, dim) and o._memory_side_by_side(beside + [tokens], dim)
+    o, chunk = HipOps.__new__(HipOps), lib.lmsf_mlstm_chunk_tokens(dim)
+    for beside, least in (([], tokens), ([1] * 15, tokens), ([tokens - 1] * 8, tokens), ([1] * 64, many),
+                          ([many - 1] * 3 + [1] * 64, many)):
+        assert not o._memory_side_by_side([least - 1] + beside, dim, vdim, chunk)
+        assert o._memory_side_by_side(beside + [least], dim, vdim, chunk)
+    assert lib.lmsf_mlstm_side_tokens(dim) == max(chunk, 16)
 
 
 @pytest.mark.parametrize("inner,rank,most", [(4096, 128, 256), (8192, 256, 64), (16384, 512, 16), (1024, 64, 2048)])

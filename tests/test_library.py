@@ -8,7 +8,7 @@ from lmsf_amd.ops.hip_ops import HipOps
 # One line a version, the newest last. A difference here means that an entry point, a structure, a route or a flag has
 # changed: raise the number in csrc/runtime.hip and ops/library.py, then add its line (never change an old one).
 VERSIONS = {38: "b3ef8bfa13f50e4e", 39: "a6516c9b237f5bb9", 40: "deeb2b301a468cfb",
-            41: "6cebad8e9d1a97df", 42: "e35e1bf0818d5850"}
+            41: "6cebad8e9d1a97df", 42: "e35e1bf0818d5850", 43: "49e3e76bff5aa5a3"}
 
 
 def shared() -> str:

@@ -44,10 +44,11 @@ def memory_by_tokens(q, k, v, gates, og, w, state, lens, H, d, dv, scale, cap, e
 
 # heads of 16 and 32 entries' multiples and not, values that end inside a block of 16 and of 64 columns, segments of a tile's, a
 # chunk's and several chunks' tokens and one more or less, a short one beside them; 200 and 260: more rows of S_0 than a
-# wave holds at a time, and smaller chunks
+# wave holds at a time, and smaller chunks; 500 and 700: chunks of 16 where the other form's have 8 and 4
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,d,dv,lens", [(2, 128, 128, (64, 65, 3)), (3, 40, 70, (100, 127)), (1, 17, 5, (65, 192)), (2, 64, 64, (128, 16)),
-                                         (2, 200, 24, (33, 47)), (1, 260, 136, (40,)), (2, 128, 65, (32, 33, 1))])
+                                         (2, 200, 24, (33, 47)), (1, 260, 136, (40,)), (2, 128, 65, (32, 33, 1)),
+                                         (1, 500, 40, (33, 3)), (1, 700, 20, (16, 17))])
 def test_matrix_memory_side_by_side(H, d, dv, lens, dtype):
     o, g = ops(), torch.Generator().manual_seed(d + dv)
     N, scale, cap, eps = sum(lens), d ** -0.5, 15.0, 1e-5
@@ -69,7 +70,7 @@ def test_matrix_memory_side_by_side(H, d, dv, lens, dtype):
     S64, m64 = S.double(), m.double()
     ref = memory_by_tokens(x[:, :cut[0]], x[:, cut[0]:cut[1]], x[:, cut[1]:cut[2]], gates.double(), x[:, cut[2]:], w.double(),
                            (S64, m64), lens, H, d, dv, scale, cap, eps)
-    # sums of up to 260 float32 products that partly cancel, against the row's root mean square; a bfloat16 result's own
+    # sums of up to 700 float32 products that partly cancel, against the row's root mean square; a bfloat16 result's own
     # rounding (8 bits) is at most 2^-8 of it
     rel = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
     err = ((out.cpu().double() - ref).abs() - rel * ref.abs()).amax(1) / ref.pow(2).mean(1).sqrt()
