@@ -1745,17 +1745,17 @@ class HipOps:
     def _memory_step(n_tokens: int, heads: int, dim: int, vdim: int, size: int) -> bool:
         """Whether a step of single tokens of ``size`` bytes an entry makes its gates itself, by the workgroups (a token, a head,
         64 columns) it takes. At heads of 128 entries and more it does, but with float32, whose product beside it is quicker, just
-        beyond 1,024, where the chip holds all but a few at once; below, where a workgroup's eight waves find little to read and its gates
+        beyond 1,024, where the chip holds all but a few at once, and beyond it with a last block of columns that is not whole; below, where a workgroup's eight waves find little to read and its gates
         are much of it, up to 4,096 (float32 2,048), below 64 entries up to 1,536 (float32, and below 32 entries, 512). Step against
         product and memory, states not in cache, bfloat16: 8 heads of 128, K 2,048, 8 / 64 / 512 tokens 10.8 / 30 / 179 against 17.0 / 37 /
         198 us; 4 heads of 256, K 1,024, 17 / 51 / 160 (256 tokens) against 28 / 53 / 188; 16 heads of 64, K 1,024, 4,096 / 6,144 / 8,192
         55 / 79 / 103 against 60 / 75 / 93; 16 heads of 32, K 512, 2,048 / 3,072 24.4 / 33.6 against 26.4 / 32.6; 4 of 16, 512 / 768 8.5 /
         12.2 against 12.4 / 11.1. float32: 4 heads of 256 at 1,024 / 1,152 / 1,280 49 / 57 / 60 against 50 / 55 / 58, 4 of 160 at 1,008 / 1,248 /
-        1,344 34 / 41 / 43 against 33 / 37 / 43; 16 of 64 at 2,048 / 3,072 31.5 / 42.9 against 32.3 / 42.3; 16 of 32 at 512 / 1,024
+        1,344 34 / 41 / 43 against 33 / 37 / 43, 8 of 130 by 66 at 2,048 / 4,096 43.9 / 78.3 against 40.7 / 71.0; 16 of 64 at 2,048 / 3,072 31.5 / 42.9 against 32.3 / 42.3; 16 of 32 at 512 / 1,024
         9.2 / 13.6 against 11.7 / 13.0."""
         groups = n_tokens * heads * -(-vdim // 64)
         if dim >= 128:
-            return size == 2 or not 1024 < groups <= 1280
+            return size == 2 or groups <= 1024 or (groups > 1280 and vdim % 64 == 0)
         if dim >= 64:
             return groups <= 8192 // size
         return groups <= (1536 if dim >= 32 and size == 2 else 512)

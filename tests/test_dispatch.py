@@ -188,6 +188,7 @@ def test_the_matrix_memory_of_single_tokens_makes_its_gates_up_to(heads, dim, vd
     assert [HipOps._memory_step(n, heads, dim, vdim, size) for n in (1, most, most + 1)] == [True, True, dim >= 128]
     # (wide heads: in float32 all but just beyond what the chip holds at once)
     assert [HipOps._memory_step(n, 8, 128, 128, size) for n in (64, 65, 80, 81, 4096)] == [True, size == 2, size == 2, True, True]
+    assert [HipOps._memory_step(n, 8, 130, 66, size) for n in (64, 65, 81, 4096)] == [True] + [size == 2] * 3
 
 
 @pytest.mark.parametrize("H,rows", [(512, 1025), (1024, 1025), (1028, 513), (2048, 513), (2052, 341), (508, 8000), (8, 8000), (64, 8000)])
