@@ -1551,18 +1551,19 @@ class HipOps:
             _ptr(y), y.stride(0), N, inner, n, self._stream()))
         return y
 
-    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 16 entries, or of
-    # 32, which a lane reads and writes whole, into chunks of 32; where the tokens times the channels are few, so that the chip is far
+    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 32 entries, which
+    # a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far
     # from full, from 41 tokens on and into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 509 tokens of 4,096 channels 49 / 47 / 67
     # us, 2,048 of 4,096 137 / 114 / 108, 8 times 256 of 4,096 105 / 101 / 104, of 1,024 46 / 46 / 68; 509 of 1,024 35 / 42 / 65,
     # 8 times 128 of 1,024 31 / 41 / 66, 70 of 4,096 26 / 38 / 63. In one piece against chunks of 16: 33 tokens of 4,096 20.6 and 23.4, 8 times
     # 33 of 2,048 by 32 entries 32 and 44, 40 beside 32 single tokens of 4,096 26.8 and 27.4, 48 beside 16 28.5 and 25.4; 8 times 64 tokens of
-    # 4,096 37, in chunks of 32 42. Many segments fill the chip by themselves, and every one launches as many workgroups as the
-    # longest: 64 tokens beside 200 single ones of 2,048 by 32 74 in one piece, 142 in chunks of 16. Other numbers of entries, read
-    # one by one, gain from 32 segments on no more (1,024 by 12, 64 beside 200 47 and 68), those of 17 to 31 not at all (4,096 by 24, 64
-    # beside 64 97 and 154, 300 beside 128 188 in chunks of 64 and 257 of 32). Larger states, 16 lanes a channel, cost more to leave
-    # and fold than short chunks save: 2,048 tokens of 2,048 channels by 64 entries 281 / 247 / 236 us, of 4,096 by 256 1,581 / 1,277
-    # / 1,111, 48 tokens beside 32 single ones of 4,096 by 256 156 / 167 / 88. Both keep chunks of 64.
+    # 4,096 37, in chunks of 32 42. More than 128 segments fill the chip by themselves, and every one launches as many workgroups as
+    # the longest: 64 tokens beside 200 single ones of 2,048 by 32 74 in one piece, 142 in chunks of 16; 128 beside 250 of 1,024 by 16
+    # 53 in chunks of 32, 72 of 16. Other numbers of entries, read one by one, lose from 40 segments on what short pieces gain: 64
+    # tokens beside 64 of 4,096 by 12 50 in one piece and 60 (100 beside 32 of 1,024 by 12 34 in chunks of 16, 48 of 32); 64 beside 64 of
+    # 4,096 by 24 97 and 154, 300 beside 128 188 in chunks of 64 and 257 of 32 (512 alone of 2,048 115 and 70 of 16). Larger states,
+    # 16 lanes a channel, cost more to leave and fold than short chunks save: 2,048 tokens of 2,048 channels by 64 entries 281 / 247 / 236
+    # us, of 4,096 by 256 1,581 / 1,277 / 1,111, 48 tokens beside 32 single ones of 4,096 by 256 156 / 167 / 88. They keep chunks of 64.
     scan_chunk_tokens = 64
     scan_cut_tokens = 32
     scan_few_work = 1 << 20        # tokens times channels
@@ -1572,11 +1573,11 @@ class HipOps:
         """Tokens of a chunk of the selective scan of ``n_tokens`` tokens in segments of ``lens``, ``inner`` channels by ``n``
         entries; segments that are longer are cut."""
         chunk = self.scan_chunk_tokens
-        if not lens or (n > 16 and n != 32):
+        many = n not in (4, 8, 16, 32) and len(lens or ()) > 40
+        if not lens or n > (16 if many else 32):
             return chunk
-        few = n_tokens * inner <= self.scan_few_work and \
-            len(lens) <= (self.scan_few_segments if n in (4, 8, 16, 32) else self.scan_few_segments // 4)
-        if max(lens) > (chunk * 5 // 8 if few else chunk):
+        few = n_tokens * inner <= self.scan_few_work and len(lens) <= self.scan_few_segments
+        if max(lens) > (chunk * 5 // 8 if few and not many else chunk):
             cut = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
             if -(-max(lens) // cut) <= 65535:      # the launch's limit; a longer segment keeps the longer chunks
                 return cut
