@@ -423,7 +423,11 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // fastest over the workgroups and fall to the dies in turn, so that an expert's rows are read by one die, whose tiles of
 // that expert share them in its L2. What bounds the kernel is these rows' way into the compute units.
 // 3,994 pairs of 16 experts, 2,048 -> 2 x 1,024 -> 2,048, all four kernels, with tiles of 128 pairs by 128 outputs copied through
-// registers 32 k at a time 217 -> 116 us; 66 pairs 77 -> 55; 8,192 pairs of 8, 4,096 -> 2 x 1,536 -> 4,096, 766 -> 583.
+// registers 32 k at a time 217 -> 116 us; 66 pairs 77 -> 55; 8,192 pairs of 8, 4,096 -> 2 x 1,536 -> 4,096, 766 -> 583. Many or small experts,
+// most of whose tiles are nearly empty, gain as well (weights not in cache): 64 of 2,048 -> 2 x 1,024, 32 / 256 / 2,048 pairs 133 / 226 / 256 ->
+// 96 / 195 / 220; 128 of 1,024 -> 2 x 256 59 / 76 / 91 -> 35 / 57 / 66; 512 of these 75 / 141 / 258 -> 41 / 97 / 186; 8 of 256 -> 2 x 256 24 / 36 / 49
+// -> 21 / 27 / 42; 64 of 512 -> 256, one matrix in, 32 / 36 / 47 -> 27 / 28 / 37. Least where the experts' rows are all there is: 32 of 4,096 ->
+// 2 x 2,048, 64 to 256 pairs 0.92 to 0.94 of the time.
 #define MOE_TILE_ROWS 256
 #define MOE_TILE_WAVES 8
 #define MOE_STAGES 3
