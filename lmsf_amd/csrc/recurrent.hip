@@ -480,6 +480,11 @@ __global__ __launch_bounds__(256) void selective_scan_lane_kernel(
     for (int n = 0; n + 3 < NS; n += 4) {
       const float4 a4 = *reinterpret_cast<const float4*>(A_log + (long)cc * NS + n);
       a[n] = a4.x; a[n + 1] = a4.y; a[n + 2] = a4.z; a[n + 3] = a4.w;
+    }
+    // (behind the rates, which come from a cache: these are worked on while the state is on its way)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n + 3 < NS; n += 4) {
       float4 s4 = make_float4(0.f, 0.f, 0.f, 0.f);
       if (!SUMMARY) s4 = *reinterpret_cast<const float4*>(from + n);
       else if (copy) *reinterpret_cast<float4*>(copy + n) = *reinterpret_cast<const float4*>(st + n);
