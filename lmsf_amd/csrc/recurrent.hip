@@ -600,8 +600,11 @@ extern "C" int lmsf_selective_scan(const void* x, int dtype, long x_stride, cons
   LMSF_CHECK(!chunked || (scratch && chunk > 0 && max_chunks >= 1 && max_chunks <= 65535),
              "selective_scan: the chunked form needs scratch, a chunk size and the number of chunks");
   if (n_tokens == 0 || n_segments == 0) return 0;
+  // (an odd number of workgroups a segment: workgroups go to the compute units in turn, and with 4 or 8 of them those of single tokens, the
+  // first of each segment, would all meet on a quarter or an eighth of the units)
+  const int y_blocks = chunked ? max_chunks | 1 : 1;
   if (nstate <= 32) {
-    dim3 lgrid((inner + 255) / 256, chunked ? max_chunks : 1, n_segments), lblock(256);
+    dim3 lgrid((inner + 255) / 256, y_blocks, n_segments), lblock(256);
     // (the kernel holds exactly these numbers of entries, and every channel's lie on a 16-byte boundary)
     const int vec = (nstate == 4 || nstate == 8 || nstate == 16 || nstate == 32) && state_stride % 4 == 0 &&
                     lmsf_aligned16(state) && lmsf_aligned16(A_log) && (!chunked || (inner % 4 == 0 && lmsf_aligned16(scratch)));
@@ -631,7 +634,7 @@ extern "C" int lmsf_selective_scan(const void* x, int dtype, long x_stride, cons
   }
   const int TT = nstate <= 64 ? 32 : nstate <= 128 ? 16 : 8;
   const size_t smem = (size_t)TT * (4 * SCAN_CH + 2 * nstate) * sizeof(float);
-  dim3 grid((inner + SCAN_CH - 1) / SCAN_CH, chunked ? max_chunks : 1, n_segments), block(256);
+  dim3 grid((inner + SCAN_CH - 1) / SCAN_CH, y_blocks, n_segments), block(256);
 #define SCAN(T, SPL, SUM)                                                                                              \
   hipLaunchKernelGGL((selective_scan_kernel<T, SPL, SUM>), grid, block, smem, stream, (const T*)x, x_stride, dt_pre,   \
                      dt_stride, (const T*)bc, bc_stride, b_at, c_at, (const T*)z, z_stride, A_log, Dw, state,          \
