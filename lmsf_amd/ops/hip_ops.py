@@ -1552,34 +1552,39 @@ class HipOps:
         return y
 
     # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 32 entries, which
-    # a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far
-    # from full, from 41 tokens on and into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 509 tokens of 4,096 channels 49 / 47 / 67
-    # us, 2,048 of 4,096 137 / 114 / 108, 8 times 256 of 4,096 105 / 101 / 104, of 1,024 46 / 46 / 68; 509 of 1,024 35 / 42 / 65,
-    # 8 times 128 of 1,024 31 / 41 / 66, 70 of 4,096 26 / 38 / 63. In one piece against chunks of 16: 33 tokens of 4,096 20.6 and 23.4, 8 times
-    # 33 of 2,048 by 32 entries 32 and 44, 40 beside 32 single tokens of 4,096 26.8 and 27.4, 48 beside 16 28.5 and 25.4; 8 times 64 tokens of
-    # 4,096 37, in chunks of 32 42. More than 128 segments fill the chip by themselves, and every one launches as many workgroups as
-    # the longest: 64 tokens beside 200 single ones of 2,048 by 32 74 in one piece, 142 in chunks of 16; 128 beside 250 of 1,024 by 16
-    # 53 in chunks of 32, 72 of 16. Other numbers of entries, read one by one, lose from 40 segments on what short pieces gain: 64
-    # tokens beside 64 of 4,096 by 12 50 in one piece and 60 (100 beside 32 of 1,024 by 12 34 in chunks of 16, 48 of 32); 64 beside 64 of
-    # 4,096 by 24 97 and 154, 300 beside 128 188 in chunks of 64 and 257 of 32 (512 alone of 2,048 115 and 70 of 16). Larger states,
-    # 16 lanes a channel, cost more to leave and fold than short chunks save: 2,048 tokens of 2,048 channels by 64 entries 281 / 247 / 236
-    # us, of 4,096 by 256 1,581 / 1,277 / 1,111, 48 tokens beside 32 single ones of 4,096 by 256 156 / 167 / 88. They keep chunks of 64.
+    # a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far from full, from 41 tokens on and
+    # into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 512 tokens of 4,096 channels 46 / 45 / 67 us, 2,048 of 4,096 129 / 107 / 104, 8
+    # times 256 of 4,096 97 / 92 / 122, of 1,024 48 / 52 / 66; 512 of 1,024 34 / 42 / 64, 8 times 128 of 1,024 34 / 39 / 63, 70 beside 8 single
+    # ones of 4,096 25 / 37 / 63, 128 beside 250 of 1,024 31 / 44 / 70. Chunks of 16 and in one piece: 33 tokens of 4,096 23 and 21, 8 times 33
+    # of 2,048 by 32 entries 41 and 32, 40 beside 32 single tokens of 4,096 27 and 27, 48 beside 16 25 and 28, 64 beside 64 31 and 41; 8 times
+    # 64 of 4,096 37 in one piece, 45 in chunks of 16. From 9 entries on other numbers than 16 and 32 are read one by one, which beside
+    # more than 16 segments costs more than pieces below 64 tokens gain: 48 tokens beside 64 of 8,192 by 12 67 and 49, 4 times 48 beside 24 of
+    # 4,096 by 24 87 and 70 (with 5 entries 64 beside 64 of 1,024 21 and 28).
+    # Larger states, 16 lanes a channel, cost more to leave and fold: chunks of 16 where the tokens times the channels are at most 3 / 8
+    # of that and the segments at most 200, a longest segment of 49 to 64 tokens at most 1 / 8; else of 64. 70 tokens beside 8 of 512 by 200
+    # 52 and 145, 96 of 4,096 by 256 88 and 175, 512 of 512 by 200 75 and 148; 100 beside 32 of 4,096 by 64 (540,672) 87 and 81, 512 beside 250
+    # of 512 by 33 135 and 61; 64 beside 64 of 1,024 by 128 59 and 65, of 2,048 by 64 64 and 47, 48 beside 64 of 1,024 by 128 58 and 51.
     scan_chunk_tokens = 64
     scan_cut_tokens = 32
     scan_few_work = 1 << 20        # tokens times channels
-    scan_few_segments = 128
 
     def _scan_chunk(self, lens, n_tokens: int, inner: int, n: int) -> int:
         """Tokens of a chunk of the selective scan of ``n_tokens`` tokens in segments of ``lens``, ``inner`` channels by ``n``
         entries; segments that are longer are cut."""
         chunk = self.scan_chunk_tokens
-        many = n not in (4, 8, 16, 32) and len(lens or ()) > 40
-        if not lens or n > (16 if many else 32):
+        if not lens:
             return chunk
-        few = n_tokens * inner <= self.scan_few_work and len(lens) <= self.scan_few_segments
-        if max(lens) > (chunk * 5 // 8 if few and not many else chunk):
+        most, work = max(lens), n_tokens * inner
+        if n > 32:
+            few = len(lens) <= 200 and most > chunk * 3 // 4 and \
+                work <= (self.scan_few_work * 3 // 8 if most > chunk else self.scan_few_work // 8)
+            least = chunk * 3 // 4
+        else:
+            few = work <= self.scan_few_work
+            least = chunk * 5 // 8 if few and (n <= 8 or n in (16, 32) or len(lens) <= 16) else chunk
+        if most > least and (few or n <= 32):
             cut = min(chunk, self.scan_cut_tokens // 2 if few else self.scan_cut_tokens)
-            if -(-max(lens) // cut) <= 65535:      # the launch's limit; a longer segment keeps the longer chunks
+            if -(-most // cut) <= 65535:      # the launch's limit; a longer segment keeps the longer chunks
                 return cut
         return chunk
 

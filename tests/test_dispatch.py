@@ -145,11 +145,12 @@ def test_decode_attention_splits(lib):
 
 @pytest.mark.parametrize("lens,inner,n,chunk", [
     ((64,) * 8, 4096, 16, 64), ((64,), 4096, 16, 16), ((41,), 1024, 16, 16), ((40,), 1024, 16, 64), ((1, 512), 4096, 16, 32),
-    ((64, 512), 4096, 33, 64), ((65,), 64, 256, 64), ((), 64, 16, 64),
-    # (many segments, and numbers of entries that a lane does not read whole)
-    ((64,) + (1,) * 127, 1024, 32, 16), ((64,) + (1,) * 128, 1024, 32, 64), ((65,) + (1,) * 128, 1024, 32, 32),
-    ((64,) + (1,) * 39, 1024, 12, 16), ((64,) + (1,) * 40, 1024, 12, 64), ((65,) + (1,) * 40, 1024, 12, 16),
-    ((65,) + (1,) * 128, 1024, 12, 32), ((64,) + (1,) * 39, 1024, 24, 16), ((512,) + (1,) * 40, 1024, 24, 64), ((512,), 4096, 17, 32),
+    ((), 64, 16, 64), ((64,) + (1,) * 250, 1024, 32, 16), ((512,), 4096, 17, 32), ((512,), 2048, 17, 16),
+    # (many segments of a number of entries that a lane does not read whole)
+    ((64,) + (1,) * 15, 1024, 12, 16), ((64,) + (1,) * 16, 1024, 9, 64), ((65,) + (1,) * 16, 1024, 24, 16), ((64,) + (1,) * 16, 1024, 7, 16),
+    # (states that a lane does not hold)
+    ((64,), 2048, 33, 16), ((64,), 2049, 33, 64), ((48,), 64, 256, 64), ((49,), 64, 256, 16), ((96,), 4096, 256, 16),
+    ((97,), 4096, 256, 64), ((65,) + (1,) * 199, 64, 33, 16), ((65,) + (1,) * 200, 64, 33, 64), ((64, 512), 4096, 33, 64),
     # (no more chunks than a launch takes: segments beyond that keep the longer ones)
     ((16 * 65535,), 1, 16, 16), ((16 * 65535 + 1,), 1, 16, 64), ((32 * 65535,), 64, 16, 32), ((3, 32 * 65535 + 1), 64, 16, 64)])
 def test_chunks_of_the_selective_scan(lens, inner, n, chunk):

@@ -113,13 +113,14 @@ def test_matrix_memory_keeps_a_value_from_earlier_tokens(token, column, value, d
 
 # one piece and cuts of 16 and of 32 tokens, pieces of fewer than 8, states that the kernel's number of entries is and is not,
 # channels that end inside a workgroup; whole segments of more tokens than lie in LDS at a time; states of more entries than a
-# lane holds, whose chunks keep 64 tokens, and several tiles (of 16 and of 8 tokens) in a chunk of 32
+# lane holds, in chunks of 16 and of 64, and several tiles (of 16 and of 8 tokens) in a chunk of 32
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("inner,n,lens,sizes,chunk", [
     (256, 16, (32,), {}, 64), (300, 16, (65, 7, 1), {}, 16), (260, 5, (97, 130), {}, 16), (512, 32, (33,), {"few_work": 0}, 64),
     (256, 4, (200, 33), {"few_work": 0}, 32), (256, 16, (129, 64), {"few_work": 0}, 32), (302, 8, (70,), {"few_work": 0}, 32),
     (300, 16, (65, 128, 129, 200), {"chunk_tokens": 256, "cut_tokens": 256, "few_work": 0}, 256),
-    (48, 33, (65, 33), {}, 64), (40, 72, (150, 31, 1), {"chunk_tokens": 32}, 32), (24, 200, (33, 100), {"chunk_tokens": 32}, 32)])
+    (48, 33, (65, 33), {}, 16), (48, 33, (65, 130), {"few_work": 0}, 64),
+    (40, 72, (150, 31, 1), {"chunk_tokens": 32, "few_work": 0}, 32), (24, 200, (33, 100), {"chunk_tokens": 32, "few_work": 0}, 32)])
 def test_selective_scan_in_pieces(inner, n, lens, sizes, chunk, dtype):
     o, g = ops(), torch.Generator().manual_seed(inner + n)
     for name, value in sizes.items():
