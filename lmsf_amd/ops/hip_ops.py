@@ -1551,19 +1551,20 @@ class HipOps:
             _ptr(y), y.stride(0), N, inner, n, self._stream()))
         return y
 
-    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 32 entries, which
-    # a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far from full, from 41 tokens on and
-    # into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 512 tokens of 4,096 channels 46 / 45 / 67 us, 2,048 of 4,096 129 / 107 / 104, 8
-    # times 256 of 4,096 97 / 92 / 122, of 1,024 48 / 52 / 66; 512 of 1,024 34 / 42 / 64, 8 times 128 of 1,024 34 / 39 / 63, 70 beside 8 single
-    # ones of 4,096 25 / 37 / 63, 128 beside 250 of 1,024 31 / 44 / 70. Chunks of 16 and in one piece: 33 tokens of 4,096 23 and 21, 8 times 33
-    # of 2,048 by 32 entries 41 and 32, 40 beside 32 single tokens of 4,096 27 and 27, 48 beside 16 25 and 28, 64 beside 64 31 and 41; 8 times
-    # 64 of 4,096 37 in one piece, 45 in chunks of 16. From 9 entries on other numbers than 16 and 32 are read one by one, which beside
-    # more than 16 segments costs more than pieces below 64 tokens gain: 48 tokens beside 64 of 8,192 by 12 67 and 49, 4 times 48 beside 24 of
-    # 4,096 by 24 87 and 70 (with 5 entries 64 beside 64 of 1,024 21 and 28).
-    # Larger states, 16 lanes a channel, cost more to leave and fold: chunks of 16 where the tokens times the channels are at most 3 / 8
-    # of that and the segments at most 200, a longest segment of 49 to 64 tokens at most 1 / 8; else of 64. 70 tokens beside 8 of 512 by 200
-    # 52 and 145, 96 of 4,096 by 256 88 and 175, 512 of 512 by 200 75 and 148; 100 beside 32 of 4,096 by 64 (540,672) 87 and 81, 512 beside 250
-    # of 512 by 33 135 and 61; 64 beside 64 of 1,024 by 128 59 and 65, of 2,048 by 64 64 and 47, 48 beside 64 of 1,024 by 128 58 and 51.
+    # The selective scan walks segments of up to 64 tokens in one piece and cuts longer ones. With states of up to 32 entries,
+    # which a lane holds, into chunks of 32; where the tokens times the channels are few, so that the chip is far from full,
+    # from 41 tokens on and into chunks of 16. Chunks of 16 / 32 / 64, 16 entries: 512 tokens of 4,096 channels 46 / 45 / 67 us,
+    # 2,048 of 4,096 129 / 107 / 104, 8 times 256 of 4,096 97 / 92 / 122, of 1,024 48 / 52 / 66; 512 of 1,024 34 / 42 / 64, 8
+    # times 128 of 1,024 34 / 39 / 63, 70 beside 8 single ones of 4,096 25 / 37 / 63, 128 beside 250 of 1,024 31 / 44 / 70.
+    # Chunks of 16 and in one piece: 33 tokens of 4,096 23 and 21, 8 times 33 of 2,048 by 32 entries 41 and 32, 40 beside 32
+    # single tokens of 4,096 27 and 27, 48 beside 16 25 and 28, 64 beside 64 31 and 41; 8 times 64 of 4,096 37 in one piece, 45
+    # in chunks of 16. From 9 entries on other numbers than 16 and 32 are read one by one, which beside more than 16 segments
+    # costs more than pieces below 64 tokens gain: 48 tokens beside 64 of 8,192 by 12 67 and 49, 4 times 48 beside 24 of 4,096
+    # by 24 87 and 70 (with 5 entries 64 beside 64 of 1,024 21 and 28). Larger states, 16 lanes a channel, cost more to leave
+    # and fold: chunks of 16 where the tokens times the channels are at most 3 / 8 of that and the segments at most 200, a
+    # longest segment of 49 to 64 tokens at most 1 / 8; else of 64. 70 tokens beside 8 of 512 by 200 52 and 145, 96 of 4,096 by
+    # 256 88 and 175, 512 of 512 by 200 75 and 148; 100 beside 32 of 4,096 by 64 (540,672) 87 and 81, 512 beside 250 of 512 by
+    # 33 135 and 61; 64 beside 64 of 1,024 by 128 59 and 65, of 2,048 by 64 64 and 47, 48 beside 64 of 1,024 by 128 58 and 51.
     scan_chunk_tokens = 64
     scan_cut_tokens = 32
     scan_few_work = 1 << 20        # tokens times channels
@@ -1591,17 +1592,19 @@ class HipOps:
     recurrent_chunked_min_tokens = 16   # segments from this many tokens on go to the matrix memory's chunked form
     recurrent_parallel_min_chunks = 3   # and from this many chunks on the chunks run side by side (retention)
     # The matrix memory's chunks run side by side where the step's longest segment has this many tokens at heads of 256 and
-    # more, 1.5 times as many from 128 on, twice from 64 on, where their values are whole blocks of 64 columns; with others twice from 64
-    # on, three times from 32 on and six times below, and six times too in steps of more than 16 segments of which fewer than a quarter are that
-    # long; anywhere from three of the other form's chunks on. The rule is for the whole step: a single token then has
-    # a chunk of its own, whose memory goes through scratch, where the other form (a workgroup a head and 32 columns) is held up
-    # by its longest segment. Side by side over the other form, bfloat16, states not in cache, 1 / 4 / 16 segments of that many tokens and
-    # the most of them beside 8, 24, 64 or 200 single tokens: 8 heads of 128, 32 tokens 0.98 / 1.03 / 0.77 and 1.14, 48 tokens 0.76 / 0.81
-    # / 0.60 and 0.89; 4 heads of 256, 24 tokens 0.93 / 1.02 / 0.79 and 1.18, 32 tokens 0.77 / 0.85 / 0.66 and 0.99; 16 heads of 64,
-    # 48 tokens 1.02 / 1.05 / 0.72 and 1.19, 64 tokens 0.85 / 0.89 / 0.61 and 1.02 (float32 up to 1.01 and 1.02 at the same lines). 8 heads of
-    # 130 by 66, 48 tokens beside 24 1.21 (float32 1.35), 64 beside 24 1.01 (1.05), 96 beside 64 1.06 (1.48); 5 of 99 by 130, 64 beside
-    # 24 1.04 (1.12), beside 200 0.9 (1.26); 16 of 32, 96 tokens 0.82 / 0.84 / 0.90, beside 24 0.9, beside 64 1.32; 4 of 16, 96
-    # tokens 1.29, 128 tokens 1.10, 191 tokens 0.81.
+    # more, 1.5 times as many from 128 on, twice from 64 on, where their values are whole blocks of 64 columns (two thirds of
+    # these where 16 segments have as many); with others twice from 64 on, three times from 32 on and six times below, and six
+    # times too in steps of more than 16 segments of which fewer than a quarter are that long; anywhere from three of the other
+    # form's chunks on. The rule is for the whole step: a single token then has a chunk of its own, whose memory goes through
+    # scratch, where the other form (a workgroup a head and 32 columns) is held up by its longest segment. Side by side over the
+    # other form, bfloat16, states not in cache, 1 / 4 / 16 segments of that many tokens and the most of them beside 8, 24, 64
+    # or 200 single tokens: 8 heads of 128, 32 tokens 0.98 / 1.03 / 0.77 and 1.14, 48 tokens 0.76 / 0.81 / 0.60 and 0.89; 4
+    # heads of 256, 24 tokens 0.93 / 1.02 / 0.79 and 1.18, 32 tokens 0.77 / 0.85 / 0.66 and 0.99; 16 heads of 64, 48 tokens 1.02
+    # / 1.05 / 0.72 and 1.19, 64 tokens 0.85 / 0.89 / 0.61 and 1.02 (float32 up to 1.01 and 1.02 at the same lines); 16 segments
+    # of two thirds beside 0 to 200 single tokens 0.67 to 0.85 (float32 to 0.97). 8 heads of 130 by 66, 48 tokens beside 24 1.21
+    # (float32 1.35), 64 beside 24 1.01 (1.05), 96 beside 64 1.06 (1.48); 5 of 99 by 130, 64 beside 24 1.04 (1.12), beside 200
+    # 0.9 (1.26); 16 of 32, 96 tokens 0.82 / 0.84 / 0.90, beside 24 0.9, beside 64 1.32; 4 of 16, 96 tokens 1.29, 128 tokens
+    # 1.10, 191 tokens 0.81.
     matrix_memory_parallel_min_tokens = 32
 
     def _memory_side_by_side(self, lens, dim: int, vdim: int, chunk: int) -> bool:
@@ -1609,6 +1612,8 @@ class HipOps:
         least = self.matrix_memory_parallel_min_tokens
         if dim >= 64 and vdim % 64 == 0:
             tokens = least * (1 if dim >= 256 else 1.5 if dim >= 128 else 2)
+            if tokens > max(lens) >= tokens * 2 / 3 and sum(n >= tokens * 2 / 3 for n in lens) >= 16:
+                return True
         else:
             tokens = least * (2 if dim >= 64 else 3 if dim >= 32 else 6)
             if len(lens) > 16 and 4 * sum(n >= tokens for n in lens) < len(lens):

@@ -173,6 +173,14 @@ def test_the_matrix_memory_goes_side_by_side(lib, dim, vdim, tokens, many):
     assert lib.lmsf_mlstm_side_tokens(dim) == max(chunk, 16)
 
 
+def test_the_matrix_memory_goes_side_by_side_sooner_for_many_segments(lib):
+    from lmsf_amd.ops.hip_ops import HipOps
+    o = HipOps.__new__(HipOps)
+    for dim, tokens in ((256, 22), (128, 32), (64, 43)):
+        f = lambda lens, vdim: o._memory_side_by_side(lens, dim, vdim, 64)      # noqa: E731
+        assert f([tokens] * 16 + [1] * 200, 128) and not f([tokens] * 15 + [tokens - 1], 128) and not f([tokens] * 32, 100)
+
+
 @pytest.mark.parametrize("inner,rank,most", [(4096, 128, 256), (8192, 256, 64), (16384, 512, 16), (1024, 64, 2048)])
 def test_scans_of_single_tokens_with_the_product_inside_end(lib, inner, rank, most):
     """Every 8 tokens read the product's matrix again: beyond 2^27 multiplications the product is a kernel of its own."""
